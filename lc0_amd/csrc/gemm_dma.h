@@ -37,8 +37,10 @@ __device__ __forceinline__ void DmaToLds16(const void* gptr, void* lds_base) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)gptr, LC0MI_LDS_PTR(lds_base), 16,
                                      0, 0);
   } else {
+    // (the no-op is the wait state that the hardware needs between a scalar write of M0 and a load into LDS, which takes
+    // its LDS address from it; the compiler adds it for its builtin and does not look into this)
     unsigned lds_addr = (unsigned)(size_t)LC0MI_LDS_PTR(lds_base);
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(gptr) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(gptr) : "memory", "m0");
   }
 }
 
