@@ -339,10 +339,13 @@ class NetworkComputation:
         return np.zeros(0, np.float32)
 
     def results(self):
-        """All outputs as arrays: dict(policy [n,1858], q [n], d [n], m [n])."""
+        """All outputs as arrays: dict(policy [n,1858], q [n], d [n], m [n]). A NaN among q, d and m is an error, as it
+        is when they are read one by one."""
         n = self.GetBatchSize()
         policy = np.empty((n, 1858), np.float32)
-        q, d, m = np.empty((3, n), np.float32)
+        q, d, m = values = np.empty((3, n), np.float32)
         if n:
             _check(self._lib.lc0mi_comp_outputs(self._h, _address(policy), _address(q), _address(d), _address(m)))
+            if np.isnan(values).any():
+                raise BackendError("NaN among the outputs of sample %d" % np.isnan(values).any(0).argmax())
         return dict(policy=policy, q=q, d=d, m=m)
