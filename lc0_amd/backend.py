@@ -333,10 +333,11 @@ class NetworkComputation:
         if self._legal is not None and 0 <= sample < len(self._legal[0]) - 1:
             off, probs = self._legal
             return probs[off[sample]:off[sample + 1]].copy()
-        n = C.c_int(0)
-        if not self._lib.lc0mi_comp_legal_policy(self._h, sample, C.byref(n)):
+        n = C.c_int(0)              # no bulk read: the library's own answer or error
+        ptr = self._lib.lc0mi_comp_legal_policy(self._h, sample, C.byref(n))
+        if not ptr:
             raise BackendError(self._lib.lc0mi_last_error().decode(errors="replace"))
-        return np.zeros(0, np.float32)
+        return np.ctypeslib.as_array(ptr, (n.value,)).copy() if n.value else np.zeros(0, np.float32)
 
     def results(self):
         """All outputs as arrays: dict(policy [n,1858], q [n], d [n], m [n]). A NaN among q, d and m is an error, as it

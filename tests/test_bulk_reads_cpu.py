@@ -76,3 +76,14 @@ def test_nan_is_an_error_in_every_reader(which):
     assert reader(0) == 3 * which
     with pytest.raises(be.BackendError):
         reader(1)
+
+
+@pytest.mark.parametrize("bulk", [True, False])
+def test_legal_policies_with_and_without_the_bulk_read(bulk):
+    comp = _computation(Library(bulk=bulk))
+    for sample, want in enumerate(([0.25, 0.75], [], [1.0])):
+        got = comp.GetLegalPolicy(sample)
+        assert got.dtype == np.float32
+        np.testing.assert_array_equal(got, np.array(want, np.float32))
+    with pytest.raises(be.BackendError, match="what the library says"):
+        comp.GetLegalPolicy(3)
