@@ -317,6 +317,7 @@ class NetworkComputation:
         ids = np.ascontiguousarray(move_ids, dtype=np.uint16)
         if ids.ndim != 1:
             raise BackendError("AddLegalMoves expects a one-dimensional list of move ids.")
+        self._values = self._legal = None
         _check(self._lib.lc0mi_comp_add_legal_moves(self._h, ids.shape[0], _address(ids)))
 
     def SetPolicySoftmaxTemperature(self, temperature):

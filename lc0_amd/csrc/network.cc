@@ -2401,6 +2401,7 @@ void Mi355xComputation::AddInputs(int n, const uint64_t* masks, const float* val
 
 void Mi355xComputation::ComputeBlocking() {
   Mi355xNetwork* net = Net();
+  computed_ = false;   // (until every slot has been evaluated: a failed pass leaves some of them half written)
   for (size_t si = 0; si < slots_.size(); si++) {
     const int n = std::min(max_batch_, batch_ - static_cast<int>(si) * max_batch_);
     HostSlot* s = slots_[si].get();
@@ -2483,6 +2484,7 @@ void Mi355xComputation::AddLegalMoves(int n, const uint16_t* move_ids) {
   s->legal_off[at + 1] = off + n;
   s->legal_samples = at + 1;
   legal_mode_ = true;
+  computed_ = false;   // (the slot holds no probabilities of these moves yet)
 }
 
 void Mi355xComputation::SetPolicySoftmaxTemperature(float temperature) {

@@ -1010,6 +1010,24 @@ def test_legal_move_policy_equals_caller_side_softmax(name, options, batch, temp
     raw.close()
 
 
+def test_moves_listed_after_a_pass_are_not_read_before_the_next_one(positions):
+    """ComputeBlocking without a list, then AddLegalMoves: no kernel has written probabilities of these moves."""
+    from lc0_amd import Network
+    net = Network(netgen.cached_config("tiny_attn"), "")
+    c = net.NewComputation()
+    c.AddInputs(positions["masks"][:1], positions["values"][:1])
+    c.ComputeBlocking()
+    q = c.GetQVal(0)
+    c.AddLegalMoves([1, 2, 3])
+    for read in (c.GetQVal, c.GetLegalPolicy):
+        with pytest.raises(Exception, match="has not been called"):
+            read(0)
+    c.ComputeBlocking()
+    assert c.GetQVal(0) == q
+    assert abs(float(c.GetLegalPolicy(0).sum()) - 1.0) < 1e-5
+    c.close()
+
+
 def test_legal_move_policy_call_order_errors(positions):
     from lc0_amd import Network
     net = Network(netgen.cached_config("tiny_attn"), "")
