@@ -11,18 +11,24 @@ namespace lc0mi {
 // A wave owns RT x CT accumulator tiles of 16x16 over its share of the reduction and takes its operand rows straight
 // from global memory (row_panel.h); the four values of a 16-byte chunk feed four matrix instructions. A workgroup is
 // WM x WN such waves by KS shares of the reduction; the KS partial tiles are added through LDS in wave order, so
-// results do not depend on timing.
+// results do not depend on timing. ONE_STEP: K <= 64 KS, a wave has one step of 64 values at most and holds one set of
+// operands instead of two (56 registers instead of 96: eight waves per SIMD).
 //
 // What bounds it: a CU multiplies 256 fp32 values per cycle and takes 64 bytes of operands per cycle, so even a 32x32
 // tile (0.125 bytes per operation) leaves the matrix cores the slower side and no LDS staging is needed, provided that
 // the loads run at that rate. The form before this one (32x32x2 instructions, 32 bytes of 32 rows per load) got a
-// quarter of it. us per launch, before -> now: 1280x256x256 10.1 -> 5.1, 1280x1024x256 24.6 -> 13.3, 1280x256x1024
-// 22.3 -> 13.1, 32x1858x2048 21.0 -> 8.4, 32x128x2048 20.4 -> 7.0, 36 x 128x64x64 6.7 -> 3.6, 16384x256x1024
-// 177 -> 103, 36 x 4096x64x64 49 -> 33.
+// quarter of it. us per launch between two events, before -> now: 1280x256x256 12.6 -> 8.4, 1280x1024x256 27.5 -> 17.0,
+// 1280x256x1024 25.3 -> 15.8, 32x1858x2048 25.2 -> 11.0, 36 x 128x64x64 10.0 -> 6.8, 36 x 4000x64x64 47.3 -> 26.1,
+// 16384x256x1024 180 -> 104.
+//
+// Rounding: a 16x16 tile adds the 64 products of a step in eight (ONE_STEP) or four sums and pairs those. One sum over a
+// wave's whole share rounds a longer chain: relative error of the result in the 2-norm at K = 64 / 256 / 1024, random
+// operands, 1.4e-7 / 1.5e-7 / 2.9e-7, now 7.2e-8 / 8.2e-8 / 1.0e-7 (the form before: 7.8e-8 / 1.2e-7 / 2.1e-7). The large
+// tile keeps one sum per quarter of K (K = 1024 2.9e-7, the form before 4.1e-7): its registers are used up.
 // ---------------------------------------------------------------------------
 namespace {
-template <int RT, int CT, int WM, int WN, int KS>
-__global__ __launch_bounds__(64 * WM * WN * KS) void gemm_f32_mfma_kernel(GemmArgsF32 p) {
+template <int RT, int CT, int WM, int WN, int KS, bool ONE_STEP = false>
+__global__ __launch_bounds__(64 * WM * WN * KS, RT * CT == 1 ? 5 : 1) void gemm_f32_mfma_kernel(GemmArgsF32 p) {
   constexpr int ROWS = 16 * RT * WM, COLS = 16 * CT * WN, NT = 64 * WM * WN * KS;
   constexpr int LD = COLS + 4;   // (rows stay 16-byte aligned)
   __shared__ __attribute__((aligned(16))) float part[KS][ROWS * LD];
@@ -44,19 +50,37 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_f32_mfma_kernel(GemmAr
   for (int t = 0; t < RT; t++)
 #pragma unroll
     for (int c = 0; c < CT; c++) acc[t][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto op = [](const intx4 (&w)[4], const intx4 (&a)[4], floatx4& c) {   // the products of one step
+    constexpr int SUMS = RT * CT > 1 ? 1 : ONE_STEP ? 8 : 4;
+    floatx4 sum[SUMS] = {};
+    if constexpr (SUMS == 1) sum[0] = c;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int l = 0; l < 4; l++) {
+        // (four sums: one per chunk, so that neighbouring instructions do not wait for each other)
+        const int j = SUMS == 4 ? l : i, e = SUMS == 4 ? i : l, n = SUMS == 4 ? j : (4 * j + e) % SUMS;
+        const floatx4 fw = __builtin_bit_cast(floatx4, w[j]), fa = __builtin_bit_cast(floatx4, a[j]);
+        sum[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[e], fa[e], sum[n], 0, 0, 0);
+      }
+#pragma unroll
+    for (int n = SUMS / 2; n > 0; n /= 2)
+#pragma unroll
+      for (int i = 0; i < n; i++) sum[i] += sum[i + n];
+    if constexpr (SUMS == 1 || ONE_STEP) c = sum[0];
+    else c += sum[0];
+  };
   // A contiguous share of the steps per wave.
-  const int steps = (4 * K + kStepBytes - 1) / kStepBytes, per_wave = (steps + KS - 1) / KS;
-  const int s_begin = min(steps, ks * per_wave), s_end = min(steps, s_begin + per_wave);
-  PanelProducts<RT, CT>(A, ta, W, tw, 4 * K, s_begin, s_end, acc,
-                        [](const intx4 (&w)[4], const intx4 (&a)[4], floatx4& c) {
-#pragma unroll
-                          for (int j = 0; j < 4; j++) {
-                            const floatx4 fw = __builtin_bit_cast(floatx4, w[j]), fa = __builtin_bit_cast(floatx4, a[j]);
-#pragma unroll
-                            for (int e = 0; e < 4; e++)
-                              c = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[e], fa[e], c, 0, 0, 0);
-                          }
-                        });
+  const int steps = (4 * K + kStepBytes - 1) / kStepBytes;
+  if constexpr (ONE_STEP) {   // (K <= 64 KS)
+    if (ks < steps) {
+      OneStep<RT, CT>(A + ks * kStepBytes, ta, W + ks * kStepBytes, tw, 4 * K - ks * kStepBytes, acc, op);
+    }
+  } else {
+    const int per_wave = (steps + KS - 1) / KS;
+    const int s_begin = min(steps, ks * per_wave), s_end = min(steps, s_begin + per_wave);
+    PanelProducts<RT, CT>(A, ta, W, tw, 4 * K, s_begin, s_end, acc, op);
+  }
   // Accumulator lane (r, g) of tile (t, c): row 16 t + r, columns 16 c + 4 g + e.
 #pragma unroll
   for (int t = 0; t < RT; t++)
@@ -83,10 +107,10 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_f32_mfma_kernel(GemmAr
   });
 }
 
-template <int RT, int CT, int WM, int WN, int KS>
+template <int RT, int CT, int WM, int WN, int KS, bool ONE_STEP = false>
 void LaunchTile(const GemmArgsF32& a, hipStream_t stream) {
   dim3 grid((a.M + 16 * RT * WM - 1) / (16 * RT * WM), (a.N + 16 * CT * WN - 1) / (16 * CT * WN), a.batch);
-  hipLaunchKernelGGL((gemm_f32_mfma_kernel<RT, CT, WM, WN, KS>), grid, dim3(64 * WM * WN * KS), 0, stream, a);
+  hipLaunchKernelGGL((gemm_f32_mfma_kernel<RT, CT, WM, WN, KS, ONE_STEP>), grid, dim3(64 * WM * WN * KS), 0, stream, a);
 }
 }  // namespace
 
@@ -96,14 +120,30 @@ void LaunchGemmF32(const GemmArgsF32& a, hipStream_t stream) {
   // traffic decides (16384x256x1024: 103 us on 64x64 tiles, 143 on 16x16 ones; 1280x256x1024: 25 against 13).
   const long long tiles16 = (long long)((a.M + 15) / 16) * ((a.N + 15) / 16) * a.batch;
   const long long tiles64 = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch;
-  if (tiles64 >= 400) {
+  if (tiles64 >= 400 && a.K >= 512) {
     // Two waves share every operand row in both; a long reduction is worth splitting (16384x1024x256: 125 us unsplit
     // against 137; 16384x256x1024: 117 against 103).
-    if (a.K >= 512) LaunchTile<4, 2, 1, 2, 4>(a, stream);
-    else LaunchTile<1, 1, 2, 2, 1>(a, stream);
+    LaunchTile<4, 2, 1, 2, 4>(a, stream);
+  } else if (a.K <= 128) {
+    // One step for each of one or two waves. 32-row workgroups once there are several for every CU; before, a few more or
+    // less than one per CU decide (a 6x64 tower at 32 positions, 1152 tiles of 36 x 128x64x64: 207 us a pass in single
+    // tiles, 219 in 288 workgroups of 32x32; at 64 positions 239 in 32x32, with four waves per tile 242).
+    if (a.K <= 64) {
+      if (tiles16 < 2048) LaunchTile<1, 1, 1, 1, 1, true>(a, stream);
+      else LaunchTile<1, 1, 2, 2, 1, true>(a, stream);
+    } else if (tiles64 >= 400) {
+      LaunchTile<1, 1, 2, 2, 1>(a, stream);
+    } else {
+      if (tiles16 < 2048) LaunchTile<1, 1, 1, 1, 2, true>(a, stream);
+      else LaunchTile<1, 1, 2, 1, 2, true>(a, stream);
+    }
+  } else if (tiles64 >= 400) {
+    LaunchTile<1, 1, 2, 2, 1>(a, stream);
   } else if (tiles16 <= 256 && a.K >= 1024) {
     // One workgroup per CU at most: eight waves share a long reduction (32x1858x2048: 8.4 us against 10.2 with four).
     LaunchTile<1, 1, 1, 1, 8>(a, stream);
+  } else if (a.K <= 256) {
+    LaunchTile<1, 1, 1, 1, 4, true>(a, stream);
   } else {
     LaunchTile<1, 1, 1, 1, 4>(a, stream);
   }
