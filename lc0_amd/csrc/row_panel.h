@@ -71,9 +71,9 @@ struct TileOffsets {
   }
 };
 
-// The products of one step, of which only `bytes` of every row may exist (a multiple of 16, at least 16): a lane without
-// bytes in it reads the step's first ones of its rows and takes zeros instead, so that there is no condition around a
-// load (with one, a rest of 8 halves made 256x256x264 2.83 us instead of 2.72).
+// The products of a wave that has one step only, with one set of operand registers. `bytes` of every row exist (a multiple
+// of 16, at least 16), masked as PanelProducts masks its last step. (A function of its own: the same code called from there
+// made its loops 3 % slower, 33x3072x256 in halves 3.38 us against 3.25.)
 template <int TA, int TW, typename Acc, typename Op>
 __device__ __forceinline__ void OneStep(const char* pa, const TileOffsets (&ta)[TA], const char* pw,
                                         const TileOffsets (&tw)[TW], int bytes, Acc (&acc)[TA][TW], Op op) {
@@ -160,7 +160,30 @@ __device__ __forceinline__ void PanelProducts(const char* a_base, const TileOffs
     }
   }
   if (begin < end && end > whole) {
-    OneStep<TA, TW>(a_base + whole * kStepBytes, ta, w_base + whole * kStepBytes, tw, row_bytes - whole * kStepBytes, acc, op);
+    // A lane without bytes in this step reads the step's first ones of its rows and takes zeros instead: no condition
+    // around a load here either (with one, a rest of 8 halves made 256x256x264 2.83 us instead of 2.72).
+    const int lane = threadIdx.x & 63, in_row = 64 * (lane >> 4) + 16 * (lane & 3);
+    const bool in = in_row < row_bytes - whole * kStepBytes;
+    const char* pa = a_base + whole * kStepBytes;
+    const char* pw = w_base + whole * kStepBytes;
+    const unsigned back = in ? 0u : (unsigned)in_row;
+#pragma unroll
+    for (int c = 0; c < TW; c++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) w0[c][i] = *reinterpret_cast<const intx4*>(pw + (tw[c].off[i] - back));
+#pragma unroll
+    for (int t = 0; t < TA; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) a0[t][i] = *reinterpret_cast<const intx4*>(pa + (ta[t].off[i] - back));
+    const intx4 zero = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+#pragma unroll
+      for (int c = 0; c < TW; c++) w0[c][i] = in ? w0[c][i] : zero;
+#pragma unroll
+      for (int t = 0; t < TA; t++) a0[t][i] = in ? a0[t][i] : zero;
+    }
+    multiply(a0, w0);
   }
 }
 
