@@ -374,6 +374,14 @@ GemmVariant PickGemmVariant(const GemmArgs& a) {
   if (a.split_k == 1 && a.K >= 256 && RowPanelWorkgroups(a.M, a.N, a.batch, kRowPanelShapes[3]) <= kRowPanelWorkgroups) {
     return kRowPanel;
   }
+  // At most 128 rows and too many columns or products for that, up to 128 tiles of 64x64: direct-to-LDS tiles where they
+  // serve (33x8192x256 3.5 us against 4.0 on 64x32 panels and 5.4 on the register-staged tiles, 33x8192x1024 5.8 against
+  // 6.2 and 12.4, 64x8192x256 3.5 against 4.2 and 5.4, 77 products of 64x64x1024 5.4 against 7.9 and 10.5), else 64x32 panels
+  // (float output: 33x8192x256 4.0 against 5.5, 128x3072x1024 6.2 against 10.0, 77 products of 64x64x1024 8.0 against 12.9).
+  const long long tiles64 = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch;
+  if (a.split_k == 1 && a.K >= 256 && a.M <= 128 && tiles64 <= 128) {
+    return !a.out_f32 && a.K % 64 == 0 && a.N >= 64 ? kDma64x64 : kRowPanel;
+  }
   // A few hundred rows (3 to 12 positions), or few columns: too small for the cost model above, too large for row
   // panels. Small direct-to-LDS tiles with three or four stages in flight stream the weights, which come from
   // memory, better than the register-staged tiles below (512x1024x1024: 6.8 against 9.9 us; a pass of 8 positions

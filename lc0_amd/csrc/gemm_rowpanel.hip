@@ -16,7 +16,7 @@ inline RowPanelShape PickRowPanelShape(int M, int N, int batch) {
   for (const RowPanelShape& c : kRowPanelShapes) {
     if (RowPanelWorkgroups(M, N, batch, c) <= kRowPanelWorkgroups) return c;
   }
-  return kRowPanelShapes[3];
+  return kRowPanelShapes[4];
 }
 
 // One step (four 16-byte chunks of both operands) of a 16x16 accumulator tile, by operand type.
@@ -138,7 +138,8 @@ void LaunchPanel(const Args& a, int batch, hipStream_t stream) {
   if (s.rt == 1 && s.ct == 1) launch(One{}, One{});
   else if (s.rt == 2 && s.ct == 1) launch(Two{}, One{});
   else if (s.rt == 1 && s.ct == 2) launch(One{}, Two{});
-  else launch(Two{}, Two{});
+  else if (std::is_same<ET, uint8_t>::value || s.rt == 2) launch(Two{}, Two{});
+  else launch(std::integral_constant<int, std::is_same<ET, uint8_t>::value ? 2 : 4>{}, Two{});
 }
 }  // namespace
 

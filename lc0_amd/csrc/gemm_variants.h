@@ -19,7 +19,7 @@ int ResolvedOutStores(const GemmArgs& a);
 
 // Row panels (gemm_rowpanel.hip): panels of 16 rt x 16 ct outputs, and how many of them cover a problem.
 struct RowPanelShape { int rt, ct; };
-constexpr RowPanelShape kRowPanelShapes[] = {{1, 1}, {2, 1}, {1, 2}, {2, 2}};
+constexpr RowPanelShape kRowPanelShapes[] = {{1, 1}, {2, 1}, {1, 2}, {2, 2}, {4, 2}};
 constexpr long long kRowPanelWorkgroups = 256;   // one per CU
 inline long long RowPanelWorkgroups(int M, int N, int batch, const RowPanelShape& c) {
   return (long long)((M + 16 * c.rt - 1) / (16 * c.rt)) * ((N + 16 * c.ct - 1) / (16 * c.ct)) * batch;

@@ -70,3 +70,17 @@ def test_small_and_batched_products_keep_their_kernels():
     assert K.gemm_variant_name(64, 64, 1024, batch=256) == "gemm_64x64x64"    # policy logits, one product per position
     assert K.gemm_variant_name(16384, 32, 1024) == "gemm_64x64x64"            # smolgen compression beside the projection
     assert K.gemm_variant_name(16384, 32, 1024, latency_first=True) == "gemm_rowpanel"
+
+
+def test_few_rows_with_many_columns_or_products():
+    """33 to 128 rows (smolgen's second dense layer, the policy logits): direct-to-LDS tiles or panels, not the tiles that walk
+    the whole reduction in one workgroup per 64x64 outputs."""
+    for latency_first in (False, True):
+        for m in (33, 48, 63, 64):
+            assert K.gemm_variant_name(m, 8192, 256, latency_first=latency_first) == "gemm_dma_64x64x64"
+            assert K.gemm_variant_name(m, 8192, 264, latency_first=latency_first) == "gemm_rowpanel"
+        assert K.gemm_variant_name(128, 3072, 256, latency_first=latency_first) == "gemm_dma_64x64x64"
+    for batch in (65, 77, 128):
+        assert K.gemm_variant_name(64, 64, 1024, batch=batch) == "gemm_dma_64x64x64"
+    assert K.gemm_variant_name(64, 64, 1024, batch=129) == "gemm_64x64x64"
+    assert K.gemm_variant_name(32, 8192, 256) == "gemm_rowpanel"
