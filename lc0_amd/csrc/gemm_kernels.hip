@@ -304,9 +304,12 @@ GemmVariant PickGemmVariant(const GemmArgs& a) {
     // 64x64 tiles while about two workgroups share a CU (M = 32 3.5 us against 5.4 on the register-staged tiles, 128
     // 4.3 / 6.1, 256 5.3 against 5.9 on 128x64; M = 384 10.8), then 128x128 alone on a CU (384: 7.1) or 128x64 tiles; with
     // narrow products 64x64 throughout (1536 x 64x64 4.2 us against 6.2).
-    if ((long long)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch <= 640) return kDma64x64;
-    if (a.N >= 128 && tiles128 <= 256) return kDma128x128;
-    if (a.M < 1024 || a.N < 128 || a.K < 128) return a.N <= 64 ? kDma64x64 : kDma128x64;
+    // (What one workgroup per CU of the row panels below covers is left to them: 16 x 64x64x256 2.7 us against 3.3, 20 x
+    // 4x256x256 2.8 against 3.3.)
+    const bool panels = a.K >= 256 && RowPanelWorkgroups(a.M, a.N, a.batch, kRowPanelShapes[3]) <= kRowPanelWorkgroups;
+    if (!panels && (long long)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch <= 640) return kDma64x64;
+    if (!panels && a.N >= 128 && tiles128 <= 256) return kDma128x128;
+    if (!panels && (a.M < 1024 || a.N < 128 || a.K < 128)) return a.N <= 64 ? kDma64x64 : kDma128x64;
   }
   if (!a.out_f32 && a.split_k == 1 && a.K % 64 == 0 && a.K >= 128 && a.N >= 128 && a.M >= (a.latency_first ? 256 : 1024) && tiles128 >= 64) {
     // Direct-to-LDS kernels. Cost = rounds over the 256 CUs x tile area x a measured cost per

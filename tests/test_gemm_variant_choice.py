@@ -84,3 +84,7 @@ def test_few_rows_with_many_columns_or_products():
         assert K.gemm_variant_name(64, 64, 1024, batch=batch) == "gemm_dma_64x64x64"
     assert K.gemm_variant_name(64, 64, 1024, batch=129) == "gemm_64x64x64"
     assert K.gemm_variant_name(32, 8192, 256) == "gemm_rowpanel"
+    # few products with a short reduction: panels as long as one workgroup per CU covers them
+    assert K.gemm_variant_name(64, 64, 256, batch=16) == "gemm_rowpanel"
+    assert K.gemm_variant_name(4, 256, 256, batch=20) == "gemm_rowpanel"
+    assert K.gemm_variant_name(64, 64, 256, batch=77) == "gemm_dma_64x64x64"
