@@ -521,8 +521,12 @@ GemmVariant PickGemmF8Variant(const GemmF8Args& a) {
   if (GemmF8TakesRowPanels(a)) return kRowPanel;
   // A few hundred to a few thousand rows: 64x64 tiles, up to three workgroups of which share a CU and fill each other's
   // gaps (us against 128x64 tiles: 1024x1024x1536 5.5 / 6.8, 2048x1024x1024 5.5 / 6.3, 2048x1536x1024 on 768 tiles
-  // 7.4 / 7.9, 4096x1024x1024 on 1024 tiles 8.9 / 8.5).
-  if (a.N >= 64 && (long long)((a.M + 63) / 64) * ((a.N + 63) / 64) <= 768) return kDma64x64;
+  // 7.4 / 7.9, 4096x1024x1024 on 1024 tiles 8.9 / 8.5). With several per CU, few rows and weights beyond the 4 MiB of an
+  // XCD's L2 the 128x64 tiles, which read them half as often, stay ahead (512x3072x1536 8.8 / 6.8, 256x8192x2048 12.2 / 9.1,
+  // 300x8192x1024 9.1 / 7.9; 256x8192x512 with 4 MiB 4.4 / 4.8, 1024x3072x1536 with twice the rows 10.6 / 11.2).
+  const long long tiles64 = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64);
+  const bool few_rows_large_weights = tiles64 > 256 && a.M < 1024 && (long long)a.N * a.K > (4LL << 20);
+  if (a.N >= 64 && tiles64 <= 768 && !few_rows_large_weights) return kDma64x64;
   if (a.M < 1024 && a.N >= 64) return kDma128x64;
   auto rounds = [&](int bm, int bn) {
     const long long tiles = (long long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
@@ -538,8 +542,8 @@ GemmVariant PickGemmF8Variant(const GemmF8Args& a) {
   if (c192 < cost) { best = kDma256x192; cost = c192; }
   if (c128 < cost) { best = kDma256x128; cost = c128; }
   if (cs < cost) { best = kDma128x128; cost = cs; }
-  const double tiles64 = (double)((a.M + 127) / 128) * ((a.N + 63) / 64);
-  const double c64 = std::max(1.0, tiles64 / 256.0) * 128 * 64 * 0.80;
+  const double tiles128x64 = (double)((a.M + 127) / 128) * ((a.N + 63) / 64);
+  const double c64 = std::max(1.0, tiles128x64 / 256.0) * 128 * 64 * 0.80;
   if (c64 < cost) { best = kDma128x64; cost = c64; }
   return best;
 }

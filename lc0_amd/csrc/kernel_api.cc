@@ -170,6 +170,13 @@ const char* lc0mi_k_gemm_variant_name(int M, int N, int K, int batch, int latenc
   return lc0mi::GemmVariantName(g);
 }
 
+const char* lc0mi_k_gemm_f8_variant_name(int M, int N, int K) {
+  lc0mi::GemmF8Args g;
+  g.M = M; g.N = N; g.K = K;
+  g.lda = K; g.ldw = K; g.ldc = N;
+  return lc0mi::GemmF8VariantName(g);
+}
+
 void lc0mi_k_set_gemm_row_split(int on) { lc0mi::SetGemmRowSplit(on != 0); }
 
 int lc0mi_k_gemm_row_split(int M, int N, int K) {

@@ -20,6 +20,8 @@ def _lib():
         lib.lc0mi_k_gemm_splitk.argtypes = [vp, ci, vp, ci, vp, ci, ci, ci, ci, cf, vp, ci]
         lib.lc0mi_k_gemm_variant_name.argtypes = [ci, ci, ci, ci, ci]
         lib.lc0mi_k_gemm_variant_name.restype = C.c_char_p
+        lib.lc0mi_k_gemm_f8_variant_name.argtypes = [ci, ci, ci]
+        lib.lc0mi_k_gemm_f8_variant_name.restype = C.c_char_p
         lib.lc0mi_k_gemm_row_split.argtypes = [ci, ci, ci]
         lib.lc0mi_k_set_gemm_row_split.argtypes = [ci]
         lib.lc0mi_k_set_gemm_row_split.restype = None
@@ -119,6 +121,11 @@ def gemm(a, w, bias=None, scale=1.0, act=ACT_NONE, out_f32=False, time_iters=0):
 def gemm_variant_name(m, n, k, batch=1, latency_first=False):
     """Tile shape the launcher picks for a half-precision product of this shape (host-side logic, no GPU needed)."""
     return _lib().lc0mi_k_gemm_variant_name(m, n, k, batch, int(latency_first)).decode()
+
+
+def gemm_f8_variant_name(m, n, k):
+    """The same for e4m3 operands."""
+    return _lib().lc0mi_k_gemm_f8_variant_name(m, n, k).decode()
 
 
 def set_gemm_row_split(on):

@@ -88,3 +88,12 @@ def test_few_rows_with_many_columns_or_products():
     assert K.gemm_variant_name(64, 64, 256, batch=16) == "gemm_rowpanel"
     assert K.gemm_variant_name(4, 256, 256, batch=20) == "gemm_rowpanel"
     assert K.gemm_variant_name(64, 64, 256, batch=77) == "gemm_dma_64x64x64"
+
+
+def test_e4m3_products_of_few_rows_with_large_weights():
+    """More than one 64x64 tile per CU and weights beyond an XCD's 4 MiB of L2: 128x64 tiles; otherwise 64x64."""
+    for m, n, k in ((512, 3072, 1536), (256, 8192, 2048), (300, 8192, 1024), (640, 3072, 2048)):
+        assert K.gemm_f8_variant_name(m, n, k) == "gemm_f8_128x64x128", (m, n, k)
+    for m, n, k in ((256, 3072, 2048), (256, 8192, 512), (832, 1536, 1024), (832, 3072, 1024), (1024, 3072, 1536)):
+        assert K.gemm_f8_variant_name(m, n, k) == "gemm_f8_64x64x128", (m, n, k)
+    assert K.gemm_f8_variant_name(64, 1024, 1024) == "gemm_f8_rowpanel"
