@@ -597,19 +597,24 @@ void LaunchGemmDma(const GemmArgs& a, hipStream_t stream) {
 // workgroup per CU nothing else hides the time a k-tile takes to arrive from memory, with several per CU they hide it
 // for each other and more stages would only lower their number (15x1024 net, per pass: 16 positions 1.91 -> 1.67 ms
 // with four stages; 64 positions 2.59 -> 2.93 ms if forced there).
+// A count of stages is an instance only where it admits more workgroups than the one tried before it.
+constexpr int WorkgroupsPerCu(int stages, int stage_bytes) { return 160 * 1024 / (stages * stage_bytes + 4096); }
+
 template <typename ET, int BM, int BN, int BK, int WAVES_M, int WAVES_N>
 void LaunchGemmDmaStaged(const GemmArgs& a, hipStream_t stream) {
-  constexpr int kStage = (BM + BN) * BK * 2, kLds = 160 * 1024, kCus = 256;
+  constexpr int kStage = (BM + BN) * BK * 2, kCus = 256;
+  constexpr int kFour = WorkgroupsPerCu(4, kStage), kThree = WorkgroupsPerCu(3, kStage);
+  constexpr bool kAlone = BM * BN <= 128 * 64;   // (an instance for one workgroup per CU, with four stages)
   const long long wgs = (long long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN) * a.batch;
   if (a.skip != nullptr || a.row_stats != nullptr) return LaunchGemmDma<ET, BM, BN, BK, WAVES_M, WAVES_N, 2>(a, stream);
-  if constexpr (BM * BN <= 128 * 64) {
+  if constexpr (kAlone) {
     if (wgs <= kCus) return LaunchGemmDma<ET, BM, BN, BK, WAVES_M, WAVES_N, 4, true>(a, stream);
   }
-  if constexpr (4 * kStage + 4096 <= kLds) {
-    if (wgs <= (long long)kCus * (kLds / (4 * kStage + 4096))) return LaunchGemmDma<ET, BM, BN, BK, WAVES_M, WAVES_N, 4>(a, stream);
+  if constexpr (kFour > (kAlone ? 1 : 0)) {
+    if (wgs <= kCus * kFour) return LaunchGemmDma<ET, BM, BN, BK, WAVES_M, WAVES_N, 4>(a, stream);
   }
-  if constexpr (3 * kStage + 4096 <= kLds) {
-    if (wgs <= (long long)kCus * (kLds / (3 * kStage + 4096))) return LaunchGemmDma<ET, BM, BN, BK, WAVES_M, WAVES_N, 3>(a, stream);
+  if constexpr (kThree > kFour) {
+    if (wgs <= kCus * kThree) return LaunchGemmDma<ET, BM, BN, BK, WAVES_M, WAVES_N, 3>(a, stream);
   }
   LaunchGemmDma<ET, BM, BN, BK, WAVES_M, WAVES_N, 2>(a, stream);
 }

@@ -35,16 +35,18 @@ void LaunchGemmDmaF8Tile(const GemmF8Args& a, hipStream_t stream) {
 // Stage count by the launch's workgroup count, as LaunchGemmDmaStaged does for fp16 operands.
 template <int BM, int BN, int WAVES_M, int WAVES_N>
 void LaunchGemmDmaF8Staged(const GemmF8Args& a, hipStream_t stream) {
-  constexpr int kStage = (BM + BN) * 128, kLds = 160 * 1024, kCus = 256;
+  constexpr int kStage = (BM + BN) * 128, kCus = 256;
+  constexpr int kFour = WorkgroupsPerCu(4, kStage), kThree = WorkgroupsPerCu(3, kStage);
+  constexpr bool kAlone = BM * BN <= 128 * 64;
   const long long wgs = (long long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-  if constexpr (BM * BN <= 128 * 64) {
+  if constexpr (kAlone) {
     if (wgs <= kCus) return LaunchGemmDmaF8Tile<BM, BN, WAVES_M, WAVES_N, 128, 4, true>(a, stream);
   }
-  if constexpr (4 * kStage + 4096 <= kLds) {
-    if (wgs <= (long long)kCus * (kLds / (4 * kStage + 4096))) return LaunchGemmDmaF8Tile<BM, BN, WAVES_M, WAVES_N, 128, 4>(a, stream);
+  if constexpr (kFour > (kAlone ? 1 : 0)) {
+    if (wgs <= kCus * kFour) return LaunchGemmDmaF8Tile<BM, BN, WAVES_M, WAVES_N, 128, 4>(a, stream);
   }
-  if constexpr (3 * kStage + 4096 <= kLds) {
-    if (wgs <= (long long)kCus * (kLds / (3 * kStage + 4096))) return LaunchGemmDmaF8Tile<BM, BN, WAVES_M, WAVES_N, 128, 3>(a, stream);
+  if constexpr (kThree > kFour) {
+    if (wgs <= kCus * kThree) return LaunchGemmDmaF8Tile<BM, BN, WAVES_M, WAVES_N, 128, 3>(a, stream);
   }
   LaunchGemmDmaF8Tile<BM, BN, WAVES_M, WAVES_N, 128, 2>(a, stream);
 }
