@@ -163,6 +163,11 @@ struct CopySegments {
     dst[count] = d; src[count] = s; words[count] = static_cast<unsigned>((bytes + 3) / 4);
     count++;
   }
+  size_t Bytes() const {
+    size_t n = 0;
+    for (int k = 0; k < count; k++) n += 4ull * words[k];
+    return n;
+  }
 };
 void LaunchCopySegments(const CopySegments& segments, hipStream_t stream);
 // Sets n floats to zero (a kernel, so that it can be captured into a graph).

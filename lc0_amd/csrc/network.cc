@@ -494,7 +494,7 @@ class Mi355xNetwork : public Network, protected ModelState {
   void ReleaseLane(Mi355xNetwork* lane);
   void AcquireAllLanes();
   void ReleaseAllLanes();
-  void EvaluateOnLane(HostSlot* slot, int batch);
+  void EvaluateOnLane(HostSlot* slot, int batch, bool others_busy);
   void DrainStreams();
   void CreateStreams();
   void AllocActivations();
@@ -2210,7 +2210,7 @@ void Mi355xNetwork::Evaluate(HostSlot* slot, int batch) {
     AcquireAllLanes();
     single_stream_ = false;
     try {
-      EvaluateOnLane(slot, batch);
+      EvaluateOnLane(slot, batch, false);
     } catch (...) {
       DrainStreams();
       ReleaseAllLanes();
@@ -2227,7 +2227,7 @@ void Mi355xNetwork::Evaluate(HostSlot* slot, int batch) {
   Mi355xNetwork* lane = AcquireLane(&others_busy);
   lane->single_stream_ = others_busy && attn_body_;   // (a residual tower uses one stream anyway)
   try {
-    lane->EvaluateOnLane(slot, batch);
+    lane->EvaluateOnLane(slot, batch, others_busy);
   } catch (...) {
     lane->DrainStreams();
     ReleaseLane(lane);
@@ -2245,15 +2245,13 @@ void Mi355xNetwork::DrainStreams() {
   (void)hipGetLastError();
 }
 
-void Mi355xNetwork::EvaluateOnLane(HostSlot* slot, int batch) {
+void Mi355xNetwork::EvaluateOnLane(HostSlot* slot, int batch, bool others_busy) {
   std::lock_guard<std::mutex> lock(eval_mutex_);
   // Argument errors are reported before anything is enqueued: the lane's streams stay idle.
   if (slot->legal_samples > 0 && slot->legal_samples != batch) {
     throw Error("legal moves were given for some inputs of the batch only");
   }
   HIP_CHECK(hipSetDevice(device_));
-  // Inputs come out of the pinned slot and outputs go back into it by kernels (CopySegments): one launch before the pass
-  // and one after it.
   CopySegments in, out;
   in.Add(d_masks_, slot->masks, sizeof(uint64_t) * kInputPlanes * batch);
   in.Add(d_values_, slot->values, sizeof(float) * kInputPlanes * batch);
@@ -2263,11 +2261,24 @@ void Mi355xNetwork::EvaluateOnLane(HostSlot* slot, int batch) {
     in.Add(d_legal_off_, slot->legal_off, sizeof(int) * (batch + 1));
     in.Add(d_legal_ids_, slot->legal_ids, sizeof(uint16_t) * total);
   }
-  LaunchCopySegments(in, stream_);
-  ForwardDevice(batch);
-  HIP_CHECK(hipGetLastError());
   out.Add(slot->wdl, d_wdl_, sizeof(float) * (wdl_ ? 3 : 1) * batch);
   if (moves_left_) out.Add(slot->mlh, d_mlh_, sizeof(float) * batch);
+  if (!legal) out.Add(slot->policy, d_policy_, sizeof(float) * kPolicyOutputs * batch);
+  // Inputs come out of the pinned slot and outputs go back into it by kernels: one launch before the pass and one after
+  // it. Beside a pass of another lane large transfers are copy commands instead, which a copy engine carries out while the
+  // CUs work for the other pass (thousands of evals/s, kernels against commands. Four threads on the 10x256 net: 1000 positions
+  // 392 / 417, 160 335 / 344, 16 84 / 69; on the 20x256 tower: 512 310 / 322, 100 level. Two threads on the 15x1024 net: 256
+  // positions 43.2 to 47.7 / 48.3 to 48.6, as the passes happen to fall).
+  const bool by_command = others_busy && in.Bytes() + out.Bytes() >= (1 << 20);
+  auto transfer = [&](const CopySegments& c) {
+    if (!by_command) return LaunchCopySegments(c, stream_);
+    for (int k = 0; k < c.count; k++) {
+      if (c.words[k] > 0) HIP_CHECK(hipMemcpyAsync(c.dst[k], c.src[k], 4ull * c.words[k], hipMemcpyDefault, stream_));
+    }
+  };
+  transfer(in);
+  ForwardDevice(batch);
+  HIP_CHECK(hipGetLastError());
   if (legal) {
     // Only the probabilities of the listed moves leave the device (tens of floats per sample instead of 1858).
     Timed("legal_softmax", 0.0, total * 10.0 + batch * 4.0, [&] {
@@ -2275,8 +2286,7 @@ void Mi355xNetwork::EvaluateOnLane(HostSlot* slot, int batch) {
                          out);
     });
   } else {
-    out.Add(slot->policy, d_policy_, sizeof(float) * kPolicyOutputs * batch);
-    LaunchCopySegments(out, stream_);
+    transfer(out);
   }
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(stream_));

@@ -1113,6 +1113,46 @@ def test_legal_and_raw_computations_interleaved_across_threads(positions):
     assert not errors, errors
 
 
+def test_large_transfers_beside_another_lane(positions):
+    """From 1 MiB up a batch's inputs and outputs go by copy commands while another lane is busy, by kernels otherwise: the
+    same bytes. 150 positions with raw policies (1.3 MB), 800 with move lists (1.1 MB of inputs, odd counts of moves)."""
+    import threading
+    from lc0_amd import Network
+    net = Network(netgen.cached_config("tiny_attn"), "lanes=3")
+
+    def evaluate(n, legal, at):
+        idx = (np.arange(n) + at) % 320
+        comp = net.NewComputation()
+        for i in idx if legal else ():
+            comp.AddInputs(positions["masks"][i:i + 1], positions["values"][i:i + 1])
+            comp.AddLegalMoves(positions["legal"][i][:1 + i % 5])
+        if not legal:
+            comp.AddInputs(positions["masks"][idx], positions["values"][idx])
+        comp.ComputeBlocking()
+        policy = [comp.GetLegalPolicy(i) if legal else comp.GetPolicyRow(i) for i in range(n)]
+        values = [(comp.GetQVal(i), comp.GetDVal(i), comp.GetMVal(i)) for i in range(n)]
+        comp.close()
+        return np.concatenate([np.concatenate(policy), np.array(values, np.float32).reshape(-1)])
+
+    jobs = [(150, False, 0), (800, True, 7), (150, False, 100)]
+    want, errors = [evaluate(*j) for j in jobs], []
+
+    def worker(t):
+        try:
+            for it in range(6):
+                j = (t + it) % len(jobs)
+                np.testing.assert_array_equal(evaluate(*jobs[j]), want[j])
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=worker, args=(t,)) for t in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not errors, errors
+
+
 def test_canonical_hectoplies_input_format_with_legal_policy():
     """A net that declares INPUT_112_WITH_CANONICALIZATION_HECTOPLIES: positions are encoded for that format
     (board transform chosen per position, en-passant plane, rule-50 plane in hundredths), the capabilities
