@@ -241,11 +241,14 @@ __device__ __forceinline__ void InputTile(const float (&d)[6][6], float (&r)[6][
 // In bulk it moves its bytes at about 4 TB/s (512 positions x 256 half channels, 92 MB: 24 us), every CU reading, then
 // computing, then writing at the same time as the others; V = 2 keeps two workgroups on a CU there (128 registers) and
 // halves the instructions (1000 positions 4082 -> 4007 us a pass; at 512 and below 300 the two forms are level, with
-// few positions V = 1 has twice the waves).
+// few positions V = 1 has twice the waves). One channel per thread in bulk (floats, and halves of 16 times an odd
+// number of channels) wants the waves more than the early requests: without them (EARLY = false) it takes 61 registers
+// instead of 114 and eight waves per SIMD instead of four (a pass of a ten-block tower in halves, 1000 positions: 176 channels
+// 1854 -> 1630 us, 240 2590 -> 2310).
 // The squeeze-and-excitation layers are spread over all threads: every wave pools the channels it needs itself, the
 // second layer is split four ways over k, and every thread adds the four partial sums of its own channels.
-template <typename T, typename MT, int V>
-__global__ __launch_bounds__(1024 / V, 4) void winograd_output_transform_tiles_kernel(
+template <typename T, typename MT, int V, bool EARLY>
+__global__ __launch_bounds__(1024 / V, EARLY ? 4 : 8) void winograd_output_transform_tiles_kernel(
     const MT* __restrict__ m, const float* __restrict__ bias, const T* skip, const float* __restrict__ se_w1,
     const float* __restrict__ se_b1, const float* __restrict__ se_w2, const float* __restrict__ se_b2, int se_k,
     T* out, T* __restrict__ v_next, int ldv, int batch, int C, int act) {
@@ -282,11 +285,12 @@ __global__ __launch_bounds__(1024 / V, 4) void winograd_output_transform_tiles_k
   // channels, four k at a time. Second layer: k = tile, tile + 4, ..., four at a time.
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
   constexpr int kMaxPerLane = 4;   // C <= 256
-  float w1[4][kMaxPerLane], b1[4];
+  constexpr int U = EARLY ? 4 : 2;
+  float w1[U][kMaxPerLane], b1[U];
   ChF wg[4], wb[4], sg, sb;
   auto load_w1 = [&](int k0) {
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
+    for (int u = 0; u < U; u++) {
       const int k = min(k0 + u * nwaves, se_k - 1);
       b1[u] = se_b1[k];
 #pragma unroll
@@ -309,7 +313,7 @@ __global__ __launch_bounds__(1024 / V, 4) void winograd_output_transform_tiles_k
       sb = *reinterpret_cast<const ChF*>(se_b2 + C + c);
     }
   };
-  if constexpr (V == 1) {
+  if constexpr (V == 1 && EARLY) {
     if (skip != nullptr) load_skip();
     ask();
   }
@@ -321,7 +325,7 @@ __global__ __launch_bounds__(1024 / V, 4) void winograd_output_transform_tiles_k
     for (int k = 0; k < 36; k++) f[k] = (float)mm[k][v];
     OutputTile(f, y[v]);
   }
-  if constexpr (V > 1) ask();   // (the registers of m are free now; the skip has to wait for those of the weights)
+  if constexpr (V > 1 && EARLY) ask();   // (the registers of m are free now; the skip has to wait for those of the weights)
   float gamma[V], beta[V];
 #pragma unroll
   for (int v = 0; v < V; v++) gamma[v] = 1.0f, beta[v] = bc[v];
@@ -342,11 +346,11 @@ __global__ __launch_bounds__(1024 / V, 4) void winograd_output_transform_tiles_k
       const int i = lane + 64 * q;
       pool[q] = i < C ? (part[i] + part[C + i] + part[2 * C + i] + part[3 * C + i]) * (1.0f / 64.0f) + bias[i] : 0.0f;
     }
-    for (int k0 = wave; k0 < se_k; k0 += 4 * nwaves) {
-      if (k0 != wave) load_w1(k0);
-      float h[4];
+    for (int k0 = wave; k0 < se_k; k0 += U * nwaves) {
+      if (!EARLY || k0 != wave) load_w1(k0);
+      float h[U];
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
+      for (int u = 0; u < U; u++) {
         h[u] = 0.0f;
 #pragma unroll
         for (int q = 0; q < kMaxPerLane; q++) h[u] += w1[u][q] * pool[q];
@@ -354,9 +358,9 @@ __global__ __launch_bounds__(1024 / V, 4) void winograd_output_transform_tiles_k
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1)
 #pragma unroll
-        for (int u = 0; u < 4; u++) h[u] += __shfl_xor(h[u], off, 64);
+        for (int u = 0; u < U; u++) h[u] += __shfl_xor(h[u], off, 64);
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
+      for (int u = 0; u < U; u++) {
         const int k = k0 + u * nwaves;
         if (lane == 0 && k < se_k) hidden[k] = RActivate(h[u] + b1[u], act);
       }
@@ -367,7 +371,7 @@ __global__ __launch_bounds__(1024 / V, 4) void winograd_output_transform_tiles_k
 #pragma unroll
     for (int v = 0; v < V; v++) pg[v] = 0.0f, pb[v] = 0.0f;
     for (int k0 = tile; k0 < se_k; k0 += 16) {
-      if (k0 != tile) load_w2(k0);
+      if (!EARLY || k0 != tile) load_w2(k0);
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const int k = k0 + 4 * u;
@@ -382,6 +386,10 @@ __global__ __launch_bounds__(1024 / V, 4) void winograd_output_transform_tiles_k
     *reinterpret_cast<ChF*>(&fc2[(tile * 2) * C + c]) = pg;
     *reinterpret_cast<ChF*>(&fc2[(tile * 2 + 1) * C + c]) = pb;
     __syncthreads();
+    if constexpr (!EARLY) {
+      sg = *reinterpret_cast<const ChF*>(se_b2 + c);
+      sb = *reinterpret_cast<const ChF*>(se_b2 + C + c);
+    }
     ChF fg[4], fb[4];
 #pragma unroll
     for (int t = 0; t < 4; t++) {
@@ -396,7 +404,7 @@ __global__ __launch_bounds__(1024 / V, 4) void winograd_output_transform_tiles_k
       beta[v] = a + gamma[v] * bc[v];
     }
   }
-  if constexpr (V > 1) {
+  if constexpr (V > 1 || !EARLY) {
     if (skip != nullptr) load_skip();
   }
   T* o = out ? out + (long long)b * 64 * C : nullptr;
@@ -510,18 +518,23 @@ void LaunchWinogradOutputTransform(const MT* m, const float* bias, const T* skip
   if (C <= 256 && C % 16 == 0) {   // 4 * C threads in whole waves (the SE reduction shuffles across a wave)
     size_t shm = sizeof(float) * (size_t)(12 * C + k + (k & 1));
     if (v_next) shm += sizeof(T) * 64 * (size_t)C;
-    auto launch = [&](auto v_tag) {
+    auto launch = [&](auto v_tag, auto early_tag) {
       constexpr int V = decltype(v_tag)::value;
-      hipLaunchKernelGGL((winograd_output_transform_tiles_kernel<T, MT, V>), dim3(batch), dim3(4 * C / V), shm, stream, m,
-                         bias, skip, se_w1, se_b1, se_w2, se_b2, se_k, out, v_next, ldv_next, batch, C, act);
+      hipLaunchKernelGGL((winograd_output_transform_tiles_kernel<T, MT, V, decltype(early_tag)::value>), dim3(batch),
+                         dim3(4 * C / V), shm, stream, m, bias, skip, se_w1, se_b1, se_w2, se_b2, se_k, out, v_next, ldv_next, batch, C, act);
     };
     // Two channels per thread (see the kernel) where a CU has more than one position; that needs 2 * C threads in whole
     // waves and whole pairs of channels in every row.
     const bool pairs = C % 32 == 0 && (v_next == nullptr || ldv_next % 2 == 0);
     if constexpr (sizeof(T) == 2) {
-      if (pairs && batch > 256) return launch(std::integral_constant<int, 2>{});
+      if (pairs && batch > 256) return launch(std::integral_constant<int, 2>{}, std::true_type{});
     }
-    launch(std::integral_constant<int, 1>{});
+    // The early requests while all positions are on the CUs at once (at four waves per SIMD a CU holds 256 / C workgroups),
+    // the form of 61 registers beyond (us of the kernel, early / late: halves of 176 channels at 300 positions 20.8 / 16.7,
+    // at 1000 41.0 / 30.2, floats of 192 22.5 / 18.0 and 54.1 / 46.2; the other way round floats of 64 at 300 13.1 / 13.5, halves
+    // of 112 8.5 / 8.7).
+    if (batch > 256 * (256 / C)) return launch(std::integral_constant<int, 1>{}, std::false_type{});
+    launch(std::integral_constant<int, 1>{}, std::true_type{});
     return;
   }
   // Wide towers: separate kernels (the caller checks WinogradFusedInputTransform before asking for v_next).
