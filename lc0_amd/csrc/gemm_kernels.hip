@@ -271,14 +271,14 @@ int PlanRowSplit(const GemmArgs& a, GemmVariant* first) {
   return best_m1;
 }
 
-// The smallest direct-to-LDS tile with which an output fits the CUs with one workgroup each (kUnused8: none does). A
+// The smallest direct-to-LDS tile with which an output fits the CUs with one workgroup each (kNoVariant: none does). A
 // workgroup's time hardly depends on how many others run (us at K = 1024 / 1536: 64x64 5.6 / 6.9, 128x64 7.1 / 8.8,
 // 128x128 9.6 / 12.2), a second workgroup on some of the CUs costs most of that time again: 832x1536x1024 8.0 us on 168
 // tiles of 128x64 against 9.4 on 312 of 64x64, 832x3072x1024 12.8 on 168 tiles of 128x128 against 13.5 on 336 of 128x64,
 // 1024x1024x1536 7.7 on 256 tiles of 64x64 against 9.2 on 128 of 128x64.
 inline GemmVariant OneRoundTile(int M, int N, int batch) {
   auto fits = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch <= 256; };
-  return fits(64, 64) ? kDma64x64 : fits(128, 64) ? kDma128x64 : fits(128, 128) ? kDma128x128 : kUnused8;
+  return fits(64, 64) ? kDma64x64 : fits(128, 64) ? kDma128x64 : fits(128, 128) ? kDma128x128 : kNoVariant;
 }
 
 GemmVariant PickGemmVariant(const GemmArgs& a) {
@@ -288,7 +288,7 @@ GemmVariant PickGemmVariant(const GemmArgs& a) {
                         g_variant_override == kDma128x64 || g_variant_override == kDma128x32 ||
                         g_variant_override == kDma64x64;
     bool ok = is_dma ? dma_ok : (g_variant_override != kRowPanel || a.split_k == 1);
-    if (g_variant_override == kUnused8) ok = false;
+    if (g_variant_override == kNoVariant) ok = false;
     if (g_variant_override == kResident) ok = GemmResidentWorkgroups(a) > 0;
     if (ok) return static_cast<GemmVariant>(g_variant_override);
   }
@@ -336,7 +336,7 @@ GemmVariant PickGemmVariant(const GemmArgs& a) {
     }
     if (a.K >= 512 && a.batch == 1) {
       const GemmVariant v = OneRoundTile(a.M, a.N, 1);
-      if (v != kUnused8) return v;
+      if (v != kNoVariant) return v;
     }
     auto rounds = [&](int bm, int bn) {
       const long long tiles = (long long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * a.batch;
@@ -393,7 +393,7 @@ GemmVariant PickGemmVariant(const GemmArgs& a) {
   // disturb it less.)
   if (!a.out_f32 && a.split_k == 1 && a.K % 64 == 0 && a.K >= (a.latency_first ? 256 : 512) && a.N >= 64 && a.M >= (a.batch == 1 ? 64 : 192)) {
     const GemmVariant v = OneRoundTile(a.M, a.N, a.batch);
-    return v != kUnused8 ? v : kDma128x64;
+    return v != kNoVariant ? v : kDma128x64;
   }
   // A single 32-column panel (the smolgen compression): one workgroup per 64 rows, K split over its waves
   // (16384x32x1024: 9.5 us against 12.3 for the 64x64 tiles, but with twice the threads on every CU).

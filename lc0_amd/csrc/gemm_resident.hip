@@ -14,11 +14,12 @@ namespace {
 //
 // A wave owns 32 rows x 128 columns (2 x 8 accumulator tiles of v_mfma_f32_16x16x32): its rows come straight from global
 // memory (row_panel.h), all 256 values of them, and the next block's are on their way while this one's are multiplied.
-// The weights come in by direct transfers of 64 bytes per four lanes and are read without bank conflicts; a CU needs 8 x 64 KiB of them per block (4096 cycles) and as many cycles
-// of its matrix cores. Output rows go through 4 KiB of LDS per wave and leave as 256-byte pieces.
+// The weights come in by direct transfers of 64 bytes per four lanes and are read without bank conflicts; a CU needs
+// 8 x 64 KiB of them per block (4096 cycles) and as many cycles of its matrix cores. Output rows go through 4 KiB of LDS per wave and leave as 256-byte pieces.
 // What bounds it: about 9 us of launch, weights and first rows before the first output, then memory: 36 products of 4096
 // rows move 156 MB in 32.2 us (37.3 on 128x64 tiles), of 2048 rows 80 MB in 21.8 (23.5 to 25.9), of 768 rows 10.6 (12.9).
-// Workgroups of one product run on the same XCD (its L2 serves the weights to all of them).
+// Consecutive workgroups run on the same XCD, so that its L2 serves the weights of a product to all of them, or to all of
+// them on two XCDs where the share of an XCD (31 or 32 of 252 workgroups) ends within a product's seven.
 // ---------------------------------------------------------------------------
 constexpr int kResRows = 128, kResCols = 256, kResK = 256;
 

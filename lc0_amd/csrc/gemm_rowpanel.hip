@@ -40,23 +40,21 @@ template <> struct PanelOp<uint8_t> {     // e4m3: 256 values, v_mfma_f32_16x16x
 
 // ---------------------------------------------------------------------------
 // Row-panel GEMM for small problems (few rows, or few columns): a workgroup owns a
-// (16 RT WM) x (16 CT WN) output panel and KS waves per part of it split the reduction
-// dimension, so even a 16 x 16 x K problem keeps KS waves busy. Such problems are bound
+// 16 RT x 16 CT output panel and its KS waves split the reduction dimension, so even a 16 x 16 x K problem keeps KS waves busy. Such problems are bound
 // by memory latency and by the rate at which a CU's address path takes operand loads,
 // not by arithmetic: fragments go from global memory straight into registers, 64 bytes
 // of a row per four lanes (row_panel.h), a whole share of K in flight at once when it is
 // one or two steps; the partial sums are added in wave order through LDS, so results do
 // not depend on timing.
 // ---------------------------------------------------------------------------
-template <typename ET, int RT, int CT, int WM, int WN, int KS, typename OutT, typename Args>
-__global__ __launch_bounds__(64 * WM * WN * KS) void gemm_rowpanel_kernel(Args p) {
+template <typename ET, int RT, int CT, int KS, typename OutT, typename Args>
+__global__ __launch_bounds__(64 * KS) void gemm_rowpanel_kernel(Args p) {
   constexpr bool F8 = std::is_same<ET, uint8_t>::value;
   constexpr int ES = F8 ? 1 : 2;
-  constexpr int ROWS = 16 * RT * WM, COLS = 16 * CT * WN, NT = 64 * WM * WN * KS, LD = COLS + 4;
+  constexpr int ROWS = 16 * RT, COLS = 16 * CT, NT = 64 * KS, LD = COLS + 4;
   __shared__ __attribute__((aligned(16))) float part[KS][ROWS * LD];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ks = wave % KS, wn = (wave / KS) % WN, wm = wave / (KS * WN);
+  const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int m0 = blockIdx.x * ROWS, n0 = blockIdx.y * COLS;
   const int M = p.M, N = p.N;
@@ -68,9 +66,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_rowpanel_kernel(Args p
   }
   TileOffsets ta[RT], tw[CT];
 #pragma unroll
-  for (int t = 0; t < RT; t++) ta[t].Set(16 * (wm * RT + t), M - m0, ES * p.lda);
+  for (int t = 0; t < RT; t++) ta[t].Set(16 * t, M - m0, ES * p.lda);
 #pragma unroll
-  for (int c = 0; c < CT; c++) tw[c].Set(16 * (wn * CT + c), N - n0, ES * p.ldw);
+  for (int c = 0; c < CT; c++) tw[c].Set(16 * c, N - n0, ES * p.ldw);
   floatx4 acc[RT][CT];
 #pragma unroll
   for (int t = 0; t < RT; t++)
@@ -85,7 +83,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_rowpanel_kernel(Args p
   for (int t = 0; t < RT; t++)
 #pragma unroll
     for (int c = 0; c < CT; c++)
-      *reinterpret_cast<floatx4*>(&part[ks][(16 * (wm * RT + t) + r) * LD + 16 * (wn * CT + c) + 4 * g]) = acc[t][c];
+      *reinterpret_cast<floatx4*>(&part[ks][(16 * t + r) * LD + 16 * c + 4 * g]) = acc[t][c];
   __syncthreads();
   OutT* C = reinterpret_cast<OutT*>(p.C);
   if constexpr (!F8) C += (long long)blockIdx.z * p.strideC;
@@ -131,7 +129,7 @@ void LaunchPanel(const Args& a, int batch, hipStream_t stream) {
   auto launch = [&](auto rt_tag, auto ct_tag) {
     constexpr int RT = decltype(rt_tag)::value, CT = decltype(ct_tag)::value, KS = kPanelWaves<ET>;
     dim3 grid((a.M + 16 * RT - 1) / (16 * RT), (a.N + 16 * CT - 1) / (16 * CT), batch);
-    hipLaunchKernelGGL((gemm_rowpanel_kernel<ET, RT, CT, 1, 1, KS, OutT, Args>), grid, dim3(64 * KS), 0, stream, a);
+    hipLaunchKernelGGL((gemm_rowpanel_kernel<ET, RT, CT, KS, OutT, Args>), grid, dim3(64 * KS), 0, stream, a);
   };
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;

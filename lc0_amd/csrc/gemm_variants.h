@@ -5,8 +5,8 @@
 
 namespace lc0mi {
 
-// (the numbers are those of SetGemmVariantOverride)
-enum GemmVariant { kDma256x256, kDma256x192, kDma256x128, kTile128, kTile64, kDma128x128, kRowPanel, kDma128x64, kUnused8 /* keeps the numbering of the variants after it */,
+// (the numbers are those of SetGemmVariantOverride; 8 is no kernel: the answer of a choice that finds none)
+enum GemmVariant { kDma256x256, kDma256x192, kDma256x128, kTile128, kTile64, kDma128x128, kRowPanel, kDma128x64, kNoVariant,
                    kDma128x32, kDma64x64, kResident };
 
 // Direct-to-LDS tiles (gemm_dma_half.hip, gemm_dma_bf16.hip, gemm_dma_f8.hip). The folded layer-norm fields of

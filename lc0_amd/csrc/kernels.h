@@ -175,7 +175,8 @@ void LaunchZero(float* p, long long n, hipStream_t stream);
 // Forces LaunchGemm to use one kernel variant (-1 = automatic choice): 0 256x256x64,
 // 1 256x192x64, 2 256x128x32 (direct-to-LDS, need K % 64 == 0 and half output),
 // 3 128x128x64, 4 64x64x64 (register-staged), 5 128x128x64 direct-to-LDS with 4 waves,
-// 6 row-panel 64x32 (K split over the waves), 7 128x64x64 direct-to-LDS with 4 waves. For tests and tuning only.
+// 6 row panels of 16x16 to 64x32 (K split over the waves), 7 128x64x64 direct-to-LDS with 4 waves, 9 128x32x64 and
+// 10 64x64x64 direct-to-LDS, 11 resident weights (K = N = 256, products in a batch). For tests and tuning only.
 void SetGemmVariantOverride(int variant);
 // Whether LaunchGemm may cut a large product along its rows (GemmRowSplit); on by default.
 void SetGemmRowSplit(bool on);
@@ -212,7 +213,8 @@ void LaunchAttention(const half_t* qkv, const half_t* bias, half_t* out, int bat
                      float scale, hipStream_t stream, int depth = 32, bool bf16 = false);
 bool AttentionDepthSupported(int depth);
 // The same contract (bias in the SmolgenBiasIndex layout, may be null) for any element type and any head depth up to
-// 128, on the vector ALUs: the float configuration, and head depths the kernel above does not take.
+// 128: the float configuration, on the fp32 matrix cores for head depths of 32, 64 and 128, and on the vector ALUs the
+// head depths that neither kernel takes.
 template <typename T>
 void LaunchAttentionGeneric(const T* qkv, const T* bias, T* out, int batch, int heads, int depth, float scale,
                             hipStream_t stream);
