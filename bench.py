@@ -203,7 +203,8 @@ def main():
 
     # Two and four search threads, each with its own computation in flight on the shared network (host I/O
     # included): how lc0 drives a backend (backendbench.cc:177-184 does the same with --threads). Passes of
-    # different lanes overlap on the GPU, so the aggregate rate is above that of one computation at a time.
+    # different lanes overlap on the GPU. With large batches, whose kernels each fill it, the aggregate rate is a few per cent
+    # above that of one computation at a time or below it, as the passes fall out of step or into it.
     import threading
 
     def threads_ms(n_threads):

@@ -396,7 +396,8 @@ GemmVariant PickGemmVariant(const GemmArgs& a) {
     return v != kNoVariant ? v : kDma128x64;
   }
   // A single 32-column panel (the smolgen compression): one workgroup per 64 rows, K split over its waves
-  // (16384x32x1024: 9.5 us against 12.3 for the 64x64 tiles, but with twice the threads on every CU).
+  // (16384x32x1024: 6.8 us against 12.8 on the 64x64 tiles and 9.6 on the 128x32 ones, but with twice the threads on
+  // every CU; 4096 rows 4.2 / 9.8 / 6.1).
   if (a.latency_first && a.split_k == 1 && a.N <= 32 && a.K >= 512) return kRowPanel;
   // Many products that each fit a 64x64 tile (the policy head's Q.K^T per position) would leave three quarters of
   // every 128x128 tile empty (256 x 64x64x1024: 14.5 against 21.4 us).
