@@ -107,7 +107,7 @@ LISTING = """
 
 @pytest.mark.parametrize("fill,rules", [(("s_nop 0", "s_nop 0", "s_nop 1"), []), (("", "", "s_nop 0"),
                                                                                  ["M0", "matrix read", "DPP read"])])
-def test_the_checker_sees_missing_wait_states(fill, rules):
+def test_missing_wait_states_are_seen(fill, rules):
     assert [h[1] for h in hazards(LISTING % fill)] == rules
 
 
