@@ -137,6 +137,14 @@ int lc0mi_k_winograd_conv(const float* x, const float* filter, const float* bias
 int lc0mi_k_gemm_f8(const uint8_t* A, int lda, const uint8_t* W, int ldw, const float* col_scale, const float* bias,
                     int M, int N, int K, int act, int out_f8, float out_mul, void* C, int ldc, int time_iters,
                     double* ms);
+/* Dense layer that normalises its input rows itself, `group` consecutive rows of A as one (gamma, beta: [group * K]; K 256):
+ * C = act(col_scale[n] * norm(A).W^T + bias[n]) with norm(A) rounded to half (bfloat16 after lc0mi_k_set_bf16(1)), or with
+ * f8 != 0 to e4m3(norm * in_mul) and W e4m3 bytes; col_scale is for f8 only. A [M][K], W [N][K], C [M][N], N % 16 == 0.
+ * Counterparts: LayerNorm2DWithSkipConnection without skip, then FullyConnectedLayer::Forward1D
+ * (src/neural/backends/blas/encoder.h:29-66, fully_connected_layer.cc:66-106). */
+int lc0mi_k_norm_gemm(int f8, const uint16_t* A, const void* W, const float* bias, const float* col_scale,
+                      const float* gamma, const float* beta, int group, int M, int N, int K, float eps, float in_mul, int act,
+                      uint16_t* C, int time_iters, double* ms);
 /* y[i] = e4m3(x[i] * mul): round to nearest even, saturating at +-448 (FP32toFP8E4M3FN,
  * src/utils/fp8_utils.h:111-138, applied to half inputs). n % 8 == 0. */
 int lc0mi_k_quantize_f8(const uint16_t* x, long long n, float mul, uint8_t* y);

@@ -19,25 +19,6 @@ inline RowPanelShape PickRowPanelShape(int M, int N, int batch) {
   return kRowPanelShapes[4];
 }
 
-// One step (four 16-byte chunks of both operands) of a 16x16 accumulator tile, by operand type.
-template <typename ET> struct PanelOp {   // half_t, bf16_t: 128 values, v_mfma_f32_16x16x32
-  __device__ __forceinline__ void operator()(const intx4 (&w)[4], const intx4 (&a)[4], floatx4& c) const {
-    using ev8 = typename Vec16<ET>::v8;
-#pragma unroll
-    for (int j = 0; j < 4; j++) c = Mfma16(__builtin_bit_cast(ev8, w[j]), __builtin_bit_cast(ev8, a[j]), c);
-  }
-};
-template <> struct PanelOp<uint8_t> {     // e4m3: 256 values, v_mfma_f32_16x16x128_f8f6f4
-  __device__ __forceinline__ void operator()(const intx4 (&w)[4], const intx4 (&a)[4], floatx4& c) const {
-#pragma unroll
-    for (int j = 0; j < 4; j += 2) {
-      const intx8 fw = {w[j][0], w[j][1], w[j][2], w[j][3], w[j + 1][0], w[j + 1][1], w[j + 1][2], w[j + 1][3]};
-      const intx8 fa = {a[j][0], a[j][1], a[j][2], a[j][3], a[j + 1][0], a[j + 1][1], a[j + 1][2], a[j + 1][3]};
-      c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw, fa, c, 0, 0, 0, 0, 0, 0);
-    }
-  }
-};
-
 // ---------------------------------------------------------------------------
 // Row-panel GEMM for small problems (few rows, or few columns): a workgroup owns a
 // 16 RT x 16 CT output panel and its KS waves split the reduction dimension, so even a 16 x 16 x K problem keeps KS waves busy. Such problems are bound

@@ -644,6 +644,32 @@ int lc0mi_k_winograd_conv(const float* x, const float* filter, const float* bias
   });
 }
 
+int lc0mi_k_norm_gemm(int f8, const uint16_t* A, const void* W, const float* bias, const float* col_scale,
+                      const float* gamma, const float* beta, int group, int M, int N, int K, float eps, float in_mul, int act,
+                      uint16_t* C, int time_iters, double* ms) {
+  return Guard([&] {
+    RequireDevice();
+    if (M < 1 || N < 1 || !lc0mi::NormGemmSupported(K, group, N) || M % group != 0 || (f8 && !col_scale)) throw Error("bad shape");
+    Dev dev;
+    lc0mi::NormGemmArgs g;
+    g.A = reinterpret_cast<const half_t*>(dev.Put(A, (size_t)M * K));
+    g.W = dev.Put(static_cast<const uint8_t*>(W), (size_t)N * K * (f8 ? 1 : 2)); g.ldw = K;
+    g.C = reinterpret_cast<half_t*>(dev.Put(C, (size_t)M * N)); g.ldc = N;
+    g.bias = bias ? dev.Put(bias, (size_t)N) : nullptr;
+    g.col_scale = f8 ? dev.Put(col_scale, (size_t)N) : nullptr;
+    g.gamma = dev.Put(gamma, (size_t)group * K);
+    g.beta = dev.Put(beta, (size_t)group * K);
+    g.M = M; g.N = N; g.K = K; g.group = group; g.eps = eps; g.in_mul = in_mul; g.act = act;
+    g.bf16 = g_bf16 && !f8;
+    g.f8 = f8 != 0;
+    lc0mi::LaunchNormGemm(g, nullptr);
+    K_CHECK(hipDeviceSynchronize());
+    K_CHECK(hipGetLastError());
+    K_CHECK(hipMemcpy(C, g.C, (size_t)M * N * 2, hipMemcpyDeviceToHost));
+    if (time_iters > 0 && ms) *ms = TimeLaunches(time_iters, [&] { lc0mi::LaunchNormGemm(g, nullptr); });
+  });
+}
+
 int lc0mi_k_gemm_f8(const uint8_t* A, int lda, const uint8_t* W, int ldw, const float* col_scale, const float* bias,
                     int M, int N, int K, int act, int out_f8, float out_mul, void* C, int ldc, int time_iters,
                     double* ms) {

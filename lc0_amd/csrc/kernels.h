@@ -191,6 +191,24 @@ void LaunchLayerNormRows(const float* x_f32, int n_partials, long long partial_s
                          int C, float alpha, float eps, hipStream_t stream, bool bf16 = false,
                          uint8_t* y_f8 = nullptr, float f8_mul = 1.0f);
 
+// C[m][n] = act(sum_k norm(A)[m][k] W[n][k] + bias[n]): a dense layer that normalises its input rows itself, `group`
+// consecutive rows (a divisor of M) as one: norm(A) = beta + gamma * (A - mean) / sqrt(var + eps), gamma and beta of
+// group * K values, rounded to the type of W's elements. A, C: halves, or with bf16 bfloat16; A has rows of K values, no
+// gap between them. f8: W holds e4m3 bytes, the normalised rows become e4m3(norm * in_mul), and the sums are multiplied
+// by col_scale[n] before the bias. For few rows: NormGemmSupported(), ldc % 16 == 0, bases 16-byte aligned.
+struct NormGemmArgs {
+  const half_t* A = nullptr;
+  const void* W = nullptr; int ldw = 0;
+  half_t* C = nullptr; int ldc = 0;
+  const float *bias = nullptr, *col_scale = nullptr, *gamma = nullptr, *beta = nullptr;
+  int M = 0, N = 0, K = 0, group = 1;
+  float eps = 1e-3f, in_mul = 1.0f;
+  int act = 3;
+  bool bf16 = false, f8 = false;
+};
+bool NormGemmSupported(int K, int group, int N);
+void LaunchNormGemm(const NormGemmArgs& args, hipStream_t stream);
+
 // rows x C layer norm: y = beta + gamma * (t - mean) / sqrt(var + eps) with
 // t = x * alpha + skip (skip may be null). x, skip, y may alias. C % 8 == 0, C <= 8192.
 // y_f8 (optional): also receives e4m3(y * f8_mul), saturating, the operand of a following fp8 GEMM.

@@ -293,6 +293,7 @@ struct ModelState {
   bool fused_smolgen_attention_ = true;
   int fused_smolgen_min_batch_ = 72;
   int dense1_split_min_batch_ = 112;   // smallest batch whose smolgen dense1 splits K between workgroups
+  int dense2_norm_max_batch_ = 64, generator_norm_max_batch_ = 48;   // largest batches whose row norms run inside the layer after them
   bool qkv_first_ = true;
   bool write_through_ = true;   // big activations go to the memory-side cache while a layer's worth fits it
   int chain_latency_max_batch_ = 128;   // largest fp16 batch whose smolgen chain takes the shortest-latency GEMM variants
@@ -442,6 +443,8 @@ class Mi355xNetwork : public Network, protected ModelState {
   void LayerNorm(const half_t* x, const half_t* skip, half_t* y, const float* gamma, const float* beta, int rows, int C,
                  float alpha, float eps, hipStream_t st = nullptr, uint8_t* y_f8 = nullptr, float f8_mul = 1.0f,
                  bool through = false);
+  void NormGemm(const char* name, const half_t* A, const Linear& lin, const LinearF8* f8, float in_mul, const float* gamma,
+                const float* beta, int group, half_t* C, int M, int act, hipStream_t st);
   void LayerNormRows(const half_t* x, half_t* y, const float* gamma, const float* beta, int rows, int C,
                      hipStream_t st);
   void Attention(const half_t* qkv, const half_t* bias, half_t* out, int B, int heads, int depth, hipStream_t st);
@@ -695,6 +698,28 @@ void Mi355xNetwork::Gemm(const char* name, const half_t* A, int lda, const Linea
   std::string label = std::string(name) + "|" + GemmVariantName(g);
   if (fold != nullptr) label += fold->skip != nullptr ? "+skip_stats" : "+row_norm";
   Timed(label.c_str(), flops, bytes, [&] { LaunchGemm(g, st); }, st);
+}
+
+// A dense layer of the smolgen chain with the norm of its input rows (`group` of them together) in the same kernel.
+// f8: the layer on e4m3 operands, whose input scale is 1 / in_mul.
+void Mi355xNetwork::NormGemm(const char* name, const half_t* A, const Linear& lin, const LinearF8* f8, float in_mul,
+                             const float* gamma, const float* beta, int group, half_t* C, int M, int act, hipStream_t st) {
+  NormGemmArgs g;
+  g.A = A;
+  g.W = f8 != nullptr ? static_cast<const void*>(f8->w) : lin.w;
+  g.ldw = f8 != nullptr ? lin.in : lin.ld;
+  g.C = C; g.ldc = lin.out;
+  g.bias = lin.b;
+  g.col_scale = f8 != nullptr ? f8->col_scale : nullptr;
+  g.gamma = gamma; g.beta = beta; g.group = group;
+  g.M = M; g.N = lin.out; g.K = lin.in;
+  g.in_mul = in_mul;
+  g.act = act;
+  g.bf16 = dtype_ == Dtype::kBf16;
+  g.f8 = f8 != nullptr;
+  const std::string label = std::string(name) + (g.f8 ? "|gemm_f8_norm" : "|gemm_norm");
+  Timed(label.c_str(), 2.0 * M * lin.out * lin.in,
+        2.0 * M * lin.in + (f8 != nullptr ? 1.0 : 2.0) * lin.out * lin.in + 2.0 * M * lin.out, [&] { LaunchNormGemm(g, st); }, st);
 }
 
 void Mi355xNetwork::LayerNorm(const half_t* x, const half_t* skip, half_t* y, const float* gamma, const float* beta,
@@ -1046,6 +1071,8 @@ Mi355xNetwork::Mi355xNetwork(const WeightsFile& file, Options& options) {
   fused_smolgen_attention_ = options.GetBool("fused_smolgen_attention", true);
   fused_smolgen_min_batch_ = options.GetInt("fused_smolgen_min_batch", 72);
   dense1_split_min_batch_ = options.GetInt("dense1_split_min_batch", 112);
+  dense2_norm_max_batch_ = options.GetInt("dense2_norm_max_batch", 64);
+  generator_norm_max_batch_ = options.GetInt("generator_norm_max_batch", 48);
   qkv_first_ = options.GetBool("qkv_first", true);
   write_through_ = options.GetBool("write_through", true);
   chain_latency_max_batch_ = options.GetInt("chain_latency_max_batch", 128);
@@ -1950,22 +1977,42 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       // or at most 128 positions): its kernels then take the variants with the shortest latency. At larger fp16
       // batches the two are balanced and the leaner variants disturb the projection less (batch 256: 1.5 %).
       const bool chain_first = f8 || B <= chain_latency_max_batch_;
+      // For few positions the two layers after a row norm normalise their rows themselves, which saves two launches of a
+      // chain of thirteen per layer (norm_gemm_kernel; us of a 15x1024 pass, neither -> dense2 -> both. fp16: 1 position 989 ->
+      // 950 -> 915, 13 1375 -> 1323 -> 1278, 32 1768 -> 1720 -> 1691, 64 2374 -> 2352 -> 2323, 71 2605 -> 2607 -> 2626; e4m3: 1
+      // 843 -> 806 -> 765, 32 1268 -> 1209 -> 1187, 48 1555 -> 1509 -> 1578). From 65 positions the products are long enough to
+      // hide the launches and the norm, repeated in every workgroup of a row, costs what it saves; the generator layer gets
+      // there earlier, with e4m3 operands at 33.
+      const bool norms_inside = !calibrating_ && dtype_ != Dtype::kFloat && B < dense1_split_min_batch_;
+      const bool norm_dense2 = norms_inside && B <= dense2_norm_max_batch_ && NormGemmSupported(sg_hs_, 1, sg_gen_);
+      const bool norm_global = norms_inside && !fused_gen && B <= std::min(generator_norm_max_batch_, chain_f8 ? 32 : 1024) &&
+                               NormGemmSupported(g, heads_, 4096);
       if (chain_f8) {
         // The whole chain on e4m3 operands: the compression reads the e4m3 copy of x that the QKV projection reads
         // and writes e4m3 itself; the two row norms write halves and their e4m3 copies.
         GemmF8("gemm_smolgen_compress", xq_, e.sg_compress, e.sg_compress8, sg1q_, T, kActNone, true, 1.0f / e.s_sg1, ss);
         GemmF8("gemm_smolgen_dense1", sg1q_, e.sg_dense1, e.sg_dense18, sg2_, B, smolgen_act_, false, 1.0f, ss);
-        Timed("layer_norm_rows", 0.0, 5.0 * B * sg_hs_, [&] {
-          LaunchLayerNormRows(nullptr, 0, 0, sg2_, kActNone, nullptr, sg2_, e.sg_ln1_g, e.sg_ln1_b, B, sg_hs_, 1.0f,
-                              1e-3f, ss, false, sg2q_, 1.0f / e.s_sg2);
-        }, ss);
-        GemmF8("gemm_smolgen_dense2", sg2q_, e.sg_dense2, e.sg_dense28, sg3_, B, smolgen_act_, false, 1.0f, ss);
-        Timed("layer_norm_rows", 0.0, (fused_gen ? 4.0 : 5.0) * B * sg_gen_, [&] {
-          LaunchLayerNormRows(nullptr, 0, 0, sg3_, kActNone, nullptr, sg3_, e.sg_ln2_g, e.sg_ln2_b, B, sg_gen_, 1.0f,
-                              1e-3f, ss, false, fused_gen ? nullptr : sg3q_, 1.0f / e.s_sg3);
-        }, ss);
-        if (!fused_gen) {
-          GemmF8("gemm_smolgen_global", sg3q_, smolgen_w_, e.sg_global8, sbias_, B * heads_, kActNone, false, 1.0f, ss);
+        if (norm_dense2) {
+          NormGemm("gemm_smolgen_dense2", sg2_, e.sg_dense2, &e.sg_dense28, 1.0f / e.s_sg2, e.sg_ln1_g, e.sg_ln1_b, 1, sg3_, B,
+                   smolgen_act_, ss);
+        } else {
+          Timed("layer_norm_rows", 0.0, 5.0 * B * sg_hs_, [&] {
+            LaunchLayerNormRows(nullptr, 0, 0, sg2_, kActNone, nullptr, sg2_, e.sg_ln1_g, e.sg_ln1_b, B, sg_hs_, 1.0f,
+                                1e-3f, ss, false, sg2q_, 1.0f / e.s_sg2);
+          }, ss);
+          GemmF8("gemm_smolgen_dense2", sg2q_, e.sg_dense2, e.sg_dense28, sg3_, B, smolgen_act_, false, 1.0f, ss);
+        }
+        if (norm_global) {
+          NormGemm("gemm_smolgen_global", sg3_, smolgen_w_, &e.sg_global8, 1.0f / e.s_sg3, e.sg_ln2_g, e.sg_ln2_b, heads_,
+                   sbias_, B * heads_, kActNone, ss);
+        } else {
+          Timed("layer_norm_rows", 0.0, (fused_gen ? 4.0 : 5.0) * B * sg_gen_, [&] {
+            LaunchLayerNormRows(nullptr, 0, 0, sg3_, kActNone, nullptr, sg3_, e.sg_ln2_g, e.sg_ln2_b, B, sg_gen_, 1.0f,
+                                1e-3f, ss, false, fused_gen ? nullptr : sg3q_, 1.0f / e.s_sg3);
+          }, ss);
+          if (!fused_gen) {
+            GemmF8("gemm_smolgen_global", sg3q_, smolgen_w_, e.sg_global8, sbias_, B * heads_, kActNone, false, 1.0f, ss);
+          }
         }
       } else if (dtype_ == Dtype::kFloat) {
         SmolgenChain(e, x_, emb_, heads_, sg_hc_, sg_hs_, sg_gen_, sg1_, sg2_, sg3_, sbias_, B, ss, chain_first);
@@ -1978,10 +2025,12 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       if (B < dense1_split_min_batch_) {
         Gemm("gemm_smolgen_dense1", sg1_, 64 * sg_hc_, e.sg_dense1, sg2_, sg_hs_, B, smolgen_act_, false, ss, 1,
              chain_first);
-        Timed("layer_norm_rows", 0.0, 4.0 * B * sg_hs_, [&] {
-          LaunchLayerNormRows(nullptr, 0, 0, sg2_, kActNone, nullptr, sg2_, e.sg_ln1_g, e.sg_ln1_b, B, sg_hs_, 1.0f,
-                              1e-3f, ss, bf16);
-        }, ss);
+        if (!norm_dense2) {
+          Timed("layer_norm_rows", 0.0, 4.0 * B * sg_hs_, [&] {
+            LaunchLayerNormRows(nullptr, 0, 0, sg2_, kActNone, nullptr, sg2_, e.sg_ln1_g, e.sg_ln1_b, B, sg_hs_, 1.0f,
+                                1e-3f, ss, bf16);
+          }, ss);
+        }
       } else {
         const int split = std::max(1, std::min(16, (64 * sg_hc_) / 256));
         Gemm("gemm_smolgen_dense1", sg1_, 64 * sg_hc_, e.sg_dense1, sg2f_, sg_hs_, B, kActNone, true, ss, split);
@@ -1994,14 +2043,23 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
         RecordAbsMax(sg1_, static_cast<size_t>(T) * sg_hc_, SmolgenSlot(li, 0), ss);
         RecordAbsMax(sg2_, static_cast<size_t>(B) * sg_hs_, SmolgenSlot(li, 1), ss);
       }
-      Gemm("gemm_smolgen_dense2", sg2_, sg_hs_, e.sg_dense2, sg3_, sg_gen_, B, smolgen_act_, false, ss, 1, chain_first);
-      Timed("layer_norm_rows", 0.0, 4.0 * B * sg_gen_, [&] {
-        LaunchLayerNormRows(nullptr, 0, 0, sg3_, kActNone, nullptr, sg3_, e.sg_ln2_g, e.sg_ln2_b, B, sg_gen_, 1.0f, 1e-3f,
-                            ss, bf16);
-      }, ss);
-      if (calibrating_ && q_smolgen_) RecordAbsMax(sg3_, static_cast<size_t>(B) * sg_gen_, SmolgenSlot(li, 2), ss);
-      if (!fused_gen) {
-        Gemm("gemm_smolgen_global", sg3_, g, smolgen_w_, sbias_, 4096, B * heads_, kActNone, false, ss, 1, chain_first);
+      if (norm_dense2) {
+        NormGemm("gemm_smolgen_dense2", sg2_, e.sg_dense2, nullptr, 1.0f, e.sg_ln1_g, e.sg_ln1_b, 1, sg3_, B, smolgen_act_, ss);
+      } else {
+        Gemm("gemm_smolgen_dense2", sg2_, sg_hs_, e.sg_dense2, sg3_, sg_gen_, B, smolgen_act_, false, ss, 1, chain_first);
+      }
+      if (norm_global) {
+        NormGemm("gemm_smolgen_global", sg3_, smolgen_w_, nullptr, 1.0f, e.sg_ln2_g, e.sg_ln2_b, heads_, sbias_, B * heads_,
+                 kActNone, ss);
+      } else {
+        Timed("layer_norm_rows", 0.0, 4.0 * B * sg_gen_, [&] {
+          LaunchLayerNormRows(nullptr, 0, 0, sg3_, kActNone, nullptr, sg3_, e.sg_ln2_g, e.sg_ln2_b, B, sg_gen_, 1.0f, 1e-3f,
+                              ss, bf16);
+        }, ss);
+        if (calibrating_ && q_smolgen_) RecordAbsMax(sg3_, static_cast<size_t>(B) * sg_gen_, SmolgenSlot(li, 2), ss);
+        if (!fused_gen) {
+          Gemm("gemm_smolgen_global", sg3_, g, smolgen_w_, sbias_, 4096, B * heads_, kActNone, false, ss, 1, chain_first);
+        }
       }
       }
       if (ss != stream_) HIP_CHECK(hipEventRecord(join_events_[li], ss));

@@ -71,6 +71,25 @@ struct TileOffsets {
   }
 };
 
+// One step (four 16-byte chunks of both operands) of a 16x16 accumulator tile, by operand type.
+template <typename ET> struct PanelOp {   // half_t, bf16_t: 128 values, v_mfma_f32_16x16x32
+  __device__ __forceinline__ void operator()(const intx4 (&w)[4], const intx4 (&a)[4], floatx4& c) const {
+    using ev8 = typename Vec16<ET>::v8;
+#pragma unroll
+    for (int j = 0; j < 4; j++) c = Mfma16(__builtin_bit_cast(ev8, w[j]), __builtin_bit_cast(ev8, a[j]), c);
+  }
+};
+template <> struct PanelOp<uint8_t> {     // e4m3: 256 values, v_mfma_f32_16x16x128_f8f6f4
+  __device__ __forceinline__ void operator()(const intx4 (&w)[4], const intx4 (&a)[4], floatx4& c) const {
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {
+      const intx8 fw = {w[j][0], w[j][1], w[j][2], w[j][3], w[j + 1][0], w[j + 1][1], w[j + 1][2], w[j + 1][3]};
+      const intx8 fa = {a[j][0], a[j][1], a[j][2], a[j][3], a[j + 1][0], a[j + 1][1], a[j + 1][2], a[j + 1][3]};
+      c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw, fa, c, 0, 0, 0, 0, 0, 0);
+    }
+  }
+};
+
 // The products of a wave that has one step only, with one set of operand registers. `bytes` of every row exist (a multiple
 // of 16, at least 16), masked as PanelProducts masks its last step. (A function of its own: the same code called from there
 // made its loops 3 % slower, 33x3072x256 in halves 3.38 us against 3.25.)

@@ -38,6 +38,7 @@ def _lib():
         lib.lc0mi_k_expand_planes_nchw.argtypes = [vp, vp, ci, vp]
         lib.lc0mi_k_attn_policy_gather.argtypes = [vp, vp, vp, ci, ci, vp]
         lib.lc0mi_k_gemm_f8.argtypes = [vp, ci, vp, ci, vp, vp, ci, ci, ci, ci, ci, cf, vp, ci, ci, cd]
+        lib.lc0mi_k_norm_gemm.argtypes = [ci] + [vp] * 6 + [ci] * 4 + [cf, cf, ci, vp, ci, cd]
         lib.lc0mi_k_quantize_f8.argtypes = [vp, ll, cf, vp]
         lib.lc0mi_k_layer_norm_f8.argtypes = [vp, vp, vp, vp, ci, ci, cf, cf, cf, vp, vp]
         lib.lc0mi_k_attention_f8.argtypes = [vp, vp, ci, ci, cf, cf, vp]
@@ -304,6 +305,21 @@ def gemm_f8(a, w, col_scale, bias=None, act=ACT_NONE, out_f8=False, out_mul=1.0,
     _check(_lib().lc0mi_k_gemm_f8(_ptr(a), k, _ptr(w), k, _ptr(cs), _ptr(b), m, n, k, act, int(out_f8),
                                   C.c_float(out_mul), _ptr(out), n, time_iters, C.byref(ms)))
     return (out, ms.value) if time_iters else out
+
+
+def norm_gemm(a, w, gamma, beta, group=1, bias=None, eps=1e-3, act=ACT_NONE, col_scale=None, in_mul=1.0, time_iters=0):
+    """act(norm(a).w^T + bias), the rows of a normalised inside the kernel, `group` of them together. col_scale (and e4m3
+    bytes as w): the e4m3 form, norm(a) * in_mul quantised."""
+    f8 = col_scale is not None
+    a, w = _h(a), np.ascontiguousarray(w, np.uint8) if f8 else _h(w)
+    (m, k), n = a.shape, w.shape[0]
+    gamma, beta = np.ascontiguousarray(gamma, np.float32), np.ascontiguousarray(beta, np.float32)
+    b = np.ascontiguousarray(bias, np.float32) if bias is not None else None
+    cs = np.ascontiguousarray(col_scale, np.float32) if f8 else None
+    out, ms = _out16((m, n)), C.c_double(0)
+    _check(_lib().lc0mi_k_norm_gemm(int(f8), _ptr(a), _ptr(w), _ptr(b), _ptr(cs), _ptr(gamma), _ptr(beta), group, m, n, k,
+                                    C.c_float(eps), C.c_float(in_mul), act, _ptr(out), time_iters, C.byref(ms)))
+    return (_ret16(out), ms.value) if time_iters else _ret16(out)
 
 
 def quantize_f8(x, mul=1.0):
