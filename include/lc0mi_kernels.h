@@ -145,6 +145,12 @@ int lc0mi_k_gemm_f8(const uint8_t* A, int lda, const uint8_t* W, int ldw, const 
 int lc0mi_k_norm_gemm(int f8, const uint16_t* A, const void* W, const float* bias, const float* col_scale,
                       const float* gamma, const float* beta, int group, int M, int N, int K, float eps, float in_mul, int act,
                       uint16_t* C, int time_iters, double* ms);
+/* Two products of the same rows in one launch: C as lc0mi_k_gemm (batch 1, 16-bit output, act none) or, with f8 != 0, as
+ * lc0mi_k_gemm_f8 (half output), and C2 = A.W2^T without bias (16-bit), or e4m3(col_scale2[n] * sum * out_mul2) bytes.
+ * A [M][K], W [N][K], W2 [N2][K]. Fails where the kernel of the first product does not serve a second one. Counterpart:
+ * two calls of FullyConnectedLayer::Forward1D (src/neural/backends/blas/fully_connected_layer.cc:66-106). */
+int lc0mi_k_gemm_second(int f8, const void* A, const void* W, const void* W2, const float* bias, const float* col_scale,
+                        const float* col_scale2, float out_mul2, int M, int N, int N2, int K, uint16_t* C, void* C2);
 /* y[i] = e4m3(x[i] * mul): round to nearest even, saturating at +-448 (FP32toFP8E4M3FN,
  * src/utils/fp8_utils.h:111-138, applied to half inputs). n % 8 == 0. */
 int lc0mi_k_quantize_f8(const uint16_t* x, long long n, float mul, uint8_t* y);

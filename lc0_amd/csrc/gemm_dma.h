@@ -130,16 +130,20 @@ void gemm_dma_kernel(Args p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  const int M = p.M, N = p.N, K = p.K;
+  // Tiles past the columns of the first product belong to the second one (small tiles only).
+  constexpr bool TWO = BM < 256 && EPI == 0;
+  const int col_tiles = TWO ? (p.N + BN - 1) / BN : 0;
+  const bool second = TWO && (int)blockIdx.y >= col_tiles;
+  const int m0 = blockIdx.x * BM, n0 = (second ? blockIdx.y - col_tiles : blockIdx.y) * BN;
+  const int M = p.M, N = second ? p.N2 : p.N, K = p.K, ldw = second ? p.ldw2 : p.ldw;
   float my_bias = 0.0f;
   [[maybe_unused]] float my_cscale = 0.0f;
   if (tid < BN && n0 + tid < N) {
-    if (p.bias != nullptr) my_bias = p.bias[n0 + tid];
-    if constexpr (F8) my_cscale = p.col_scale[n0 + tid];
+    if (p.bias != nullptr && !second) my_bias = p.bias[n0 + tid];
+    if constexpr (F8) my_cscale = (second ? p.col_scale2 : p.col_scale)[n0 + tid];
   }
   const char* A = reinterpret_cast<const char*>(p.A);
-  const char* W = reinterpret_cast<const char*>(p.W);
+  const char* W = second ? reinterpret_cast<const char*>(p.W2) : reinterpret_cast<const char*>(p.W);
   if constexpr (!F8) {
     A += (long long)blockIdx.z * p.strideA * ES;
     W += (long long)blockIdx.z * p.strideW * ES;
@@ -157,7 +161,7 @@ void gemm_dma_kernel(Args p) {
   for (int i = 0; i < W_CPW; i++) {
     const int row = (wave * W_CPW + i) * ROWS_PER_CHUNK + lane / CPR;
     const int c = (lane % CPR) ^ ((row >> SWZ_SHIFT) % CPR);
-    w_ptr[i] = W + (long long)min(n0 + row, N - 1) * p.ldw * ES + c * 16;
+    w_ptr[i] = W + (long long)min(n0 + row, N - 1) * ldw * ES + c * 16;
   }
   auto issue = [&](char* As, char* Ws, int kbyte) {
 #pragma unroll
@@ -342,6 +346,34 @@ void gemm_dma_kernel(Args p) {
   for (; kt + NSTAGES - 1 < nk; kt++) k_tile(kt, std::true_type{});
   for (; kt < nk; kt++) k_tile(kt, std::false_type{});
 
+  if constexpr (TWO) {
+    if (second) {   // few columns: straight from the accumulators, four neighbouring columns of a row per lane
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int blk = 0; blk < 4; blk++) {
+            const int m = m0 + wm * WM + i * 32 + r, col = wn * WN + j * 32 + blk * 8 + g * 4, n = n0 + col;
+            if (m >= M || n >= N) continue;
+            if constexpr (F8) {
+              const floatx4 cs = *reinterpret_cast<const floatx4*>(colv + BN + col);
+              float v[4];
+#pragma unroll
+              for (int rr = 0; rr < 4; rr++) v[rr] = acc[i][j][blk * 4 + rr] * cs[rr] * p.out_mul2;
+              *reinterpret_cast<unsigned*>(reinterpret_cast<uint8_t*>(p.C2) + (long long)m * p.ldc2 + n) =
+                  PackFp8x4(v[0], v[1], v[2], v[3]);
+            } else {
+              using ov4 = typename Vec16<ET>::v4;
+              ov4 h;
+#pragma unroll
+              for (int rr = 0; rr < 4; rr++) h[rr] = (ET)acc[i][j][blk * 4 + rr];
+              *reinterpret_cast<ov4*>(reinterpret_cast<ET*>(p.C2) + (long long)m * p.ldc2 + n) = h;
+            }
+          }
+      return;
+    }
+  }
   // Epilogue through LDS (the stage buffers are free after the barrier).
   __syncthreads();
   if constexpr (EPI == 2) {
@@ -562,7 +594,7 @@ inline int OutputStores(int requested, long long m, long long n, long long batch
 
 template <typename ET, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int NSTAGES = 2, bool ALONE = false>
 void LaunchGemmDma(const GemmArgs& a, hipStream_t stream) {
-  dim3 grid((a.M + BM - 1) / BM, (a.N + BN - 1) / BN, a.batch);
+  dim3 grid((a.M + BM - 1) / BM, (a.N + BN - 1) / BN + (a.N2 + BN - 1) / BN, a.batch);
   const dim3 block(WAVES_M * WAVES_N * 64);
   auto launch = [&](auto stores_tag) {
     constexpr int S = decltype(stores_tag)::value;
@@ -605,7 +637,7 @@ void LaunchGemmDmaStaged(const GemmArgs& a, hipStream_t stream) {
   constexpr int kStage = (BM + BN) * BK * 2, kCus = 256;
   constexpr int kFour = WorkgroupsPerCu(4, kStage), kThree = WorkgroupsPerCu(3, kStage);
   constexpr bool kAlone = BM * BN <= 128 * 64;   // (an instance for one workgroup per CU, with four stages)
-  const long long wgs = (long long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN) * a.batch;
+  const long long wgs = (long long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN + (a.N2 + BN - 1) / BN) * a.batch;
   if (a.skip != nullptr || a.row_stats != nullptr) return LaunchGemmDma<ET, BM, BN, BK, WAVES_M, WAVES_N, 2>(a, stream);
   if constexpr (kAlone) {
     if (wgs <= kCus) return LaunchGemmDma<ET, BM, BN, BK, WAVES_M, WAVES_N, 4, true>(a, stream);

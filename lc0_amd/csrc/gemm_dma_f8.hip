@@ -6,7 +6,7 @@ namespace lc0mi {
 namespace {
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BKB = 128, int NSTAGES = 2, bool ALONE = false>
 void LaunchGemmDmaF8Tile(const GemmF8Args& a, hipStream_t stream) {
-  dim3 grid((a.M + BM - 1) / BM, (a.N + BN - 1) / BN, 1);
+  dim3 grid((a.M + BM - 1) / BM, (a.N + BN - 1) / BN + (a.N2 + BN - 1) / BN);
   const dim3 block(WAVES_M * WAVES_N * 64);
   if constexpr (BM == 256) {
     const int stores = OutputStores(a.out_stores, a.M, a.N, 1, a.out_f8 ? 1 : 2);
@@ -38,7 +38,7 @@ void LaunchGemmDmaF8Staged(const GemmF8Args& a, hipStream_t stream) {
   constexpr int kStage = (BM + BN) * 128, kCus = 256;
   constexpr int kFour = WorkgroupsPerCu(4, kStage), kThree = WorkgroupsPerCu(3, kStage);
   constexpr bool kAlone = BM * BN <= 128 * 64;
-  const long long wgs = (long long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
+  const long long wgs = (long long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN + (a.N2 + BN - 1) / BN);
   if constexpr (kAlone) {
     if (wgs <= kCus) return LaunchGemmDmaF8Tile<BM, BN, WAVES_M, WAVES_N, 128, 4, true>(a, stream);
   }

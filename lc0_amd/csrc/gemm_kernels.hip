@@ -438,6 +438,30 @@ bool GemmSupportsNormFolding(const GemmArgs& a) {
   return true;
 }
 
+namespace {
+// Whether the workgroups of a second product of N2 columns are no more per CU than those of the first one alone: the
+// launch then takes no longer than without them.
+bool SecondFits(GemmVariant v, int M, int N, int N2) {
+  if (v == kRowPanel) {
+    for (const RowPanelShape& c : kRowPanelShapes) {   // (the panel that the first product gets)
+      const long long first = RowPanelWorkgroups(M, N, 1, c);
+      if (first <= kRowPanelWorkgroups) return first + RowPanelWorkgroups(M, N2, 1, c) <= kRowPanelWorkgroups;
+    }
+    return false;
+  }
+  const int bm = v == kDma64x64 ? 64 : 128, bn = v == kDma128x128 ? 128 : 64;
+  if (v != kDma64x64 && v != kDma128x64 && v != kDma128x128) return false;
+  const long long rows = (M + bm - 1) / bm, first = rows * ((N + bn - 1) / bn), both = first + rows * ((N2 + bn - 1) / bn);
+  return (both + 255) / 256 == (first + 255) / 256;
+}
+}  // namespace
+
+bool GemmTakesSecond(const GemmArgs& a) {
+  GemmVariant first = kDma256x256;
+  return a.batch == 1 && a.split_k == 1 && !a.out_f32 && a.skip == nullptr && a.row_stats == nullptr && a.N2 % 8 == 0 &&
+         a.ldw2 % 8 == 0 && a.ldc2 % 8 == 0 && PlanRowSplit(a, &first) == 0 && SecondFits(PickGemmVariant(a), a.M, a.N, a.N2);
+}
+
 int GemmStatsParts(const GemmArgs& a) {
   const int bn = DmaTileN(PickGemmVariant(a));
   return bn == 0 ? 0 : (a.N + bn - 1) / bn;
@@ -486,6 +510,7 @@ void LaunchGemmOne(const GemmArgs& a, hipStream_t stream) {
 
 void LaunchGemm(const GemmArgs& a, hipStream_t stream) {
   if (a.M <= 0 || a.N <= 0 || a.batch <= 0) return;
+  if (a.N2 > 0 && !GemmTakesSecond(a)) throw std::runtime_error("LaunchGemm: no kernel with a second product for this shape");
   if ((a.skip != nullptr || a.row_stats != nullptr) && !GemmSupportsNormFolding(a)) {
     throw std::runtime_error("LaunchGemm: no kernel variant with the folded layer-norm epilogue for this shape");
   }
@@ -527,7 +552,11 @@ GemmVariant PickGemmF8Variant(const GemmF8Args& a) {
   // 300x8192x1024 9.1 / 7.9; 256x8192x512 with 4 MiB 4.4 / 4.8, 1024x3072x1536 with twice the rows 10.6 / 11.2).
   const long long tiles64 = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64);
   const bool few_rows_large_weights = tiles64 > 256 && a.M < 1024 && (long long)a.N * a.K > (4LL << 20);
-  if (a.N >= 64 && tiles64 <= 768 && !few_rows_large_weights) return kDma64x64;
+  if (a.N >= 64 && tiles64 <= 768 && !few_rows_large_weights) {
+    // (A second product whose tiles would make a fourth per CU: the next larger tiles, 1024x3072x1024 8.1 us against 7.9, and one launch less.)
+    const bool larger = a.N2 > 0 && !SecondFits(kDma64x64, a.M, a.N, a.N2) && SecondFits(kDma128x64, a.M, a.N, a.N2);
+    return larger ? kDma128x64 : kDma64x64;
+  }
   if (a.M < 1024 && a.N >= 64) return kDma128x64;
   auto rounds = [&](int bm, int bn) {
     const long long tiles = (long long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
@@ -550,6 +579,10 @@ GemmVariant PickGemmF8Variant(const GemmF8Args& a) {
 }
 }  // namespace
 
+bool GemmF8TakesSecond(const GemmF8Args& a) {
+  return !a.out_f8 && a.N2 % 4 == 0 && a.ldw2 % 16 == 0 && a.ldc2 % 4 == 0 && SecondFits(PickGemmF8Variant(a), a.M, a.N, a.N2);
+}
+
 const char* GemmF8VariantName(const GemmF8Args& a) {
   switch (PickGemmF8Variant(a)) {
     case kDma256x256: return "gemm_f8_256x256x128";
@@ -564,6 +597,7 @@ const char* GemmF8VariantName(const GemmF8Args& a) {
 
 void LaunchGemmF8(const GemmF8Args& a, hipStream_t stream) {
   if (a.M <= 0 || a.N <= 0) return;
+  if (a.N2 > 0 && !GemmF8TakesSecond(a)) throw std::runtime_error("LaunchGemmF8: no kernel with a second product for this shape");
   const GemmVariant v = PickGemmF8Variant(a);
   if (v == kRowPanel) LaunchGemmF8RowPanel(a, stream);
   else LaunchGemmDmaF8(v, a, stream);

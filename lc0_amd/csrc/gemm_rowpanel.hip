@@ -37,10 +37,13 @@ __global__ __launch_bounds__(64 * KS) void gemm_rowpanel_kernel(Args p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int m0 = blockIdx.x * ROWS, n0 = blockIdx.y * COLS;
-  const int M = p.M, N = p.N;
+  // Panels past the columns of the first product belong to the second one.
+  const int panels = (p.N + COLS - 1) / COLS;
+  const bool second = (int)blockIdx.y >= panels;
+  const int m0 = blockIdx.x * ROWS, n0 = (second ? blockIdx.y - panels : blockIdx.y) * COLS;
+  const int M = p.M, N = second ? p.N2 : p.N, ldw = second ? p.ldw2 : p.ldw;
   const char* A = reinterpret_cast<const char*>(p.A) + (long long)m0 * p.lda * ES;
-  const char* W = reinterpret_cast<const char*>(p.W) + (long long)n0 * p.ldw * ES;
+  const char* W = (second ? reinterpret_cast<const char*>(p.W2) : reinterpret_cast<const char*>(p.W)) + (long long)n0 * ldw * ES;
   if constexpr (!F8) {
     A += (long long)blockIdx.z * p.strideA * ES;
     W += (long long)blockIdx.z * p.strideW * ES;
@@ -49,7 +52,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_rowpanel_kernel(Args p) {
 #pragma unroll
   for (int t = 0; t < RT; t++) ta[t].Set(16 * t, M - m0, ES * p.lda);
 #pragma unroll
-  for (int c = 0; c < CT; c++) tw[c].Set(16 * c, N - n0, ES * p.ldw);
+  for (int c = 0; c < CT; c++) tw[c].Set(16 * c, N - n0, ES * ldw);
   floatx4 acc[RT][CT];
 #pragma unroll
   for (int t = 0; t < RT; t++)
@@ -66,6 +69,24 @@ __global__ __launch_bounds__(64 * KS) void gemm_rowpanel_kernel(Args p) {
     for (int c = 0; c < CT; c++)
       *reinterpret_cast<floatx4*>(&part[ks][(16 * t + r) * LD + 16 * c + 4 * g]) = acc[t][c];
   __syncthreads();
+  if (second) {   // (an epilogue of its own: neither bias nor activation, and e4m3 output with e4m3 operands)
+#pragma unroll
+    for (int i = 0; i < (ROWS * COLS + NT - 1) / NT; i++) {
+      const int idx = tid + NT * i, row = idx / COLS, col = idx % COLS;
+      const int m = m0 + row, n = n0 + col;
+      if (row >= ROWS || m >= M || n >= N) continue;
+      float sum = part[0][row * LD + col];
+#pragma unroll
+      for (int w = 1; w < KS; w++) sum += part[w][row * LD + col];
+      if constexpr (F8) {
+        reinterpret_cast<uint8_t*>(p.C2)[(long long)m * p.ldc2 + n] =
+            (uint8_t)(PackFp8x4(sum * p.col_scale2[n] * p.out_mul2, 0.0f, 0.0f, 0.0f) & 0xFFu);
+      } else if constexpr (sizeof(OutT) == 2) {
+        reinterpret_cast<OutT*>(p.C2)[(long long)m * p.ldc2 + n] = (OutT)sum;
+      }
+    }
+    return;
+  }
   OutT* C = reinterpret_cast<OutT*>(p.C);
   if constexpr (!F8) C += (long long)blockIdx.z * p.strideC;
   DispatchAct(p.act, [&](auto act_fn) {
@@ -109,7 +130,7 @@ void LaunchPanel(const Args& a, int batch, hipStream_t stream) {
   const RowPanelShape s = PickRowPanelShape(a.M, a.N, batch);
   auto launch = [&](auto rt_tag, auto ct_tag) {
     constexpr int RT = decltype(rt_tag)::value, CT = decltype(ct_tag)::value, KS = kPanelWaves<ET>;
-    dim3 grid((a.M + 16 * RT - 1) / (16 * RT), (a.N + 16 * CT - 1) / (16 * CT), batch);
+    dim3 grid((a.M + 16 * RT - 1) / (16 * RT), (a.N + 16 * CT - 1) / (16 * CT) + (a.N2 + 16 * CT - 1) / (16 * CT), batch);
     hipLaunchKernelGGL((gemm_rowpanel_kernel<ET, RT, CT, KS, OutT, Args>), grid, dim3(64 * KS), 0, stream, a);
   };
   using One = std::integral_constant<int, 1>;

@@ -670,6 +670,43 @@ int lc0mi_k_norm_gemm(int f8, const uint16_t* A, const void* W, const float* bia
   });
 }
 
+int lc0mi_k_gemm_second(int f8, const void* A, const void* W, const void* W2, const float* bias, const float* col_scale,
+                        const float* col_scale2, float out_mul2, int M, int N, int N2, int K, uint16_t* C, void* C2) {
+  return Guard([&] {
+    RequireDevice();
+    if (M < 1 || N < 1 || N2 < 1 || K < 8 || K % (f8 ? 128 : 8) || (f8 && (!col_scale || !col_scale2))) throw Error("bad gemm shape");
+    Dev dev;
+    const size_t es = f8 ? 1 : 2;
+    auto put = [&](const void* p, size_t rows) { return dev.Put(static_cast<const uint8_t*>(p), rows * K * es); };
+    uint8_t *dA = put(A, M), *dW = put(W, N), *dW2 = put(W2, N2);
+    void *dC = dev.Alloc((size_t)M * N * 2), *dC2 = dev.Alloc((size_t)M * N2 * es);
+    const float* db = bias ? dev.Put(bias, (size_t)N) : nullptr;
+    if (f8) {
+      lc0mi::GemmF8Args g;
+      g.A = dA; g.lda = K; g.W = dW; g.ldw = K; g.C = dC; g.ldc = N; g.bias = db;
+      g.col_scale = dev.Put(col_scale, (size_t)N);
+      g.M = M; g.N = N; g.K = K;
+      g.W2 = dW2; g.ldw2 = K; g.C2 = dC2; g.ldc2 = N2; g.N2 = N2;
+      g.col_scale2 = dev.Put(col_scale2, (size_t)N2);
+      g.out_mul2 = out_mul2;
+      if (!lc0mi::GemmF8TakesSecond(g)) throw Error("no kernel with a second product for this shape");
+      lc0mi::LaunchGemmF8(g, nullptr);
+    } else {
+      lc0mi::GemmArgs g;
+      g.A = reinterpret_cast<const half_t*>(dA); g.lda = K; g.W = reinterpret_cast<const half_t*>(dW); g.ldw = K;
+      g.C = dC; g.ldc = N; g.bias = db;
+      g.M = M; g.N = N; g.K = K; g.bf16 = g_bf16;
+      g.W2 = reinterpret_cast<const half_t*>(dW2); g.ldw2 = K; g.C2 = dC2; g.ldc2 = N2; g.N2 = N2;
+      if (!lc0mi::GemmTakesSecond(g)) throw Error("no kernel with a second product for this shape");
+      lc0mi::LaunchGemm(g, nullptr);
+    }
+    K_CHECK(hipDeviceSynchronize());
+    K_CHECK(hipGetLastError());
+    K_CHECK(hipMemcpy(C, dC, (size_t)M * N * 2, hipMemcpyDeviceToHost));
+    K_CHECK(hipMemcpy(C2, dC2, (size_t)M * N2 * es, hipMemcpyDeviceToHost));
+  });
+}
+
 int lc0mi_k_gemm_f8(const uint8_t* A, int lda, const uint8_t* W, int ldw, const float* col_scale, const float* bias,
                     int M, int N, int K, int act, int out_f8, float out_mul, void* C, int ldc, int time_iters,
                     double* ms) {

@@ -78,12 +78,21 @@ struct GemmArgs {
   float* stats_out = nullptr;
   int norm_n = 0;        // length of the normalised rows (consumer: K of the real problem; producer: N)
   float norm_eps = 0.0f;
+
+  // A second product of the same A in the same launch: C2[m][n] = sum_k A[m][k] W2[n][k] for n < N2 (16-bit output, no
+  // bias, activation or scale; N2, ldw2 and ldc2 multiples of 8). Only where GemmTakesSecond().
+  const half_t* W2 = nullptr; int ldw2 = 0;
+  void* C2 = nullptr; int ldc2 = 0;
+  int N2 = 0;
 };
 void LaunchGemm(const GemmArgs& args, hipStream_t stream);
 // Whether LaunchGemm serves the folded layer-norm fields of these arguments (the kernel variant it picks has the
 // epilogue), and the number of partial sums per row a producer launch writes to stats_out.
 bool GemmSupportsNormFolding(const GemmArgs& args);
 int GemmStatsParts(const GemmArgs& args);
+// Whether LaunchGemm serves a second product of N2 columns: the kernel it picks for the first one is for few rows, and
+// the workgroups of both fit the CUs with one each.
+bool GemmTakesSecond(const GemmArgs& args);
 // Name of the kernel variant LaunchGemm picks for these arguments (tile shape; "...+rest" when it cuts the product
 // along its rows into whole rounds of large tiles and a rest, GemmRowSplit() rows in the first launch).
 const char* GemmVariantName(const GemmArgs& args);
@@ -105,7 +114,15 @@ struct GemmF8Args {
   bool out_f8 = false;
   float out_mul = 1.0f;
   int out_stores = kStoresAuto;
+  // A second product of the same A, as in GemmArgs, with e4m3 output: C2 = e4m3(col_scale2[n] * sum * out_mul2). N2, ldc2
+  // multiples of 4. Only with half output of the first product and where GemmF8TakesSecond().
+  const uint8_t* W2 = nullptr; int ldw2 = 0;
+  void* C2 = nullptr; int ldc2 = 0;
+  int N2 = 0;
+  const float* col_scale2 = nullptr;
+  float out_mul2 = 1.0f;
 };
+bool GemmF8TakesSecond(const GemmF8Args& args);
 void LaunchGemmF8(const GemmF8Args& args, hipStream_t stream);
 const char* GemmF8VariantName(const GemmF8Args& args);
 

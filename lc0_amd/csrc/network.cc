@@ -143,6 +143,17 @@ struct NormFold {
   float eps = 0.0f;
 };
 
+// A second layer that reads the rows of a GEMM launch and may share it (GemmArgs::W2): the smolgen compression beside Q/K/V.
+struct Linear;
+struct LinearF8;
+// With one given, nothing is launched unless the launch takes both.
+struct SecondProduct {
+  const Linear* lin = nullptr;
+  const LinearF8* f8 = nullptr;
+  void* C = nullptr;
+  float out_mul = 1.0f;
+};
+
 int RoundUp(int v, int m) { return (v + m - 1) / m * m; }
 
 // Residual-tower device weights (element type chosen by the precision option).
@@ -294,6 +305,7 @@ struct ModelState {
   int fused_smolgen_min_batch_ = 72;
   int dense1_split_min_batch_ = 112;   // smallest batch whose smolgen dense1 splits K between workgroups
   int dense2_norm_max_batch_ = 64, generator_norm_max_batch_ = 48;   // largest batches whose row norms run inside the layer after them
+  bool compress_with_qkv_ = true;
   bool qkv_first_ = true;
   bool write_through_ = true;   // big activations go to the memory-side cache while a layer's worth fits it
   int chain_latency_max_batch_ = 128;   // largest fp16 batch whose smolgen chain takes the shortest-latency GEMM variants
@@ -403,8 +415,9 @@ class Mi355xNetwork : public Network, protected ModelState {
   Linear MakeLinear(const Vec& w, const Vec& b, int out, int in, int pad_to = 8);
   Linear MakeLinearNormFolded(const Vec& w, const Vec& b, const Vec& gamma, const Vec& beta, int out, int in);
   LinearF8 MakeLinearF8(const Vec& w, int out, int in);
-  void GemmF8(const char* name, const uint8_t* A, const Linear& lin, const LinearF8& q, void* C, int M, int act,
-              bool out_f8, float out_mul, hipStream_t st = nullptr, int out_stores = kStoresAuto);
+  bool GemmF8(const char* name, const uint8_t* A, const Linear& lin, const LinearF8& q, void* C, int M, int act,
+              bool out_f8, float out_mul, hipStream_t st = nullptr, int out_stores = kStoresAuto,
+              const SecondProduct& second = {});
   void RecordAbsMax(const half_t* x, size_t n, int slot, hipStream_t st = nullptr);
   // Slot of the calibration maxima: 4 per layer plus the last layer's output, then 3 per layer for the smolgen chain.
   int SmolgenSlot(size_t li, int which) const { return static_cast<int>(4 * encoders_.size() + 1 + 3 * li + which); }
@@ -433,9 +446,9 @@ class Mi355xNetwork : public Network, protected ModelState {
   // Launch helpers (profiling aware).
   template <typename F>
   void Timed(const char* name, double flops, double bytes, F&& launch, hipStream_t st = nullptr);
-  void Gemm(const char* name, const half_t* A, int lda, const Linear& lin, void* C, int ldc, int M, int act,
+  bool Gemm(const char* name, const half_t* A, int lda, const Linear& lin, void* C, int ldc, int M, int act,
             bool out_f32 = false, hipStream_t st = nullptr, int split_k = 1, bool latency_first = false,
-            const NormFold* fold = nullptr, int out_stores = kStoresAuto);
+            const NormFold* fold = nullptr, int out_stores = kStoresAuto, const SecondProduct& second = {});
   GemmArgs MakeGemmArgs(const half_t* A, int lda, const Linear& lin, void* C, int ldc, int M, int act, bool out_f32,
                         int split_k, bool latency_first, const NormFold* fold) const;
   // Kernels other than the dense layers, by the network's element type (and, for 16-bit types, by whether the tuned
@@ -668,12 +681,13 @@ GemmArgs Mi355xNetwork::MakeGemmArgs(const half_t* A, int lda, const Linear& lin
   return g;
 }
 
-void Mi355xNetwork::Gemm(const char* name, const half_t* A, int lda, const Linear& lin, void* C, int ldc, int M,
+bool Mi355xNetwork::Gemm(const char* name, const half_t* A, int lda, const Linear& lin, void* C, int ldc, int M,
                          int act, bool out_f32, hipStream_t st, int split_k, bool latency_first,
-                         const NormFold* fold, int out_stores) {
+                         const NormFold* fold, int out_stores, const SecondProduct& second) {
   if (st == nullptr) st = stream_;
   if (dtype_ == Dtype::kFloat) {
     if (split_k != 1 || fold != nullptr) throw Error("internal: split or folded GEMM requested in the float configuration");
+    if (second.lin != nullptr) return false;
     GemmArgsF32 g;
     g.A = reinterpret_cast<const float*>(A); g.lda = lda;
     g.W = reinterpret_cast<const float*>(lin.w); g.ldw = lin.ld;
@@ -685,19 +699,27 @@ void Mi355xNetwork::Gemm(const char* name, const half_t* A, int lda, const Linea
     Timed(label.c_str(), 2.0 * M * lin.out * lin.in,
           4.0 * (static_cast<double>(M) * lin.in + static_cast<double>(lin.out) * lin.in + static_cast<double>(M) * lin.out),
           [&] { LaunchGemmF32(g, st); }, st);
-    return;
+    return false;
   }
   GemmArgs g = MakeGemmArgs(A, lda, lin, C, ldc, M, act, out_f32, split_k, latency_first, fold);
   g.bf16 = dtype_ == Dtype::kBf16;
   g.out_stores = out_stores;
+  if (second.lin != nullptr) {
+    g.W2 = second.lin->w; g.ldw2 = second.lin->ld;
+    g.C2 = second.C; g.ldc2 = second.lin->out;
+    g.N2 = second.lin->out;
+    if (!GemmTakesSecond(g)) return false;
+  }
   if (fold != nullptr && fold->parts_out != nullptr) *fold->parts_out = GemmStatsParts(g);
-  const double flops = 2.0 * M * lin.out * lin.in;
+  const double flops = 2.0 * M * (lin.out + g.N2) * lin.in;
   const double bytes = 2.0 * (static_cast<double>(M) * lin.in + static_cast<double>(lin.out) * lin.in) +
                        static_cast<double>(M) * lin.out * (out_f32 ? 4 : 2) +
                        (fold != nullptr && fold->skip != nullptr ? 2.0 * M * lin.out : 0.0);
   std::string label = std::string(name) + "|" + GemmVariantName(g);
   if (fold != nullptr) label += fold->skip != nullptr ? "+skip_stats" : "+row_norm";
+  if (g.N2 > 0) label += "+second";
   Timed(label.c_str(), flops, bytes, [&] { LaunchGemm(g, st); }, st);
+  return g.N2 > 0;
 }
 
 // A dense layer of the smolgen chain with the norm of its input rows (`group` of them together) in the same kernel.
@@ -845,8 +867,9 @@ LinearF8 Mi355xNetwork::MakeLinearF8(const Vec& w, int out, int in) {
   return q;
 }
 
-void Mi355xNetwork::GemmF8(const char* name, const uint8_t* A, const Linear& lin, const LinearF8& q, void* C, int M,
-                           int act, bool out_f8, float out_mul, hipStream_t st, int out_stores) {
+bool Mi355xNetwork::GemmF8(const char* name, const uint8_t* A, const Linear& lin, const LinearF8& q, void* C, int M,
+                           int act, bool out_f8, float out_mul, hipStream_t st, int out_stores,
+                           const SecondProduct& second) {
   if (st == nullptr) st = stream_;
   GemmF8Args g;
   g.A = A; g.lda = lin.in;
@@ -859,11 +882,20 @@ void Mi355xNetwork::GemmF8(const char* name, const uint8_t* A, const Linear& lin
   g.out_f8 = out_f8;
   g.out_mul = out_mul;
   g.out_stores = out_stores;
-  const double flops = 2.0 * M * lin.out * lin.in;
+  if (second.lin != nullptr) {
+    g.W2 = second.f8->w; g.ldw2 = second.lin->in;
+    g.col_scale2 = second.f8->col_scale;
+    g.C2 = second.C; g.ldc2 = second.lin->out;
+    g.N2 = second.lin->out;
+    g.out_mul2 = second.out_mul;
+    if (!GemmF8TakesSecond(g)) return false;
+  }
+  const double flops = 2.0 * M * (lin.out + g.N2) * lin.in;
   const double bytes = static_cast<double>(M) * lin.in + static_cast<double>(lin.out) * lin.in +
                        static_cast<double>(M) * lin.out * (out_f8 ? 1 : 2);
-  const std::string label = std::string(name) + "|" + GemmF8VariantName(g);
+  const std::string label = std::string(name) + "|" + GemmF8VariantName(g) + (g.N2 > 0 ? "+second" : "");
   Timed(label.c_str(), flops, bytes, [&] { LaunchGemmF8(g, st); }, st);
+  return g.N2 > 0;
 }
 
 void Mi355xNetwork::RecordAbsMax(const half_t* x, size_t n, int slot, hipStream_t st) {
@@ -1071,6 +1103,7 @@ Mi355xNetwork::Mi355xNetwork(const WeightsFile& file, Options& options) {
   fused_smolgen_attention_ = options.GetBool("fused_smolgen_attention", true);
   fused_smolgen_min_batch_ = options.GetInt("fused_smolgen_min_batch", 72);
   dense1_split_min_batch_ = options.GetInt("dense1_split_min_batch", 112);
+  compress_with_qkv_ = options.GetBool("compress_with_qkv", true);
   dense2_norm_max_batch_ = options.GetInt("dense2_norm_max_batch", 64);
   generator_norm_max_batch_ = options.GetInt("generator_norm_max_batch", 48);
   qkv_first_ = options.GetBool("qkv_first", true);
@@ -1954,14 +1987,27 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
     // plus the plain attention kernel. An explicit fp8_gemms=...+smolgen keeps all four layers in e4m3.
     const bool fused_gen = e.has_smolgen && smolgen_wfrag_ != nullptr && B >= fused_smolgen_min_batch_ &&
                            (!chain_f8 || q_smolgen_auto_);
-    auto launch_qkv = [&] {
+    auto launch_qkv = [&](const SecondProduct& second = {}) {
       if (f8 && q_qkv_) {
-        GemmF8("gemm_qkv", xq_, e.qkv, e.qkv8, qkv_, T, kActNone, false, 1.0f, nullptr, keep);
-      } else {
-        Gemm("gemm_qkv", x_, emb_, norm_in ? e.qkv_n : e.qkv, qkv_, 3 * d_model_, T, kActNone, false, nullptr, 1, false,
-             norm_in ? &cons_in : nullptr, keep);
+        return GemmF8("gemm_qkv", xq_, e.qkv, e.qkv8, qkv_, T, kActNone, false, 1.0f, nullptr, keep, second);
       }
+      return Gemm("gemm_qkv", x_, emb_, norm_in ? e.qkv_n : e.qkv, qkv_, 3 * d_model_, T, kActNone, false, nullptr, 1, false,
+                  norm_in ? &cons_in : nullptr, keep, second);
     };
+    // On one stream, the smolgen compression (a few columns of the same rows) is a second product of the projection's
+    // launch where its workgroups find free CUs (GemmTakesSecond): one launch less in a chain of dependent ones. us of a
+    // 15x1024 pass, own launch -> with the projection: fp16 1 position 923 -> 833, 13 1296 -> 1230, 21 1574 -> 1502, 48 2219 ->
+    // 2136; e4m3 1 791 -> 729, 16 979 -> 929, 48 1545 -> 1486. (Not when profiling: every layer then has a launch and a time of
+    // its own.)
+    bool with_compress = false;
+    if (e.has_smolgen && ss == stream_ && compress_with_qkv_ && !profiling_ && !norm_in && !calibrating_ && chain_f8 == (f8 && q_qkv_)) {
+      SecondProduct compress;
+      compress.lin = &e.sg_compress;
+      compress.f8 = &e.sg_compress8;
+      compress.C = chain_f8 ? static_cast<void*>(sg1q_) : sg1_;
+      compress.out_mul = 1.0f / e.s_sg1;
+      with_compress = launch_qkv(compress);
+    }
     // With two streams the projection is recorded before the chain: a replayed graph then keeps it on the hardware
     // queue of the layer norm before it and of the attention after it, and only the chain, which has slack, pays the
     // dependencies between queues.
@@ -1990,7 +2036,9 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       if (chain_f8) {
         // The whole chain on e4m3 operands: the compression reads the e4m3 copy of x that the QKV projection reads
         // and writes e4m3 itself; the two row norms write halves and their e4m3 copies.
-        GemmF8("gemm_smolgen_compress", xq_, e.sg_compress, e.sg_compress8, sg1q_, T, kActNone, true, 1.0f / e.s_sg1, ss);
+        if (!with_compress) {
+          GemmF8("gemm_smolgen_compress", xq_, e.sg_compress, e.sg_compress8, sg1q_, T, kActNone, true, 1.0f / e.s_sg1, ss);
+        }
         GemmF8("gemm_smolgen_dense1", sg1q_, e.sg_dense1, e.sg_dense18, sg2_, B, smolgen_act_, false, 1.0f, ss);
         if (norm_dense2) {
           NormGemm("gemm_smolgen_dense2", sg2_, e.sg_dense2, &e.sg_dense28, 1.0f / e.s_sg2, e.sg_ln1_g, e.sg_ln1_b, 1, sg3_, B,
@@ -2017,8 +2065,10 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       } else if (dtype_ == Dtype::kFloat) {
         SmolgenChain(e, x_, emb_, heads_, sg_hc_, sg_hs_, sg_gen_, sg1_, sg2_, sg3_, sbias_, B, ss, chain_first);
       } else {
-      Gemm("gemm_smolgen_compress", x_, emb_, norm_in ? e.sg_compress_n : e.sg_compress, sg1_, sg_hc_, T, kActNone,
-           false, ss, 1, chain_first, norm_in ? &cons_in : nullptr);
+      if (!with_compress) {
+        Gemm("gemm_smolgen_compress", x_, emb_, norm_in ? e.sg_compress_n : e.sg_compress, sg1_, sg_hc_, T, kActNone,
+             false, ss, 1, chain_first, norm_in ? &cons_in : nullptr);
+      }
       // dense1 has a long reduction and few outputs. With few rows one workgroup per 16x16 outputs splits K over
       // its waves; from dense1_split_min_batch_ rows on, workgroups split K between them, accumulate in float, and
       // the layer norm kernel adds the slices and applies the activation.
@@ -2065,7 +2115,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       if (ss != stream_) HIP_CHECK(hipEventRecord(join_events_[li], ss));
       bias = sbias_;
     }
-    if (!qkv_before_chain) launch_qkv();
+    if (!qkv_before_chain && !with_compress) launch_qkv();
     if (e.has_smolgen && ss != stream_) HIP_CHECK(hipStreamWaitEvent(stream_, join_events_[li], 0));
     const int gen_sz = e.has_smolgen ? sg_gen_ / heads_ : 0;
     const double att_flops = 4.0 * 64 * 64 * depth_ * B * heads_ + (fused_gen ? 2.0 * 4096 * gen_sz * B * heads_ : 0.0);

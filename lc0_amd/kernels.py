@@ -39,6 +39,7 @@ def _lib():
         lib.lc0mi_k_attn_policy_gather.argtypes = [vp, vp, vp, ci, ci, vp]
         lib.lc0mi_k_gemm_f8.argtypes = [vp, ci, vp, ci, vp, vp, ci, ci, ci, ci, ci, cf, vp, ci, ci, cd]
         lib.lc0mi_k_norm_gemm.argtypes = [ci] + [vp] * 6 + [ci] * 4 + [cf, cf, ci, vp, ci, cd]
+        lib.lc0mi_k_gemm_second.argtypes = [ci] + [vp] * 6 + [cf] + [ci] * 4 + [vp, vp]
         lib.lc0mi_k_quantize_f8.argtypes = [vp, ll, cf, vp]
         lib.lc0mi_k_layer_norm_f8.argtypes = [vp, vp, vp, vp, ci, ci, cf, cf, cf, vp, vp]
         lib.lc0mi_k_attention_f8.argtypes = [vp, vp, ci, ci, cf, cf, vp]
@@ -320,6 +321,19 @@ def norm_gemm(a, w, gamma, beta, group=1, bias=None, eps=1e-3, act=ACT_NONE, col
     _check(_lib().lc0mi_k_norm_gemm(int(f8), _ptr(a), _ptr(w), _ptr(b), _ptr(cs), _ptr(gamma), _ptr(beta), group, m, n, k,
                                     C.c_float(eps), C.c_float(in_mul), act, _ptr(out), time_iters, C.byref(ms)))
     return (_ret16(out), ms.value) if time_iters else _ret16(out)
+
+
+def gemm_second(a, w, w2, bias=None, col_scale=None, col_scale2=None, out_mul2=1.0):
+    """(a.w^T + bias, a.w2^T) in one launch; with col_scale on e4m3 bytes: (col_scale * a.w^T + bias as half, e4m3 bytes of
+    col_scale2 * a.w2^T * out_mul2)."""
+    f8 = col_scale is not None
+    a, w, w2 = (np.ascontiguousarray(x, np.uint8) if f8 else _h(x) for x in (a, w, w2))
+    b, cs, cs2 = (np.ascontiguousarray(x, np.float32) if x is not None else None for x in (bias, col_scale, col_scale2))
+    (m, k), n, n2 = a.shape, w.shape[0], w2.shape[0]
+    out, out2 = _out16((m, n)), np.zeros((m, n2), np.uint8) if f8 else _out16((m, n2))
+    _check(_lib().lc0mi_k_gemm_second(int(f8), _ptr(a), _ptr(w), _ptr(w2), _ptr(b), _ptr(cs), _ptr(cs2), C.c_float(out_mul2),
+                                      m, n, n2, k, _ptr(out), _ptr(out2)))
+    return _ret16(out), _ret16(out2)
 
 
 def quantize_f8(x, mul=1.0):
