@@ -145,6 +145,18 @@ int lc0mi_k_gemm_f8(const uint8_t* A, int lda, const uint8_t* W, int ldw, const 
 int lc0mi_k_norm_gemm(int f8, const uint16_t* A, const void* W, const float* bias, const float* col_scale,
                       const float* gamma, const float* beta, int group, int M, int N, int K, float eps, float in_mul, int act,
                       uint16_t* C, int time_iters, double* ms);
+/* Q/K/V projection and attention of heads of depth 32 in one kernel (emb 128 or 256, an even number of heads, no smolgen):
+ * x [batch * 64][emb], W [3 * 32 heads][emb] (Q, K, V), bias [3 * 32 heads] or NULL, out [batch * 64][32 heads]; 16-bit.
+ * Counterpart: src/neural/backends/blas/network_blas.cc:352-439. */
+int lc0mi_k_qkv_attention(const uint16_t* x, const uint16_t* W, const float* bias, int batch, int emb, int heads, float scale,
+                          uint16_t* out, int time_iters, double* ms);
+/* The rest of an encoder layer in one kernel (emb 128 or 256; d_model and dff multiples of emb; M a multiple of 64):
+ * u = LN1(alpha (att.dense^T + b) + x), x = LN2(alpha (act(u.ffn1^T + b).ffn2^T + b) + u), in place. biases: dense, ffn1 and
+ * ffn2 one after the other, or NULL; norms: gamma, beta of the first, then of the second. After time_iters runs the
+ * device's x is no longer what is returned. Counterpart: network_blas.cc:441-486, blas/encoder.h:29-66. */
+int lc0mi_k_encoder_tail(const uint16_t* att, uint16_t* x, const uint16_t* dense, const uint16_t* ffn1, const uint16_t* ffn2,
+                         const float* biases, const float* norms, int M, int emb, int d_model, int dff, float alpha, float eps,
+                         int act, int time_iters, double* ms);
 /* Two products of the same rows in one launch: C as lc0mi_k_gemm (batch 1, 16-bit output, act none) or, with f8 != 0, as
  * lc0mi_k_gemm_f8 (half output), and C2 = A.W2^T without bias (16-bit), or e4m3(col_scale2[n] * sum * out_mul2) bytes.
  * A [M][K], W [N][K], W2 [N2][K]. Fails where the kernel of the first product does not serve a second one. Counterpart:

@@ -670,6 +670,64 @@ int lc0mi_k_norm_gemm(int f8, const uint16_t* A, const void* W, const float* bia
   });
 }
 
+int lc0mi_k_qkv_attention(const uint16_t* x, const uint16_t* W, const float* bias, int batch, int emb, int heads, float scale,
+                          uint16_t* out, int time_iters, double* ms) {
+  return Guard([&] {
+    RequireDevice();
+    if (batch < 1 || batch > 65535 || !lc0mi::QkvAttentionSupported(emb, heads, 32)) throw Error("bad shape");
+    const int d_model = 32 * heads;
+    Dev dev;
+    std::vector<uint16_t> packed((size_t)3 * d_model * emb);
+    for (int o = 0; o < 3 * d_model; o++)
+      for (int i = 0; i < emb; i++) packed[lc0mi::QkvFragmentIndex(o, i, emb, d_model)] = W[(size_t)o * emb + i];
+    lc0mi::QkvAttentionArgs a;
+    a.x = reinterpret_cast<const half_t*>(dev.Put(x, (size_t)batch * 64 * emb));
+    a.packed = reinterpret_cast<const half_t*>(dev.Put(packed.data(), packed.size()));
+    a.bias = bias ? dev.Put(bias, (size_t)3 * d_model) : nullptr;
+    a.out = reinterpret_cast<half_t*>(dev.Put(out, (size_t)batch * 64 * d_model));
+    a.batch = batch; a.emb = emb; a.heads = heads; a.scale = scale; a.bf16 = g_bf16;
+    lc0mi::LaunchQkvAttention(a, nullptr);
+    K_CHECK(hipDeviceSynchronize());
+    K_CHECK(hipGetLastError());
+    K_CHECK(hipMemcpy(out, a.out, (size_t)batch * 64 * d_model * 2, hipMemcpyDeviceToHost));
+    if (time_iters > 0 && ms) *ms = TimeLaunches(time_iters, [&] { lc0mi::LaunchQkvAttention(a, nullptr); });
+  });
+}
+
+int lc0mi_k_encoder_tail(const uint16_t* att, uint16_t* x, const uint16_t* dense, const uint16_t* ffn1, const uint16_t* ffn2,
+                         const float* biases, const float* norms, int M, int emb, int d_model, int dff, float alpha, float eps,
+                         int act, int time_iters, double* ms) {
+  return Guard([&] {
+    RequireDevice();
+    if (M < 64 || M % 64 || !lc0mi::EncoderTailSupported(emb, d_model, dff)) throw Error("bad shape");
+    Dev dev;
+    std::vector<uint16_t> packed((size_t)emb * (d_model + 2 * dff));
+    auto pack = [&](int layer, const uint16_t* m, int out, int in) {
+      for (int o = 0; o < out; o++)
+        for (int i = 0; i < in; i++) packed[lc0mi::EncoderTailFragmentIndex(layer, o, i, emb, d_model)] = m[(size_t)o * in + i];
+    };
+    pack(0, dense, emb, d_model);
+    pack(1, ffn1, dff, emb);
+    pack(2, ffn2, emb, dff);
+    lc0mi::EncoderTailArgs a;
+    a.att = reinterpret_cast<const half_t*>(dev.Put(att, (size_t)M * d_model));
+    a.packed = reinterpret_cast<const half_t*>(dev.Put(packed.data(), packed.size()));
+    a.x = reinterpret_cast<half_t*>(dev.Put(x, (size_t)M * emb));
+    if (biases) {
+      const float* b = dev.Put(biases, (size_t)2 * emb + dff);
+      a.dense_b = b; a.ffn1_b = b + emb; a.ffn2_b = b + emb + dff;
+    }
+    const float* n = dev.Put(norms, (size_t)4 * emb);
+    a.ln1_g = n; a.ln1_b = n + emb; a.ln2_g = n + 2 * emb; a.ln2_b = n + 3 * emb;
+    a.M = M; a.emb = emb; a.d_model = d_model; a.dff = dff; a.alpha = alpha; a.eps = eps; a.act = act; a.bf16 = g_bf16;
+    lc0mi::LaunchEncoderTail(a, nullptr);
+    K_CHECK(hipDeviceSynchronize());
+    K_CHECK(hipGetLastError());
+    K_CHECK(hipMemcpy(x, a.x, (size_t)M * emb * 2, hipMemcpyDeviceToHost));
+    if (time_iters > 0 && ms) *ms = TimeLaunches(time_iters, [&] { lc0mi::LaunchEncoderTail(a, nullptr); });
+  });
+}
+
 int lc0mi_k_gemm_second(int f8, const void* A, const void* W, const void* W2, const float* bias, const float* col_scale,
                         const float* col_scale2, float out_mul2, int M, int N, int N2, int K, uint16_t* C, void* C2) {
   return Guard([&] {

@@ -273,6 +273,42 @@ void LaunchSmolgenAttentionF8Out(const half_t* qkv, const half_t* gen, const hal
                                  float out_mul, int batch, int heads, int depth, int gen_sz, float scale,
                                  hipStream_t stream);
 
+// Encoder layers of narrow bodies in two kernels (encoder_narrow.hip), 16-bit types, 64 rows per position.
+//
+// out[b*64+i][h*32+d] = the attention of heads of depth 32 over x.W^T + bias (W, bias: the rows of Q, K and V one after the
+// other, [3 d_model][emb] with d_model = 32 heads; bias may be null), without smolgen logits. packed: W with element
+// (row, col) at QkvFragmentIndex.
+struct QkvAttentionArgs {
+  const half_t *x = nullptr, *packed = nullptr;
+  const float* bias = nullptr;
+  half_t* out = nullptr;
+  int batch = 0, emb = 0, heads = 0;
+  float scale = 1.0f;
+  bool bf16 = false;
+};
+bool QkvAttentionSupported(int emb, int heads, int depth);
+long long QkvFragmentIndex(int row, int col, int emb, int d_model);
+void LaunchQkvAttention(const QkvAttentionArgs& args, hipStream_t stream);
+
+// u = LN1(alpha (att.dense^T + dense_b) + x), x <- LN2(alpha (act(u.ffn1^T + ffn1_b).ffn2^T + ffn2_b) + u) for M rows
+// (a multiple of 64): x [M][emb], att [M][d_model], biases may be null, u is rounded to 16 bits. packed: the three weight
+// matrices, element (row, col) of dense (layer 0: [emb][d_model]), ffn1 (1: [dff][emb]) and ffn2 (2: [emb][dff]) at
+// EncoderTailFragmentIndex.
+struct EncoderTailArgs {
+  const half_t *att = nullptr, *packed = nullptr;
+  half_t* x = nullptr;
+  const float *dense_b = nullptr, *ffn1_b = nullptr, *ffn2_b = nullptr;
+  const float *ln1_g = nullptr, *ln1_b = nullptr, *ln2_g = nullptr, *ln2_b = nullptr;
+  int M = 0, emb = 0, d_model = 0, dff = 0;
+  float alpha = 1.0f, eps = 1e-6f;
+  int act = 3;
+  bool bf16 = false;
+};
+bool EncoderTailSupported(int emb, int d_model, int dff);
+int EncoderTailRows(int M);   // rows of a workgroup
+long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_model);
+void LaunchEncoderTail(const EncoderTailArgs& args, hipStream_t stream);
+
 // Attention policy tail: promotion offsets + gather to 1858 moves.
 // logits: [B][64*64] float (already scaled), kq: [B*64][ld_kq] with keys at column
 // offset key_off, ppo: [4][pd] float, inv_map: [1858] source index into the

@@ -202,6 +202,8 @@ struct EncoderDev {
   // ffn1: this layer's first norm), and the biases of the two layers before a norm times the DeepNorm alpha.
   Linear qkv_n, sg_compress_n, ffn1_n;
   float *dense_ab = nullptr, *ffn2_ab = nullptr;
+  // Weights in the orders of the two kernels of narrow bodies (null: the general path).
+  half_t *qkv_packed = nullptr, *tail_packed = nullptr;
 };
 
 // Pinned host staging of one batch (inputs and outputs).
@@ -306,6 +308,7 @@ struct ModelState {
   int dense1_split_min_batch_ = 112;   // smallest batch whose smolgen dense1 splits K between workgroups
   int dense2_norm_max_batch_ = 64, generator_norm_max_batch_ = 48;   // largest batches whose row norms run inside the layer after them
   bool compress_with_qkv_ = true;
+  bool narrow_layers_ = true;   // the two kernels of narrow bodies
   bool qkv_first_ = true;
   bool write_through_ = true;   // big activations go to the memory-side cache while a layer's worth fits it
   int chain_latency_max_batch_ = 128;   // largest fp16 batch whose smolgen chain takes the shortest-latency GEMM variants
@@ -1104,6 +1107,7 @@ Mi355xNetwork::Mi355xNetwork(const WeightsFile& file, Options& options) {
   fused_smolgen_min_batch_ = options.GetInt("fused_smolgen_min_batch", 72);
   dense1_split_min_batch_ = options.GetInt("dense1_split_min_batch", 112);
   compress_with_qkv_ = options.GetBool("compress_with_qkv", true);
+  narrow_layers_ = options.GetBool("narrow_layers", true);
   dense2_norm_max_batch_ = options.GetInt("dense2_norm_max_batch", 64);
   generator_norm_max_batch_ = options.GetInt("generator_norm_max_batch", 48);
   qkv_first_ = options.GetBool("qkv_first", true);
@@ -1586,6 +1590,25 @@ void Mi355xNetwork::BuildAttentionBody(const WeightsFile& file) {
       ab = l.ffn.dense2_b;
       for (float& v : ab) v *= alpha_;
       e.ffn2_ab = UploadF(ab);
+    }
+    if (narrow_layers_ && !fold_layer_norm_ && !fp8_ && dtype_ != Dtype::kFloat) {
+      if (!e.has_smolgen && QkvAttentionSupported(emb_, heads_, depth_)) {
+        Vec packed(qkv_w.size());
+        for (int o = 0; o < 3 * d_model_; o++)
+          for (int i = 0; i < emb_; i++) packed[QkvFragmentIndex(o, i, emb_, d_model_)] = qkv_w[static_cast<size_t>(o) * emb_ + i];
+        e.qkv_packed = UploadElems(packed);
+      }
+      if (EncoderTailSupported(emb_, d_model_, dff_)) {
+        Vec packed(l.mha.dense_w.size() + l.ffn.dense1_w.size() + l.ffn.dense2_w.size());
+        auto pack = [&](int layer, const Vec& m, int out, int in) {
+          for (int o = 0; o < out; o++)
+            for (int i = 0; i < in; i++) packed[EncoderTailFragmentIndex(layer, o, i, emb_, d_model_)] = m[static_cast<size_t>(o) * in + i];
+        };
+        pack(0, l.mha.dense_w, emb_, d_model_);
+        pack(1, l.ffn.dense1_w, dff_, emb_);
+        pack(2, l.ffn.dense2_w, emb_, dff_);
+        e.tail_packed = UploadElems(packed);
+      }
     }
     encoders_.push_back(e);
   }
@@ -2115,7 +2138,9 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       if (ss != stream_) HIP_CHECK(hipEventRecord(join_events_[li], ss));
       bias = sbias_;
     }
-    if (!qkv_before_chain && !with_compress) launch_qkv();
+    // Narrow bodies: projection and attention in one kernel, everything after them in another.
+    const bool qkv_attention = e.qkv_packed != nullptr;
+    if (!qkv_before_chain && !with_compress && !qkv_attention) launch_qkv();
     if (e.has_smolgen && ss != stream_) HIP_CHECK(hipStreamWaitEvent(stream_, join_events_[li], 0));
     const int gen_sz = e.has_smolgen ? sg_gen_ / heads_ : 0;
     const double att_flops = 4.0 * 64 * 64 * depth_ * B * heads_ + (fused_gen ? 2.0 * 4096 * gen_sz * B * heads_ : 0.0);
@@ -2135,12 +2160,29 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
             [&] { LaunchAttentionF8Out(qkv_, bias, attq_, 1.0f / e.s_att, B, heads_, att_scale, stream_, depth_); });
       GemmF8("gemm_mha_dense", attq_, e.dense, e.dense8, t_, T, kActNone, false, 1.0f, nullptr, keep);
     } else {
-      if (fused_gen) {
+      if (qkv_attention) {
+        QkvAttentionArgs a;
+        a.x = x_; a.packed = e.qkv_packed; a.bias = e.qkv.b; a.out = att_;
+        a.batch = B; a.emb = emb_; a.heads = heads_; a.scale = att_scale; a.bf16 = bf16;
+        Timed("qkv_attention", 6.0 * T * emb_ * d_model_ + att_flops, 2.0 * T * (emb_ + d_model_) + 6.0 * emb_ * d_model_,
+              [&] { LaunchQkvAttention(a, stream_); });
+      } else if (fused_gen) {
         Timed("smolgen_attention", att_flops, att_bytes, [&] {
           LaunchSmolgenAttention(qkv_, sg3_, smolgen_wfrag_, att_, B, heads_, depth_, gen_sz, att_scale, stream_, bf16);
         });
       } else {
         Timed("attention", att_flops, att_bytes, [&] { Attention(qkv_, bias, att_, B, heads_, depth_, stream_); });
+      }
+      if (e.tail_packed != nullptr) {
+        EncoderTailArgs a;
+        a.att = att_; a.packed = e.tail_packed; a.x = x_;
+        a.dense_b = e.dense.b; a.ffn1_b = e.ffn1.b; a.ffn2_b = e.ffn2.b;
+        a.ln1_g = e.ln1_g; a.ln1_b = e.ln1_b; a.ln2_g = e.ln2_g; a.ln2_b = e.ln2_b;
+        a.M = T; a.emb = emb_; a.d_model = d_model_; a.dff = dff_;
+        a.alpha = alpha_; a.eps = eps_; a.act = ffn_act_; a.bf16 = bf16;
+        const double weights = static_cast<double>(emb_) * (d_model_ + 2 * dff_);
+        Timed("encoder_tail", 2.0 * T * weights, 2.0 * (weights + T * (2.0 * emb_ + d_model_)), [&] { LaunchEncoderTail(a, stream_); });
+        continue;
       }
       if (calibrating_) RecordAbsMax(att_, static_cast<size_t>(T) * d_model_, static_cast<int>(4 * li + 1));
       if (fold) {

@@ -39,6 +39,8 @@ def _lib():
         lib.lc0mi_k_attn_policy_gather.argtypes = [vp, vp, vp, ci, ci, vp]
         lib.lc0mi_k_gemm_f8.argtypes = [vp, ci, vp, ci, vp, vp, ci, ci, ci, ci, ci, cf, vp, ci, ci, cd]
         lib.lc0mi_k_norm_gemm.argtypes = [ci] + [vp] * 6 + [ci] * 4 + [cf, cf, ci, vp, ci, cd]
+        lib.lc0mi_k_qkv_attention.argtypes = [vp] * 3 + [ci] * 3 + [cf, vp, ci, cd]
+        lib.lc0mi_k_encoder_tail.argtypes = [vp] * 7 + [ci] * 4 + [cf, cf, ci, ci, cd]
         lib.lc0mi_k_gemm_second.argtypes = [ci] + [vp] * 6 + [cf] + [ci] * 4 + [vp, vp]
         lib.lc0mi_k_quantize_f8.argtypes = [vp, ll, cf, vp]
         lib.lc0mi_k_layer_norm_f8.argtypes = [vp, vp, vp, vp, ci, ci, cf, cf, cf, vp, vp]
@@ -320,6 +322,30 @@ def norm_gemm(a, w, gamma, beta, group=1, bias=None, eps=1e-3, act=ACT_NONE, col
     out, ms = _out16((m, n)), C.c_double(0)
     _check(_lib().lc0mi_k_norm_gemm(int(f8), _ptr(a), _ptr(w), _ptr(b), _ptr(cs), _ptr(gamma), _ptr(beta), group, m, n, k,
                                     C.c_float(eps), C.c_float(in_mul), act, _ptr(out), time_iters, C.byref(ms)))
+    return (_ret16(out), ms.value) if time_iters else _ret16(out)
+
+
+def qkv_attention(x, w, heads, bias=None, scale=None, time_iters=0):
+    """Attention (heads of depth 32) over x.w^T + bias in one kernel; x [batch * 64][emb], w [3 * 32 heads][emb]."""
+    x, w = _h(x), _h(w)
+    (m, emb) = x.shape
+    b = np.ascontiguousarray(bias, np.float32) if bias is not None else None
+    out, ms = _out16((m, 32 * heads)), C.c_double(0)
+    _check(_lib().lc0mi_k_qkv_attention(_ptr(x), _ptr(w), _ptr(b), m // 64, emb, heads,
+                                        C.c_float(32 ** -0.5 if scale is None else scale), _ptr(out), time_iters, C.byref(ms)))
+    return (_ret16(out), ms.value) if time_iters else _ret16(out)
+
+
+def encoder_tail(att, x, dense, ffn1, ffn2, norms, biases=None, alpha=1.0, eps=1e-6, act=ACT_NONE, time_iters=0):
+    """Output projection, norm with skip x, FFN, norm with skip, in one kernel. biases: (dense, ffn1, ffn2); norms:
+    (gamma1, beta1, gamma2, beta2)."""
+    att, dense, ffn1, ffn2 = _h(att), _h(dense), _h(ffn1), _h(ffn2)
+    out, ms = _h(x).copy(), C.c_double(0)
+    (m, d_model), (dff, emb) = att.shape, ffn1.shape
+    b = np.concatenate(biases).astype(np.float32) if biases is not None else None
+    n = np.concatenate(norms).astype(np.float32)
+    _check(_lib().lc0mi_k_encoder_tail(_ptr(att), _ptr(out), _ptr(dense), _ptr(ffn1), _ptr(ffn2), _ptr(b), _ptr(n), m, emb, d_model,
+                                       dff, C.c_float(alpha), C.c_float(eps), act, time_iters, C.byref(ms)))
     return (_ret16(out), ms.value) if time_iters else _ret16(out)
 
 
