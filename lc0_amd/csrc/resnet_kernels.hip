@@ -12,6 +12,7 @@
 // instead of 16): the same convolution with 2.25x fewer multiplications.
 #include "kernels.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace lc0mi {
@@ -233,7 +234,7 @@ __device__ __forceinline__ void InputTile(const float (&d)[6][6], float (&r)[6][
 }
 
 // Same for C <= 256 with one thread per (tile, V neighbouring channels), blockDim.x == 4 * C / V.
-// Shared memory: part[4][C] | hidden[K] | fc2[4][2][C] floats | xs[64][C].
+// Shared memory: part[4][C] | hidden[K] | fc2[4][2][C] floats | xs[64][C]; with WIDTH xs[64][WIDTH].
 //
 // With few positions the chain of memory latencies bounds it (m, first squeeze-and-excitation layer, second one, skip):
 // the skip and the first four weights of either layer are asked for together with m (per launch, 32 positions x 64
@@ -245,10 +246,11 @@ __device__ __forceinline__ void InputTile(const float (&d)[6][6], float (&r)[6][
 // number of channels) wants the waves more than the early requests: without them (EARLY = false) it takes 61 registers
 // instead of 114 and eight waves per SIMD instead of four (a pass of a ten-block tower in halves, 1000 positions: 176 channels
 // 1854 -> 1630 us, 240 2590 -> 2310).
+// WIDTH > 0: no squeeze-and-excitation, and a workgroup takes WIDTH channels from blockIdx.y * WIDTH instead of all C.
 // The squeeze-and-excitation layers are spread over all threads: every wave pools the channels it needs itself, the
 // second layer is split four ways over k, and every thread adds the four partial sums of its own channels.
-template <typename T, typename MT, int V, bool EARLY>
-__global__ __launch_bounds__(1024 / V, EARLY ? 4 : 8) void winograd_output_transform_tiles_kernel(
+template <typename T, typename MT, int V, bool EARLY, int WIDTH>
+__global__ __launch_bounds__((WIDTH > 0 ? 4 * WIDTH : 1024) / V, EARLY ? 4 : WIDTH > 0 ? 6 : 8) void winograd_output_transform_tiles_kernel(
     const MT* __restrict__ m, const float* __restrict__ bias, const T* skip, const float* __restrict__ se_w1,
     const float* __restrict__ se_b1, const float* __restrict__ se_w2, const float* __restrict__ se_b2, int se_k,
     T* out, T* __restrict__ v_next, int ldv, int batch, int C, int act) {
@@ -259,10 +261,13 @@ __global__ __launch_bounds__(1024 / V, EARLY ? 4 : 8) void winograd_output_trans
   float* part = shm;               // [4][C]
   float* hidden = shm + 4 * C;     // [K]
   float* fc2 = hidden + se_k + (se_k & 1);   // [4][gamma | beta][C] partial sums of the second layer
-  T* xs = reinterpret_cast<T*>(fc2 + 8 * C);   // [64][C] activations for the fused input transform
+  // activations [64][width] for the fused input transform
+  T* xs = reinterpret_cast<T*>(WIDTH > 0 ? shm : fc2 + 8 * C);
   const int b = blockIdx.x;
-  const int per_tile = C / V;
-  const int tile = threadIdx.x / per_tile, c = V * (threadIdx.x - tile * per_tile);
+  const int width = WIDTH > 0 ? WIDTH : C;
+  const int per_tile = width / V;
+  const int tile = threadIdx.x / per_tile, c_in = V * (threadIdx.x - tile * per_tile);
+  const int c = WIDTH > 0 ? (int)blockIdx.y * WIDTH + c_in : c_in;
   const int ty = (tile >> 1) * 4, tx = (tile & 1) * 4;
   const long long kstride = (long long)batch * 4 * C;
   // (a base that all lanes share and a 32-bit lane offset: one address register for the 36 loads)
@@ -272,7 +277,7 @@ __global__ __launch_bounds__(1024 / V, EARLY ? 4 : 8) void winograd_output_trans
 #pragma unroll
   for (int k = 0; k < 36; k++) mm[k] = *reinterpret_cast<const ChM*>(mp + (long long)k * kstride + m_off);
   const ChF bc = *reinterpret_cast<const ChF*>(bias + c);
-  const unsigned sq_off = (ty * 8 + tx) * C + c;
+  const unsigned sq_off = (ty * 8 + tx) * C + c, xs_off = WIDTH > 0 ? (ty * 8 + tx) * width + c_in : sq_off;
   using Raw = std::conditional_t<sizeof(Ch) == 4, uint32_t, uint16_t>;   // (as halves the pairs would be split into registers)
   static_assert(sizeof(Ch) == sizeof(Raw), "2 or 4 bytes per lane");
   Raw sk[16];
@@ -306,7 +311,7 @@ __global__ __launch_bounds__(1024 / V, EARLY ? 4 : 8) void winograd_output_trans
     }
   };
   auto ask = [&]() {
-    if (se_k > 0) {
+    if (WIDTH == 0 && se_k > 0) {
       load_w1(wave);
       load_w2(tile);
       sg = *reinterpret_cast<const ChF*>(se_b2 + c);
@@ -329,7 +334,7 @@ __global__ __launch_bounds__(1024 / V, EARLY ? 4 : 8) void winograd_output_trans
   float gamma[V], beta[V];
 #pragma unroll
   for (int v = 0; v < V; v++) gamma[v] = 1.0f, beta[v] = bc[v];
-  if (se_k > 0) {
+  if (WIDTH == 0 && se_k > 0) {
     ChF sum;
 #pragma unroll
     for (int v = 0; v < V; v++) {
@@ -421,7 +426,7 @@ __global__ __launch_bounds__(1024 / V, EARLY ? 4 : 8) void winograd_output_trans
         r[v] = (T)RActivate(x, act);
       }
       if (o) *reinterpret_cast<Ch*>(o + sq * C + sq_off) = r;
-      if (v_next) *reinterpret_cast<Ch*>(&xs[sq * C + sq_off]) = r;
+      if (v_next) *reinterpret_cast<Ch*>(&xs[sq * width + xs_off]) = r;
     }
   if (!v_next) return;
   // Fused input transform of the next convolution: this thread's tile reads its 6x6
@@ -435,7 +440,7 @@ __global__ __launch_bounds__(1024 / V, EARLY ? 4 : 8) void winograd_output_trans
     for (int j = 0; j < 6; j++) {
       const int yy = y0 + i, xx = x0 + j;
       if (yy >= 0 && yy < 8 && xx >= 0 && xx < 8) {
-        patch[i][j] = *reinterpret_cast<const Ch*>(&xs[(yy * 8 + xx) * C + c]);
+        patch[i][j] = *reinterpret_cast<const Ch*>(&xs[(yy * 8 + xx) * width + c_in]);
       } else {
 #pragma unroll
         for (int v = 0; v < V; v++) patch[i][j][v] = (T)0.0f;
@@ -516,25 +521,34 @@ void LaunchWinogradOutputTransform(const MT* m, const float* bias, const T* skip
   if (batch <= 0) return;
   const int k = se_k > 0 ? se_k : 0;
   if (C <= 256 && C % 16 == 0) {   // 4 * C threads in whole waves (the SE reduction shuffles across a wave)
-    size_t shm = sizeof(float) * (size_t)(12 * C + k + (k & 1));
-    if (v_next) shm += sizeof(T) * 64 * (size_t)C;
-    auto launch = [&](auto v_tag, auto early_tag) {
-      constexpr int V = decltype(v_tag)::value;
-      hipLaunchKernelGGL((winograd_output_transform_tiles_kernel<T, MT, V, decltype(early_tag)::value>), dim3(batch),
-                         dim3(4 * C / V), shm, stream, m, bias, skip, se_w1, se_b1, se_w2, se_b2, se_k, out, v_next, ldv_next, batch, C, act);
+    // Without squeeze-and-excitation the channels of a position need nothing of each other: while the positions do not fill the
+    // CUs, 64 of them to a workgroup (at six waves per SIMD: eight spill), so that few positions lie on more CUs (a 20x256 pass in
+    // halves, half of its transforms, us, whole positions -> 64 channels: 1 position 686 -> 622, 13 736 -> 671, 64 977 -> 917, 200 1331
+    // -> 1296; 512 1910 -> 1943; in floats 1 742 -> 728, 13 963 -> 943, 64 1523 -> 1520, 200
+    // 3291 -> 3318. 16 and 32 channels are level with 64).
+    const bool split = k == 0 && C > 64 && C % 64 == 0 && batch <= (sizeof(T) == 2 ? 256 : 64);
+    size_t shm = split ? 0 : sizeof(float) * (size_t)(12 * C + k + (k & 1));
+    if (v_next) shm += sizeof(T) * 64 * (size_t)(split ? 64 : C);
+    auto launch = [&](auto v_tag, auto early_tag, auto width_tag) {
+      constexpr int V = decltype(v_tag)::value, W = decltype(width_tag)::value;
+      hipLaunchKernelGGL((winograd_output_transform_tiles_kernel<T, MT, V, decltype(early_tag)::value, W>), dim3(batch, W > 0 ? C / std::max(W, 1) : 1),
+                         dim3(4 * (W > 0 ? W : C) / V), shm, stream, m, bias, skip, se_w1, se_b1, se_w2, se_b2, se_k, out, v_next,
+                         ldv_next, batch, C, act);
     };
+    using Whole = std::integral_constant<int, 0>;
+    if (split) return launch(std::integral_constant<int, 1>{}, std::false_type{}, std::integral_constant<int, 64>{});
     // Two channels per thread (see the kernel) where a CU has more than one position; that needs 2 * C threads in whole
     // waves and whole pairs of channels in every row.
     const bool pairs = C % 32 == 0 && (v_next == nullptr || ldv_next % 2 == 0);
     if constexpr (sizeof(T) == 2) {
-      if (pairs && batch > 256) return launch(std::integral_constant<int, 2>{}, std::true_type{});
+      if (pairs && batch > 256) return launch(std::integral_constant<int, 2>{}, std::true_type{}, Whole{});
     }
     // The early requests while all positions are on the CUs at once (at four waves per SIMD a CU holds 256 / C workgroups),
     // the form of 61 registers beyond (us of the kernel, early / late: halves of 176 channels at 300 positions 20.8 / 16.7,
     // at 1000 41.0 / 30.2, floats of 192 22.5 / 18.0 and 54.1 / 46.2; the other way round floats of 64 at 300 13.1 / 13.5, halves
     // of 112 8.5 / 8.7).
-    if (batch > 256 * (256 / C)) return launch(std::integral_constant<int, 1>{}, std::false_type{});
-    launch(std::integral_constant<int, 1>{}, std::true_type{});
+    if (batch > 256 * (256 / C)) return launch(std::integral_constant<int, 1>{}, std::false_type{}, Whole{});
+    launch(std::integral_constant<int, 1>{}, std::true_type{}, Whole{});
     return;
   }
   // Wide towers: separate kernels (the caller checks WinogradFusedInputTransform before asking for v_next).
