@@ -157,6 +157,11 @@ int lc0mi_k_qkv_attention(const uint16_t* x, const uint16_t* W, const float* bia
 int lc0mi_k_encoder_tail(const uint16_t* att, uint16_t* x, const uint16_t* dense, const uint16_t* ffn1, const uint16_t* ffn2,
                          const float* biases, const float* norms, int M, int emb, int d_model, int dff, float alpha, float eps,
                          int act, int time_iters, double* ms);
+/* One or two heads of an attention body, each embedding, first and second dense layer, in one kernel: x [batch * 64][emb],
+ * dims {ch, fc, out_n, out_act} per head, weights {[ch][emb], [fc][64 ch], [out_n][fc]} and biases (entries may be NULL) per head,
+ * outs [batch][out_n] floats per head; 16-bit. ch even and at most 32, fc at most 128. Counterpart: network_blas.cc:725-772. */
+int lc0mi_k_value_heads(const uint16_t* x, int batch, int emb, int act, int heads, const int* dims, const uint16_t* const* weights,
+                        const float* const* biases, float* const* outs, int time_iters, double* ms);
 /* Two products of the same rows in one launch: C as lc0mi_k_gemm (batch 1, 16-bit output, act none) or, with f8 != 0, as
  * lc0mi_k_gemm_f8 (half output), and C2 = A.W2^T without bias (16-bit), or e4m3(col_scale2[n] * sum * out_mul2) bytes.
  * A [M][K], W [N][K], W2 [N2][K]. Fails where the kernel of the first product does not serve a second one. Counterpart:

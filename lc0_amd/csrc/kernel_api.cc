@@ -728,6 +728,43 @@ int lc0mi_k_encoder_tail(const uint16_t* att, uint16_t* x, const uint16_t* dense
   });
 }
 
+int lc0mi_k_value_heads(const uint16_t* x, int batch, int emb, int act, int heads, const int* dims, const uint16_t* const* weights,
+                        const float* const* biases, float* const* outs, int time_iters, double* ms) {
+  return Guard([&] {
+    RequireDevice();
+    if (batch < 1 || heads < 1 || heads > 2) throw Error("bad shape");
+    Dev dev;
+    lc0mi::ValueHeadsArgs a;
+    a.x = reinterpret_cast<const half_t*>(dev.Put(x, (size_t)batch * 64 * emb));
+    a.ldx = emb; a.emb = emb; a.batch = batch; a.act = act; a.heads = heads; a.bf16 = g_bf16;
+    for (int i = 0; i < heads; i++) {
+      lc0mi::HeadLayers& h = a.head[i];
+      h.ch = dims[4 * i]; h.fc = dims[4 * i + 1]; h.out_n = dims[4 * i + 2]; h.out_act = dims[4 * i + 3];
+      if (!lc0mi::ValueHeadSupported(emb, h.ch, h.fc, h.out_n)) throw Error("bad shape");
+      h.ld_fc2 = h.fc;
+      auto packed = [&](bool embed, const uint16_t* w, int out, int in) {
+        std::vector<uint16_t> v(lc0mi::HeadFragments(embed, emb, h.ch), 0);
+        for (int o = 0; o < out; o++)
+          for (int k = 0; k < in; k++) v[lc0mi::HeadFragmentIndex(embed, o, k, emb, h.ch)] = w[(size_t)o * in + k];
+        return reinterpret_cast<const half_t*>(dev.Put(v.data(), v.size()));
+      };
+      h.w_embed = packed(true, weights[3 * i], h.ch, emb);
+      h.w_fc1 = packed(false, weights[3 * i + 1], h.fc, 64 * h.ch);
+      h.w_fc2 = reinterpret_cast<const half_t*>(dev.Put(weights[3 * i + 2], (size_t)h.out_n * h.fc));
+      auto bias = [&](int k, int n) { return biases[3 * i + k] ? dev.Put(biases[3 * i + k], (size_t)n) : nullptr; };
+      h.b_embed = bias(0, h.ch); h.b_fc1 = bias(1, h.fc); h.b_fc2 = bias(2, h.out_n);
+      h.out = static_cast<float*>(dev.Alloc((size_t)batch * h.out_n * 4));
+    }
+    lc0mi::LaunchValueHeads(a, nullptr);
+    K_CHECK(hipDeviceSynchronize());
+    K_CHECK(hipGetLastError());
+    for (int i = 0; i < heads; i++) {
+      K_CHECK(hipMemcpy(outs[i], a.head[i].out, (size_t)batch * a.head[i].out_n * 4, hipMemcpyDeviceToHost));
+    }
+    if (time_iters > 0 && ms) *ms = TimeLaunches(time_iters, [&] { lc0mi::LaunchValueHeads(a, nullptr); });
+  });
+}
+
 int lc0mi_k_gemm_second(int f8, const void* A, const void* W, const void* W2, const float* bias, const float* col_scale,
                         const float* col_scale2, float out_mul2, int M, int N, int N2, int K, uint16_t* C, void* C2) {
   return Guard([&] {

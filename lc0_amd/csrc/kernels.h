@@ -309,6 +309,29 @@ int EncoderTailRows(int M);   // rows of a workgroup
 long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_model);
 void LaunchEncoderTail(const EncoderTailArgs& args, hipStream_t stream);
 
+// Value and moves-left heads of a 16-bit attention body (value_heads.hip), for few positions: per head
+//   out[b][o] = out_act(sum_n act(sum_k e[b][k] w_fc1[n][k] + b_fc1[n]) w_fc2[o][n] + b_fc2[o]),
+//   e[b][sq * ch + c] = act(sum_j x[b*64+sq][j] w_embed[c][j] + b_embed[c]), rounded to 16 bits.
+// w_embed and w_fc1 are HeadFragments() elements, element (row, col) at HeadFragmentIndex() and zeros elsewhere; w_fc2 is
+// [out_n][ld_fc2]; biases may be null. Only where ValueHeadSupported(); ldx % 8 == 0, 16-byte aligned bases.
+struct HeadLayers {
+  const half_t *w_embed = nullptr, *w_fc1 = nullptr, *w_fc2 = nullptr;
+  const float *b_embed = nullptr, *b_fc1 = nullptr, *b_fc2 = nullptr;
+  int ld_fc2 = 0, ch = 0, fc = 0, out_n = 0;
+  int out_act = 3;
+  float* out = nullptr;
+};
+struct ValueHeadsArgs {
+  const half_t* x = nullptr;
+  int ldx = 0, emb = 0, batch = 0, heads = 0, act = 3;
+  HeadLayers head[2];
+  bool bf16 = false;
+};
+long long HeadFragments(bool embed, int emb, int ch);
+long long HeadFragmentIndex(bool embed, int row, int col, int emb, int ch);
+bool ValueHeadSupported(int emb, int ch, int fc, int out_n);
+void LaunchValueHeads(const ValueHeadsArgs& args, hipStream_t stream);
+
 // Attention policy tail: promotion offsets + gather to 1858 moves.
 // logits: [B][64*64] float (already scaled), kq: [B*64][ld_kq] with keys at column
 // offset key_off, ppo: [4][pd] float, inv_map: [1858] source index into the

@@ -309,6 +309,8 @@ struct ModelState {
   int dense2_norm_max_batch_ = 64, generator_norm_max_batch_ = 48;   // largest batches whose row norms run inside the layer after them
   bool compress_with_qkv_ = true;
   bool narrow_layers_ = true;   // the two kernels of narrow bodies
+  int fused_heads_max_batch_ = -1;   // largest batch whose value and moves-left heads are one kernel (-1: automatic)
+  half_t *val_packed_[2] = {}, *mov_packed_[2] = {};   // embedding and first layer of either head in that kernel's order (null: never)
   bool qkv_first_ = true;
   bool write_through_ = true;   // big activations go to the memory-side cache while a layer's worth fits it
   int chain_latency_max_batch_ = 128;   // largest fp16 batch whose smolgen chain takes the shortest-latency GEMM variants
@@ -1108,6 +1110,7 @@ Mi355xNetwork::Mi355xNetwork(const WeightsFile& file, Options& options) {
   dense1_split_min_batch_ = options.GetInt("dense1_split_min_batch", 112);
   compress_with_qkv_ = options.GetBool("compress_with_qkv", true);
   narrow_layers_ = options.GetBool("narrow_layers", true);
+  fused_heads_max_batch_ = options.GetInt("fused_heads_max_batch", -1);
   dense2_norm_max_batch_ = options.GetInt("dense2_norm_max_batch", 64);
   generator_norm_max_batch_ = options.GetInt("generator_norm_max_batch", 48);
   qkv_first_ = options.GetBool("qkv_first", true);
@@ -1653,7 +1656,21 @@ void Mi355xNetwork::BuildAttentionBody(const WeightsFile& file) {
     mov_fc1_ = MakeLinear(w.ip1_mov_w, w.ip1_mov_b, mov_fc_, 64 * mov_ch_);
     mov_fc2_ = MakeLinear(w.ip2_mov_w, w.ip2_mov_b, 1, mov_fc_);
   }
-
+  if (dtype_ != Dtype::kFloat && ValueHeadSupported(emb_, val_ch_, val_fc_, val_out_) &&
+      (!moves_left_ || ValueHeadSupported(emb_, mov_ch_, mov_fc_, 1))) {
+    auto pack = [&](half_t* (&packed)[2], const Vec& embed, const Vec& fc1, int ch, int fc) {
+      Vec v(HeadFragments(true, emb_, ch), 0.0f);
+      for (int o = 0; o < ch; o++)
+        for (int k = 0; k < emb_; k++) v[HeadFragmentIndex(true, o, k, emb_, ch)] = embed[static_cast<size_t>(o) * emb_ + k];
+      packed[0] = UploadElems(v);
+      v.assign(HeadFragments(false, emb_, ch), 0.0f);
+      for (int o = 0; o < fc; o++)
+        for (int k = 0; k < 64 * ch; k++) v[HeadFragmentIndex(false, o, k, emb_, ch)] = fc1[static_cast<size_t>(o) * 64 * ch + k];
+      packed[1] = UploadElems(v);
+    };
+    pack(val_packed_, vh.ip_val_w, vh.ip1_val_w, val_ch_, val_fc_);
+    if (moves_left_) pack(mov_packed_, w.ip_mov_w, w.ip1_mov_w, mov_ch_, mov_fc_);
+  }
 }
 
 
@@ -2251,13 +2268,35 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
     HIP_CHECK(hipEventRecord(heads_fork_, stream_));
     HIP_CHECK(hipStreamWaitEvent(hs, heads_fork_, 0));
   }
-  Gemm("gemm_value_embed", x_, emb_, val_emb_lin_, head1_, val_ch_, T, default_act_, false, hs);
-  Gemm("gemm_value_fc1", head1_, 64 * val_ch_, val_fc1_, head2_, val_fc_, B, default_act_, false, hs);
-  Gemm("gemm_value_fc2", head2_, val_fc_, val_fc2_, d_wdl_, val_out_, B, kActNone, /*out_f32=*/true, hs);
-  if (moves_left_) {
-    Gemm("gemm_mlh_embed", x_, emb_, mov_emb_lin_, head1_, mov_ch_, T, default_act_, false, hs);
-    Gemm("gemm_mlh_fc1", head1_, 64 * mov_ch_, mov_fc1_, head2_, mov_fc_, B, default_act_, false, hs);
-    Gemm("gemm_mlh_fc2", head2_, mov_fc_, mov_fc2_, d_mlh_, 1, B, kActRelu, /*out_f32=*/true, hs);
+  // The two heads in one launch while their workgroups find a place at once (two per CU at width 256, else one). us of a pass,
+  // six launches -> one: 10x256 fp16 1 position 291 -> 278, 64 323 -> 310, 200 545 -> 528, 1024 1865 -> 1889; 15x1024 fp16 1 831 -> 822, 13
+  // 1234 -> 1217, 77 2776 -> 2764, 128 level, 256 5603 -> 5633; e4m3 16 934 -> 916.
+  const int fused_heads_max = fused_heads_max_batch_ >= 0 ? fused_heads_max_batch_ : emb_ <= 256 ? 256 : 128;
+  if (val_packed_[0] != nullptr && B <= fused_heads_max) {
+    ValueHeadsArgs a;
+    a.x = x_; a.ldx = emb_; a.emb = emb_; a.batch = B; a.act = default_act_; a.bf16 = dtype_ == Dtype::kBf16;
+    double weights = 0.0;
+    auto add = [&](half_t* const (&packed)[2], const Linear& embed, const Linear& fc1, const Linear& fc2, int out_act, float* out) {
+      HeadLayers& h = a.head[a.heads++];
+      h.w_embed = packed[0]; h.b_embed = embed.b; h.ch = embed.out;
+      h.w_fc1 = packed[1]; h.b_fc1 = fc1.b; h.fc = fc1.out;
+      h.w_fc2 = fc2.w; h.ld_fc2 = fc2.ld; h.b_fc2 = fc2.b; h.out_n = fc2.out;
+      h.out_act = out_act; h.out = out;
+      weights += static_cast<double>(embed.out) * emb_ + static_cast<double>(fc1.out) * fc1.in + fc2.out * fc2.in;
+    };
+    add(val_packed_, val_emb_lin_, val_fc1_, val_fc2_, kActNone, d_wdl_);
+    if (moves_left_) add(mov_packed_, mov_emb_lin_, mov_fc1_, mov_fc2_, kActRelu, d_mlh_);
+    Timed("value_heads", 2.0 * B * (weights + 63.0 * emb_ * (val_ch_ + (moves_left_ ? mov_ch_ : 0))),
+          2.0 * (weights + static_cast<double>(T) * emb_), [&] { LaunchValueHeads(a, hs); }, hs);
+  } else {
+    Gemm("gemm_value_embed", x_, emb_, val_emb_lin_, head1_, val_ch_, T, default_act_, false, hs);
+    Gemm("gemm_value_fc1", head1_, 64 * val_ch_, val_fc1_, head2_, val_fc_, B, default_act_, false, hs);
+    Gemm("gemm_value_fc2", head2_, val_fc_, val_fc2_, d_wdl_, val_out_, B, kActNone, /*out_f32=*/true, hs);
+    if (moves_left_) {
+      Gemm("gemm_mlh_embed", x_, emb_, mov_emb_lin_, head1_, mov_ch_, T, default_act_, false, hs);
+      Gemm("gemm_mlh_fc1", head1_, 64 * mov_ch_, mov_fc1_, head2_, mov_fc_, B, default_act_, false, hs);
+      Gemm("gemm_mlh_fc2", head2_, mov_fc_, mov_fc2_, d_mlh_, 1, B, kActRelu, /*out_f32=*/true, hs);
+    }
   }
   if (heads_beside) HIP_CHECK(hipEventRecord(heads_join_, hs));
   // Policy head.

@@ -41,6 +41,7 @@ def _lib():
         lib.lc0mi_k_norm_gemm.argtypes = [ci] + [vp] * 6 + [ci] * 4 + [cf, cf, ci, vp, ci, cd]
         lib.lc0mi_k_qkv_attention.argtypes = [vp] * 3 + [ci] * 3 + [cf, vp, ci, cd]
         lib.lc0mi_k_encoder_tail.argtypes = [vp] * 7 + [ci] * 4 + [cf, cf, ci, ci, cd]
+        lib.lc0mi_k_value_heads.argtypes = [vp, ci, ci, ci, ci, vp, vp, vp, vp, ci, cd]
         lib.lc0mi_k_gemm_second.argtypes = [ci] + [vp] * 6 + [cf] + [ci] * 4 + [vp, vp]
         lib.lc0mi_k_quantize_f8.argtypes = [vp, ll, cf, vp]
         lib.lc0mi_k_layer_norm_f8.argtypes = [vp, vp, vp, vp, ci, ci, cf, cf, cf, vp, vp]
@@ -347,6 +348,22 @@ def encoder_tail(att, x, dense, ffn1, ffn2, norms, biases=None, alpha=1.0, eps=1
     _check(_lib().lc0mi_k_encoder_tail(_ptr(att), _ptr(out), _ptr(dense), _ptr(ffn1), _ptr(ffn2), _ptr(b), _ptr(n), m, emb, d_model,
                                        dff, C.c_float(alpha), C.c_float(eps), act, time_iters, C.byref(ms)))
     return (_ret16(out), ms.value) if time_iters else _ret16(out)
+
+
+def value_heads(x, heads, act=ACT_NONE, time_iters=0):
+    """Heads of an attention body in one kernel. heads: one or two of (w_embed, b_embed, w_fc1, b_fc1, w_fc2, b_fc2, out_act),
+    biases or None. Returns one [batch][out_n] float array per head."""
+    x = _h(x)
+    (m, emb) = x.shape
+    w = [[_h(h[i]) for i in (0, 2, 4)] for h in heads]
+    b = [[np.ascontiguousarray(h[i], np.float32) if h[i] is not None else None for i in (1, 3, 5)] for h in heads]
+    dims = np.array([[hw[0].shape[0], hw[1].shape[0], hw[2].shape[0], h[6]] for hw, h in zip(w, heads)], np.int32)
+    outs = [np.zeros((m // 64, hw[2].shape[0]), np.float32) for hw in w]
+    table = lambda arrays: (C.c_void_p * len(arrays))(*[_ptr(v) for v in arrays])
+    ms = C.c_double(0)
+    _check(_lib().lc0mi_k_value_heads(_ptr(x), m // 64, emb, act, len(heads), _ptr(dims), table(sum(w, [])), table(sum(b, [])),
+                                      table(outs), time_iters, C.byref(ms)))
+    return (outs, ms.value) if time_iters else outs
 
 
 def gemm_second(a, w, w2, bias=None, col_scale=None, col_scale2=None, out_mul2=1.0):
