@@ -162,6 +162,12 @@ int lc0mi_k_encoder_tail(const uint16_t* att, uint16_t* x, const uint16_t* dense
  * outs [batch][out_n] floats per head; 16-bit. ch even and at most 32, fc at most 128. Counterpart: network_blas.cc:725-772. */
 int lc0mi_k_value_heads(const uint16_t* x, int batch, int emb, int act, int heads, const int* dims, const uint16_t* const* weights,
                         const float* const* biases, float* const* outs, int time_iters, double* ms);
+/* Row norm, smolgen generator (gen_sz 256) and attention in one kernel: gen [batch][heads * 256] before the norm, gamma and beta
+ * [heads * 256], otherwise as lc0mi_k_smolgen_attention; heads a multiple of four up to 32. Counterpart:
+ * src/neural/backends/blas/network_blas.cc:326-439. */
+int lc0mi_k_smolgen_attention_few(const uint16_t* qkv, const uint16_t* gen, const uint16_t* w, const float* gamma, const float* beta,
+                                  float eps, int batch, int heads, float scale, int f8_out, float out_mul, void* out,
+                                  int time_iters, double* ms);
 /* Two products of the same rows in one launch: C as lc0mi_k_gemm (batch 1, 16-bit output, act none) or, with f8 != 0, as
  * lc0mi_k_gemm_f8 (half output), and C2 = A.W2^T without bias (16-bit), or e4m3(col_scale2[n] * sum * out_mul2) bytes.
  * A [M][K], W [N][K], W2 [N2][K]. Fails where the kernel of the first product does not serve a second one. Counterpart:

@@ -921,6 +921,37 @@ int lc0mi_k_smolgen_attention(const uint16_t* qkv, const uint16_t* gen, const ui
   });
 }
 
+int lc0mi_k_smolgen_attention_few(const uint16_t* qkv, const uint16_t* gen, const uint16_t* w, const float* gamma, const float* beta,
+                                  float eps, int batch, int heads, float scale, int f8_out, float out_mul, void* out,
+                                  int time_iters, double* ms) {
+  return Guard([&] {
+    RequireDevice();
+    constexpr int gen_sz = 256;
+    if (batch < 1 || !lc0mi::SmolgenAttentionFewSupported(heads, 32, gen_sz)) throw Error("bad smolgen attention shape");
+    Dev dev;
+    const int d = heads * 32;
+    std::vector<uint16_t> frag((size_t)4096 * gen_sz);
+    for (int row = 0; row < 4096; row++)
+      for (int col = 0; col < gen_sz; col++)
+        frag[lc0mi::SmolgenFragmentIndex(row, col, gen_sz)] = w[(size_t)row * gen_sz + col];
+    lc0mi::SmolgenFewArgs a;
+    a.qkv = reinterpret_cast<const half_t*>(dev.Put(qkv, (size_t)batch * 64 * 3 * d));
+    a.gen = reinterpret_cast<const half_t*>(dev.Put(gen, (size_t)batch * heads * gen_sz));
+    a.wfrag = reinterpret_cast<const half_t*>(dev.Put(frag.data(), frag.size()));
+    a.gamma = dev.Put(gamma, (size_t)heads * gen_sz);
+    a.beta = dev.Put(beta, (size_t)heads * gen_sz);
+    const size_t out_bytes = (size_t)batch * 64 * d * (f8_out ? 1 : 2);
+    a.out = dev.Alloc(out_bytes);
+    a.batch = batch; a.heads = heads; a.scale = scale; a.eps = eps; a.out_mul = out_mul;
+    a.bf16 = g_bf16; a.out_f8 = f8_out != 0;
+    lc0mi::LaunchSmolgenAttentionFew(a, nullptr);
+    K_CHECK(hipDeviceSynchronize());
+    K_CHECK(hipGetLastError());
+    K_CHECK(hipMemcpy(out, a.out, out_bytes, hipMemcpyDeviceToHost));
+    if (time_iters > 0 && ms) *ms = TimeLaunches(time_iters, [&] { lc0mi::LaunchSmolgenAttentionFew(a, nullptr); });
+  });
+}
+
 int lc0mi_k_copy(long long bytes, int iters, double* ms) {
   return Guard([&] {
     RequireDevice();

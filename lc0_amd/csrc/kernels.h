@@ -309,6 +309,20 @@ int EncoderTailRows(int M);   // rows of a workgroup
 long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_model);
 void LaunchEncoderTail(const EncoderTailArgs& args, hipStream_t stream);
 
+// For few positions the same with the norm before the generator layer inside (smolgen_attention_few.hip): gen holds the rows of
+// heads * 256 values before the norm, gamma and beta as many floats. out: 16 bits, or with out_f8 e4m3(result * out_mul).
+// SmolgenAttentionFewSupported: head depth 32, a multiple of four heads up to 32, gen_sz 256.
+struct SmolgenFewArgs {
+  const half_t *qkv = nullptr, *gen = nullptr, *wfrag = nullptr;
+  const float *gamma = nullptr, *beta = nullptr;
+  void* out = nullptr;
+  int batch = 0, heads = 0;
+  float scale = 1.0f, eps = 1e-3f, out_mul = 1.0f;
+  bool bf16 = false, out_f8 = false;
+};
+bool SmolgenAttentionFewSupported(int heads, int depth, int gen_sz);
+void LaunchSmolgenAttentionFew(const SmolgenFewArgs& args, hipStream_t stream);
+
 // Value and moves-left heads of a 16-bit attention body (value_heads.hip), for few positions: per head
 //   out[b][o] = out_act(sum_n act(sum_k e[b][k] w_fc1[n][k] + b_fc1[n]) w_fc2[o][n] + b_fc2[o]),
 //   e[b][sq * ch + c] = act(sum_j x[b*64+sq][j] w_embed[c][j] + b_embed[c]), rounded to 16 bits.

@@ -307,6 +307,7 @@ struct ModelState {
   int fused_smolgen_min_batch_ = 72;
   int dense1_split_min_batch_ = 112;   // smallest batch whose smolgen dense1 splits K between workgroups
   int dense2_norm_max_batch_ = 64, generator_norm_max_batch_ = 48;   // largest batches whose row norms run inside the layer after them
+  int smolgen_few_max_batch_ = 64;   // largest batch whose generator layer and norm run in the attention kernel for few positions
   bool compress_with_qkv_ = true;
   bool narrow_layers_ = true;   // the two kernels of narrow bodies
   int fused_heads_max_batch_ = -1;   // largest batch whose value and moves-left heads are one kernel (-1: automatic)
@@ -1110,6 +1111,7 @@ Mi355xNetwork::Mi355xNetwork(const WeightsFile& file, Options& options) {
   dense1_split_min_batch_ = options.GetInt("dense1_split_min_batch", 112);
   compress_with_qkv_ = options.GetBool("compress_with_qkv", true);
   narrow_layers_ = options.GetBool("narrow_layers", true);
+  smolgen_few_max_batch_ = options.GetInt("smolgen_few_max_batch", 64);
   fused_heads_max_batch_ = options.GetInt("fused_heads_max_batch", -1);
   dense2_norm_max_batch_ = options.GetInt("dense2_norm_max_batch", 64);
   generator_norm_max_batch_ = options.GetInt("generator_norm_max_batch", 48);
@@ -2027,6 +2029,12 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
     // plus the plain attention kernel. An explicit fp8_gemms=...+smolgen keeps all four layers in e4m3.
     const bool fused_gen = e.has_smolgen && smolgen_wfrag_ != nullptr && B >= fused_smolgen_min_batch_ &&
                            (!chain_f8 || q_smolgen_auto_);
+    // Few positions: the norm before the generator layer, that layer and the attention in one kernel, while that is one
+    // workgroup per CU. us of a 15x1024 pass, two or three launches -> one: fp16 1 position 824 -> 814, 13 1219 -> 1187, 17 1348 -> 1306, 32
+    // 1690 -> 1647, 48 2135 -> 2066, 64 2390 -> 2238, 70 2731 -> 2835; bf16 64 2328 -> 2186; e4m3 16 920 -> 901, 32 1222 -> 1198, 64 1708 -> 1610.
+    const bool gen_inside = e.has_smolgen && smolgen_wfrag_ != nullptr && !fused_gen && !calibrating_ && B <= smolgen_few_max_batch_ &&
+                            B < dense1_split_min_batch_ && (!chain_f8 || q_smolgen_auto_) &&
+                            SmolgenAttentionFewSupported(heads_, depth_, sg_gen_ / heads_);
     auto launch_qkv = [&](const SecondProduct& second = {}) {
       if (f8 && q_qkv_) {
         return GemmF8("gemm_qkv", xq_, e.qkv, e.qkv8, qkv_, T, kActNone, false, 1.0f, nullptr, keep, second);
@@ -2071,7 +2079,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       // there earlier, with e4m3 operands at 33.
       const bool norms_inside = !calibrating_ && dtype_ != Dtype::kFloat && B < dense1_split_min_batch_;
       const bool norm_dense2 = norms_inside && B <= dense2_norm_max_batch_ && NormGemmSupported(sg_hs_, 1, sg_gen_);
-      const bool norm_global = norms_inside && !fused_gen && B <= std::min(generator_norm_max_batch_, chain_f8 ? 32 : 1024) &&
+      const bool norm_global = norms_inside && !fused_gen && !gen_inside && B <= std::min(generator_norm_max_batch_, chain_f8 ? 32 : 1024) &&
                                NormGemmSupported(g, heads_, 4096);
       if (chain_f8) {
         // The whole chain on e4m3 operands: the compression reads the e4m3 copy of x that the QKV projection reads
@@ -2090,7 +2098,9 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
           }, ss);
           GemmF8("gemm_smolgen_dense2", sg2q_, e.sg_dense2, e.sg_dense28, sg3_, B, smolgen_act_, false, 1.0f, ss);
         }
-        if (norm_global) {
+        if (gen_inside) {
+          // (in the attention kernel)
+        } else if (norm_global) {
           NormGemm("gemm_smolgen_global", sg3_, smolgen_w_, &e.sg_global8, 1.0f / e.s_sg3, e.sg_ln2_g, e.sg_ln2_b, heads_,
                    sbias_, B * heads_, kActNone, ss);
         } else {
@@ -2138,7 +2148,9 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       } else {
         Gemm("gemm_smolgen_dense2", sg2_, sg_hs_, e.sg_dense2, sg3_, sg_gen_, B, smolgen_act_, false, ss, 1, chain_first);
       }
-      if (norm_global) {
+      if (gen_inside) {
+        // (in the attention kernel)
+      } else if (norm_global) {
         NormGemm("gemm_smolgen_global", sg3_, smolgen_w_, nullptr, 1.0f, e.sg_ln2_g, e.sg_ln2_b, heads_, sbias_, B * heads_,
                  kActNone, ss);
       } else {
@@ -2166,7 +2178,18 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
         B * heads_ * (2.0 * 3 * 64 * depth_ + (att_f8 ? 1.0 : 2.0) * 64 * depth_ +
                       (fused_gen ? 2.0 * gen_sz : bias ? 2.0 * 4096 : 0.0));
     const float att_scale = 1.0f / std::sqrt(static_cast<float>(depth_));
-    if (att_f8 && fused_gen) {
+    if (gen_inside) {
+      SmolgenFewArgs a;
+      a.qkv = qkv_; a.gen = sg3_; a.wfrag = smolgen_wfrag_;
+      a.gamma = e.sg_ln2_g; a.beta = e.sg_ln2_b;
+      a.out = att_f8 ? static_cast<void*>(attq_) : att_;
+      a.batch = B; a.heads = heads_; a.scale = att_scale; a.out_mul = att_f8 ? 1.0f / e.s_att : 1.0f;
+      a.bf16 = bf16; a.out_f8 = att_f8;
+      Timed("smolgen_attention_few", att_flops + 2.0 * 4096 * gen_sz * B * heads_, att_bytes, [&] { LaunchSmolgenAttentionFew(a, stream_); });
+    }
+    if (att_f8 && gen_inside) {
+      GemmF8("gemm_mha_dense", attq_, e.dense, e.dense8, t_, T, kActNone, false, 1.0f, nullptr, keep);
+    } else if (att_f8 && fused_gen) {
       Timed("smolgen_attention", att_flops, att_bytes, [&] {
         LaunchSmolgenAttentionF8Out(qkv_, sg3_, smolgen_wfrag_, attq_, 1.0f / e.s_att, B, heads_, depth_, gen_sz,
                                     att_scale, stream_);
@@ -2183,6 +2206,8 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
         a.batch = B; a.emb = emb_; a.heads = heads_; a.scale = att_scale; a.bf16 = bf16;
         Timed("qkv_attention", 6.0 * T * emb_ * d_model_ + att_flops, 2.0 * T * (emb_ + d_model_) + 6.0 * emb_ * d_model_,
               [&] { LaunchQkvAttention(a, stream_); });
+      } else if (gen_inside) {
+        // (launched above)
       } else if (fused_gen) {
         Timed("smolgen_attention", att_flops, att_bytes, [&] {
           LaunchSmolgenAttention(qkv_, sg3_, smolgen_wfrag_, att_, B, heads_, depth_, gen_sz, att_scale, stream_, bf16);

@@ -42,6 +42,7 @@ def _lib():
         lib.lc0mi_k_qkv_attention.argtypes = [vp] * 3 + [ci] * 3 + [cf, vp, ci, cd]
         lib.lc0mi_k_encoder_tail.argtypes = [vp] * 7 + [ci] * 4 + [cf, cf, ci, ci, cd]
         lib.lc0mi_k_value_heads.argtypes = [vp, ci, ci, ci, ci, vp, vp, vp, vp, ci, cd]
+        lib.lc0mi_k_smolgen_attention_few.argtypes = [vp] * 5 + [cf, ci, ci, cf, ci, cf, vp, ci, cd]
         lib.lc0mi_k_gemm_second.argtypes = [ci] + [vp] * 6 + [cf] + [ci] * 4 + [vp, vp]
         lib.lc0mi_k_quantize_f8.argtypes = [vp, ll, cf, vp]
         lib.lc0mi_k_layer_norm_f8.argtypes = [vp, vp, vp, vp, ci, ci, cf, cf, cf, vp, vp]
@@ -414,6 +415,18 @@ def smolgen_attention(qkv, gen, w, batch, heads, scale, f8_out=False, out_mul=1.
     ms = C.c_double(0)
     _check(_lib().lc0mi_k_smolgen_attention(_ptr(qkv), _ptr(gen), _ptr(w), batch, heads, w.shape[1], scale,
                                             int(f8_out), out_mul, _ptr(out), time_iters, C.byref(ms)))
+    out = _ret16(out)
+    return (out, ms.value) if time_iters else out
+
+
+def smolgen_attention_few(qkv, gen, w, gamma, beta, batch, heads, scale, eps=1e-3, f8_out=False, out_mul=1.0, time_iters=0):
+    """As smolgen_attention (gen_sz 256), with the norm of every position's heads * 256 generator values inside."""
+    qkv, gen, w = _h(qkv), _h(gen), _h(w)
+    gamma, beta = np.ascontiguousarray(gamma, np.float32), np.ascontiguousarray(beta, np.float32)
+    out = np.zeros((batch * 64, heads * 32), np.uint8) if f8_out else _out16((batch * 64, heads * 32))
+    ms = C.c_double(0)
+    _check(_lib().lc0mi_k_smolgen_attention_few(_ptr(qkv), _ptr(gen), _ptr(w), _ptr(gamma), _ptr(beta), C.c_float(eps), batch, heads,
+                                                C.c_float(scale), int(f8_out), C.c_float(out_mul), _ptr(out), time_iters, C.byref(ms)))
     out = _ret16(out)
     return (out, ms.value) if time_iters else out
 
