@@ -404,6 +404,29 @@ void LaunchWinogradOutputTransform(const MT* m, const float* bias, const T* skip
                                    int ldv_next = 0);
 bool WinogradFusedInputTransform(int C, int elem_size, int se_k);
 
+// A whole tower in one launch (resident_tower.hip): out[b][sq][c] after the last of `blocks` residual blocks, from the bit
+// planes. packed: TowerFragments() elements, the weight of convolution `conv` (0: input, then two per block), tap 3 y + x, output
+// and input channel at TowerFragmentIndex() and zeros elsewhere; biases: [1 + 2 blocks][filters]; se: one entry per block, k = 0
+// without squeeze-and-excitation, layers as above. act: mish or relu. Only where TowerSupported().
+constexpr int kTowerMaxSe = 256;
+struct TowerSe {
+  const float *w1 = nullptr, *b1 = nullptr, *w2 = nullptr, *b2 = nullptr;
+  int k = 0;
+};
+struct TowerArgs {
+  const uint64_t* masks = nullptr;
+  const float *values = nullptr, *biases = nullptr;
+  const void* packed = nullptr;
+  const TowerSe* se = nullptr;
+  void* out = nullptr;
+  int batch = 0, blocks = 0, act = 2;
+};
+bool TowerSupported(int filters, bool f32);
+long long TowerFragments(int blocks, bool f32);
+long long TowerFragmentIndex(int blocks, bool f32, int conv, int tap, int out, int in);
+bool TowerFaster(int batch, bool f32);   // than winograd convolutions
+void LaunchTower(const TowerArgs& args, bool f32, hipStream_t stream);
+
 // Gather of the convolutional policy head: out[b][j] = t[b][sq][plane] for
 // kConvPolicyMap[plane*64+sq] = j. t: [B][64][ld] (NHWC), inv_map: [1858] holding plane*64+sq.
 template <typename T>

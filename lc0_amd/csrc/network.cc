@@ -359,6 +359,12 @@ struct ModelState {
   bool classical_value_ = false;
   ConvDev res_input_, res_policy1_, res_policy_conv_;
   std::vector<ResBlockDev> res_blocks_;
+  // The tower as one kernel reads it (null where the shape has no such kernel), and option resident_tower: 0 never, 1 for every
+  // batch, -1 by batch size.
+  void* tower_packed_ = nullptr;
+  float* tower_biases_ = nullptr;
+  TowerSe* tower_se_ = nullptr;
+  int resident_tower_ = -1;
   LinearT res_pol_conv1x1_, res_pol_fc_, res_val_conv_, res_val_fc1_, res_val_fc2_, res_mov_conv_, res_mov_fc1_,
       res_mov_fc2_;
   int16_t* conv_inv_map_ = nullptr;
@@ -409,6 +415,8 @@ class Mi355xNetwork : public Network, protected ModelState {
   void EnsureSmolgenGlobal(const NetWeights& w, int g);
   template <typename T>
   void ForwardResnet(int B);
+  template <typename T>
+  bool ForwardTowerWinograd(int B);
   template <typename T>
   bool WinogradConv(const char* name, const struct ConvDev& conv, const void* x, const void* skip, const struct SeDev* se,
                     int act, void* out, int B, bool have_v = false, const struct ConvDev* next = nullptr);
@@ -1120,6 +1128,8 @@ Mi355xNetwork::Mi355xNetwork(const WeightsFile& file, Options& options) {
   chain_latency_max_batch_ = options.GetInt("chain_latency_max_batch", 128);
   fp8_fp16_layers_ = options.GetInt("fp8_fp16_layers", 0);
   if (fp8_fp16_layers_ < 0) throw Error("fp8_fp16_layers must not be negative.");
+  resident_tower_ = options.GetInt("resident_tower", -1);
+  if (resident_tower_ < -1 || resident_tower_ > 1) throw Error("resident_tower must be in -1..1.");
   use_graphs_ = options.GetBool("graphs", true);
   // Running the smolgen chain beside the QKV projection costs two cross-queue dependencies per layer; below
   // this batch size the chain on the main stream is faster (measured on the 15x1024 net, chain on the main stream
@@ -1773,6 +1783,30 @@ void Mi355xNetwork::BuildResnet(const WeightsFile& file) {
     }
     res_blocks_.push_back(b);
   }
+  if (!res_blocks_.empty() && resident_tower_ != 0 && TowerSupported(filters_, fp32_)) {
+    const int blocks = static_cast<int>(res_blocks_.size());
+    std::vector<T> packed(TowerFragments(blocks, fp32_), (T)0.0f);
+    Vec biases;
+    auto pack = [&](int conv, const ConvBlock& cb, int cin) {
+      for (int o = 0; o < filters_; o++)
+        for (int i = 0; i < cin; i++)
+          for (int tap = 0; tap < 9; tap++) {
+            packed[TowerFragmentIndex(blocks, fp32_, conv, tap, o, i)] = (T)cb.weights[(static_cast<size_t>(o) * cin + i) * 9 + tap];
+          }
+      biases.insert(biases.end(), cb.biases.begin(), cb.biases.end());
+    };
+    pack(0, w.input, kInputPlanes);
+    std::vector<TowerSe> se(blocks);
+    for (int i = 0; i < blocks; i++) {
+      pack(1 + 2 * i, w.residual[i].conv1, filters_);
+      pack(2 + 2 * i, w.residual[i].conv2, filters_);
+      const SeDev& d = res_blocks_[i].se;
+      if (res_blocks_[i].has_se) se[i] = TowerSe{d.w1, d.b1, d.w2, d.b2, d.k};
+    }
+    tower_packed_ = arena_.Upload(packed);
+    tower_biases_ = arena_.Upload(biases);
+    tower_se_ = arena_.Upload(se);
+  }
 
   // A dense layer fed by a flattened [C][64] head tensor: this backend keeps heads as
   // [64][C], so the columns are reordered once here (c*64+sq -> sq*C+c).
@@ -1866,9 +1900,9 @@ bool Mi355xNetwork::WinogradConv(const char* name, const ConvDev& conv, const vo
   return fuse;
 }
 
+// The tower as winograd convolutions into r_x_; whether r_v_ holds the transformed input of the policy head's convolution.
 template <typename T>
-void Mi355xNetwork::ForwardResnet(int B) {
-  const int T64 = B * 64;
+bool Mi355xNetwork::ForwardTowerWinograd(int B) {
   Timed("expand_planes", 0.0, B * (112.0 * 12 + sizeof(T) * 64.0 * 112), [&] {
     LaunchExpandPlanesNhwc<T>(d_masks_, d_values_, static_cast<T*>(r_in_), B, stream_);
   });
@@ -1887,6 +1921,23 @@ void Mi355xNetwork::ForwardResnet(int B) {
                              have_v, &blk.conv2);
     have_v = WinogradConv<T>("gemm_winograd", blk.conv2, r_y_, r_x_, blk.has_se ? &blk.se : nullptr, default_act_, r_x_,
                              B, have_v, next);
+  }
+  return have_v;
+}
+
+template <typename T>
+void Mi355xNetwork::ForwardResnet(int B) {
+  const int T64 = B * 64;
+  bool have_v = false;
+  if (tower_packed_ != nullptr && (resident_tower_ == 1 || TowerFaster(B, fp32_))) {
+    TowerArgs t;
+    t.masks = d_masks_; t.values = d_values_; t.biases = tower_biases_; t.packed = tower_packed_; t.se = tower_se_;
+    t.out = r_x_; t.batch = B; t.blocks = static_cast<int>(res_blocks_.size()); t.act = default_act_;
+    const double convs = 9.0 * filters_ * (kInputPlanes + 2.0 * filters_ * t.blocks);
+    Timed("resident_tower", 2.0 * 64 * B * convs, sizeof(T) * convs + B * (112.0 * 12 + sizeof(T) * 64.0 * filters_),
+          [&] { LaunchTower(t, fp32_, stream_); });
+  } else {
+    have_v = ForwardTowerWinograd<T>(B);
   }
   const bool policy_have_v = have_v;
   auto fc = [&](const char* name, const void* a, const LinearT& l, void* c, int m, int act, bool out_f32) {

@@ -1,0 +1,417 @@
+// A whole residual tower in one kernel: plane expansion, input convolution, every block with its squeeze-and-excitation.
+//
+//   resident_tower_kernel   EncodePlanes, the 3x3 convolutions, BiasActivate / BiasResidual / ApplySEUnit
+//                           blas/network_blas.cc:640-713, blas/winograd_convolution3.cc:326-382,
+//                           shared/activation.cc:166-267, blas/se_unit.cc:31-91
+#include "kernel_common.h"
+
+#include <algorithm>
+#include <stdexcept>
+#include <type_traits>
+
+namespace lc0mi {
+
+namespace {
+
+// A step of a convolution is 64 bytes of one tap's inputs: 32 halves or 16 floats. Products are tiles of TILE rows (squares) and
+// TILE output channels: 32 for halves (v_mfma_f32_32x32x16, whose rate per operation is twice that of the 16x16x32 form: 32.5
+// and 30.2 cycles an instruction, measured), 16 for floats (v_mfma_f32_16x16x4; the two forms are level). Weights are 1 KiB
+// fragments of TILE channels (lane l: channel l % TILE, 16 bytes of inputs from l / TILE), a wave's in the order in which it
+// multiplies them, over all convolutions of the tower.
+constexpr int kWaves = 4;                 // that share the channels of a product
+constexpr int kChunk = 8;                 // steps of a turn of the main loop, the most that are in flight per wave
+constexpr int kPlanes = 128;              // the 112 input planes, padded
+
+template <typename T, int C> struct TowerShape {
+  static constexpr int V = 16 / (int)sizeof(T);                    // values of a 16-byte vector
+  static constexpr int KS = 4 * V;                                 // inputs of a step
+  static constexpr int TILE = sizeof(T) == 4 ? 16 : 32, G = 64 / TILE;
+  static constexpr int SUB = KS / (G * V);                         // fragments of a tile in a step
+  static constexpr int CT = C / (TILE * kWaves);                   // channel tiles of a wave
+  static constexpr int F = CT * SUB;                               // weight fragments of a step
+  static constexpr int NS = C / KS, NS_IN = kPlanes / KS;          // steps of a tap
+  static constexpr int STEPS = (9 * NS + kChunk - 1) / kChunk * kChunk, STEPS_IN = (9 * NS_IN + kChunk - 1) / kChunk * kChunk;
+  static constexpr int LD = (C > kPlanes ? C : kPlanes) + V;       // an odd number of vectors: 16 rows meet different banks
+  static_assert(kChunk % NS == 0 && kChunk % NS_IN == 0, "a turn does whole taps");
+};
+
+// The tower's activations: mish and relu.
+template <typename F>
+__device__ __forceinline__ void TowerAct(int act, F&& f) {
+  if (act == kActMish) f([](float v) { return ActMish(v); });
+  else f([](float v) { return v > 0.0f ? v : 0.0f; });
+}
+
+// Sum over the 16 lanes of a row of lanes.
+__device__ __forceinline__ float Sum16(float v) {
+  v += DppMove<0xB1>(v);
+  v += DppMove<0x4E>(v);
+  v += DppMove<0x141>(v);
+  v += DppMove<0x140>(v);   // mirrored within 16
+  return v;
+}
+
+// ---------------------------------------------------------------------------
+// A workgroup owns POS positions from the bit planes to the last block: their activations never leave LDS (a block's input
+// and its inner activations, 64 POS rows each), and the weights stream from L2 once per workgroup, four to eight steps ahead, across
+// the ends of the convolutions too. Convolutions are direct: nine shifted products whose rows past the board's edge read a row
+// of zeros. Four times the multiplications of winograd F(4x4,3x3), but no transforms, no winograd domain in memory (2 x 38 MB
+// per convolution at 512 positions) and no launches; and sums in float over all of a convolution, where the winograd products
+// of a half tower are rounded to halves twice. Float sums run over one tap at a time, to keep the chains short.
+// ---------------------------------------------------------------------------
+template <typename T, int C, int POS, int RG>
+__global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(TowerArgs p) {
+  using S = TowerShape<T, C>;
+  constexpr int V = S::V, KS = S::KS, CT = S::CT, LD = S::LD, R = 64 * POS;
+  constexpr int THREADS = 64 * kWaves * RG;
+  constexpr int TILE = S::TILE, SUB = S::SUB, F = S::F, RT = R / TILE / RG, PT = RT / POS;   // a wave's row tiles, of a position
+  constexpr int Q = TILE * TILE / 256;                   // a lane's output channels of a tile: Q times four, 8 apart
+  using Acc = std::conditional_t<sizeof(T) == 4, floatx4, floatx16>;
+  constexpr int kRing = POS == 1 ? 8 : 4;                // steps of weights in flight
+  constexpr bool kFloat = sizeof(T) == 4;
+  using Tv4 = T __attribute__((ext_vector_type(4)));
+  constexpr int kOther = R * LD, kZero = 2 * R * LD;     // the two activation buffers, then a row of zeros
+  __shared__ __attribute__((aligned(16))) T lds[2 * R * LD + LD];
+  __shared__ __attribute__((aligned(16))) float pool[RG][POS][C];
+  __shared__ float hidden[POS][kTowerMaxSe];
+  __shared__ __attribute__((aligned(16))) float scale_shift[POS][2][C];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), cg = wave % kWaves, rg = wave / kWaves;
+  const int r = lane % TILE, g = lane / TILE;
+  const int pos0 = blockIdx.x * POS;
+  const int ch0 = cg * TILE * CT + 4 * g;              // this lane's first output channel
+
+  const int row0 = rg * (64 / RG) + r;                   // this lane's row of its first tile (with RG > 1 of one position)
+  static_assert(RG == 1 || POS == 1, "row groups share one position");
+
+  const long long steps = S::STEPS_IN + 2LL * p.blocks * S::STEPS;
+  const intx4* ws = reinterpret_cast<const intx4*>(p.packed) + cg * steps * F * 64 + lane;
+  intx4 w[kRing][F];
+#pragma unroll
+  for (int j = 0; j < kRing; j++)
+#pragma unroll
+    for (int f = 0; f < F; f++) w[j][f] = ws[(j * F + f) * 64];
+
+  // Planes of the positions into the second buffer.
+  {
+    constexpr int PER_ROW = kPlanes / V, STRIDE = THREADS / PER_ROW;
+    const int v = tid % PER_ROW;
+#pragma unroll
+    for (int q = 0; q < POS; q++) {
+      const long long at = (long long)min(pos0 + q, p.batch - 1) * 112;
+      uint64_t mask[V];
+      T value[V];
+#pragma unroll
+      for (int e = 0; e < V; e++) {
+        const int plane = v * V + e;
+        mask[e] = plane < 112 ? p.masks[at + plane] : 0;
+        value[e] = (T)(plane < 112 ? p.values[at + plane] : 0.0f);
+      }
+      for (int sq = tid / PER_ROW; sq < 64; sq += STRIDE) {
+        T x[V];
+#pragma unroll
+        for (int e = 0; e < V; e++) x[e] = ((mask[e] >> sq) & 1) ? value[e] : (T)0.0f;
+        *reinterpret_cast<intx4*>(lds + kOther + (q * 64 + sq) * LD + v * V) = *reinterpret_cast<const intx4*>(x);
+      }
+    }
+    if (tid < LD / V) *reinterpret_cast<intx4*>(lds + kZero + tid * V) = intx4{0, 0, 0, 0};
+  }
+  __syncthreads();
+
+  Acc acc[RT][CT];
+  // acc = the convolution of the rows at src (element offset), NS_ steps per tap, STEPS_ in all.
+  auto convolve = [&](int src, auto ns, auto total) {
+    constexpr int NS_ = decltype(ns)::value, STEPS_ = decltype(total)::value;
+    int at[RT];
+    auto aim = [&](int tap) {
+      const int dy = tap / 3 - 1, dx = tap - tap / 3 * 3 - 1, x = (r & 7) + dx;
+#pragma unroll
+      for (int t = 0; t < RT; t++) {
+        const int y = (TILE * t + row0 >> 3 & 7) + dy;
+        const bool on = (unsigned)x < 8u && (unsigned)y < 8u && tap < 9;
+        at[t] = (on ? src + (t / PT * 64 + y * 8 + x) * LD : kZero) + V * g;
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+      for (int c = 0; c < CT; c++) acc[t][c] = Acc{};
+    Acc part[kFloat ? RT : 1][kFloat ? CT : 1];
+    intx4 a[2][RT][SUB];
+    auto load_rows = [&](intx4 (&x)[RT][SUB], int s) {
+#pragma unroll
+      for (int u = 0; u < SUB; u++)
+#pragma unroll
+        for (int t = 0; t < RT; t++) x[t][u] = *reinterpret_cast<const intx4*>(lds + at[t] + s * KS + u * (KS / SUB));
+    };
+    aim(0);
+    load_rows(a[0], 0);
+    for (int base = 0; base < STEPS_; base += kChunk) {
+#pragma unroll
+      for (int j = 0; j < kChunk; j++) {
+        if ((j + 1) % NS_ == 0) aim((base + j + 1) / NS_);   // (past the last tap: the zeros, not used)
+        load_rows(a[(j + 1) & 1], (j + 1) % NS_);
+        if constexpr (kFloat) {
+          if (j % NS_ == 0) {
+#pragma unroll
+            for (int t = 0; t < RT; t++)
+#pragma unroll
+              for (int c = 0; c < CT; c++) part[t][c] = Acc{};
+          }
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int t = 0; t < RT; t++)
+#pragma unroll
+              for (int c = 0; c < CT; c++)
+                part[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(floatx4, w[j % kRing][c])[e],
+                                                                  __builtin_bit_cast(floatx4, a[j & 1][t][0])[e], part[t][c], 0, 0, 0);
+          if ((j + 1) % NS_ == 0) {
+#pragma unroll
+            for (int t = 0; t < RT; t++)
+#pragma unroll
+              for (int c = 0; c < CT; c++) acc[t][c] += part[t][c];
+          }
+        } else {
+          using ev8 = typename Vec16<T>::v8;
+#pragma unroll
+          for (int u = 0; u < SUB; u++)
+#pragma unroll
+            for (int t = 0; t < RT; t++)
+#pragma unroll
+              for (int c = 0; c < CT; c++)
+                acc[t][c] = Mfma32(__builtin_bit_cast(ev8, w[j % kRing][c * SUB + u]), __builtin_bit_cast(ev8, a[j & 1][t][u]), acc[t][c]);
+        }
+#pragma unroll
+        for (int f = 0; f < F; f++) w[j % kRing][f] = ws[((j + kRing) * F + f) * 64];
+        // The next step's rows go out one by one between this step's products, and nothing moves to another step (the compiler's
+        // own order reads a fragment right before its products and waits for it).
+#pragma unroll
+        for (int i = 0; i < RT * SUB; i++) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, kFloat ? 4 * CT : CT, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      ws += kChunk * F * 64;
+    }
+  };
+  // Output channels ch0 + TILE c + 8 q .. + 3: element 4 q .. + 3 of acc[.][c].
+  auto load_bias = [&](int conv, floatx4 (&b)[CT][Q]) {
+#pragma unroll
+    for (int c = 0; c < CT; c++)
+#pragma unroll
+      for (int q = 0; q < Q; q++) b[c][q] = *reinterpret_cast<const floatx4*>(p.biases + (long long)conv * C + ch0 + TILE * c + 8 * q);
+  };
+  auto four = [&](int t, int c, int q) {
+    return floatx4{acc[t][c][4 * q], acc[t][c][4 * q + 1], acc[t][c][4 * q + 2], acc[t][c][4 * q + 3]};
+  };
+  auto store = [&](int dst, int t, int c, int q, const floatx4& v) {
+    *reinterpret_cast<Tv4*>(lds + dst + (TILE * t + row0) * LD + ch0 + TILE * c + 8 * q) = Tv4{(T)v[0], (T)v[1], (T)v[2], (T)v[3]};
+  };
+
+  floatx4 bias[CT][Q];
+  auto plain_tail = [&](int dst) {
+    TowerAct(p.act, [&](auto act) {
+#pragma unroll
+      for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int c = 0; c < CT; c++)
+#pragma unroll
+          for (int q = 0; q < Q; q++) {
+            const floatx4 v = four(t, c, q) + bias[c][q];
+            store(dst, t, c, q, floatx4{act(v[0]), act(v[1]), act(v[2]), act(v[3])});
+          }
+    });
+    __syncthreads();
+  };
+  load_bias(0, bias);
+  convolve(kOther, std::integral_constant<int, S::NS_IN>(), std::integral_constant<int, S::STEPS_IN>());
+  plain_tail(0);
+
+  for (int conv = 1; conv <= 2 * p.blocks; conv++) {
+    const bool second = (conv & 1) == 0;
+    load_bias(conv, bias);
+    convolve(second ? kOther : 0, std::integral_constant<int, S::NS>(), std::integral_constant<int, S::STEPS>());
+    if (!second) {
+      plain_tail(kOther);
+      continue;
+    }
+    const TowerSe se = p.se[conv / 2 - 1];
+    if (se.k > 0) {
+      // First layer: a wave does 16 hidden values, lane l value l % 16 and every fourth vector of the channels. Second layer: a
+      // thread does four outputs and every KP-th hidden value. The first weights of either are asked for a barrier early.
+      constexpr int S1 = C / 16, O4 = 2 * C / 4, KP = THREADS / O4, U = 16;
+      const int k_lane = lane & 15, v_lane = lane >> 4, o4 = tid % O4, kp = tid / O4;
+      floatx4 w1[S1], w2[U];
+      auto load_w1 = [&](int k0) {
+        const float* w = se.w1 + (long long)min(k0 + k_lane, se.k - 1) * C + 4 * v_lane;
+#pragma unroll
+        for (int i = 0; i < S1; i++) w1[i] = *reinterpret_cast<const floatx4*>(w + 16 * i);
+      };
+      auto load_w2 = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          w2[u] = *reinterpret_cast<const floatx4*>(se.w2 + (long long)min(k0 + u * KP, se.k - 1) * 2 * C + 4 * o4);
+      };
+      load_w1(16 * wave);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < POS; b++)
+#pragma unroll
+        for (int c = 0; c < CT; c++)
+#pragma unroll
+          for (int q = 0; q < Q; q++) {
+            floatx4 s = four(b * PT, c, q);
+#pragma unroll
+            for (int t = 1; t < PT; t++) s += four(b * PT + t, c, q);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              s[e] = Sum16(s[e]);
+              if (TILE == 32) s[e] += __shfl_xor(s[e], 16, 64);
+              s[e] = s[e] * (1.0f / 64.0f) + (rg == 0 ? bias[c][q][e] : 0.0f);
+            }
+            if (r == 0) *reinterpret_cast<floatx4*>(&pool[rg][b][ch0 + TILE * c + 8 * q]) = s;
+          }
+      __syncthreads();
+      for (int k0 = 16 * wave; k0 < se.k; k0 += 16 * kWaves * RG) {
+        if (k0 > 16 * wave) load_w1(k0);
+#pragma unroll
+        for (int b = 0; b < POS; b++) {
+          floatx4 h4 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int i = 0; i < S1; i++) {
+            floatx4 x = *reinterpret_cast<const floatx4*>(&pool[0][b][16 * i + 4 * v_lane]);
+#pragma unroll
+            for (int j = 1; j < RG; j++) x += *reinterpret_cast<const floatx4*>(&pool[j][b][16 * i + 4 * v_lane]);
+            h4 += w1[i] * x;
+          }
+          float h = (h4[0] + h4[1]) + (h4[2] + h4[3]);
+          h += __shfl_xor(h, 16, 64);
+          h += __shfl_xor(h, 32, 64);
+          const int k = k0 + k_lane;
+          if (v_lane == 0 && k < se.k) TowerAct(p.act, [&](auto act) { hidden[b][k] = act(h + se.b1[k]); });
+        }
+      }
+      load_w2(kp);
+      __syncthreads();
+      floatx4 out[POS];
+#pragma unroll
+      for (int b = 0; b < POS; b++) out[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int k0 = kp; k0 < se.k; k0 += U * KP) {
+        if (k0 > kp) load_w2(k0);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int b = 0; b < POS; b++) {
+            const int k = k0 + u * KP;
+            const float h = hidden[b][min(k, se.k - 1)];
+            out[b] += w2[u] * (k < se.k ? h : 0.0f);
+          }
+      }
+      // The partial sums take the place of the block's inner activations: no wave reads those any more.
+      float* part = reinterpret_cast<float*>(lds + kOther);
+#pragma unroll
+      for (int b = 0; b < POS; b++) *reinterpret_cast<floatx4*>(part + (kp * POS + b) * 2 * C + 4 * o4) = out[b];
+      __syncthreads();
+      for (int i = tid; i < POS * 2 * C; i += THREADS) {
+        const int b = i / (2 * C), o = i % (2 * C);
+        float v = se.b2[o];
+#pragma unroll
+        for (int j = 0; j < KP; j++) v += part[j * POS * 2 * C + i];
+        scale_shift[b][o / C][o % C] = o < C ? 1.0f / (1.0f + __expf(-v)) : v;
+      }
+      __syncthreads();
+    }
+    TowerAct(p.act, [&](auto act) {
+#pragma unroll
+      for (int b = 0; b < POS; b++)
+#pragma unroll
+        for (int c = 0; c < CT; c++)
+#pragma unroll
+          for (int q = 0; q < Q; q++) {
+            const int ch = ch0 + TILE * c + 8 * q;
+            floatx4 gamma = {1.0f, 1.0f, 1.0f, 1.0f}, beta = bias[c][q];
+            if (se.k > 0) {
+              gamma = *reinterpret_cast<const floatx4*>(&scale_shift[b][0][ch]);
+              beta = *reinterpret_cast<const floatx4*>(&scale_shift[b][1][ch]) + gamma * bias[c][q];
+            }
+#pragma unroll
+            for (int t = b * PT; t < (b + 1) * PT; t++) {
+              const Tv4 skip = *reinterpret_cast<const Tv4*>(lds + (TILE * t + row0) * LD + ch);
+              const floatx4 y = four(t, c, q);
+              floatx4 v;
+#pragma unroll
+              for (int e = 0; e < 4; e++) v[e] = act(gamma[e] * y[e] + beta[e] + (float)skip[e]);
+              store(0, t, c, q, v);
+            }
+          }
+    });
+    __syncthreads();
+  }
+
+  T* out = static_cast<T*>(p.out) + (long long)pos0 * 64 * C;
+  for (int i = tid; i < R * (C / V); i += THREADS) {
+    const int row = i / (C / V), v = i % (C / V);
+    if (pos0 + row / 64 < p.batch)
+      *reinterpret_cast<intx4*>(out + (long long)row * C + v * V) = *reinterpret_cast<const intx4*>(lds + row * LD + v * V);
+  }
+}
+
+template <typename T, int C>
+long long FragmentIndex(int blocks, int conv, int tap, int out, int in) {
+  using S = TowerShape<T, C>;
+  const long long steps = S::STEPS_IN + 2LL * blocks * S::STEPS;
+  const int wave = out / (S::TILE * S::CT), c = out / S::TILE % S::CT, sub = in % S::KS / (S::G * S::V);
+  const long long first = conv == 0 ? 0 : S::STEPS_IN + (conv - 1LL) * S::STEPS;
+  const long long step = wave * steps + first + tap * (conv == 0 ? S::NS_IN : S::NS) + in / S::KS;
+  return ((step * S::F + c * S::SUB + sub) * 64 + in / S::V % S::G * S::TILE + out % S::TILE) * S::V + in % S::V;
+}
+template <typename T, int C>
+long long Fragments(int blocks) {   // (and a turn's worth that is asked for past the end)
+  using S = TowerShape<T, C>;
+  return ((S::STEPS_IN + 2LL * blocks * S::STEPS) * kWaves + kChunk) * S::F * 64 * S::V;
+}
+
+}  // namespace
+
+bool TowerSupported(int filters, bool f32) { return filters == (f32 ? 64 : 256); }
+
+long long TowerFragments(int blocks, bool f32) { return f32 ? Fragments<float, 64>(blocks) : Fragments<half_t, 256>(blocks); }
+
+long long TowerFragmentIndex(int blocks, bool f32, int conv, int tap, int out, int in) {
+  return f32 ? FragmentIndex<float, 64>(blocks, conv, tap, out, in) : FragmentIndex<half_t, 256>(blocks, conv, tap, out, in);
+}
+
+// From how many positions on the kernel is faster than winograd convolutions, whose launches spread few positions over more CUs,
+// and up to how many. us a batch through the interface, winograd and this: 20x256 halves 3 positions 680 / 715, 13 696 / 725, 32 811 / 702,
+// 64 963 / 712, 256 1457 / 929, 512 2163 / 1558, 1000 3661 / 2984; 6x64 floats 3 187 / 206, 32 228 / 221, 64 272 / 245, 256 514 / 358, 512
+// 725 / 654, 600 813 / 869, 1000 1174 / 1217.
+bool TowerFaster(int batch, bool f32) { return f32 ? batch > 24 && batch <= 512 : batch > 16; }
+
+// Halves: full rounds of 256 workgroups with two positions each, then the rest, with one position each where that makes one round
+// of cheaper workgroups (20x256: a round of one 0.8 ms, of two 1.4 ms).
+void LaunchTower(const TowerArgs& a, bool f32, hipStream_t stream) {
+  if (a.batch <= 0) return;
+  if (a.blocks < 1 || (a.act != kActMish && a.act != kActRelu)) throw std::runtime_error("LaunchTower: no kernel");
+  if (f32) {
+    resident_tower_kernel<float, 64, 1, 2><<<dim3(a.batch), dim3(128 * kWaves), 0, stream>>>(a);
+    return;
+  }
+  const int rest = a.batch % 512, pairs = rest > 256 ? a.batch : a.batch - rest;
+  if (pairs > 0) {
+    TowerArgs b = a;
+    b.batch = pairs;
+    resident_tower_kernel<half_t, 256, 2, 1><<<dim3((pairs + 1) / 2), dim3(64 * kWaves), 0, stream>>>(b);
+  }
+  if (pairs < a.batch) {
+    TowerArgs b = a;
+    b.batch = a.batch - pairs;
+    b.masks += 112LL * pairs;
+    b.values += 112LL * pairs;
+    b.out = static_cast<half_t*>(a.out) + 64LL * 256 * pairs;
+    resident_tower_kernel<half_t, 256, 1, 1><<<dim3(b.batch), dim3(64 * kWaves), 0, stream>>>(b);
+  }
+}
+
+}  // namespace lc0mi

@@ -175,6 +175,36 @@ def test_random_residual_tower_shapes_match_oracle(seed, positions, tmp_path):
                  tie_flips=3)
 
 
+@pytest.mark.parametrize("filters,options,se,mish,batch", [
+    (256, "precision=fp16", 64, False, 1), (256, "precision=fp16", 0, True, 3), (256, "precision=fp16", 8, False, 259),
+    (256, "precision=fp16", 200, True, 515), (64, "precision=fp32", 16, False, 1), (64, "precision=fp32", 0, False, 5),
+    (64, "precision=fp32", 250, True, 300)])
+def test_tower_in_one_kernel_matches_oracle(filters, options, se, mish, batch, positions, tmp_path):
+    """The tower as one kernel, at one and two positions per workgroup (256 half filters: two from 257 positions on, odd counts and
+    a rest after 512 among them), with and without squeeze-and-excitation of widths that fill no whole tile. Eight positions
+    are repeated, so that every workgroup is compared with the oracle; the bounds are those of the other towers."""
+    from lc0_amd import netproto
+    net = netgen.se_resnet(filters, 2, se, seed=7000 + filters + se)
+    if mish:
+        net["format"]["network_format"]["default_activation"] = 1
+    path = str(tmp_path / "net.pb.gz")
+    netproto.write_pb_gz(path, net)
+    rows = np.arange(batch) % 8
+    want = onn.BlasNetwork(nr.load(path)).forward(positions["masks"][:8], positions["values"][:8])
+    net, res = _run_gpu(path, positions["masks"][rows], positions["values"][rows], options + ",resident_tower=1")
+    want = {k: v[rows] for k, v in want.items() if v is not None}
+    legal = [positions["legal"][i] for i in rows]
+    if "fp32" in options:
+        _compare(res, want, legal, tol=1e-3)
+    else:
+        _compare(res, want, legal, tie_flips=3 * ((batch + 7) // 8))
+    net.SetProfiling(True)
+    comp = net.NewComputation()
+    comp.AddInputs(positions["masks"][:2], positions["values"][:2])
+    comp.ComputeBlocking()
+    assert "resident_tower" in str(net.TakeProfile())
+
+
 @pytest.mark.parametrize("name,batch,options", [("tiny_attn", 37, ""), ("c2_bt4_15x1024", 33, ""),
                                                 ("tiny_attn_f8", 21, "precision=fp8,")])
 def test_smolgen_generator_inside_attention_and_as_a_gemm_of_its_own(name, batch, options, positions):
