@@ -58,6 +58,19 @@ __device__ __forceinline__ float Sum16(float v) {
 // of zeros. Four times the multiplications of winograd F(4x4,3x3), but no transforms, no winograd domain in memory (2 x 38 MB
 // per convolution at 512 positions) and no launches; and sums in float over all of a convolution, where the winograd products
 // of a half tower are rounded to halves twice. Float sums run over one tap at a time, to keep the chains short.
+//
+// Split: with one wave per SIMD each takes 64 channels of all rows, so that a weight fragment and a row fragment are both used
+// twice or more (two positions, a 64-byte step: 512 cycles of products, 256 of LDS reads, 256 of weights at 64 bytes a cycle); half
+// the channels per wave would read the rows twice as often. One position per workgroup has half the products for the same
+// weights and serves up to one round of the CUs. 64 float channels: two waves per SIMD with half the rows each, which hide the
+// ends of a tap (243 -> 221 us a pass of 32 positions).
+// What bounds it, in cycles of a wave over the 20x256 tower: two positions 2.80 M, of which products 1.47 M (1.75 M with
+// the waits between them), squeeze-and-excitation 0.72 M (192 KiB of float weights per block and workgroup, four barriers), the
+// additions of skip, bias and activation 0.31 M; with all CUs busy the clock falls to 1.9 GHz on top. One position 1.46 M, products
+// 0.74 M. 6x64 in floats 0.35 M, products 0.26 M. 512 positions: 1.04 PFLOP/s of direct products over a round of 1.5 ms, and 24 us
+// per transform and 22 us per product of 36 x 2048x256x256 before.
+// Tried and not kept: the next squeeze-and-excitation weights touched during a convolution, so that they wait in the L2 (the stream
+// waits for them in order: 512 positions 1558 -> 1727 us a pass); zeros in the banks of the rows they stand for (level).
 // ---------------------------------------------------------------------------
 template <typename T, int C, int POS, int RG>
 __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(TowerArgs p) {
@@ -68,12 +81,14 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
   constexpr int Q = TILE * TILE / 256;                   // a lane's output channels of a tile: Q times four, 8 apart
   using Acc = std::conditional_t<sizeof(T) == 4, floatx4, floatx16>;
   constexpr int kRing = POS == 1 ? 8 : 4;                // steps of weights in flight
+  constexpr int H = POS == 1 ? SUB : 1, ST = SUB / H;    // fragments of a tile that are read ahead together, and such reads in a step
   constexpr bool kFloat = sizeof(T) == 4;
   using Tv4 = T __attribute__((ext_vector_type(4)));
   constexpr int kOther = R * LD, kZero = 2 * R * LD;     // the two activation buffers, then a row of zeros
   __shared__ __attribute__((aligned(16))) T lds[2 * R * LD + LD];
   __shared__ __attribute__((aligned(16))) float pool[RG][POS][C];
   __shared__ float hidden[POS][kTowerMaxSe];
+  __shared__ __attribute__((aligned(16))) float biases[2][C];   // of this convolution and the next
   __shared__ __attribute__((aligned(16))) float scale_shift[POS][2][C];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), cg = wave % kWaves, rg = wave / kWaves;
@@ -115,6 +130,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
       }
     }
     if (tid < LD / V) *reinterpret_cast<intx4*>(lds + kZero + tid * V) = intx4{0, 0, 0, 0};
+    if (tid < C) biases[0][tid] = p.biases[tid];
   }
   __syncthreads();
 
@@ -137,71 +153,78 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
 #pragma unroll
       for (int c = 0; c < CT; c++) acc[t][c] = Acc{};
     Acc part[kFloat ? RT : 1][kFloat ? CT : 1];
-    intx4 a[2][RT][SUB];
-    auto load_rows = [&](intx4 (&x)[RT][SUB], int s) {
+    intx4 a[2][RT][H];
+    auto load_rows = [&](intx4 (&x)[RT][H], int s, int u0) {
 #pragma unroll
-      for (int u = 0; u < SUB; u++)
+      for (int h = 0; h < H; h++)
 #pragma unroll
-        for (int t = 0; t < RT; t++) x[t][u] = *reinterpret_cast<const intx4*>(lds + at[t] + s * KS + u * (KS / SUB));
+        for (int t = 0; t < RT; t++) x[t][h] = *reinterpret_cast<const intx4*>(lds + at[t] + s * KS + (u0 + h) * (KS / SUB));
     };
     aim(0);
-    load_rows(a[0], 0);
+    load_rows(a[0], 0, 0);
     for (int base = 0; base < STEPS_; base += kChunk) {
 #pragma unroll
       for (int j = 0; j < kChunk; j++) {
-        if ((j + 1) % NS_ == 0) aim((base + j + 1) / NS_);   // (past the last tap: the zeros, not used)
-        load_rows(a[(j + 1) & 1], (j + 1) % NS_);
-        if constexpr (kFloat) {
-          if (j % NS_ == 0) {
 #pragma unroll
-            for (int t = 0; t < RT; t++)
+        for (int st = 0; st < ST; st++) {
+          const int now = (j * ST + st) & 1;
+          if (st == ST - 1 && (j + 1) % NS_ == 0) aim((base + j + 1) / NS_);   // (past the last tap: the zeros, not used)
+          load_rows(a[now ^ 1], (j + (st + 1) / ST) % NS_, (st + 1) % ST * H);
+          if constexpr (kFloat) {
+            if (j % NS_ == 0) {
 #pragma unroll
-              for (int c = 0; c < CT; c++) part[t][c] = Acc{};
+              for (int t = 0; t < RT; t++)
+#pragma unroll
+                for (int c = 0; c < CT; c++) part[t][c] = Acc{};
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+              for (int t = 0; t < RT; t++)
+#pragma unroll
+                for (int c = 0; c < CT; c++)
+                  part[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(floatx4, w[j % kRing][c])[e],
+                                                                    __builtin_bit_cast(floatx4, a[now][t][0])[e], part[t][c], 0, 0, 0);
+            if ((j + 1) % NS_ == 0) {
+#pragma unroll
+              for (int t = 0; t < RT; t++)
+#pragma unroll
+                for (int c = 0; c < CT; c++) acc[t][c] += part[t][c];
+            }
+          } else {
+            using ev8 = typename Vec16<T>::v8;
+#pragma unroll
+            for (int h = 0; h < H; h++)
+#pragma unroll
+              for (int t = 0; t < RT; t++)
+#pragma unroll
+                for (int c = 0; c < CT; c++)
+                  acc[t][c] = Mfma32(__builtin_bit_cast(ev8, w[j % kRing][c * SUB + st * H + h]), __builtin_bit_cast(ev8, a[now][t][h]),
+                                     acc[t][c]);
           }
+          if (st == ST - 1) {
 #pragma unroll
-          for (int e = 0; e < 4; e++)
-#pragma unroll
-            for (int t = 0; t < RT; t++)
-#pragma unroll
-              for (int c = 0; c < CT; c++)
-                part[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(floatx4, w[j % kRing][c])[e],
-                                                                  __builtin_bit_cast(floatx4, a[j & 1][t][0])[e], part[t][c], 0, 0, 0);
-          if ((j + 1) % NS_ == 0) {
-#pragma unroll
-            for (int t = 0; t < RT; t++)
-#pragma unroll
-              for (int c = 0; c < CT; c++) acc[t][c] += part[t][c];
+            for (int f = 0; f < F; f++) w[j % kRing][f] = ws[((j + kRing) * F + f) * 64];
           }
-        } else {
-          using ev8 = typename Vec16<T>::v8;
+          // The next rows go out one by one between these products, and nothing moves past them (the compiler's own order reads a
+          // fragment right before its products and waits for it).
 #pragma unroll
-          for (int u = 0; u < SUB; u++)
-#pragma unroll
-            for (int t = 0; t < RT; t++)
-#pragma unroll
-              for (int c = 0; c < CT; c++)
-                acc[t][c] = Mfma32(__builtin_bit_cast(ev8, w[j % kRing][c * SUB + u]), __builtin_bit_cast(ev8, a[j & 1][t][u]), acc[t][c]);
+          for (int i = 0; i < RT * H; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, kFloat ? 4 * CT : CT, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int f = 0; f < F; f++) w[j % kRing][f] = ws[((j + kRing) * F + f) * 64];
-        // The next step's rows go out one by one between this step's products, and nothing moves to another step (the compiler's
-        // own order reads a fragment right before its products and waits for it).
-#pragma unroll
-        for (int i = 0; i < RT * SUB; i++) {
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, kFloat ? 4 * CT : CT, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
       }
       ws += kChunk * F * 64;
     }
   };
   // Output channels ch0 + TILE c + 8 q .. + 3: element 4 q .. + 3 of acc[.][c].
-  auto load_bias = [&](int conv, floatx4 (&b)[CT][Q]) {
-#pragma unroll
-    for (int c = 0; c < CT; c++)
-#pragma unroll
-      for (int q = 0; q < Q; q++) b[c][q] = *reinterpret_cast<const floatx4*>(p.biases + (long long)conv * C + ch0 + TILE * c + 8 * q);
+  auto bias4 = [&](int conv, int c, int q) { return *reinterpret_cast<const floatx4*>(&biases[conv & 1][ch0 + TILE * c + 8 * q]); };
+  float next_bias = 0.0f;
+  auto ask_bias = [&](int conv) { next_bias = p.biases[(long long)min(conv, 2 * p.blocks) * C + tid % C]; };
+  auto keep_bias = [&](int conv) {
+    if (tid < C) biases[conv & 1][tid] = next_bias;
   };
   auto four = [&](int t, int c, int q) {
     return floatx4{acc[t][c][4 * q], acc[t][c][4 * q + 1], acc[t][c][4 * q + 2], acc[t][c][4 * q + 3]};
@@ -210,8 +233,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
     *reinterpret_cast<Tv4*>(lds + dst + (TILE * t + row0) * LD + ch0 + TILE * c + 8 * q) = Tv4{(T)v[0], (T)v[1], (T)v[2], (T)v[3]};
   };
 
-  floatx4 bias[CT][Q];
-  auto plain_tail = [&](int dst) {
+  auto plain_tail = [&](int conv, int dst) {
     TowerAct(p.act, [&](auto act) {
 #pragma unroll
       for (int t = 0; t < RT; t++)
@@ -219,22 +241,23 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
         for (int c = 0; c < CT; c++)
 #pragma unroll
           for (int q = 0; q < Q; q++) {
-            const floatx4 v = four(t, c, q) + bias[c][q];
+            const floatx4 v = four(t, c, q) + bias4(conv, c, q);
             store(dst, t, c, q, floatx4{act(v[0]), act(v[1]), act(v[2]), act(v[3])});
           }
     });
+    keep_bias(conv + 1);
     __syncthreads();
   };
-  load_bias(0, bias);
+  ask_bias(1);
   convolve(kOther, std::integral_constant<int, S::NS_IN>(), std::integral_constant<int, S::STEPS_IN>());
-  plain_tail(0);
+  plain_tail(0, 0);
 
   for (int conv = 1; conv <= 2 * p.blocks; conv++) {
     const bool second = (conv & 1) == 0;
-    load_bias(conv, bias);
+    ask_bias(conv + 1);
     convolve(second ? kOther : 0, std::integral_constant<int, S::NS>(), std::integral_constant<int, S::STEPS>());
     if (!second) {
-      plain_tail(kOther);
+      plain_tail(conv, kOther);
       continue;
     }
     const TowerSe se = p.se[conv / 2 - 1];
@@ -262,16 +285,17 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
         for (int c = 0; c < CT; c++)
 #pragma unroll
           for (int q = 0; q < Q; q++) {
+            const floatx4 bias = bias4(conv, c, q);
             floatx4 s = four(b * PT, c, q);
 #pragma unroll
             for (int t = 1; t < PT; t++) s += four(b * PT + t, c, q);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
               s[e] = Sum16(s[e]);
-              if (TILE == 32) s[e] += __shfl_xor(s[e], 16, 64);
-              s[e] = s[e] * (1.0f / 64.0f) + (rg == 0 ? bias[c][q][e] : 0.0f);
+              if (TILE == 32) s[e] += DppMove<0x142>(s[e]);   // (the row of lanes before: the upper 16 hold the sum of 32)
+              s[e] = s[e] * (1.0f / 64.0f) + (rg == 0 ? bias[e] : 0.0f);
             }
-            if (r == 0) *reinterpret_cast<floatx4*>(&pool[rg][b][ch0 + TILE * c + 8 * q]) = s;
+            if (r == TILE - 16) *reinterpret_cast<floatx4*>(&pool[rg][b][ch0 + TILE * c + 8 * q]) = s;
           }
       __syncthreads();
       for (int k0 = 16 * wave; k0 < se.k; k0 += 16 * kWaves * RG) {
@@ -331,10 +355,10 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
 #pragma unroll
           for (int q = 0; q < Q; q++) {
             const int ch = ch0 + TILE * c + 8 * q;
-            floatx4 gamma = {1.0f, 1.0f, 1.0f, 1.0f}, beta = bias[c][q];
+            floatx4 gamma = {1.0f, 1.0f, 1.0f, 1.0f}, beta = bias4(conv, c, q);
             if (se.k > 0) {
               gamma = *reinterpret_cast<const floatx4*>(&scale_shift[b][0][ch]);
-              beta = *reinterpret_cast<const floatx4*>(&scale_shift[b][1][ch]) + gamma * bias[c][q];
+              beta = *reinterpret_cast<const floatx4*>(&scale_shift[b][1][ch]) + gamma * beta;
             }
 #pragma unroll
             for (int t = b * PT; t < (b + 1) * PT; t++) {
@@ -347,6 +371,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
             }
           }
     });
+    keep_bias(conv + 1);
     __syncthreads();
   }
 
@@ -384,9 +409,9 @@ long long TowerFragmentIndex(int blocks, bool f32, int conv, int tap, int out, i
 }
 
 // From how many positions on the kernel is faster than winograd convolutions, whose launches spread few positions over more CUs,
-// and up to how many. us a batch through the interface, winograd and this: 20x256 halves 3 positions 680 / 715, 13 696 / 725, 32 811 / 702,
-// 64 963 / 712, 256 1457 / 929, 512 2163 / 1558, 1000 3661 / 2984; 6x64 floats 3 187 / 206, 32 228 / 221, 64 272 / 245, 256 514 / 358, 512
-// 725 / 654, 600 813 / 869, 1000 1174 / 1217.
+// and up to how many. us a batch through the interface, winograd and this: 20x256 halves 1 position 639 / 683, 13 686 / 726, 32 850 / 702,
+// 200 1426 / 840, 256 1477 / 943, 300 1777 / 1285, 512 2146 / 1571, 600 2601 / 2240, 768 3008 / 2446, 1000 3505 / 3061; 6x64 floats 1 175 /
+// 199, 16 205 / 209, 32 225 / 216, 64 263 / 234, 256 509 / 352, 512 728 / 636, and before the last trim 600 813 / 869, 1000 1174 / 1217.
 bool TowerFaster(int batch, bool f32) { return f32 ? batch > 24 && batch <= 512 : batch > 16; }
 
 // Halves: full rounds of 256 workgroups with two positions each, then the rest, with one position each where that makes one round
