@@ -52,7 +52,7 @@ WORKLOADS = {
     "c1_attn_10x256": dict(batch=64, desc="attention body: 10 layers, d=256, 8 heads, dff 1024, fp16"),
     "c0_resnet_6x64": dict(batch=32, options="precision=fp32", dtype="fp32",
                            desc="SE-ResNet 6x64, SE ratio 4, classical policy, WDL, fp32"),
-    "c3_resnet_20x256": dict(batch=512, desc="SE-ResNet 20x256, SE ratio 4, winograd F(4x4,3x3), fp16"),
+    "c3_resnet_20x256": dict(batch=512, desc="SE-ResNet 20x256, SE ratio 4, fp16"),
     "c4_bt4_fp8": dict(batch=1024, net="c2_bt4_15x1024", options="precision=fp8", dtype="fp8_e4m3",
                        desc="BT4-shape attention body with e4m3 operands (fp32 accumulation) in the QKV, attention-output "
                             "and FFN GEMMs; weights scaled per output row, activations per tensor; the rest fp16"),
@@ -257,7 +257,7 @@ def main():
     net.SetProfiling(False)
     total_kernel_ms = sum(k.ms for k in prof) / prof_iters
     kernels = sorted(prof, key=lambda k: -k.ms)
-    matrix = [k for k in prof if k.name.startswith("gemm") or k.name in ("attention", "smolgen_attention")]
+    matrix = [k for k in prof if k.name.startswith(("gemm", "tower", "encoder_tail")) or k.name in ("attention", "smolgen_attention", "qkv_attention")]
     gemm_ms = sum(k.ms for k in matrix) / prof_iters
     gemm_flops = sum(k.flops for k in matrix) / prof_iters
     # Group call sites by the kernel that ran them ("call_site|kernel_variant"): the
@@ -271,7 +271,7 @@ def main():
         groups[variant] = Agg(variant, g.ms + k.ms, g.launches + k.launches, g.flops + k.flops, g.bytes + k.bytes)
     dom = max(groups.values(), key=lambda g: g.ms)
     peak = (PEAK_FP8_TFLOPS if dom.name.startswith("gemm_f8") else
-            PEAK_FP32_TFLOPS if dom.name.startswith("gemm_f32") else PEAK_FP16_TFLOPS)   # (bf16 has the fp16 peak)
+            PEAK_FP32_TFLOPS if dom.name.startswith("gemm_f32") or dom.name.endswith("_f32") else PEAK_FP16_TFLOPS)   # (bf16 has the fp16 peak)
     # A matrix kernel is priced against the MFMA peak only when its flops per algorithmic byte lie above the ridge
     # point peak flops / peak bandwidth (fp16: 312 flop/B); below it the memory roofline is the one that bounds it
     # (the 36 batched winograd-domain GEMMs of a 256-filter convolution: 121 flop/B).

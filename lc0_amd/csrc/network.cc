@@ -1934,7 +1934,7 @@ void Mi355xNetwork::ForwardResnet(int B) {
     t.masks = d_masks_; t.values = d_values_; t.biases = tower_biases_; t.packed = tower_packed_; t.se = tower_se_;
     t.out = r_x_; t.batch = B; t.blocks = static_cast<int>(res_blocks_.size()); t.act = default_act_;
     const double convs = 9.0 * filters_ * (kInputPlanes + 2.0 * filters_ * t.blocks);
-    Timed("resident_tower", 2.0 * 64 * B * convs, sizeof(T) * convs + B * (112.0 * 12 + sizeof(T) * 64.0 * filters_),
+    Timed(fp32_ ? "tower|resident_tower_f32" : "tower|resident_tower", 2.0 * 64 * B * convs, sizeof(T) * convs + B * (112.0 * 12 + sizeof(T) * 64.0 * filters_),
           [&] { LaunchTower(t, fp32_, stream_); });
   } else {
     have_v = ForwardTowerWinograd<T>(B);

@@ -64,11 +64,10 @@ __device__ __forceinline__ float Sum16(float v) {
 // the channels per wave would read the rows twice as often. One position per workgroup has half the products for the same
 // weights and serves up to one round of the CUs. 64 float channels: two waves per SIMD with half the rows each, which hide the
 // ends of a tap (243 -> 221 us a pass of 32 positions).
-// What bounds it, in cycles of a wave over the 20x256 tower: two positions 2.80 M, of which products 1.47 M (1.75 M with
-// the waits between them), squeeze-and-excitation 0.72 M (192 KiB of float weights per block and workgroup, four barriers), the
-// additions of skip, bias and activation 0.31 M; with all CUs busy the clock falls to 1.9 GHz on top. One position 1.46 M, products
-// 0.74 M. 6x64 in floats 0.35 M, products 0.26 M. 512 positions: 1.04 PFLOP/s of direct products over a round of 1.5 ms, and 24 us
-// per transform and 22 us per product of 36 x 2048x256x256 before.
+// What bounds it, by cycle counters over the 20x256 tower: two positions 52 % products, 10 % waits between them, 26 %
+// squeeze-and-excitation (192 KiB of float weights per block and workgroup, four barriers), 11 % additions of skip and bias and
+// activations; with all CUs busy the clock falls to 1.9 GHz on top. One position 50 % products, 6x64 in floats 75 %. A round of 512
+// positions takes 1.25 ms (1.2 PFLOP/s of direct products), where 41 transforms of 24 us and 40 launches of 36 x 2048x256x256 of 22 took 1.86.
 // Tried and not kept: the next squeeze-and-excitation weights touched during a convolution, so that they wait in the L2 (the stream
 // waits for them in order: 512 positions 1558 -> 1727 us a pass); zeros in the banks of the rows they stand for (level).
 // ---------------------------------------------------------------------------

@@ -205,6 +205,18 @@ def test_tower_in_one_kernel_matches_oracle(filters, options, se, mish, batch, p
     assert "resident_tower" in str(net.TakeProfile())
 
 
+@pytest.mark.parametrize("name,options,batch,tol", [("c3_resnet_20x256", "precision=fp16", 140, 5e-3), ("c0_resnet_6x64", "precision=fp32", 40, 1e-3)])
+def test_towers_of_the_one_kernel_as_winograd_convolutions(name, options, batch, tol, positions):
+    """The shapes that the tower kernel takes, on the winograd convolutions that it takes over from (products with resident weights from
+    512 rows up): against the oracle on the first eight positions and the last eight of the batch, the same ones again."""
+    path = netgen.cached_config(name)
+    rows = np.concatenate([np.arange(8), np.arange(batch - 16) % 60, np.arange(8)])
+    want = onn.BlasNetwork(nr.load(path)).forward(positions["masks"][:8], positions["values"][:8])
+    _, res = _run_gpu(path, positions["masks"][rows], positions["values"][rows], options + ",resident_tower=0")
+    for part in (slice(0, 8), slice(batch - 8, batch)):
+        _compare({k: v[part] for k, v in res.items()}, want, positions["legal"][:8], tol=tol)
+
+
 @pytest.mark.parametrize("name,batch,options", [("tiny_attn", 37, ""), ("c2_bt4_15x1024", 33, ""),
                                                 ("tiny_attn_f8", 21, "precision=fp8,")])
 def test_smolgen_generator_inside_attention_and_as_a_gemm_of_its_own(name, batch, options, positions):
