@@ -102,7 +102,8 @@ const char* lc0mi_last_error(void);
 /* Turns per-kernel HIP-event timing of subsequent compute calls on or off. */
 int lc0mi_net_set_profiling(lc0mi_net* net, int on);
 /* Writes the accumulated per-kernel records as text lines
- * "name ms launches flops bytes\n" into buf (truncated to cap, NUL-terminated),
+ * "name ms launches flops bytes\n" into buf (truncated to cap, NUL-terminated;
+ * 0 ms and 0 launches: a layer that shares the launch of another record),
  * clears them and returns the number of bytes needed. */
 int lc0mi_net_take_profile(lc0mi_net* net, char* buf, int cap);
 /* Re-runs the device pass for `batch` positions already resident in HBM `iters`

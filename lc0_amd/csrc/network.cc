@@ -148,11 +148,15 @@ struct Linear;
 struct LinearF8;
 // With one given, nothing is launched unless the launch takes both.
 struct SecondProduct {
+  const char* name = nullptr;   // in profiles
   const Linear* lin = nullptr;
   const LinearF8* f8 = nullptr;
   void* C = nullptr;
   float out_mul = 1.0f;
 };
+
+constexpr int kOverlapMinBatch = 80;                              // option overlap_min_batch
+constexpr int kCompressWithQkvMaxBatch = kOverlapMinBatch - 1;   // largest batch whose compression is such a second product
 
 int RoundUp(int v, int m) { return (v + m - 1) / m * m; }
 
@@ -460,6 +464,8 @@ class Mi355xNetwork : public Network, protected ModelState {
   // Launch helpers (profiling aware).
   template <typename F>
   void Timed(const char* name, double flops, double bytes, F&& launch, hipStream_t st = nullptr);
+  void TimedElsewhere(const std::string& name, double flops, double bytes);
+  void AddToProfile(const KernelTime& t);
   bool Gemm(const char* name, const half_t* A, int lda, const Linear& lin, void* C, int ldc, int M, int act,
             bool out_f32 = false, hipStream_t st = nullptr, int split_k = 1, bool latency_first = false,
             const NormFold* fold = nullptr, int out_stores = kStoresAuto, const SecondProduct& second = {});
@@ -573,19 +579,28 @@ void Mi355xNetwork::Timed(const char* name, double flops, double bytes, F&& laun
   pending_.push_back(p);
 }
 
+// Work done inside the launch of another label, whose time holds it.
+void Mi355xNetwork::TimedElsewhere(const std::string& name, double flops, double bytes) {
+  if (profiling_) AddToProfile(KernelTime{name, 0.0, 0, flops, bytes});
+}
+
+void Mi355xNetwork::AddToProfile(const KernelTime& t) {
+  auto it = std::find_if(profile_.begin(), profile_.end(), [&](const KernelTime& k) { return k.name == t.name; });
+  if (it == profile_.end()) {
+    profile_.push_back(t);
+    return;
+  }
+  it->ms += t.ms;
+  it->launches += t.launches;
+  it->flops += t.flops;
+  it->bytes += t.bytes;
+}
+
 void Mi355xNetwork::CollectPending() {
   for (Pending& p : pending_) {
     float ms = 0.0f;
     HIP_CHECK(hipEventElapsedTime(&ms, p.start, p.stop));
-    auto it = std::find_if(profile_.begin(), profile_.end(), [&](const KernelTime& k) { return k.name == p.name; });
-    if (it == profile_.end()) {
-      profile_.push_back(KernelTime{p.name, 0.0, 0, 0.0, 0.0});
-      it = profile_.end() - 1;
-    }
-    it->ms += ms;
-    it->launches += 1;
-    it->flops += p.flops;
-    it->bytes += p.bytes;
+    AddToProfile(KernelTime{p.name, ms, 1, p.flops, p.bytes});
     event_pool_.push_back(p.start);
     event_pool_.push_back(p.stop);
   }
@@ -725,14 +740,15 @@ bool Mi355xNetwork::Gemm(const char* name, const half_t* A, int lda, const Linea
     if (!GemmTakesSecond(g)) return false;
   }
   if (fold != nullptr && fold->parts_out != nullptr) *fold->parts_out = GemmStatsParts(g);
-  const double flops = 2.0 * M * (lin.out + g.N2) * lin.in;
+  const double flops = 2.0 * M * lin.out * lin.in;
   const double bytes = 2.0 * (static_cast<double>(M) * lin.in + static_cast<double>(lin.out) * lin.in) +
                        static_cast<double>(M) * lin.out * (out_f32 ? 4 : 2) +
                        (fold != nullptr && fold->skip != nullptr ? 2.0 * M * lin.out : 0.0);
-  std::string label = std::string(name) + "|" + GemmVariantName(g);
-  if (fold != nullptr) label += fold->skip != nullptr ? "+skip_stats" : "+row_norm";
-  if (g.N2 > 0) label += "+second";
-  Timed(label.c_str(), flops, bytes, [&] { LaunchGemm(g, st); }, st);
+  std::string variant = std::string("|") + GemmVariantName(g);
+  if (fold != nullptr) variant += fold->skip != nullptr ? "+skip_stats" : "+row_norm";
+  if (g.N2 > 0) variant += "+second";
+  Timed((name + variant).c_str(), flops, bytes, [&] { LaunchGemm(g, st); }, st);
+  if (g.N2 > 0) TimedElsewhere(second.name + variant, 2.0 * M * g.N2 * lin.in, 2.0 * g.N2 * (M + lin.in));
   return g.N2 > 0;
 }
 
@@ -904,11 +920,12 @@ bool Mi355xNetwork::GemmF8(const char* name, const uint8_t* A, const Linear& lin
     g.out_mul2 = second.out_mul;
     if (!GemmF8TakesSecond(g)) return false;
   }
-  const double flops = 2.0 * M * (lin.out + g.N2) * lin.in;
+  const double flops = 2.0 * M * lin.out * lin.in;
   const double bytes = static_cast<double>(M) * lin.in + static_cast<double>(lin.out) * lin.in +
                        static_cast<double>(M) * lin.out * (out_f8 ? 1 : 2);
-  const std::string label = std::string(name) + "|" + GemmF8VariantName(g) + (g.N2 > 0 ? "+second" : "");
-  Timed(label.c_str(), flops, bytes, [&] { LaunchGemmF8(g, st); }, st);
+  const std::string variant = std::string("|") + GemmF8VariantName(g) + (g.N2 > 0 ? "+second" : "");
+  Timed((name + variant).c_str(), flops, bytes, [&] { LaunchGemmF8(g, st); }, st);
+  if (g.N2 > 0) TimedElsewhere(second.name + variant, 2.0 * M * g.N2 * lin.in, 1.0 * g.N2 * (M + lin.in));
   return g.N2 > 0;
 }
 
@@ -1136,7 +1153,7 @@ Mi355xNetwork::Mi355xNetwork(const WeightsFile& file, Options& options) {
   // against beside the projection: fp16 batch 8 1.26 against 1.45 ms, batch 64 2.50 against 2.53, batch 96 3.43
   // against 3.24; fp8 batch 64 2.00 against 2.25, batch 96 2.60 against 2.54).
   overlap_min_batch_ = options.GetInt("overlap_min_batch", -1);
-  if (overlap_min_batch_ < 0) overlap_min_batch_ = 80;
+  if (overlap_min_batch_ < 0) overlap_min_batch_ = kOverlapMinBatch;
   heads_overlap_min_batch_ = options.GetInt("heads_overlap_min_batch", -1);
   lane_count_ = options.GetInt("lanes", 4);
   if (lane_count_ < 1 || lane_count_ > 8) throw Error("lanes must be in 1..8.");
@@ -2093,14 +2110,16 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       return Gemm("gemm_qkv", x_, emb_, norm_in ? e.qkv_n : e.qkv, qkv_, 3 * d_model_, T, kActNone, false, nullptr, 1, false,
                   norm_in ? &cons_in : nullptr, keep, second);
     };
-    // On one stream, the smolgen compression (a few columns of the same rows) is a second product of the projection's
+    // With few positions the smolgen compression (a few columns of the same rows) is a second product of the projection's
     // launch where its workgroups find free CUs (GemmTakesSecond): one launch less in a chain of dependent ones. us of a
     // 15x1024 pass, own launch -> with the projection: fp16 1 position 923 -> 833, 13 1296 -> 1230, 21 1574 -> 1502, 48 2219 ->
-    // 2136; e4m3 1 791 -> 729, 16 979 -> 929, 48 1545 -> 1486. (Not when profiling: every layer then has a launch and a time of
-    // its own.)
+    // 2136; e4m3 1 791 -> 729, 16 979 -> 929, 48 1545 -> 1486. Its sums are added in another order than in a launch of its own, so
+    // nothing but the batch decides: a pass has the same bits on one stream and on two, beside other passes and when profiled. The
+    // limit is where the chain leaves the projection's stream by default: beside the projection it has no launch to save.
     bool with_compress = false;
-    if (e.has_smolgen && ss == stream_ && compress_with_qkv_ && !profiling_ && !norm_in && !calibrating_ && chain_f8 == (f8 && q_qkv_)) {
+    if (e.has_smolgen && B <= kCompressWithQkvMaxBatch && compress_with_qkv_ && !norm_in && !calibrating_ && chain_f8 == (f8 && q_qkv_)) {
       SecondProduct compress;
+      compress.name = "gemm_smolgen_compress";
       compress.lin = &e.sg_compress;
       compress.f8 = &e.sg_compress8;
       compress.C = chain_f8 ? static_cast<void*>(sg1q_) : sg1_;
@@ -2115,7 +2134,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       const int g = sg_gen_ / heads_;
       if (ss != stream_) {
         HIP_CHECK(hipEventRecord(fork_events_[li], stream_));
-        if (qkv_before_chain) launch_qkv();
+        if (qkv_before_chain && !with_compress) launch_qkv();
         HIP_CHECK(hipStreamWaitEvent(ss, fork_events_[li], 0));
       }
       // The chain is the critical path of this phase when the QKV projection beside it is short (e4m3 operands,

@@ -84,7 +84,7 @@ class Options {
 struct KernelTime {
   std::string name;
   double ms = 0.0;       // summed HIP-event time of all launches with this label
-  int launches = 0;
+  int launches = 0;      // 0: work inside the launches of another label, which have its time
   double flops = 0.0;    // algorithmic flops of those launches
   double bytes = 0.0;    // algorithmic bytes moved by those launches
 };

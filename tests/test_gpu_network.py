@@ -871,6 +871,74 @@ def test_concurrent_computations_from_several_threads(name, options, positions):
             np.testing.assert_array_equal(got[key][field], w[field])
 
 
+def _evaluate(net, positions, n, at=0):
+    idx = (np.arange(n) * 3 + at) % 320
+    comp = net.NewComputation()
+    comp.AddInputs(positions["masks"][idx], positions["values"][idx])
+    comp.ComputeBlocking()
+    res = comp.results()
+    comp.close()
+    return res
+
+
+def _names_of_a_profiled_pass(net, positions, n, at=0):
+    net.SetProfiling(True)
+    res = _evaluate(net, positions, n, at)
+    names = [k.name for k in net.TakeProfile()]
+    net.SetProfiling(False)
+    return names, res
+
+
+@pytest.fixture(scope="module")
+def smolgen_nets(tmp_path_factory):
+    """Two layers of the published shape at two widths: with few positions their launches are those of the full-size nets."""
+    from lc0_amd import netproto
+    paths = {}
+    for emb in (256, 1024):
+        paths[emb] = str(tmp_path_factory.mktemp("nets") / ("smolgen_%d.pb.gz" % emb))
+        netproto.write_pb_gz(paths[emb], netgen.attention_body(emb, 2, emb // 32, 512, seed=2030 + emb, smolgen=(32, 256, 256),
+                                                               perturb_ln=True, std=0.5 * emb ** -0.5))
+    return paths
+
+
+@pytest.mark.parametrize("emb,options", [(256, ""), (1024, ""), (1024, "precision=fp8,")])
+def test_a_pass_has_the_same_bits_beside_others_on_other_streams_and_profiled(emb, options, smolgen_nets, positions):
+    """Which kernels run follows from the batch alone. Beside another thread's passes a computation keeps to one stream, options
+    move the smolgen chain to another one, a profiled pass uses one stream: the results are bitwise those of a lone pass, around
+    the batch from which the chain has its own stream and at the sizes where the compression shares the projection's launch."""
+    import threading
+    from lc0_amd import Network
+    net = Network(smolgen_nets[emb], options + "lanes=2")
+    sizes = (1, 13, 33, 48, 64, 79, 80, 85, 92, 98, 110, 118, 128)
+    want = {n: _evaluate(net, positions, n) for n in sizes}
+    stop, errors = threading.Event(), []
+
+    def others():
+        try:
+            while not stop.is_set():
+                _evaluate(net, positions, 320)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    th = threading.Thread(target=others)
+    th.start()
+    try:
+        beside = [(n, _evaluate(net, positions, n)) for _ in range(4) for n in sizes]
+    finally:
+        stop.set()
+        th.join()
+    assert not errors, errors
+    profiled = [(n, _names_of_a_profiled_pass(net, positions, n)[1]) for n in sizes]
+    moved = []
+    for chain in (0, 100000):
+        other = Network(smolgen_nets[emb], options + "overlap_min_batch=%d" % chain)
+        moved += [(n, _evaluate(other, positions, n)) for n in sizes]
+    for what, runs in (("beside", beside), ("profiled", profiled), ("moved", moved)):
+        for n, res in runs:
+            for field in ("policy", "q", "d", "m"):
+                np.testing.assert_array_equal(res[field], want[n][field], err_msg="%s %s %d" % (what, field, n))
+
+
 @pytest.mark.parametrize("name,batch", [("tiny_attn_d64", 40), ("tiny_resnet_attnpolicy", 33)])
 def test_head_depth_64_policy_encoders_and_attention_policy_on_a_tower(name, batch, positions):
     """tiny_attn_d64: attention heads of depth 64 and two encoder layers inside the policy head
