@@ -5,6 +5,7 @@
 //                                                                   blas/network_blas.cc:441-486, blas/encoder.h:29-66
 #include "kernel_common.h"
 
+#include <algorithm>
 #include <stdexcept>
 #include <type_traits>
 
@@ -24,7 +25,7 @@ constexpr int kPad = 8;   // 16-bit values between the rows of an LDS tile: 16-b
 // the 16 queries from 16 w of both heads. V is multiplied with its operands exchanged, so that it comes out transposed, as the
 // second product wants it.
 // Bound by latency and by the 130 KiB of rows and weights a workgroup reads. us back to back at width 256 (8 heads): 1 position 5.7,
-// 64 6.6, 256 16.2, 1024 48 (34 GFLOP: 710 TFLOP/s).
+// 64 6.6, 256 16.2, 1024 48 (30 GFLOP: 626 TFLOP/s).
 // ---------------------------------------------------------------------------
 template <typename ET, int C>
 __global__ __launch_bounds__(256, 2) void qkv_attention_kernel(const half_t* __restrict__ x, const half_t* __restrict__ packed,
@@ -163,8 +164,10 @@ __global__ __launch_bounds__(256, 2) void qkv_attention_kernel(const half_t* __r
 // Bound by the weight stream (1.18 MB at width 256, d_model 256 and 1024 hidden columns; a CU takes 64 bytes per cycle from L2,
 // here 88 GB/s per CU) up to 32 rows per workgroup, with 64 rows by that, the matrix cores and the LDS reads alike. us back to back at
 // that width: 16 rows on 4 CUs 13.3, on 256 CUs 16.3; 32 rows on 256 CUs 19.8; 64 rows on 256 CUs 27.9 = 690 TFLOP/s. A pass
-// of the 10x256 net, seven kernels per layer -> these two: 1 position 294 -> 290, 16 389 -> 305, 64 477 -> 330, 256 926 -> 526, 1024 2687
-// -> 1690. One launch at a width of 512 or more would stream more bytes through every CU than the separate products take.
+// of the 10x256 net, seven kernels per layer -> these two: 16 positions 389 -> 305, 64 477 -> 330, 256 926 -> 526, 1024 2687 -> 1690
+// (below five positions: EncoderTailMinBatch); of ten layers of width 128 (4 heads, 512 hidden columns) 1 361 -> 209, 64 452 -> 250, 256
+// 740 -> 471, 1000 1946 -> 1270, with smolgen, where only this kernel is used, 64 654 -> 497, 1000 3721 -> 3166; width 256 with smolgen
+// 64 712 -> 606, 1000 4986 -> 4216. One launch at a width of 512 or more would stream more bytes through every CU than the separate products take.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void MergeMoments(float& mean, float& m2, float mean_b, float m2_b, float n) {
   const float d = mean_b - mean;   // (two sets of n values each)
@@ -412,6 +415,16 @@ bool EncoderTailSupported(int emb, int d_model, int dff) {
 // 16 rows per workgroup while they all fit the CUs, else 32, else 64: a workgroup takes the weights through its CU once
 // whatever its rows, so more of them per workgroup cost nothing until their products take longer than the stream.
 int EncoderTailRows(int M) { return M <= 16 * 256 ? 16 : M <= 32 * 256 ? 32 : 64; }
+
+// A few workgroups stream all weights through one CU each, whatever the batch, where five launches spread them over the chip;
+// how many positions that costs follows from their bytes. us of a ten-layer pass, layers one by one -> the kernel. Width 256,
+// 0.66 MB (512 hidden columns) 1 position 275 -> 255; 1.2 MB (1024) 1 287 -> 304, 4 302 -> 311, 8 341 -> 310, with smolgen 1 440 ->
+// 453, 4 463 -> 469, 8 559 -> 522; 2.2 MB (2048) 1 305 -> 406, 12 392 -> 411, 16 386 -> 410, 24 460 -> 418. Width 128, whose own
+// products have short reductions, 0.3 MB 1 292 -> 200, 1.1 MB (2048) 1 330 -> 319, 16 378 -> 329.
+int EncoderTailMinBatch(int emb, int d_model, int dff) {
+  const int kib = 2 * emb * (d_model + 2 * dff) / 1024;
+  return emb <= 128 ? 1 : std::max(1, (kib - 768 + 79) / 80);
+}
 
 long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_model) {
   // Parts of emb x emb: those of the output projection, then of the FFN's two layers in turn.

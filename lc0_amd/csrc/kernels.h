@@ -306,6 +306,7 @@ struct EncoderTailArgs {
 };
 bool EncoderTailSupported(int emb, int d_model, int dff);
 int EncoderTailRows(int M);   // rows of a workgroup
+int EncoderTailMinBatch(int emb, int d_model, int dff);   // smallest batch at which it is faster than its layers one by one
 long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_model);
 void LaunchEncoderTail(const EncoderTailArgs& args, hipStream_t stream);
 

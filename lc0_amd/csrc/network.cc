@@ -2285,7 +2285,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       } else {
         Timed("attention", att_flops, att_bytes, [&] { Attention(qkv_, bias, att_, B, heads_, depth_, stream_); });
       }
-      if (e.tail_packed != nullptr) {
+      if (e.tail_packed != nullptr && B >= EncoderTailMinBatch(emb_, d_model_, dff_)) {
         EncoderTailArgs a;
         a.att = att_; a.packed = e.tail_packed; a.x = x_;
         a.dense_b = e.dense.b; a.ffn1_b = e.ffn1.b; a.ffn2_b = e.ffn2.b;

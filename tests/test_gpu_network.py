@@ -939,6 +939,21 @@ def test_a_pass_has_the_same_bits_beside_others_on_other_streams_and_profiled(em
                 np.testing.assert_array_equal(res[field], want[n][field], err_msg="%s %s %d" % (what, field, n))
 
 
+@pytest.mark.parametrize("dff,smolgen,first", [(512, None, 1), (1024, None, 5), (1024, (32, 256, 256), 5), (2048, None, 18)])
+def test_rest_of_a_layer_is_one_kernel_from_as_many_positions_as_its_weights_need(dff, smolgen, first, positions, tmp_path):
+    """The kernel streams a layer's weights through every CU that it uses: with few positions and many weights the layers one by
+    one are faster. Both sides of the line against the oracle, by the names in the profile."""
+    from lc0_amd import Network, netproto
+    path = str(tmp_path / "net.pb.gz")
+    netproto.write_pb_gz(path, netgen.attention_body(256, 2, 8, dff, seed=2050, smolgen=smolgen, perturb_ln=True, std=0.03))
+    net, bn = Network(path), onn.BlasNetwork(nr.load(path))
+    for n in sorted({1, max(first - 1, 1), first}):
+        names, res = _names_of_a_profiled_pass(net, positions, n)
+        assert ("encoder_tail" in names) == (n >= first) and any(k.startswith("gemm_ffn1") for k in names) == (n < first), (n, names)
+        idx = (np.arange(n) * 3) % 320
+        _compare(res, bn.forward(positions["masks"][idx], positions["values"][idx]), [positions["legal"][i] for i in idx])
+
+
 @pytest.mark.parametrize("name,batch", [("tiny_attn_d64", 40), ("tiny_resnet_attnpolicy", 33)])
 def test_head_depth_64_policy_encoders_and_attention_policy_on_a_tower(name, batch, positions):
     """tiny_attn_d64: attention heads of depth 64 and two encoder layers inside the policy head
