@@ -420,12 +420,12 @@ struct TowerArgs {
   const void* packed = nullptr;
   const TowerSe* se = nullptr;
   void* out = nullptr;
-  int batch = 0, blocks = 0, act = 2;
+  int batch = 0, blocks = 0, filters = 0, act = 2;
 };
 bool TowerSupported(int filters, bool f32);
-long long TowerFragments(int blocks, bool f32);
-long long TowerFragmentIndex(int blocks, bool f32, int conv, int tap, int out, int in);
-bool TowerFaster(int batch, bool f32);   // than winograd convolutions
+long long TowerFragments(int blocks, int filters, bool f32);
+long long TowerFragmentIndex(int blocks, int filters, bool f32, int conv, int tap, int out, int in);
+bool TowerFaster(int batch, int filters, bool f32);   // than winograd convolutions
 void LaunchTower(const TowerArgs& args, bool f32, hipStream_t stream);
 
 // Gather of the convolutional policy head: out[b][j] = t[b][sq][plane] for

@@ -1802,13 +1802,13 @@ void Mi355xNetwork::BuildResnet(const WeightsFile& file) {
   }
   if (!res_blocks_.empty() && resident_tower_ != 0 && TowerSupported(filters_, fp32_)) {
     const int blocks = static_cast<int>(res_blocks_.size());
-    std::vector<T> packed(TowerFragments(blocks, fp32_), (T)0.0f);
+    std::vector<T> packed(TowerFragments(blocks, filters_, fp32_), (T)0.0f);
     Vec biases;
     auto pack = [&](int conv, const ConvBlock& cb, int cin) {
       for (int o = 0; o < filters_; o++)
         for (int i = 0; i < cin; i++)
           for (int tap = 0; tap < 9; tap++) {
-            packed[TowerFragmentIndex(blocks, fp32_, conv, tap, o, i)] = (T)cb.weights[(static_cast<size_t>(o) * cin + i) * 9 + tap];
+            packed[TowerFragmentIndex(blocks, filters_, fp32_, conv, tap, o, i)] = (T)cb.weights[(static_cast<size_t>(o) * cin + i) * 9 + tap];
           }
       biases.insert(biases.end(), cb.biases.begin(), cb.biases.end());
     };
@@ -1946,10 +1946,10 @@ template <typename T>
 void Mi355xNetwork::ForwardResnet(int B) {
   const int T64 = B * 64;
   bool have_v = false;
-  if (tower_packed_ != nullptr && (resident_tower_ == 1 || TowerFaster(B, fp32_))) {
+  if (tower_packed_ != nullptr && (resident_tower_ == 1 || TowerFaster(B, filters_, fp32_))) {
     TowerArgs t;
     t.masks = d_masks_; t.values = d_values_; t.biases = tower_biases_; t.packed = tower_packed_; t.se = tower_se_;
-    t.out = r_x_; t.batch = B; t.blocks = static_cast<int>(res_blocks_.size()); t.act = default_act_;
+    t.out = r_x_; t.batch = B; t.blocks = static_cast<int>(res_blocks_.size()); t.filters = filters_; t.act = default_act_;
     const double convs = 9.0 * filters_ * (kInputPlanes + 2.0 * filters_ * t.blocks);
     Timed(fp32_ ? "tower|resident_tower_f32" : "tower|resident_tower", 2.0 * 64 * B * convs, sizeof(T) * convs + B * (112.0 * 12 + sizeof(T) * 64.0 * filters_),
           [&] { LaunchTower(t, fp32_, stream_); });

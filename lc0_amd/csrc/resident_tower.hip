@@ -400,42 +400,60 @@ long long Fragments(int blocks) {   // (and a turn's worth that is asked for pas
 
 }  // namespace
 
-bool TowerSupported(int filters, bool f32) { return filters == (f32 ? 64 : 256); }
+// 64 float, 128 and 256 half filters. A wave takes whole tiles of TILE channels, so there are 64 n float or 128 n half filters
+// (not 64 in halves); a turn of kChunk steps does whole taps, so a tap has one, two, four or eight (not 192 or 256 floats, 384
+// halves). 128 float filters fit but gain nothing: one position per workgroup is 0.87 ms of products on its CU
+// (us of a 10x128 pass, winograd / this: 8 positions 313 / 880, 64 487 / 914, 256 937 / 1032, 512 1543 / 2013).
+bool TowerSupported(int filters, bool f32) { return f32 ? filters == 64 : filters == 128 || filters == 256; }
 
-long long TowerFragments(int blocks, bool f32) { return f32 ? Fragments<float, 64>(blocks) : Fragments<half_t, 256>(blocks); }
+long long TowerFragments(int blocks, int filters, bool f32) {
+  if (f32) return Fragments<float, 64>(blocks);
+  return filters == 128 ? Fragments<half_t, 128>(blocks) : Fragments<half_t, 256>(blocks);
+}
 
-long long TowerFragmentIndex(int blocks, bool f32, int conv, int tap, int out, int in) {
-  return f32 ? FragmentIndex<float, 64>(blocks, conv, tap, out, in) : FragmentIndex<half_t, 256>(blocks, conv, tap, out, in);
+long long TowerFragmentIndex(int blocks, int filters, bool f32, int conv, int tap, int out, int in) {
+  if (f32) return FragmentIndex<float, 64>(blocks, conv, tap, out, in);
+  return filters == 128 ? FragmentIndex<half_t, 128>(blocks, conv, tap, out, in) : FragmentIndex<half_t, 256>(blocks, conv, tap, out, in);
 }
 
 // From how many positions on the kernel is faster than winograd convolutions, whose launches spread few positions over more CUs,
-// and up to how many. us a batch through the interface, winograd and this: 20x256 halves 1 position 639 / 683, 13 686 / 726, 32 850 / 702,
-// 200 1426 / 840, 256 1477 / 943, 300 1777 / 1285, 512 2146 / 1571, 600 2601 / 2240, 768 3008 / 2446, 1000 3505 / 3061; 6x64 floats 1 175 /
-// 199, 16 205 / 209, 32 225 / 216, 64 263 / 234, 256 509 / 352, 512 728 / 636, and before the last trim 600 813 / 869, 1000 1174 / 1217.
-bool TowerFaster(int batch, bool f32) { return f32 ? batch > 24 && batch <= 512 : batch > 16; }
+// and up to how many. us a batch through the interface, winograd / this. 20x256 halves 1 position 639 / 683, 13 686 / 726, 32 850 / 702,
+// 200 1426 / 840, 512 2146 / 1571, 1000 3505 / 3061; 10x256 without squeeze-and-excitation 13 299 / 309, 17 328 / 307, 64 454 / 319, 512
+// 1158 / 876, 1000 1993 / 1606; 10x128 1 284 / 195, 8 302 / 199, 64 392 / 217, 256 655 / 319, 512 915 / 518, 1000 1338 / 963, mish without
+// squeeze-and-excitation 8 261 / 183, 1000 1332 / 929; 6x64 floats 1 175 / 199, 16 205 / 209, 32 229 / 221, 64 267 / 243, 256 513 / 349, without
+// squeeze-and-excitation 24 213 / 205, 64 254 / 229. With 257 to 512 float positions a second round is 6 to 13 % faster alone
+// (512 718 / 637) but slower where passes overlap. Thousands of evals/s of two and of four threads, winograd / this: floats 32 233 / 224 and
+// 340 / 362, 64 400 / 432 and 567 / 660, 256 870 / 945 and 1260 / 1325, 512 1180 / 1017 and 1540 / 1385; 20x256 halves 17 40 / 44 and 58 / 66, 64 120 / 163
+// and 156 / 247, 512 313 / 366 and 321 / 406.
+bool TowerFaster(int batch, int filters, bool f32) { return f32 ? batch > 24 && batch <= 256 : filters <= 128 || batch > 16; }
+
+namespace {
+template <typename T, int C, int POS, int RG>
+void LaunchTowerT(TowerArgs a, int first, int count, hipStream_t stream) {
+  if (count <= 0) return;
+  a.masks += 112LL * first;
+  a.values += 112LL * first;
+  a.out = static_cast<T*>(a.out) + 64LL * C * first;
+  a.batch = count;
+  resident_tower_kernel<T, C, POS, RG><<<dim3((count + POS - 1) / POS), dim3(64 * kWaves * RG), 0, stream>>>(a);
+}
+}  // namespace
 
 // Halves: full rounds of 256 workgroups with two positions each, then the rest, with one position each where that makes one round
 // of cheaper workgroups (20x256: a round of one 0.8 ms, of two 1.4 ms).
 void LaunchTower(const TowerArgs& a, bool f32, hipStream_t stream) {
   if (a.batch <= 0) return;
-  if (a.blocks < 1 || (a.act != kActMish && a.act != kActRelu)) throw std::runtime_error("LaunchTower: no kernel");
-  if (f32) {
-    resident_tower_kernel<float, 64, 1, 2><<<dim3(a.batch), dim3(128 * kWaves), 0, stream>>>(a);
-    return;
+  if (a.blocks < 1 || (a.act != kActMish && a.act != kActRelu) || !TowerSupported(a.filters, f32)) {
+    throw std::runtime_error("LaunchTower: no kernel");
   }
+  if (f32) return LaunchTowerT<float, 64, 1, 2>(a, 0, a.batch, stream);
   const int rest = a.batch % 512, pairs = rest > 256 ? a.batch : a.batch - rest;
-  if (pairs > 0) {
-    TowerArgs b = a;
-    b.batch = pairs;
-    resident_tower_kernel<half_t, 256, 2, 1><<<dim3((pairs + 1) / 2), dim3(64 * kWaves), 0, stream>>>(b);
-  }
-  if (pairs < a.batch) {
-    TowerArgs b = a;
-    b.batch = a.batch - pairs;
-    b.masks += 112LL * pairs;
-    b.values += 112LL * pairs;
-    b.out = static_cast<half_t*>(a.out) + 64LL * 256 * pairs;
-    resident_tower_kernel<half_t, 256, 1, 1><<<dim3(b.batch), dim3(64 * kWaves), 0, stream>>>(b);
+  if (a.filters == 128) {
+    LaunchTowerT<half_t, 128, 2, 1>(a, 0, pairs, stream);
+    LaunchTowerT<half_t, 128, 1, 1>(a, pairs, a.batch - pairs, stream);
+  } else {
+    LaunchTowerT<half_t, 256, 2, 1>(a, 0, pairs, stream);
+    LaunchTowerT<half_t, 256, 1, 1>(a, pairs, a.batch - pairs, stream);
   }
 }
 

@@ -178,7 +178,8 @@ def test_random_residual_tower_shapes_match_oracle(seed, positions, tmp_path):
 @pytest.mark.parametrize("filters,options,se,mish,batch", [
     (256, "precision=fp16", 64, False, 1), (256, "precision=fp16", 0, True, 3), (256, "precision=fp16", 8, False, 259),
     (256, "precision=fp16", 200, True, 515), (64, "precision=fp32", 16, False, 1), (64, "precision=fp32", 0, False, 5),
-    (64, "precision=fp32", 250, True, 300)])
+    (64, "precision=fp32", 250, True, 300), (128, "precision=fp16", 32, False, 1), (128, "precision=fp16", 0, True, 259),
+    (128, "precision=fp16", 250, False, 515)])
 def test_tower_in_one_kernel_matches_oracle(filters, options, se, mish, batch, positions, tmp_path):
     """The tower as one kernel, at one and two positions per workgroup (256 half filters: two from 257 positions on, odd counts and
     a rest after 512 among them), with and without squeeze-and-excitation of widths that fill no whole tile. Eight positions
@@ -203,6 +204,20 @@ def test_tower_in_one_kernel_matches_oracle(filters, options, se, mish, batch, p
     comp.AddInputs(positions["masks"][:2], positions["values"][:2])
     comp.ComputeBlocking()
     assert "resident_tower" in str(net.TakeProfile())
+
+
+@pytest.mark.parametrize("filters,options,inside,outside", [(64, "precision=fp32", (25, 256), (24, 257)), (128, "precision=fp16", (1, 300), ()),
+                                                            (256, "precision=fp16", (17, 300), (16,)), (128, "precision=fp32", (), (64,)),
+                                                            (64, "precision=fp16", (), (64,)), (256, "precision=fp32", (), (64,))])
+def test_batches_that_the_tower_kernel_takes_by_itself(filters, options, inside, outside, positions, tmp_path):
+    """The widths that it has and the batches at which it is the faster one, by the names in the profile."""
+    from lc0_amd import Network, netproto
+    path = str(tmp_path / "net.pb.gz")
+    netproto.write_pb_gz(path, netgen.se_resnet(filters, 1, 16, seed=7100 + filters))
+    net = Network(path, options)
+    for n in inside + outside:
+        names, _ = _names_of_a_profiled_pass(net, positions, n)
+        assert any("resident_tower" in k for k in names) == (n in inside) and ("expand_planes" in names) == (n in outside), (n, names)
 
 
 @pytest.mark.parametrize("name,options,batch,tol", [("c3_resnet_20x256", "precision=fp16", 140, 5e-3), ("c0_resnet_6x64", "precision=fp32", 40, 1e-3)])
