@@ -408,8 +408,8 @@ bool WinogradFusedInputTransform(int C, int elem_size, int se_k);
 // A whole tower in one launch (resident_tower.hip): out[b][sq][c] after the last of `blocks` residual blocks, from the bit
 // planes. packed: TowerFragments() elements, the weight of convolution `conv` (0: input, then two per block), tap 3 y + x, output
 // and input channel at TowerFragmentIndex() and zeros elsewhere; biases: [1 + 2 blocks][filters]; se: one entry per block, k = 0
-// without squeeze-and-excitation, layers as above. act: mish or relu. Only where TowerSupported().
-constexpr int kTowerMaxSe = 256;
+// without squeeze-and-excitation, at most kTowerMaxSe, layers as above. act: mish or relu. Only where TowerSupported().
+constexpr int kTowerMaxSe = 256;   // (the caller checks it: the widths lie on the device)
 struct TowerSe {
   const float *w1 = nullptr, *b1 = nullptr, *w2 = nullptr, *b2 = nullptr;
   int k = 0;

@@ -1800,7 +1800,9 @@ void Mi355xNetwork::BuildResnet(const WeightsFile& file) {
     }
     res_blocks_.push_back(b);
   }
-  if (!res_blocks_.empty() && resident_tower_ != 0 && TowerSupported(filters_, fp32_)) {
+  int widest_se = 0;
+  for (const ResBlockDev& b : res_blocks_) widest_se = std::max(widest_se, b.se.k);
+  if (!res_blocks_.empty() && resident_tower_ != 0 && widest_se <= kTowerMaxSe && TowerSupported(filters_, fp32_)) {
     const int blocks = static_cast<int>(res_blocks_.size());
     std::vector<T> packed(TowerFragments(blocks, filters_, fp32_), (T)0.0f);
     Vec biases;

@@ -179,7 +179,8 @@ def test_random_residual_tower_shapes_match_oracle(seed, positions, tmp_path):
     (256, "precision=fp16", 64, False, 1), (256, "precision=fp16", 0, True, 3), (256, "precision=fp16", 8, False, 259),
     (256, "precision=fp16", 200, True, 515), (64, "precision=fp32", 16, False, 1), (64, "precision=fp32", 0, False, 5),
     (64, "precision=fp32", 250, True, 300), (128, "precision=fp16", 32, False, 1), (128, "precision=fp16", 0, True, 259),
-    (128, "precision=fp16", 250, False, 515)])
+    (128, "precision=fp16", 250, False, 515), (128, "precision=fp16", 256, False, 3), (256, "precision=fp16", 256, True, 2),
+    (64, "precision=fp32", 256, False, 2)])
 def test_tower_in_one_kernel_matches_oracle(filters, options, se, mish, batch, positions, tmp_path):
     """The tower as one kernel, at one and two positions per workgroup (256 half filters: two from 257 positions on, odd counts and
     a rest after 512 among them), with and without squeeze-and-excitation of widths that fill no whole tile. Eight positions
