@@ -588,16 +588,17 @@ def _legal_logit_rms(a, b, legal):
 
 
 FUSED_SMOLGEN_MIN_BATCH = 72   # default of the option fused_smolgen_min_batch
+SMOLGEN_FEW_MAX_BATCH = 64     # default of the option smolgen_few_max_batch
 
 
 def _emulation_of(path, net, gemms=None, batch=1, **kw):
     """oracle/fp8_net.py with the activation scales the backend is using and, unless told, with the smolgen chain in
-    e4m3 exactly when the backend reports scales for it: all four of its layers, or, from the batch size on at which
-    the default fp8_gemms=auto runs the generator layer inside the attention kernel, the first three."""
+    e4m3 exactly when the backend reports scales for it: all four of its layers, or the first three at the batch sizes where
+    the default fp8_gemms=auto runs the generator layer inside one of the two attention kernels that have it."""
     from oracle import fp8_net
     sc = net.Fp8Scales()
     if gemms is None:
-        chain = "smolgen_chain" if batch >= FUSED_SMOLGEN_MIN_BATCH else "smolgen"
+        chain = "smolgen" if SMOLGEN_FEW_MAX_BATCH < batch < FUSED_SMOLGEN_MIN_BATCH else "smolgen_chain"
         gemms = ALL_FP8_GEMMS + ((chain,) if (sc[:, 4:] != 1.0).any() else ())
     return fp8_net.Fp8BlasNetwork(nr.load(path), scales=sc[:, :4], smolgen_scales=sc[:, 4:], gemms=gemms, **kw)
 
@@ -968,6 +969,77 @@ def test_rest_of_a_layer_is_one_kernel_from_as_many_positions_as_its_weights_nee
         assert ("encoder_tail" in names) == (n >= first) and any(k.startswith("gemm_ffn1") for k in names) == (n < first), (n, names)
         idx = (np.arange(n) * 3) % 320
         _compare(res, bn.forward(positions["masks"][idx], positions["values"][idx]), [positions["legal"][i] for i in idx])
+
+
+FUSED_KERNELS = [
+    (1024, "compress_with_qkv", "false", "", 1, "+second", "gemm_smolgen_compress|"),
+    (1024, "compress_with_qkv", "false", "", 16, "+second", "gemm_smolgen_compress|"),
+    (1024, "compress_with_qkv", "false", "", 48, "+second", "gemm_smolgen_compress|"),
+    (256, "compress_with_qkv", "false", "", 33, "+second", "gemm_smolgen_compress|"),
+    (256, "dense2_norm_max_batch", "0", "", 13, "gemm_smolgen_dense2|gemm{}_norm", "gemm_smolgen_dense2|"),
+    (1024, "dense2_norm_max_batch", "0", "", 64, "gemm_smolgen_dense2|gemm{}_norm", "gemm_smolgen_dense2|"),
+    (1024, "generator_norm_max_batch", "0", "smolgen_few_max_batch=0", 13, "gemm_smolgen_global|gemm{}_norm", "gemm_smolgen_global|"),
+    (256, "generator_norm_max_batch", "0", "smolgen_few_max_batch=0", 32, "gemm_smolgen_global|gemm{}_norm", "gemm_smolgen_global|"),
+    (256, "smolgen_few_max_batch", "0", "", 5, "smolgen_attention_few", "attention"),
+    (1024, "smolgen_few_max_batch", "0", "", 64, "smolgen_attention_few", "attention"),
+    (1024, "fused_heads_max_batch", "0", "", 33, "value_heads", "gemm_value_fc1|"),
+    (256, "fused_heads_max_batch", "0", "", 200, "value_heads", "gemm_value_fc1|"),
+    (256, "narrow_layers", "false", "", 40, "encoder_tail", "gemm_ffn1|"),
+    (256, "narrow_layers", "false", "nosmolgen", 40, "qkv_attention", "gemm_qkv|")]
+
+
+@pytest.mark.parametrize("emb,option,off,base,batch,fused,separate,precision",
+                         [c + (p,) for c in FUSED_KERNELS for p in ("fp16", "bf16", "fp8") if (c[1], p) != ("narrow_layers", "fp8")])
+def test_kernels_of_several_layers_and_the_layers_one_by_one(emb, option, off, base, batch, fused, separate, precision, smolgen_nets,
+                                                             tmp_path, positions):
+    """Every option that turns one of the kernels of several layers off: with and without it against the oracle, and by the names in
+    the profile. Both are the same roundings to 16 bits but for those that the fused form keeps in float, so they differ from each
+    other by no more than either may differ from the oracle."""
+    from lc0_amd import Network, netproto
+    path = smolgen_nets[emb]
+    if base == "nosmolgen":
+        path, base = str(tmp_path / "net.pb.gz"), ""
+        netproto.write_pb_gz(path, netgen.attention_body(emb, 2, emb // 32, 512, seed=2060, perturb_ln=True, std=0.03))
+    idx = (np.arange(batch) * 3) % 320
+    legal = [positions["legal"][i] for i in idx]
+    want = onn.BlasNetwork(nr.load(path)).forward(positions["masks"][idx], positions["values"][idx])
+    fused = fused.format("_f8" if precision == "fp8" else "")
+    results = []
+    for extra in ("", ",%s=%s" % (option, off)):
+        net = Network(path, "precision=" + precision + ("," + base if base else "") + extra)
+        names, res = _names_of_a_profiled_pass(net, positions, batch)
+        is_fused = any(n.endswith(fused) if fused[0] == "+" else n.startswith(fused) for n in names)
+        is_separate = any(n.startswith(separate) and not n.endswith("+second") and "_norm" not in n if separate.endswith("|") else n == separate
+                          for n in names)
+        assert (is_fused, is_separate) == (not extra, bool(extra)), names
+        results.append(res)
+        if precision == "fp16":
+            _compare(res, want, legal)
+        elif precision == "fp8":
+            st = _fp8_report(res, want, legal)
+            assert st["logit_rms"] <= 0.1 * st["logit_std"] and st["kl_max"] <= 1e-3
+        else:
+            st = _fp8_report(res, want, legal)   # (bfloat16: eight bits against e4m3's four)
+            assert st["logit_rms"] <= 0.03 * st["logit_std"] and st["kl_max"] <= 1e-4
+    spread = float(want["policy"].std())
+    apart = float(np.sqrt(np.mean((results[0]["policy"] - results[1]["policy"]) ** 2)))
+    print("apart: %.2e of the spread" % (apart / spread))
+    assert apart <= {"fp16": 0.005, "bf16": 0.03, "fp8": 0.1}[precision] * spread
+
+
+def test_explicit_e4m3_generator_normalises_its_rows_itself_with_few_positions(smolgen_nets, positions):
+    """fp8_gemms=...+smolgen keeps the generator layer in e4m3, which no attention kernel has inside: up to 32 positions it takes its
+    row norm along. Against the emulation of the same arithmetic."""
+    from lc0_amd import Network
+    path, batch = smolgen_nets[1024], 24
+    gemms = ALL_FP8_GEMMS + ("smolgen",)
+    net = Network(path, "precision=fp8,fp8_gemms=" + "+".join(gemms))
+    names, res = _names_of_a_profiled_pass(net, positions, batch)
+    assert "gemm_smolgen_global|gemm_f8_norm" in names and "gemm_smolgen_dense2|gemm_f8_norm" in names, names
+    idx = (np.arange(batch) * 3) % 320
+    masks, values, legal = positions["masks"][idx], positions["values"][idx], [positions["legal"][i] for i in idx]
+    want = onn.BlasNetwork(nr.load(path)).forward(masks, values)
+    _check_fp8_against_emulation(res, _emulation_of(path, net, gemms=gemms).forward(masks, values), want, legal, "generator with its norm")
 
 
 @pytest.mark.parametrize("name,batch", [("tiny_attn_d64", 40), ("tiny_resnet_attnpolicy", 33)])
