@@ -169,12 +169,6 @@ __global__ __launch_bounds__(256, 2) void qkv_attention_kernel(const half_t* __r
 // 740 -> 471, 1000 1946 -> 1270, with smolgen, where only this kernel is used, 64 654 -> 497, 1000 3721 -> 3166; width 256 with smolgen
 // 64 712 -> 606, 1000 4986 -> 4216. One launch at a width of 512 or more would stream more bytes through every CU than the separate products take.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void MergeMoments(float& mean, float& m2, float mean_b, float m2_b, float n) {
-  const float d = mean_b - mean;   // (two sets of n values each)
-  m2 += m2_b + d * d * (0.5f * n);
-  mean = 0.5f * (mean + mean_b);
-}
-
 template <typename ET, int CT, int RT>
 __global__ __launch_bounds__(512) void encoder_tail_kernel(EncoderTailArgs p) {
   using ev8 = typename Vec16<ET>::v8;

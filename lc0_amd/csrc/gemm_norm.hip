@@ -15,14 +15,6 @@ namespace {
 
 constexpr int kNormK = 256;        // columns of the input rows
 
-// (mean, sum of squared differences from it) of two sets of n values each, merged. Exact in the order of the merges, and
-// free of the cancellation that a sum of squares has.
-__device__ __forceinline__ void MergeMoments(float& mean, float& m2, float mean_b, float m2_b, float n) {
-  const float d = mean_b - mean;
-  m2 += m2_b + d * d * (0.5f * n);
-  mean = 0.5f * (mean + mean_b);
-}
-
 // ---------------------------------------------------------------------------
 // C[m][n] = act(sum_k norm(A)[m][k] W[n][k] + bias[n]) with rows of 256 values, `group` consecutive rows normalised
 // together (1: smolgen's second dense layer, one row per position; the number of heads: the shared generator layer, whose

@@ -76,6 +76,13 @@ __device__ __forceinline__ float DppMove(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
 }
 
+// (mean, sum of squared differences from it) of two sets of n values each, merged, free of the cancellation that a sum of squares has.
+__device__ __forceinline__ void MergeMoments(float& mean, float& m2, float mean_b, float m2_b, float n) {
+  const float d = mean_b - mean;
+  m2 += m2_b + d * d * (0.5f * n);
+  mean = 0.5f * (mean + mean_b);
+}
+
 // Mean and 1 / sqrt(variance + eps) of row m from its partial (sum, sum of squares) pairs over n values.
 __device__ __forceinline__ void RowMeanRstd(const float* stats, int parts, long long m, int n, float eps, float& mean,
                                             float& rstd) {
