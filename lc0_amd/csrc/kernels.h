@@ -90,8 +90,9 @@ void LaunchGemm(const GemmArgs& args, hipStream_t stream);
 // epilogue), and the number of partial sums per row a producer launch writes to stats_out.
 bool GemmSupportsNormFolding(const GemmArgs& args);
 int GemmStatsParts(const GemmArgs& args);
-// Whether LaunchGemm serves a second product of N2 columns: the kernel it picks for the first one is for few rows, and
-// the workgroups of both fit the CUs with one each.
+// Whether LaunchGemm serves a second product of N2 columns: the kernel it picks for the first one is a row panel, and the
+// workgroups of both fit the CUs with one each; or it has tiles of up to 128 rows, and the second product's tiles add no
+// round of one workgroup per CU.
 bool GemmTakesSecond(const GemmArgs& args);
 // Name of the kernel variant LaunchGemm picks for these arguments (tile shape; "...+rest" when it cuts the product
 // along its rows into whole rounds of large tiles and a rest, GemmRowSplit() rows in the first launch).
@@ -114,15 +115,15 @@ struct GemmF8Args {
   bool out_f8 = false;
   float out_mul = 1.0f;
   int out_stores = kStoresAuto;
-  // A second product of the same A, as in GemmArgs, with e4m3 output: C2 = e4m3(col_scale2[n] * sum * out_mul2). N2, ldc2
-  // multiples of 4. Only with half output of the first product and where GemmF8TakesSecond().
+  // A second product of the same A, as in GemmArgs, with e4m3 output: C2 = e4m3(col_scale2[n] * sum * out_mul2). N2 and ldc2
+  // multiples of 4, ldw2 of 16. Only with half output of the first product and where GemmF8TakesSecond().
   const uint8_t* W2 = nullptr; int ldw2 = 0;
   void* C2 = nullptr; int ldc2 = 0;
   int N2 = 0;
   const float* col_scale2 = nullptr;
   float out_mul2 = 1.0f;
 };
-bool GemmF8TakesSecond(const GemmF8Args& args);
+bool GemmF8TakesSecond(const GemmF8Args& args);   // by the rule of GemmTakesSecond
 void LaunchGemmF8(const GemmF8Args& args, hipStream_t stream);
 const char* GemmF8VariantName(const GemmF8Args& args);
 
@@ -273,6 +274,20 @@ void LaunchSmolgenAttentionF8Out(const half_t* qkv, const half_t* gen, const hal
                                  float out_mul, int batch, int heads, int depth, int gen_sz, float scale,
                                  hipStream_t stream);
 
+// The same for few positions with the norm before the generator layer inside (smolgen_attention_few.hip): gen holds the rows of
+// heads * 256 values before the norm, gamma and beta as many floats. out: 16 bits, or with out_f8 e4m3(result * out_mul).
+// SmolgenAttentionFewSupported: head depth 32, a multiple of four heads up to 32, gen_sz 256.
+struct SmolgenFewArgs {
+  const half_t *qkv = nullptr, *gen = nullptr, *wfrag = nullptr;
+  const float *gamma = nullptr, *beta = nullptr;
+  void* out = nullptr;
+  int batch = 0, heads = 0;
+  float scale = 1.0f, eps = 1e-3f, out_mul = 1.0f;
+  bool bf16 = false, out_f8 = false;
+};
+bool SmolgenAttentionFewSupported(int heads, int depth, int gen_sz);
+void LaunchSmolgenAttentionFew(const SmolgenFewArgs& args, hipStream_t stream);
+
 // Encoder layers of narrow bodies in two kernels (encoder_narrow.hip), 16-bit types, 64 rows per position.
 //
 // out[b*64+i][h*32+d] = the attention of heads of depth 32 over x.W^T + bias (W, bias: the rows of Q, K and V one after the
@@ -309,20 +324,6 @@ int EncoderTailRows(int M);   // rows of a workgroup
 int EncoderTailMinBatch(int emb, int d_model, int dff);   // smallest batch at which it is faster than its layers one by one
 long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_model);
 void LaunchEncoderTail(const EncoderTailArgs& args, hipStream_t stream);
-
-// For few positions the same with the norm before the generator layer inside (smolgen_attention_few.hip): gen holds the rows of
-// heads * 256 values before the norm, gamma and beta as many floats. out: 16 bits, or with out_f8 e4m3(result * out_mul).
-// SmolgenAttentionFewSupported: head depth 32, a multiple of four heads up to 32, gen_sz 256.
-struct SmolgenFewArgs {
-  const half_t *qkv = nullptr, *gen = nullptr, *wfrag = nullptr;
-  const float *gamma = nullptr, *beta = nullptr;
-  void* out = nullptr;
-  int batch = 0, heads = 0;
-  float scale = 1.0f, eps = 1e-3f, out_mul = 1.0f;
-  bool bf16 = false, out_f8 = false;
-};
-bool SmolgenAttentionFewSupported(int heads, int depth, int gen_sz);
-void LaunchSmolgenAttentionFew(const SmolgenFewArgs& args, hipStream_t stream);
 
 // Value and moves-left heads of a 16-bit attention body (value_heads.hip), for few positions: per head
 //   out[b][o] = out_act(sum_n act(sum_k e[b][k] w_fc1[n][k] + b_fc1[n]) w_fc2[o][n] + b_fc2[o]),
