@@ -86,7 +86,7 @@ __device__ __forceinline__ void StoreOut16(void* dst, intx4 val) {
 // (3072x3072x1024 on 128x128 30.5 -> 32.5; 77 positions of the 15x1024 net 2830 -> 2874 a pass), and the 256-row tiles
 // lose 2 to 5 % (16384x1024x1024 35.4 -> 36.7): both keep the transfers at the head of the k-tile.
 template <int BM, int BN, int BKB, int WAVES_M, int WAVES_N, typename Args, typename OutT, int STORES = 0,
-          int EPI = 0, int NSTAGES = 2, typename ET = half_t, bool ALONE = false>
+          int EPI = 0, int NSTAGES = 2, typename ET = half_t, bool ALONE = false, bool TWO = false>
 // Second launch bound = waves per SIMD: with small wave tiles two workgroups share a CU
 // (4 waves per SIMD, at most 128 VGPRs) and overlap each other's prologue and epilogue.
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64,
@@ -130,8 +130,9 @@ void gemm_dma_kernel(Args p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  // Tiles past the columns of the first product belong to the second one (small tiles only).
-  constexpr bool TWO = BM < 256 && EPI == 0;
+  // With TWO tiles past the columns of the first product belong to a second one. (An instance of its own: the choice costs launches
+  // that have no second product, e4m3 19200x32x1024 on 128x64 tiles 11.5 us instead of 10.85, 300x8192x256 on 64x64 8.75 instead of 8.45.)
+  static_assert(!TWO || (BM < 256 && EPI == 0 && sizeof(OutT) == 2), "small tiles, 16-bit output");
   const int col_tiles = TWO ? (p.N + BN - 1) / BN : 0;
   const bool second = TWO && (int)blockIdx.y >= col_tiles;
   const int m0 = blockIdx.x * BM, n0 = (second ? blockIdx.y - col_tiles : blockIdx.y) * BN;
@@ -611,6 +612,13 @@ void LaunchGemmDma(const GemmArgs& a, hipStream_t stream) {
       if (a.row_stats != nullptr) {
         hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, BK * 2, WAVES_M, WAVES_N, GemmArgs, half_t, SF, 1, 2>), grid, block, 0,
                            stream, a);
+        return;
+      }
+    }
+    if constexpr (BM < 256 && BN >= 64) {
+      if (a.N2 > 0) {
+        hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, BK * 2, WAVES_M, WAVES_N, GemmArgs, ET, S, 0, NSTAGES, ET, ALONE, true>), grid,
+                           block, 0, stream, a);
         return;
       }
     }

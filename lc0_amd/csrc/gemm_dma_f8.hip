@@ -23,6 +23,13 @@ void LaunchGemmDmaF8Tile(const GemmF8Args& a, hipStream_t stream) {
     if (stores == 1) return launch(std::integral_constant<int, 1>{});
     if (stores == 2) return launch(std::integral_constant<int, 2>{});
   }
+  if constexpr (BM < 256) {
+    if (a.N2 > 0) {
+      hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, BKB, WAVES_M, WAVES_N, GemmF8Args, half_t, 0, 0, NSTAGES,
+                                          half_t, ALONE, true>), grid, block, 0, stream, a);
+      return;
+    }
+  }
   if (a.out_f8) {
     hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, BKB, WAVES_M, WAVES_N, GemmF8Args, uint8_t, 0, 0, NSTAGES,
                                         half_t, ALONE>), grid, block, 0, stream, a);

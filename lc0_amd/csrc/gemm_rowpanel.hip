@@ -28,7 +28,7 @@ inline RowPanelShape PickRowPanelShape(int M, int N, int batch) {
 // one or two steps; the partial sums are added in wave order through LDS, so results do
 // not depend on timing.
 // ---------------------------------------------------------------------------
-template <typename ET, int RT, int CT, int KS, typename OutT, typename Args>
+template <typename ET, int RT, int CT, int KS, typename OutT, typename Args, bool TWO>
 __global__ __launch_bounds__(64 * KS) void gemm_rowpanel_kernel(Args p) {
   constexpr bool F8 = std::is_same<ET, uint8_t>::value;
   constexpr int ES = F8 ? 1 : 2;
@@ -37,9 +37,9 @@ __global__ __launch_bounds__(64 * KS) void gemm_rowpanel_kernel(Args p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int ks = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
-  // Panels past the columns of the first product belong to the second one.
-  const int panels = (p.N + COLS - 1) / COLS;
-  const bool second = (int)blockIdx.y >= panels;
+  // With TWO panels past the columns of the first product belong to a second one.
+  const int panels = TWO ? (p.N + COLS - 1) / COLS : 0;
+  const bool second = TWO && (int)blockIdx.y >= panels;
   const int m0 = blockIdx.x * ROWS, n0 = (second ? blockIdx.y - panels : blockIdx.y) * COLS;
   const int M = p.M, N = second ? p.N2 : p.N, ldw = second ? p.ldw2 : p.ldw;
   const char* A = reinterpret_cast<const char*>(p.A) + (long long)m0 * p.lda * ES;
@@ -131,7 +131,13 @@ void LaunchPanel(const Args& a, int batch, hipStream_t stream) {
   auto launch = [&](auto rt_tag, auto ct_tag) {
     constexpr int RT = decltype(rt_tag)::value, CT = decltype(ct_tag)::value, KS = kPanelWaves<ET>;
     dim3 grid((a.M + 16 * RT - 1) / (16 * RT), (a.N + 16 * CT - 1) / (16 * CT) + (a.N2 + 16 * CT - 1) / (16 * CT), batch);
-    hipLaunchKernelGGL((gemm_rowpanel_kernel<ET, RT, CT, KS, OutT, Args>), grid, dim3(64 * KS), 0, stream, a);
+    if constexpr (sizeof(OutT) == 2) {
+      if (a.N2 > 0) {
+        hipLaunchKernelGGL((gemm_rowpanel_kernel<ET, RT, CT, KS, OutT, Args, true>), grid, dim3(64 * KS), 0, stream, a);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((gemm_rowpanel_kernel<ET, RT, CT, KS, OutT, Args, false>), grid, dim3(64 * KS), 0, stream, a);
   };
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;
