@@ -310,7 +310,7 @@ struct ModelState {
   bool fused_smolgen_attention_ = true;
   int fused_smolgen_min_batch_ = 72;
   int dense1_split_min_batch_ = 112;   // smallest batch whose smolgen dense1 splits K between workgroups
-  int dense2_norm_max_batch_ = 64, generator_norm_max_batch_ = 48;   // largest batches whose row norms run inside the layer after them
+  int dense2_norm_max_batch_ = 64, generator_norm_max_batch_ = 32;   // largest batches whose row norms run inside the layer after them
   int smolgen_few_max_batch_ = 64;   // largest batch whose generator layer and norm run in the attention kernel for few positions
   bool compress_with_qkv_ = true;
   bool narrow_layers_ = true;   // the two kernels of narrow bodies
@@ -1139,7 +1139,7 @@ Mi355xNetwork::Mi355xNetwork(const WeightsFile& file, Options& options) {
   smolgen_few_max_batch_ = options.GetInt("smolgen_few_max_batch", 64);
   fused_heads_max_batch_ = options.GetInt("fused_heads_max_batch", -1);
   dense2_norm_max_batch_ = options.GetInt("dense2_norm_max_batch", 64);
-  generator_norm_max_batch_ = options.GetInt("generator_norm_max_batch", 48);
+  generator_norm_max_batch_ = options.GetInt("generator_norm_max_batch", 32);
   qkv_first_ = options.GetBool("qkv_first", true);
   write_through_ = options.GetBool("write_through", true);
   chain_latency_max_batch_ = options.GetInt("chain_latency_max_batch", 128);
@@ -2143,15 +2143,19 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       // or at most 128 positions): its kernels then take the variants with the shortest latency. At larger fp16
       // batches the two are balanced and the leaner variants disturb the projection less (batch 256: 1.5 %).
       const bool chain_first = f8 || B <= chain_latency_max_batch_;
-      // For few positions the two layers after a row norm normalise their rows themselves, which saves two launches of a
-      // chain of thirteen per layer (norm_gemm_kernel; us of a 15x1024 pass, neither -> dense2 -> both. fp16: 1 position 989 ->
-      // 950 -> 915, 13 1375 -> 1323 -> 1278, 32 1768 -> 1720 -> 1691, 64 2374 -> 2352 -> 2323, 71 2605 -> 2607 -> 2626; e4m3: 1
-      // 843 -> 806 -> 765, 32 1268 -> 1209 -> 1187, 48 1555 -> 1509 -> 1578). From 65 positions the products are long enough to
-      // hide the launches and the norm, repeated in every workgroup of a row, costs what it saves; the generator layer gets
-      // there earlier, with e4m3 operands at 33.
+      // For few positions the layers after a row norm normalise their rows themselves (norm_gemm_kernel), which saves a launch each
+      // of a chain of dependent ones. Second dense layer, us of a 15x1024 pass: fp16 1 position 989 -> 950, 13 1375 -> 1323, 32 1768 ->
+      // 1720, 64 2374 -> 2352, 71 2605 -> 2607; e4m3 1 843 -> 806, 32 1268 -> 1209, 48 1555 -> 1509. From 65 positions the product is
+      // long enough to hide the launch, and the norm, repeated in every workgroup of a row, costs what it saves.
+      // The generator layer comes to this where no attention kernel has it inside: heads of another depth than 32, a number of them
+      // that is no multiple of four, an explicit fp8_gemms=...+smolgen, or those kernels turned off. Every wave adds up every group
+      // of its workgroup's 32 or 64 rows, so few heads make a long chain; gamma and beta, 2 KiB per head and workgroup, tell sooner. us
+      // of a ten-layer pass, own norm -> inside. 2 heads of depth 64 1 position 441 -> 442, 16 481 -> 524; 4 1 416 -> 410, 8 485 -> 501, 48
+      // 506 -> 519; 6 of depth 32 13 642 -> 638, 32 601 -> 609; 8 of depth 64 1 479 -> 473, 13 607 -> 598, 32 668 -> 670, e4m3 8 529 -> 514;
+      // 14 of depth 32 8 658 -> 637, 32 654 -> 642, 48 748 -> 765; 16 of depth 64 1 564 -> 555, 24 970 -> 954, 48 1319 -> 1314, e4m3 32 795 -> 773.
       const bool norms_inside = !calibrating_ && dtype_ != Dtype::kFloat && B < dense1_split_min_batch_;
       const bool norm_dense2 = norms_inside && B <= dense2_norm_max_batch_ && NormGemmSupported(sg_hs_, 1, sg_gen_);
-      const bool norm_global = norms_inside && !fused_gen && !gen_inside && B <= std::min(generator_norm_max_batch_, chain_f8 ? 32 : 1024) &&
+      const bool norm_global = norms_inside && !fused_gen && !gen_inside && B <= generator_norm_max_batch_ && heads_ >= 8 &&
                                NormGemmSupported(g, heads_, 4096);
       if (chain_f8) {
         // The whole chain on e4m3 operands: the compression reads the e4m3 copy of x that the QKV projection reads

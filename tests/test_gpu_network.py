@@ -956,6 +956,21 @@ def test_a_pass_has_the_same_bits_beside_others_on_other_streams_and_profiled(em
                 np.testing.assert_array_equal(res[field], want[n][field], err_msg="%s %s %d" % (what, field, n))
 
 
+@pytest.mark.parametrize("heads,inside,outside", [(2, (), (1, 13)), (4, (), (8,)), (8, (1, 13, 32), (33,))])
+def test_generator_layer_normalises_its_rows_itself_where_that_is_faster(heads, inside, outside, positions, tmp_path):
+    """Heads of depth 64 have no attention kernel with the generator inside. The layer takes its row norm along from eight heads up
+    and for up to 32 positions, by the names in the profile; either form against the oracle."""
+    from lc0_amd import Network, netproto
+    path = str(tmp_path / "net.pb.gz")
+    netproto.write_pb_gz(path, netgen.attention_body(64 * heads, 2, heads, 256, seed=2070 + heads, smolgen=(32, 256, 256), perturb_ln=True, std=0.03))
+    net, bn = Network(path), onn.BlasNetwork(nr.load(path))
+    for n in inside + outside:
+        names, res = _names_of_a_profiled_pass(net, positions, n)
+        assert ("gemm_smolgen_global|gemm_norm" in names) == (n in inside) and any(k.startswith("gemm_smolgen_global|") for k in names), (n, names)
+        idx = (np.arange(n) * 3) % 320
+        _compare(res, bn.forward(positions["masks"][idx], positions["values"][idx]), [positions["legal"][i] for i in idx])
+
+
 @pytest.mark.parametrize("dff,smolgen,first", [(512, None, 1), (1024, None, 5), (1024, (32, 256, 256), 5), (2048, None, 18)])
 def test_rest_of_a_layer_is_one_kernel_from_as_many_positions_as_its_weights_need(dff, smolgen, first, positions, tmp_path):
     """The kernel streams a layer's weights through every CU that it uses: with few positions and many weights the layers one by
