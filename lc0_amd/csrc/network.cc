@@ -2101,8 +2101,11 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
                            (!chain_f8 || q_smolgen_auto_);
     // Few positions: the norm before the generator layer, that layer and the attention in one kernel, while that is one
     // workgroup per CU. us of a 15x1024 pass, two or three launches -> one: fp16 1 position 824 -> 814, 13 1219 -> 1187, 17 1348 -> 1306, 32
-    // 1690 -> 1647, 48 2135 -> 2066, 64 2390 -> 2238, 70 2731 -> 2835; bf16 64 2328 -> 2186; e4m3 16 920 -> 901, 32 1222 -> 1198, 64 1708 -> 1610.
-    const bool gen_inside = e.has_smolgen && smolgen_wfrag_ != nullptr && !fused_gen && !calibrating_ && B <= smolgen_few_max_batch_ &&
+    // 1690 -> 1647, 48 2135 -> 2066, 64 2390 -> 2238, 70 2731 -> 2835; bf16 64 2328 -> 2186; e4m3 16 920 -> 901, 32 1222 -> 1198, 64 1708 -> 1610. Ten
+    // layers of 8 heads fp16 16 491 -> 442, 33 492 -> 474, 64 507 -> 490; 12 heads 33 698 -> 694, 64 725 -> 715; 4 heads, where one wave of eight
+    // has an attention to do, 16 462 -> 421, 32 470 -> 445, but with the 16 queries of a workgroup from 33 on 33 481 -> 490, 48 434 -> 437, 64 446 -> 444.
+    const int few_max = heads_ > 4 ? smolgen_few_max_batch_ : std::min(smolgen_few_max_batch_, 32);
+    const bool gen_inside = e.has_smolgen && smolgen_wfrag_ != nullptr && !fused_gen && !calibrating_ && B <= few_max &&
                             B < dense1_split_min_batch_ && (!chain_f8 || q_smolgen_auto_) &&
                             SmolgenAttentionFewSupported(heads_, depth_, sg_gen_ / heads_);
     auto launch_qkv = [&](const SecondProduct& second = {}) {

@@ -971,6 +971,20 @@ def test_generator_layer_normalises_its_rows_itself_where_that_is_faster(heads, 
         _compare(res, bn.forward(positions["masks"][idx], positions["values"][idx]), [positions["legal"][i] for i in idx])
 
 
+@pytest.mark.parametrize("heads,inside,outside", [(4, (32,), (33,)), (8, (33, 64), (65,))])
+def test_attention_kernel_of_few_positions_where_it_is_faster(heads, inside, outside, positions, tmp_path):
+    """Up to 64 positions, with four heads (one busy wave of eight) up to 32, by the names in the profile; either form against the oracle."""
+    from lc0_amd import Network, netproto
+    path = str(tmp_path / "net.pb.gz")
+    netproto.write_pb_gz(path, netgen.attention_body(32 * heads, 2, heads, 256, seed=2080 + heads, smolgen=(32, 256, 256), perturb_ln=True, std=0.03))
+    net, bn = Network(path), onn.BlasNetwork(nr.load(path))
+    for n in inside + outside:
+        names, res = _names_of_a_profiled_pass(net, positions, n)
+        assert ("smolgen_attention_few" in names) == (n in inside) and ("attention" in names) == (n in outside), (n, names)
+        idx = (np.arange(n) * 3) % 320
+        _compare(res, bn.forward(positions["masks"][idx], positions["values"][idx]), [positions["legal"][i] for i in idx])
+
+
 @pytest.mark.parametrize("dff,smolgen,first", [(512, None, 1), (1024, None, 5), (1024, (32, 256, 256), 5), (2048, None, 18)])
 def test_rest_of_a_layer_is_one_kernel_from_as_many_positions_as_its_weights_need(dff, smolgen, first, positions, tmp_path):
     """The kernel streams a layer's weights through every CU that it uses: with few positions and many weights the layers one by
