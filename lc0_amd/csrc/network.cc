@@ -2374,7 +2374,8 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
   }
   // The two heads in one launch while their workgroups find a place at once (two per CU at width 256, else one). us of a pass,
   // six launches -> one: 10x256 fp16 1 position 291 -> 278, 64 323 -> 310, 200 545 -> 528, 1024 1865 -> 1889; 15x1024 fp16 1 831 -> 822, 13
-  // 1234 -> 1217, 77 2776 -> 2764, 128 level, 256 5603 -> 5633; e4m3 16 934 -> 916.
+  // 1234 -> 1217, 77 2776 -> 2764, 128 level, 256 5603 -> 5633; e4m3 16 934 -> 916. Ten layers with smolgen, width 512 fp16 1 459 -> 447, 64 883 ->
+  // 865, 128 1483 -> 1459, 256 2132 -> 2098, 1000 level; width 768 1 530 -> 518, 16 707 -> 695, from 24 on level, 256 3100 -> 3118.
   const int fused_heads_max = fused_heads_max_batch_ >= 0 ? fused_heads_max_batch_ : emb_ <= 256 ? 256 : 128;
   if (val_packed_[0] != nullptr && B <= fused_heads_max) {
     ValueHeadsArgs a;

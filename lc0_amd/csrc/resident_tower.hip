@@ -64,10 +64,10 @@ __device__ __forceinline__ float Sum16(float v) {
 // the channels per wave would read the rows twice as often. One position per workgroup has half the products for the same
 // weights and serves up to one round of the CUs. 64 float channels: two waves per SIMD with half the rows each, which hide the
 // ends of a tap (243 -> 221 us a pass of 32 positions).
-// What bounds it: with two positions the matrix cores are busy 60 % of a wave's 2.5 M cycles (20x256 tower, 512 positions); what runs between
-// the products on the same waves is squeeze-and-excitation (192 KiB of float weights per block and workgroup, four barriers; about
-// a quarter), the additions of skip and bias and activations (a tenth) and waits; with all CUs busy the clock falls to 1.9 GHz on top. One
-// position 50 % products, 6x64 in floats 75 %. A round of 512 positions takes 1.25 ms (1.2 PFLOP/s of direct products), where 41
+// What bounds it: with two positions the matrix cores are busy 60 % of a wave's 2.5 M cycles (20x256 tower, 512 positions). By phases the
+// convolutions take 69 % (their waits included), squeeze-and-excitation 22 % (192 KiB of float weights per block and workgroup, four
+// barriers: 28 k cycles a block where the weights alone take 3 k), biases, skip and activations 9 %; with all CUs busy the clock falls to
+// 1.9 GHz on top. One position: 65, 28 and 7 %; 6x64 in floats 68, 18 and 14 %. A round of 512 positions takes 1.25 ms (1.2 PFLOP/s of direct products), where 41
 // transforms of 24 us and 40 launches of 36 x 2048x256x256 of 22 us took 1.86.
 // Tried and not kept: the next squeeze-and-excitation weights touched during a convolution, so that they wait in the L2 (the stream
 // waits for them in order: 512 positions 1558 -> 1727 us a pass); zeros in the banks of the rows they stand for (level).
