@@ -424,10 +424,16 @@ struct TowerArgs {
   int batch = 0, blocks = 0, filters = 0, act = 2;
 };
 bool TowerSupported(int filters, bool f32);
-long long TowerFragments(int blocks, int filters, bool f32);
-long long TowerFragmentIndex(int blocks, int filters, bool f32, int conv, int tap, int out, int in);
-bool TowerFaster(int batch, int filters, bool f32);   // than winograd convolutions
-void LaunchTower(const TowerArgs& args, bool f32, hipStream_t stream);
+bool TowerFaster(int batch, int filters, bool f32, int blocks);   // than winograd convolutions
+long long TowerFragments(int blocks, int filters);
+long long TowerFragmentIndex(int blocks, int filters, int conv, int tap, int out, int in);
+void LaunchTower(const TowerArgs& args, hipStream_t stream);
+// The same for 64 float filters (resident_tower_f32.hip). packed: bfloat16, the first of a weight's three parts at
+// TowerF32FragmentIndex(), the others kTowerF32Part and twice that behind it.
+constexpr int kTowerF32Part = 512;
+long long TowerF32Fragments(int blocks);
+long long TowerF32FragmentIndex(int blocks, int conv, int tap, int out, int in);
+void LaunchTowerF32(const TowerArgs& args, hipStream_t stream);
 
 // Gather of the convolutional policy head: out[b][j] = t[b][sq][plane] for
 // kConvPolicyMap[plane*64+sq] = j. t: [B][64][ld] (NHWC), inv_map: [1858] holding plane*64+sq.

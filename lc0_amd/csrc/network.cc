@@ -632,18 +632,33 @@ Linear Mi355xNetwork::MakeLinear(const Vec& w, const Vec& b, int out, int in, in
   return l;
 }
 
+namespace {
+// Round to nearest even on the upper 16 bits of the float.
+uint16_t Bf16Bits(float v) {
+  uint32_t u;
+  std::memcpy(&u, &v, 4);
+  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40);   // NaN stays NaN
+  return static_cast<uint16_t>((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+}
+
+// v as the exact sum of three bfloat16 (an infinity: its first part).
+void SplitBf16(float v, uint16_t (&part)[3]) {
+  for (uint16_t& b : part) {
+    b = Bf16Bits(v);
+    const uint32_t u = static_cast<uint32_t>(b) << 16;
+    float f;
+    std::memcpy(&f, &u, 4);
+    v = std::isinf(f) ? 0.0f : v - f;
+  }
+}
+}  // namespace
+
 half_t* Mi355xNetwork::UploadElems(const std::vector<float>& v) {
   if (dtype_ == Dtype::kFloat) return reinterpret_cast<half_t*>(arena_.Upload(v));
   std::vector<uint16_t> bits(v.size());
   for (size_t i = 0; i < v.size(); i++) {
-    if (dtype_ == Dtype::kBf16) {   // round to nearest even on the upper 16 bits of the float
-      uint32_t u;
-      std::memcpy(&u, &v[i], 4);
-      if ((u & 0x7fffffffu) > 0x7f800000u) {
-        bits[i] = static_cast<uint16_t>((u >> 16) | 0x40);   // NaN stays NaN
-      } else {
-        bits[i] = static_cast<uint16_t>((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-      }
+    if (dtype_ == Dtype::kBf16) {
+      bits[i] = Bf16Bits(v[i]);
     } else {
       const half_t h = (half_t)v[i];
       std::memcpy(&bits[i], &h, 2);
@@ -1804,13 +1819,21 @@ void Mi355xNetwork::BuildResnet(const WeightsFile& file) {
   for (const ResBlockDev& b : res_blocks_) widest_se = std::max(widest_se, b.se.k);
   if (!res_blocks_.empty() && resident_tower_ != 0 && widest_se <= kTowerMaxSe && TowerSupported(filters_, fp32_)) {
     const int blocks = static_cast<int>(res_blocks_.size());
-    std::vector<T> packed(TowerFragments(blocks, filters_, fp32_), (T)0.0f);
+    using Packed = std::conditional_t<sizeof(T) == 4, uint16_t, T>;   // (floats: three bfloat16 parts each)
+    std::vector<Packed> packed(fp32_ ? TowerF32Fragments(blocks) : TowerFragments(blocks, filters_), Packed{});
     Vec biases;
     auto pack = [&](int conv, const ConvBlock& cb, int cin) {
       for (int o = 0; o < filters_; o++)
         for (int i = 0; i < cin; i++)
           for (int tap = 0; tap < 9; tap++) {
-            packed[TowerFragmentIndex(blocks, filters_, fp32_, conv, tap, o, i)] = (T)cb.weights[(static_cast<size_t>(o) * cin + i) * 9 + tap];
+            const float v = cb.weights[(static_cast<size_t>(o) * cin + i) * 9 + tap];
+            if constexpr (sizeof(T) == 4) {
+              uint16_t part[3];
+              SplitBf16(v, part);
+              for (int f = 0; f < 3; f++) packed[TowerF32FragmentIndex(blocks, conv, tap, o, i) + f * kTowerF32Part] = part[f];
+            } else {
+              packed[TowerFragmentIndex(blocks, filters_, conv, tap, o, i)] = (T)v;
+            }
           }
       biases.insert(biases.end(), cb.biases.begin(), cb.biases.end());
     };
@@ -1948,13 +1971,13 @@ template <typename T>
 void Mi355xNetwork::ForwardResnet(int B) {
   const int T64 = B * 64;
   bool have_v = false;
-  if (tower_packed_ != nullptr && (resident_tower_ == 1 || TowerFaster(B, filters_, fp32_))) {
+  if (tower_packed_ != nullptr && (resident_tower_ == 1 || TowerFaster(B, filters_, fp32_, static_cast<int>(res_blocks_.size())))) {
     TowerArgs t;
     t.masks = d_masks_; t.values = d_values_; t.biases = tower_biases_; t.packed = tower_packed_; t.se = tower_se_;
     t.out = r_x_; t.batch = B; t.blocks = static_cast<int>(res_blocks_.size()); t.filters = filters_; t.act = default_act_;
     const double convs = 9.0 * filters_ * (kInputPlanes + 2.0 * filters_ * t.blocks);
     Timed(fp32_ ? "tower|resident_tower_f32" : "tower|resident_tower", 2.0 * 64 * B * convs, sizeof(T) * convs + B * (112.0 * 12 + sizeof(T) * 64.0 * filters_),
-          [&] { LaunchTower(t, fp32_, stream_); });
+          [&] { fp32_ ? LaunchTowerF32(t, stream_) : LaunchTower(t, stream_); });
   } else {
     have_v = ForwardTowerWinograd<T>(B);
   }

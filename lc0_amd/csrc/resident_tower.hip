@@ -3,7 +3,7 @@
 //   resident_tower_kernel   EncodePlanes, the 3x3 convolutions, BiasActivate / BiasResidual / ApplySEUnit
 //                           blas/network_blas.cc:640-713, blas/winograd_convolution3.cc:326-382,
 //                           shared/activation.cc:166-267, blas/se_unit.cc:31-91
-#include "kernel_common.h"
+#include "tower_common.h"
 
 #include <algorithm>
 #include <stdexcept>
@@ -13,19 +13,17 @@ namespace lc0mi {
 
 namespace {
 
-// A step of a convolution is 64 bytes of one tap's inputs: 32 halves or 16 floats. Products are tiles of TILE rows (squares) and
-// TILE output channels: 32 for halves (v_mfma_f32_32x32x16, whose rate per operation is twice that of the 16x16x32 form: 32.5
-// and 30.2 cycles an instruction, measured), 16 for floats (v_mfma_f32_16x16x4; the two forms are level). Weights are 1 KiB
-// fragments of TILE channels (lane l: channel l % TILE, 16 bytes of inputs from l / TILE), a wave's in the order in which it
-// multiplies them, over all convolutions of the tower.
+// A step of a convolution is 32 of one tap's inputs. Products are tiles of TILE rows (squares) and TILE output channels
+// (v_mfma_f32_32x32x16, whose rate per operation is twice that of the 16x16x32 form: 32.5 and 30.2 cycles an instruction,
+// measured). Weights are 1 KiB fragments of TILE channels (lane l: channel l % TILE, 16 bytes of inputs from l / TILE), a wave's in
+// the order in which it multiplies them, over all convolutions of the tower.
 constexpr int kWaves = 4;                 // that share the channels of a product
 constexpr int kChunk = 8;                 // steps of a turn of the main loop, the most that are in flight per wave
-constexpr int kPlanes = 128;              // the 112 input planes, padded
 
-template <typename T, int C> struct TowerShape {
-  static constexpr int V = 16 / (int)sizeof(T);                    // values of a 16-byte vector
+template <int C> struct TowerShape {
+  static constexpr int V = 8;                                      // values of a 16-byte vector
   static constexpr int KS = 4 * V;                                 // inputs of a step
-  static constexpr int TILE = sizeof(T) == 4 ? 16 : 32, G = 64 / TILE;
+  static constexpr int TILE = 32, G = 64 / TILE;
   static constexpr int SUB = KS / (G * V);                         // fragments of a tile in a step
   static constexpr int CT = C / (TILE * kWaves);                   // channel tiles of a wave
   static constexpr int F = CT * SUB;                               // weight fragments of a step
@@ -35,72 +33,49 @@ template <typename T, int C> struct TowerShape {
   static_assert(kChunk % NS == 0 && kChunk % NS_IN == 0, "a turn does whole taps");
 };
 
-// The tower's activations: mish and relu.
-template <typename F>
-__device__ __forceinline__ void TowerAct(int act, F&& f) {
-  if (act == kActMish) f([](float v) { return ActMish(v); });
-  else f([](float v) { return v > 0.0f ? v : 0.0f; });
-}
-
-// Sum over the 16 lanes of a row of lanes.
-__device__ __forceinline__ float Sum16(float v) {
-  v += DppMove<0xB1>(v);
-  v += DppMove<0x4E>(v);
-  v += DppMove<0x141>(v);
-  v += DppMove<0x140>(v);   // mirrored within 16
-  return v;
-}
-
 // ---------------------------------------------------------------------------
 // A workgroup owns POS positions from the bit planes to the last block: their activations never leave LDS (a block's input
 // and its inner activations, 64 POS rows each), and the weights stream from L2 once per workgroup, four to eight steps ahead, across
 // the ends of the convolutions too. Convolutions are direct: nine shifted products whose rows past the board's edge read a row
 // of zeros. Four times the multiplications of winograd F(4x4,3x3), but no transforms, no winograd domain in memory (2 x 38 MB
 // per convolution at 512 positions) and no launches; and sums in float over all of a convolution, where the winograd products
-// of a half tower are rounded to halves twice. Float sums run over one tap at a time, to keep the chains short.
+// of a half tower are rounded to halves twice.
 //
 // Split: with one wave per SIMD each takes 64 channels of all rows, so that a weight fragment and a row fragment are both used
 // twice or more (two positions, a 64-byte step: 512 cycles of products, 256 of LDS reads, 256 of weights at 64 bytes a cycle); half
 // the channels per wave would read the rows twice as often. One position per workgroup has half the products for the same
-// weights and serves up to one round of the CUs. 64 float channels: two waves per SIMD with half the rows each, which hide the
-// ends of a tap (243 -> 221 us a pass of 32 positions).
+// weights and serves up to one round of the CUs.
 // What bounds it: with two positions the matrix cores are busy 60 % of a wave's 2.5 M cycles (20x256 tower, 512 positions). By phases the
 // convolutions take 69 % (their waits included), squeeze-and-excitation 22 % (192 KiB of float weights per block and workgroup, four
 // barriers: 28 k cycles a block where the weights alone take 3 k), biases, skip and activations 9 %; with all CUs busy the clock falls to
-// 1.9 GHz on top. One position: 65, 28 and 7 %; 6x64 in floats 68, 18 and 14 %. A round of 512 positions takes 1.25 ms (1.2 PFLOP/s of direct products), where 41
+// 1.9 GHz on top. One position: 65, 28 and 7 %. A round of 512 positions takes 1.25 ms (1.2 PFLOP/s of direct products), where 41
 // transforms of 24 us and 40 launches of 36 x 2048x256x256 of 22 us took 1.86.
 // Tried and not kept: the next squeeze-and-excitation weights touched during a convolution, so that they wait in the L2 (the stream
 // waits for them in order: 512 positions 1558 -> 1727 us a pass); zeros in the banks of the rows they stand for (level).
 // ---------------------------------------------------------------------------
-template <typename T, int C, int POS, int RG>
-__global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(TowerArgs p) {
-  using S = TowerShape<T, C>;
+template <int C, int POS>
+__global__ __launch_bounds__(64 * kWaves, 1) void resident_tower_kernel(TowerArgs p) {
+  using S = TowerShape<C>;
   constexpr int V = S::V, KS = S::KS, CT = S::CT, LD = S::LD, R = 64 * POS;
-  constexpr int THREADS = 64 * kWaves * RG;
-  constexpr int TILE = S::TILE, SUB = S::SUB, F = S::F, RT = R / TILE / RG, PT = RT / POS;   // a wave's row tiles, of a position
+  constexpr int THREADS = 64 * kWaves;
+  constexpr int TILE = S::TILE, SUB = S::SUB, F = S::F, RT = R / TILE, PT = RT / POS;   // a wave's row tiles, of a position
   constexpr int Q = TILE * TILE / 256;                   // a lane's output channels of a tile: Q times four, 8 apart
-  using Acc = std::conditional_t<sizeof(T) == 4, floatx4, floatx16>;
   constexpr int kRing = POS == 1 ? 8 : 4;                // steps of weights in flight
   constexpr int H = POS == 1 ? SUB : 1, ST = SUB / H;    // fragments of a tile that are read ahead together, and such reads in a step
-  constexpr bool kFloat = sizeof(T) == 4;
-  using Tv4 = T __attribute__((ext_vector_type(4)));
   constexpr int kOther = R * LD, kZero = 2 * R * LD;     // the two activation buffers, then a row of zeros
-  __shared__ __attribute__((aligned(16))) T lds[2 * R * LD + LD];
-  __shared__ __attribute__((aligned(16))) float pool[RG][POS][C];
+  __shared__ __attribute__((aligned(16))) half_t lds[2 * R * LD + LD];
+  __shared__ __attribute__((aligned(16))) float pool[POS][C];
   __shared__ float hidden[POS][kTowerMaxSe];
   __shared__ __attribute__((aligned(16))) float biases[2][C];   // of this convolution and the next
   __shared__ __attribute__((aligned(16))) float scale_shift[POS][2][C];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), cg = wave % kWaves, rg = wave / kWaves;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane % TILE, g = lane / TILE;
   const int pos0 = blockIdx.x * POS;
-  const int ch0 = cg * TILE * CT + 4 * g;              // this lane's first output channel
-
-  const int row0 = rg * (64 / RG) + r;                   // this lane's row of its first tile (with RG > 1 of one position)
-  static_assert(RG == 1 || POS == 1, "row groups share one position");
+  const int ch0 = wave * TILE * CT + 4 * g;              // this lane's first output channel
 
   const long long steps = S::STEPS_IN + 2LL * p.blocks * S::STEPS;
-  const intx4* ws = reinterpret_cast<const intx4*>(p.packed) + cg * steps * F * 64 + lane;
+  const intx4* ws = reinterpret_cast<const intx4*>(p.packed) + wave * steps * F * 64 + lane;
   intx4 w[kRing][F];
 #pragma unroll
   for (int j = 0; j < kRing; j++)
@@ -115,17 +90,17 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
     for (int q = 0; q < POS; q++) {
       const long long at = (long long)min(pos0 + q, p.batch - 1) * 112;
       uint64_t mask[V];
-      T value[V];
+      half_t value[V];
 #pragma unroll
       for (int e = 0; e < V; e++) {
         const int plane = v * V + e;
         mask[e] = plane < 112 ? p.masks[at + plane] : 0;
-        value[e] = (T)(plane < 112 ? p.values[at + plane] : 0.0f);
+        value[e] = (half_t)(plane < 112 ? p.values[at + plane] : 0.0f);
       }
       for (int sq = tid / PER_ROW; sq < 64; sq += STRIDE) {
-        T x[V];
+        half_t x[V];
 #pragma unroll
-        for (int e = 0; e < V; e++) x[e] = ((mask[e] >> sq) & 1) ? value[e] : (T)0.0f;
+        for (int e = 0; e < V; e++) x[e] = ((mask[e] >> sq) & 1) ? value[e] : (half_t)0.0f;
         *reinterpret_cast<intx4*>(lds + kOther + (q * 64 + sq) * LD + v * V) = *reinterpret_cast<const intx4*>(x);
       }
     }
@@ -134,7 +109,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
   }
   __syncthreads();
 
-  Acc acc[RT][CT];
+  floatx16 acc[RT][CT];
   // acc = the convolution of the rows at src (element offset), NS_ steps per tap, STEPS_ in all.
   auto convolve = [&](int src, auto ns, auto total) {
     constexpr int NS_ = decltype(ns)::value, STEPS_ = decltype(total)::value;
@@ -143,7 +118,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
       const int dy = tap / 3 - 1, dx = tap - tap / 3 * 3 - 1, x = (r & 7) + dx;
 #pragma unroll
       for (int t = 0; t < RT; t++) {
-        const int y = (TILE * t + row0 >> 3 & 7) + dy;
+        const int y = ((TILE * t + r) >> 3 & 7) + dy;
         const bool on = (unsigned)x < 8u && (unsigned)y < 8u && tap < 9;
         at[t] = (on ? src + (t / PT * 64 + y * 8 + x) * LD : kZero) + V * g;
       }
@@ -151,8 +126,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
-      for (int c = 0; c < CT; c++) acc[t][c] = Acc{};
-    Acc part[kFloat ? RT : 1][kFloat ? CT : 1];
+      for (int c = 0; c < CT; c++) acc[t][c] = floatx16{};
     intx4 a[2][RT][H];
     auto load_rows = [&](intx4 (&x)[RT][H], int s, int u0) {
 #pragma unroll
@@ -170,38 +144,14 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
           const int now = (j * ST + st) & 1;
           if (st == ST - 1 && (j + 1) % NS_ == 0) aim((base + j + 1) / NS_);   // (past the last tap: the zeros, not used)
           load_rows(a[now ^ 1], (j + (st + 1) / ST) % NS_, (st + 1) % ST * H);
-          if constexpr (kFloat) {
-            if (j % NS_ == 0) {
 #pragma unroll
-              for (int t = 0; t < RT; t++)
+          for (int h = 0; h < H; h++)
 #pragma unroll
-                for (int c = 0; c < CT; c++) part[t][c] = Acc{};
-            }
+            for (int t = 0; t < RT; t++)
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-              for (int t = 0; t < RT; t++)
-#pragma unroll
-                for (int c = 0; c < CT; c++)
-                  part[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(floatx4, w[j % kRing][c])[e],
-                                                                    __builtin_bit_cast(floatx4, a[now][t][0])[e], part[t][c], 0, 0, 0);
-            if ((j + 1) % NS_ == 0) {
-#pragma unroll
-              for (int t = 0; t < RT; t++)
-#pragma unroll
-                for (int c = 0; c < CT; c++) acc[t][c] += part[t][c];
-            }
-          } else {
-            using ev8 = typename Vec16<T>::v8;
-#pragma unroll
-            for (int h = 0; h < H; h++)
-#pragma unroll
-              for (int t = 0; t < RT; t++)
-#pragma unroll
-                for (int c = 0; c < CT; c++)
-                  acc[t][c] = Mfma32(__builtin_bit_cast(ev8, w[j % kRing][c * SUB + st * H + h]), __builtin_bit_cast(ev8, a[now][t][h]),
-                                     acc[t][c]);
-          }
+              for (int c = 0; c < CT; c++)
+                acc[t][c] = Mfma32(__builtin_bit_cast(half8, w[j % kRing][c * SUB + st * H + h]), __builtin_bit_cast(half8, a[now][t][h]),
+                                   acc[t][c]);
           if (st == ST - 1) {
 #pragma unroll
             for (int f = 0; f < F; f++) w[j % kRing][f] = ws[((j + kRing) * F + f) * 64];
@@ -211,7 +161,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
 #pragma unroll
           for (int i = 0; i < RT * H; i++) {
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, kFloat ? 4 * CT : CT, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -230,7 +180,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
     return floatx4{acc[t][c][4 * q], acc[t][c][4 * q + 1], acc[t][c][4 * q + 2], acc[t][c][4 * q + 3]};
   };
   auto store = [&](int dst, int t, int c, int q, const floatx4& v) {
-    *reinterpret_cast<Tv4*>(lds + dst + (TILE * t + row0) * LD + ch0 + TILE * c + 8 * q) = Tv4{(T)v[0], (T)v[1], (T)v[2], (T)v[3]};
+    *reinterpret_cast<half4*>(lds + dst + (TILE * t + r) * LD + ch0 + TILE * c + 8 * q) = half4{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
   };
 
   auto plain_tail = [&](int conv, int dst) {
@@ -291,24 +241,19 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
             for (int t = 1; t < PT; t++) s += four(b * PT + t, c, q);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-              s[e] = Sum16(s[e]);
-              if (TILE == 32) s[e] += DppMove<0x142>(s[e]);   // (the row of lanes before: the upper 16 hold the sum of 32)
-              s[e] = s[e] * (1.0f / 64.0f) + (rg == 0 ? bias[e] : 0.0f);
+              s[e] = Sum32(s[e]) * (1.0f / 64.0f) + bias[e];
             }
-            if (r == TILE - 16) *reinterpret_cast<floatx4*>(&pool[rg][b][ch0 + TILE * c + 8 * q]) = s;
+            if (r == TILE - 16) *reinterpret_cast<floatx4*>(&pool[b][ch0 + TILE * c + 8 * q]) = s;
           }
       __syncthreads();
-      for (int k0 = 16 * wave; k0 < se.k; k0 += 16 * kWaves * RG) {
+      for (int k0 = 16 * wave; k0 < se.k; k0 += 16 * kWaves) {
         if (k0 > 16 * wave) load_w1(k0);
 #pragma unroll
         for (int b = 0; b < POS; b++) {
           floatx4 h4 = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
           for (int i = 0; i < S1; i++) {
-            floatx4 x = *reinterpret_cast<const floatx4*>(&pool[0][b][16 * i + 4 * v_lane]);
-#pragma unroll
-            for (int j = 1; j < RG; j++) x += *reinterpret_cast<const floatx4*>(&pool[j][b][16 * i + 4 * v_lane]);
-            h4 += w1[i] * x;
+            h4 += w1[i] * *reinterpret_cast<const floatx4*>(&pool[b][16 * i + 4 * v_lane]);
           }
           float h = (h4[0] + h4[1]) + (h4[2] + h4[3]);
           h += __shfl_xor(h, 16, 64);
@@ -362,7 +307,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
             }
 #pragma unroll
             for (int t = b * PT; t < (b + 1) * PT; t++) {
-              const Tv4 skip = *reinterpret_cast<const Tv4*>(lds + (TILE * t + row0) * LD + ch);
+              const half4 skip = *reinterpret_cast<const half4*>(lds + (TILE * t + r) * LD + ch);
               const floatx4 y = four(t, c, q);
               floatx4 v;
 #pragma unroll
@@ -375,7 +320,7 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
     __syncthreads();
   }
 
-  T* out = static_cast<T*>(p.out) + (long long)pos0 * 64 * C;
+  half_t* out = static_cast<half_t*>(p.out) + (long long)pos0 * 64 * C;
   for (int i = tid; i < R * (C / V); i += THREADS) {
     const int row = i / (C / V), v = i % (C / V);
     if (pos0 + row / 64 < p.batch)
@@ -383,77 +328,73 @@ __global__ __launch_bounds__(64 * kWaves * RG, 1) void resident_tower_kernel(Tow
   }
 }
 
-template <typename T, int C>
+template <int C>
 long long FragmentIndex(int blocks, int conv, int tap, int out, int in) {
-  using S = TowerShape<T, C>;
+  using S = TowerShape<C>;
   const long long steps = S::STEPS_IN + 2LL * blocks * S::STEPS;
   const int wave = out / (S::TILE * S::CT), c = out / S::TILE % S::CT, sub = in % S::KS / (S::G * S::V);
   const long long first = conv == 0 ? 0 : S::STEPS_IN + (conv - 1LL) * S::STEPS;
   const long long step = wave * steps + first + tap * (conv == 0 ? S::NS_IN : S::NS) + in / S::KS;
   return ((step * S::F + c * S::SUB + sub) * 64 + in / S::V % S::G * S::TILE + out % S::TILE) * S::V + in % S::V;
 }
-template <typename T, int C>
+template <int C>
 long long Fragments(int blocks) {   // (and a turn's worth that is asked for past the end)
-  using S = TowerShape<T, C>;
+  using S = TowerShape<C>;
   return ((S::STEPS_IN + 2LL * blocks * S::STEPS) * kWaves + kChunk) * S::F * 64 * S::V;
 }
 
 }  // namespace
 
-// 64 float, 128 and 256 half filters. A wave takes whole tiles of TILE channels, so there are 64 n float or 128 n half filters
-// (not 64 in halves); a turn of kChunk steps does whole taps, so a tap has one, two, four or eight (not 192 or 256 floats, 384
-// halves). 128 float filters fit but gain nothing: one position per workgroup is 0.87 ms of products on its CU
-// (us of a 10x128 pass, winograd / this: 8 positions 313 / 880, 64 487 / 914, 256 937 / 1032, 512 1543 / 2013).
+// 64 float (resident_tower_f32.hip), 128 and 256 half filters. A wave takes whole tiles of TILE channels, so there are 128 n half
+// filters (not 64); a turn of kChunk steps does whole taps, so a tap has one, two, four or eight (not 384).
 bool TowerSupported(int filters, bool f32) { return f32 ? filters == 64 : filters == 128 || filters == 256; }
 
-long long TowerFragments(int blocks, int filters, bool f32) {
-  if (f32) return Fragments<float, 64>(blocks);
-  return filters == 128 ? Fragments<half_t, 128>(blocks) : Fragments<half_t, 256>(blocks);
+long long TowerFragments(int blocks, int filters) { return filters == 128 ? Fragments<128>(blocks) : Fragments<256>(blocks); }
+
+long long TowerFragmentIndex(int blocks, int filters, int conv, int tap, int out, int in) {
+  return filters == 128 ? FragmentIndex<128>(blocks, conv, tap, out, in) : FragmentIndex<256>(blocks, conv, tap, out, in);
 }
 
-long long TowerFragmentIndex(int blocks, int filters, bool f32, int conv, int tap, int out, int in) {
-  if (f32) return FragmentIndex<float, 64>(blocks, conv, tap, out, in);
-  return filters == 128 ? FragmentIndex<half_t, 128>(blocks, conv, tap, out, in) : FragmentIndex<half_t, 256>(blocks, conv, tap, out, in);
-}
-
-// From how many positions on the kernel is faster than winograd convolutions, whose launches spread few positions over more CUs,
-// and up to how many. us a batch through the interface, winograd / this. 20x256 halves 1 position 639 / 683, 13 686 / 726, 32 850 / 702,
+// Where the kernel is faster than winograd convolutions, whose launches spread few positions over more CUs. us a batch through the
+// interface, winograd / this. 20x256 halves 1 position 639 / 683, 13 686 / 726, 32 850 / 702,
 // 200 1426 / 840, 512 2146 / 1571, 1000 3505 / 3061; 10x256 without squeeze-and-excitation 13 299 / 309, 17 328 / 307, 64 454 / 319, 512
 // 1158 / 876, 1000 1993 / 1606; 10x128 1 284 / 195, 8 302 / 199, 64 392 / 217, 256 655 / 319, 512 915 / 518, 1000 1338 / 963, mish without
-// squeeze-and-excitation 8 261 / 183, 1000 1332 / 929; 6x64 floats 1 175 / 199, 16 205 / 209, 32 229 / 221, 64 267 / 243, 256 513 / 349, without
-// squeeze-and-excitation 24 213 / 205, 64 254 / 229. With 257 to 512 float positions a second round is 6 to 13 % faster alone
-// (512 718 / 637) but slower where passes overlap. Thousands of evals/s of two and of four threads, winograd / this: floats 32 233 / 224 and
-// 340 / 362, 64 400 / 432 and 567 / 660, 256 870 / 945 and 1260 / 1325, 512 1180 / 1017 and 1540 / 1385; 20x256 halves 17 40 / 44 and 58 / 66, 64 120 / 163
-// and 156 / 247, 512 313 / 366 and 321 / 406.
-bool TowerFaster(int batch, int filters, bool f32) { return f32 ? batch > 24 && batch <= 256 : filters <= 128 || batch > 16; }
+// squeeze-and-excitation 8 261 / 183, 1000 1332 / 929; thousands of evals/s of two and of four threads, 20x256 halves 17 40 / 44 and 58 / 66, 64
+// 120 / 163 and 156 / 247, 512 313 / 366 and 321 / 406.
+// 64 floats: 6 blocks 1 position 172 / 124, 32 225 / 139, 256 509 / 269, 512 708 / 486, 1000 1133 / 892, of four threads 1 15.1 / 17.5, 32 349 / 519,
+// 256 1267 / 2018, 1000 1602 / 2352; 2 blocks 1 102 / 86, 24 125 / 94, 1000 848 / 745. One block, more than half of it the input
+// convolution, gains less (24 103 / 84, four threads 508 / 503; 257 263 / 234) and keeps to the batches of one round.
+bool TowerFaster(int batch, int filters, bool f32, int blocks) {
+  if (f32) return blocks > 1 || (batch > 24 && batch <= 256);
+  return filters <= 128 || batch > 16;
+}
 
 namespace {
-template <typename T, int C, int POS, int RG>
+template <int C, int POS>
 void LaunchTowerT(TowerArgs a, int first, int count, hipStream_t stream) {
   if (count <= 0) return;
   a.masks += 112LL * first;
   a.values += 112LL * first;
-  a.out = static_cast<T*>(a.out) + 64LL * C * first;
+  a.out = static_cast<half_t*>(a.out) + 64LL * C * first;
   a.batch = count;
-  resident_tower_kernel<T, C, POS, RG><<<dim3((count + POS - 1) / POS), dim3(64 * kWaves * RG), 0, stream>>>(a);
+  resident_tower_kernel<C, POS><<<dim3((count + POS - 1) / POS), dim3(64 * kWaves), 0, stream>>>(a);
 }
 }  // namespace
 
-// Halves: full rounds of 256 workgroups with two positions each, then the rest, with one position each where that makes one round
+// Full rounds of 256 workgroups with two positions each, then the rest, with one position each where that makes one round
 // of cheaper workgroups (20x256: a round of one 0.8 ms, of two 1.4 ms).
-void LaunchTower(const TowerArgs& a, bool f32, hipStream_t stream) {
+void LaunchTower(const TowerArgs& a, hipStream_t stream) {
   if (a.batch <= 0) return;
-  if (a.blocks < 1 || (a.act != kActMish && a.act != kActRelu) || !TowerSupported(a.filters, f32)) {
+  if (a.blocks < 1 || (a.act != kActMish && a.act != kActRelu) || !TowerSupported(a.filters, false)) {
     throw std::runtime_error("LaunchTower: no kernel");
   }
-  if (f32) return LaunchTowerT<float, 64, 1, 2>(a, 0, a.batch, stream);
   const int rest = a.batch % 512, pairs = rest > 256 ? a.batch : a.batch - rest;
   if (a.filters == 128) {
-    LaunchTowerT<half_t, 128, 2, 1>(a, 0, pairs, stream);
-    LaunchTowerT<half_t, 128, 1, 1>(a, pairs, a.batch - pairs, stream);
+    LaunchTowerT<128, 2>(a, 0, pairs, stream);
+    LaunchTowerT<128, 1>(a, pairs, a.batch - pairs, stream);
   } else {
-    LaunchTowerT<half_t, 256, 2, 1>(a, 0, pairs, stream);
-    LaunchTowerT<half_t, 256, 1, 1>(a, pairs, a.batch - pairs, stream);
+    LaunchTowerT<256, 2>(a, 0, pairs, stream);
+    LaunchTowerT<256, 1>(a, pairs, a.batch - pairs, stream);
   }
 }
 

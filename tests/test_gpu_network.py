@@ -221,6 +221,34 @@ def test_batches_that_the_tower_kernel_takes_by_itself(filters, options, inside,
         assert any("resident_tower" in k for k in names) == (n in inside) and ("expand_planes" in names) == (n in outside), (n, names)
 
 
+@pytest.mark.parametrize("se,mish,batch", [(16, False, 1), (0, True, 24), (96, True, 257)])
+def test_float_tower_on_split_operands_keeps_float_precision(se, mish, batch, positions, tmp_path):
+    """Two blocks of 64 float filters against the float64 model, at batches that the tower kernel takes by itself, on planes whose
+    values need all three bfloat16 parts and differ by ten powers of ten. A float pass rounds each sum to 2^-24 of its largest
+    term or so: 1e-6 of the result over five convolutions and the heads, where two parts alone (16 bits) leave 1e-5 and more."""
+    from blas_model_f64 import BlasModelF64
+    from lc0_amd import netproto
+    net = netgen.se_resnet(64, 2, se, seed=7200 + se)
+    if mish:
+        net["format"]["network_format"]["default_activation"] = 1
+    path = str(tmp_path / "net.pb.gz")
+    netproto.write_pb_gz(path, net)
+    values = positions["values"][:8].copy()
+    values[:, 0:104:3] = 0.1
+    values[:, 104:109] = 1.0 / 3.0
+    values[:, 109] = np.float32(1234.5678) * np.arange(8)
+    values[:, 1:104:7] = 1.0e-7
+    rows = np.arange(batch) % 8
+    gpu, res = _run_gpu(path, positions["masks"][rows], values[rows], "precision=fp32")
+    want = BlasModelF64(net).forward(positions["masks"][:8], values)
+    policy = np.asarray(want["policy"])[rows]
+    for at in range(0, batch, 8):   # (every group of positions by itself)
+        part = slice(at, min(at + 8, batch))
+        assert np.linalg.norm(res["policy"][part] - policy[part]) <= 1e-6 * np.linalg.norm(policy[part])
+    names, _ = _names_of_a_profiled_pass(gpu, positions, batch)
+    assert any("resident_tower" in k for k in names)
+
+
 @pytest.mark.parametrize("name,options,batch,tol", [("c3_resnet_20x256", "precision=fp16", 140, 5e-3), ("c0_resnet_6x64", "precision=fp32", 40, 1e-3)])
 def test_towers_of_the_one_kernel_as_winograd_convolutions(name, options, batch, tol, positions):
     """The shapes that the tower kernel takes, on the winograd convolutions that it takes over from (products with resident weights from
