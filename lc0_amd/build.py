@@ -7,7 +7,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liblc0mi.so")
 SOURCES = ["weights.cc", "tables.cc", "network.cc", "capi.cc", "kernel_api.cc", "kernels.hip", "gemm_kernels.hip", "gemm_dma_half.hip",
-           "gemm_dma_bf16.hip", "gemm_dma_f8.hip", "gemm_rowpanel.hip", "gemm_resident.hip", "gemm_norm.hip", "gemm_f32.hip", "smolgen_attention.hip", "smolgen_attention_few.hip", "encoder_narrow.hip", "value_heads.hip", "resnet_kernels.hip", "resident_tower.hip", "resident_tower_f32.hip"]
+           "gemm_dma_bf16.hip", "gemm_dma_f8.hip", "gemm_rowpanel.hip", "gemm_resident.hip", "gemm_norm.hip", "gemm_f32.hip", "smolgen_attention.hip", "smolgen_attention_few.hip", "encoder_narrow.hip", "encoder_narrow_f32.hip", "value_heads.hip", "resnet_kernels.hip", "resident_tower.hip", "resident_tower_f32.hip"]
 # -packed-fp32-ops off: packed fp32 forms are not trusted on this hardware pool.
 DEVICE_FLAGS = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result", "-Wno-unknown-warning-option"]

@@ -318,12 +318,22 @@ struct EncoderTailArgs {
   float alpha = 1.0f, eps = 1e-6f;
   int act = 3;
   bool bf16 = false;
+  float *u = nullptr, *partial = nullptr;   // floats with several slices: [M][emb], [slices][M][emb], slices at most dff / emb
 };
 bool EncoderTailSupported(int emb, int d_model, int dff);
 int EncoderTailRows(int M);   // rows of a workgroup
 int EncoderTailMinBatch(int emb, int d_model, int dff);   // smallest batch at which it is faster than its layers one by one
 long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_model);
 void LaunchEncoderTail(const EncoderTailArgs& args, hipStream_t stream);
+// The same two for floats (encoder_narrow_f32.hip): x, att and out hold floats, u stays one. packed: bfloat16, the first of a weight's
+// three parts at the index, the others kSplitPart and twice that behind it.
+constexpr int kSplitPart = 512;
+long long QkvF32FragmentIndex(int row, int col, int emb, int d_model);
+void LaunchQkvAttentionF32(const QkvAttentionArgs& args, hipStream_t stream);
+int NarrowF32MinBatch(int emb, int dff);   // smallest batch at which the two are faster than their layers one by one
+int EncoderTailF32Slices(int M, int emb, int dff);   // workgroups that share the FFN of a row, each with a sum of its own
+long long EncoderTailF32FragmentIndex(int layer, int row, int col, int emb, int d_model);
+void LaunchEncoderTailF32(const EncoderTailArgs& args, hipStream_t stream);
 
 // Value and moves-left heads of a 16-bit attention body (value_heads.hip), for few positions: per head
 //   out[b][o] = out_act(sum_n act(sum_k e[b][k] w_fc1[n][k] + b_fc1[n]) w_fc2[o][n] + b_fc2[o]),
@@ -429,8 +439,7 @@ long long TowerFragments(int blocks, int filters);
 long long TowerFragmentIndex(int blocks, int filters, int conv, int tap, int out, int in);
 void LaunchTower(const TowerArgs& args, hipStream_t stream);
 // The same for 64 float filters (resident_tower_f32.hip). packed: bfloat16, the first of a weight's three parts at
-// TowerF32FragmentIndex(), the others kTowerF32Part and twice that behind it.
-constexpr int kTowerF32Part = 512;
+// TowerF32FragmentIndex(), the others kSplitPart and twice that behind it.
 long long TowerF32Fragments(int blocks);
 long long TowerF32FragmentIndex(int blocks, int conv, int tap, int out, int in);
 void LaunchTowerF32(const TowerArgs& args, hipStream_t stream);

@@ -642,7 +642,8 @@ uint16_t Bf16Bits(float v) {
 }
 
 // v as the exact sum of three bfloat16 (an infinity: its first part).
-void SplitBf16(float v, uint16_t (&part)[3]) {
+constexpr int kSplitPartCount = 3;
+void SplitBf16(float v, uint16_t (&part)[kSplitPartCount]) {
   for (uint16_t& b : part) {
     b = Bf16Bits(v);
     const uint32_t u = static_cast<uint32_t>(b) << 16;
@@ -1638,23 +1639,43 @@ void Mi355xNetwork::BuildAttentionBody(const WeightsFile& file) {
       for (float& v : ab) v *= alpha_;
       e.ffn2_ab = UploadF(ab);
     }
-    if (narrow_layers_ && !fold_layer_norm_ && !fp8_ && dtype_ != Dtype::kFloat) {
+    if (narrow_layers_ && !fold_layer_norm_ && !fp8_) {
+      // Elements of a weight in the order in which the kernels multiply them; floats as their three bfloat16 parts.
+      const bool f32 = dtype_ == Dtype::kFloat;
+      std::vector<uint16_t> parts;
+      Vec elems;
+      auto start = [&](size_t n) { f32 ? parts.assign(kSplitPartCount * n, 0) : elems.assign(n, 0.0f); };
+      auto put = [&](long long at, float v) {
+        if (!f32) {
+          elems[at] = v;
+          return;
+        }
+        uint16_t part[kSplitPartCount];
+        SplitBf16(v, part);
+        for (int f = 0; f < kSplitPartCount; f++) parts[at + f * kSplitPart] = part[f];
+      };
+      auto upload = [&] { return f32 ? reinterpret_cast<half_t*>(arena_.Upload(parts)) : UploadElems(elems); };
       if (!e.has_smolgen && QkvAttentionSupported(emb_, heads_, depth_)) {
-        Vec packed(qkv_w.size());
+        start(qkv_w.size());
         for (int o = 0; o < 3 * d_model_; o++)
-          for (int i = 0; i < emb_; i++) packed[QkvFragmentIndex(o, i, emb_, d_model_)] = qkv_w[static_cast<size_t>(o) * emb_ + i];
-        e.qkv_packed = UploadElems(packed);
+          for (int i = 0; i < emb_; i++) {
+            put(f32 ? QkvF32FragmentIndex(o, i, emb_, d_model_) : QkvFragmentIndex(o, i, emb_, d_model_), qkv_w[static_cast<size_t>(o) * emb_ + i]);
+          }
+        e.qkv_packed = upload();
       }
       if (EncoderTailSupported(emb_, d_model_, dff_)) {
-        Vec packed(l.mha.dense_w.size() + l.ffn.dense1_w.size() + l.ffn.dense2_w.size());
+        start(l.mha.dense_w.size() + l.ffn.dense1_w.size() + l.ffn.dense2_w.size());
         auto pack = [&](int layer, const Vec& m, int out, int in) {
           for (int o = 0; o < out; o++)
-            for (int i = 0; i < in; i++) packed[EncoderTailFragmentIndex(layer, o, i, emb_, d_model_)] = m[static_cast<size_t>(o) * in + i];
+            for (int i = 0; i < in; i++) {
+              put(f32 ? EncoderTailF32FragmentIndex(layer, o, i, emb_, d_model_) : EncoderTailFragmentIndex(layer, o, i, emb_, d_model_),
+                  m[static_cast<size_t>(o) * in + i]);
+            }
         };
         pack(0, l.mha.dense_w, emb_, d_model_);
         pack(1, l.ffn.dense1_w, dff_, emb_);
         pack(2, l.ffn.dense2_w, emb_, dff_);
-        e.tail_packed = UploadElems(packed);
+        e.tail_packed = upload();
       }
     }
     encoders_.push_back(e);
@@ -1828,9 +1849,9 @@ void Mi355xNetwork::BuildResnet(const WeightsFile& file) {
           for (int tap = 0; tap < 9; tap++) {
             const float v = cb.weights[(static_cast<size_t>(o) * cin + i) * 9 + tap];
             if constexpr (sizeof(T) == 4) {
-              uint16_t part[3];
+              uint16_t part[kSplitPartCount];
               SplitBf16(v, part);
-              for (int f = 0; f < 3; f++) packed[TowerF32FragmentIndex(blocks, conv, tap, o, i) + f * kTowerF32Part] = part[f];
+              for (int f = 0; f < kSplitPartCount; f++) packed[TowerF32FragmentIndex(blocks, conv, tap, o, i) + f * kSplitPart] = part[f];
             } else {
               packed[TowerFragmentIndex(blocks, filters_, conv, tap, o, i)] = (T)v;
             }
@@ -2270,7 +2291,8 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       bias = sbias_;
     }
     // Narrow bodies: projection and attention in one kernel, everything after them in another.
-    const bool qkv_attention = e.qkv_packed != nullptr;
+    const bool f32 = dtype_ == Dtype::kFloat;
+    const bool qkv_attention = e.qkv_packed != nullptr && (!f32 || B >= NarrowF32MinBatch(emb_, dff_));
     if (!qkv_before_chain && !with_compress && !qkv_attention) launch_qkv();
     if (e.has_smolgen && ss != stream_) HIP_CHECK(hipStreamWaitEvent(stream_, join_events_[li], 0));
     const int gen_sz = e.has_smolgen ? sg_gen_ / heads_ : 0;
@@ -2306,8 +2328,8 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
         QkvAttentionArgs a;
         a.x = x_; a.packed = e.qkv_packed; a.bias = e.qkv.b; a.out = att_;
         a.batch = B; a.emb = emb_; a.heads = heads_; a.scale = att_scale; a.bf16 = bf16;
-        Timed("qkv_attention", 6.0 * T * emb_ * d_model_ + att_flops, 2.0 * T * (emb_ + d_model_) + 6.0 * emb_ * d_model_,
-              [&] { LaunchQkvAttention(a, stream_); });
+        Timed("qkv_attention", 6.0 * T * emb_ * d_model_ + att_flops, es_ * T * (emb_ + d_model_) + (f32 ? 18.0 : 6.0) * emb_ * d_model_,
+              [&] { f32 ? LaunchQkvAttentionF32(a, stream_) : LaunchQkvAttention(a, stream_); });
       } else if (gen_inside) {
         // (launched above)
       } else if (fused_gen) {
@@ -2317,15 +2339,17 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       } else {
         Timed("attention", att_flops, att_bytes, [&] { Attention(qkv_, bias, att_, B, heads_, depth_, stream_); });
       }
-      if (e.tail_packed != nullptr && B >= EncoderTailMinBatch(emb_, d_model_, dff_)) {
+      if (e.tail_packed != nullptr &&
+          B >= (f32 ? NarrowF32MinBatch(emb_, dff_) : EncoderTailMinBatch(emb_, d_model_, dff_))) {
         EncoderTailArgs a;
         a.att = att_; a.packed = e.tail_packed; a.x = x_;
         a.dense_b = e.dense.b; a.ffn1_b = e.ffn1.b; a.ffn2_b = e.ffn2.b;
         a.ln1_g = e.ln1_g; a.ln1_b = e.ln1_b; a.ln2_g = e.ln2_g; a.ln2_b = e.ln2_b;
         a.M = T; a.emb = emb_; a.d_model = d_model_; a.dff = dff_;
         a.alpha = alpha_; a.eps = eps_; a.act = ffn_act_; a.bf16 = bf16;
+        a.u = reinterpret_cast<float*>(t_); a.partial = reinterpret_cast<float*>(ffn_);
         const double weights = static_cast<double>(emb_) * (d_model_ + 2 * dff_);
-        Timed("encoder_tail", 2.0 * T * weights, 2.0 * (weights + T * (2.0 * emb_ + d_model_)), [&] { LaunchEncoderTail(a, stream_); });
+        Timed("encoder_tail", 2.0 * T * weights, (f32 ? 6.0 : 2.0) * weights + es_ * T * (2.0 * emb_ + d_model_), [&] { f32 ? LaunchEncoderTailF32(a, stream_) : LaunchEncoderTail(a, stream_); });
         continue;
       }
       if (calibrating_) RecordAbsMax(att_, static_cast<size_t>(T) * d_model_, static_cast<int>(4 * li + 1));

@@ -3,6 +3,7 @@
 //   resident_tower_f32_kernel   EncodePlanes, the 3x3 convolutions, BiasActivate / BiasResidual / ApplySEUnit
 //                               blas/network_blas.cc:640-713, blas/winograd_convolution3.cc:326-382,
 //                               shared/activation.cc:166-267, blas/se_unit.cc:31-91
+#include "split_bf16.h"
 #include "tower_common.h"
 
 #include <stdexcept>
@@ -12,36 +13,19 @@ namespace lc0mi {
 namespace {
 
 constexpr int C = 64;
-constexpr int kParts = 3;                     // bfloat16 parts of a float: 3 x 8 significant bits, exact
 constexpr int kLd = kParts * C + 8;           // of a row of activations: [part][channel], 16-byte reads of 16 rows meet different banks
 constexpr int kLdPlanes = kParts * kPlanes + 8;
 constexpr int kTaps = 9;
 constexpr int kRing = 3;                      // steps (tap and 16 inputs) of weights in flight
 constexpr int kThreads = 512;
 
-// v = hi + mid + lo exactly (each rounded to nearest, the remainder exact), for |v| up to the largest bfloat16; smaller parts than
-// the least float are lost. An infinity is its first part.
-__device__ __forceinline__ void Split3(const floatx4& v, bf16x4 (&part)[kParts]) {
-  floatx4 rest = v;
-#pragma unroll
-  for (int p = 0; p < kParts; p++) {
-    part[p] = __builtin_convertvector(rest, bf16x4);
-    rest -= __builtin_convertvector(part[p], floatx4);
-    if (p == 0) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) rest[e] = rest[e] == rest[e] ? rest[e] : 0.0f;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // A workgroup owns one position from the bit planes to the last block, as resident_tower_kernel does: activations stay in LDS,
 // weights stream from L2 three steps ahead, convolutions are nine shifted products whose rows past the board's edge read a
 // row of zeros.
 //
-// Products: a float is the exact sum of three bfloat16, hi + mid + lo, weights split at load and activations where they are
-// stored. Of the nine products of two such sums the six that reach 2^-24 of the result are taken: hi hi in one accumulator, the
-// five small ones in another. v_mfma_f32_32x32x16_bf16 does 16 times the work of v_mfma_f32_16x16x4_f32 in the same time, so six
+// Products: floats are sums of three bfloat16 (split_bf16.h), weights split at load and activations where they are stored, six
+// products for one. v_mfma_f32_32x32x16_bf16 does 16 times the work of v_mfma_f32_16x16x4_f32 in the same time, so six
 // of it are 2.7 times faster, and an accumulator takes 9 roundings per convolution where the float instructions took 16 per tap.
 //
 // Split: wave (kq, cg) multiplies all 64 rows by 32 output channels over a quarter of the inputs, so that a fragment of weights is
@@ -124,17 +108,13 @@ __global__ __launch_bounds__(kThreads, 1) void resident_tower_f32_kernel(TowerAr
 #pragma unroll
       for (int j = 0; j < kTaps; j++) {
         if (j + 1 < kTaps) load_rows(a[(j + 1) & 1], j + 1);
-        auto product = [&](floatx16 (&acc)[2], int fw, int fa) {
 #pragma unroll
-          for (int t = 0; t < 2; t++)
-            acc[t] = Mfma32(__builtin_bit_cast(bf16x8, w[j % kRing][fw]), __builtin_bit_cast(bf16x8, a[j & 1][t][fa]), acc[t]);
-        };
-        product(lo, 1, 1);
-        product(lo, 2, 0);
-        product(lo, 0, 2);
-        product(lo, 1, 0);
-        product(lo, 0, 1);
-        product(hi, 0, 0);
+        for (int i = 0; i < kProducts; i++)
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            floatx16& acc = i + 1 < kProducts ? lo[t] : hi[t];
+            acc = Mfma32(__builtin_bit_cast(bf16x8, w[j % kRing][kFirst[i]]), __builtin_bit_cast(bf16x8, a[j & 1][t][kSecond[i]]), acc);
+          }
 #pragma unroll
         for (int f = 0; f < kParts; f++) w[j % kRing][f] = ws[((kRing + j) * kParts + f) * 64];
         // The next rows go out one by one between these products, and nothing moves past them.
@@ -180,12 +160,6 @@ __global__ __launch_bounds__(kThreads, 1) void resident_tower_f32_kernel(TowerAr
     Split3(v, part);
 #pragma unroll
     for (int f = 0; f < kParts; f++) *reinterpret_cast<bf16x4*>(lds + dst + row * kLd + f * C + ch0 + 8 * i) = part[f];
-  };
-  auto whole = [&](const bf16_t* at) {   // four values from their parts
-    floatx4 v = __builtin_convertvector(*reinterpret_cast<const bf16x4*>(at), floatx4);
-#pragma unroll
-    for (int f = 1; f < kParts; f++) v += __builtin_convertvector(*reinterpret_cast<const bf16x4*>(at + f * C), floatx4);
-    return v;
   };
   auto plain_tail = [&](int conv, int dst) {
     TowerAct(p.act, [&](auto act) {
@@ -271,7 +245,7 @@ __global__ __launch_bounds__(kThreads, 1) void resident_tower_f32_kernel(TowerAr
           gamma = *reinterpret_cast<const floatx4*>(&scale_shift[0][ch]);
           beta = *reinterpret_cast<const floatx4*>(&scale_shift[1][ch]) + gamma * beta;
         }
-        const floatx4 skip = whole(lds + row * kLd + ch);
+        const floatx4 skip = Join3(lds + row * kLd + ch, C);
         floatx4 v;
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = act(gamma[e] * sum[i][e] + beta[e] + skip[e]);

@@ -1028,6 +1028,39 @@ def test_rest_of_a_layer_is_one_kernel_from_as_many_positions_as_its_weights_nee
         _compare(res, bn.forward(positions["masks"][idx], positions["values"][idx]), [positions["legal"][i] for i in idx])
 
 
+@pytest.mark.parametrize("emb,heads,dff,smolgen,batch", [(128, 4, 128, None, 1), (128, 12, 640, None, 9), (256, 8, 768, None, 40), (256, 16, 512, None, 70),
+                                                         (256, 8, 1024, (32, 256, 256), 6)])
+def test_narrow_float_layers_on_split_operands_keep_float_precision(emb, heads, dff, smolgen, batch, positions, tmp_path):
+    """Two layers of a float body against the float64 model: one and two heads per workgroup, one and several parts of the attention
+    output, one to five workgroups on the FFN of a row, with and without the biases of output projection and second FFN layer.
+    Float sums leave about 3e-7 of the logits' norm over a pass; operands of two parts instead of three (16 bits) would leave 1e-5."""
+    from blas_model_f64 import BlasModelF64
+    from lc0_amd import Network, netproto
+    net = netgen.attention_body(emb, 2, heads, dff, seed=2300 + heads + dff, smolgen=smolgen, perturb_ln=True, std=0.05, d_model=32 * heads)
+    idx = np.arange(batch) % 16
+    want = BlasModelF64(net).forward(positions["masks"][:16], positions["values"][:16])
+    for biased in (True, False):
+        if not biased:
+            for layer in net["weights"]["encoder"]:
+                layer["mha"]["dense_b"] = np.zeros(emb, np.float32)
+                layer["ffn"]["dense2_b"] = np.zeros(emb, np.float32)
+            want = BlasModelF64(net).forward(positions["masks"][:16], positions["values"][:16])
+            for layer in net["weights"]["encoder"]:
+                del layer["mha"]["dense_b"], layer["ffn"]["dense2_b"]
+        path = str(tmp_path / ("net%d.pb.gz" % biased))
+        netproto.write_pb_gz(path, net)
+        gpu, res = _run_gpu(path, positions["masks"][idx], positions["values"][idx], "precision=fp32")
+        policy = np.asarray(want["policy"])[idx]
+        for at in range(0, batch, 16):
+            part = slice(at, min(at + 16, batch))
+            assert np.linalg.norm(res["policy"][part] - policy[part]) <= 1e-6 * np.linalg.norm(policy[part])
+        names, _ = _names_of_a_profiled_pass(gpu, positions, batch)
+        assert "encoder_tail" in names and ("qkv_attention" in names) == (smolgen is None)
+    if emb == 256 and smolgen is None:
+        names, _ = _names_of_a_profiled_pass(gpu, positions, 3)   # (fewer positions than the weights need)
+        assert "encoder_tail" not in names and "qkv_attention" not in names
+
+
 FUSED_KERNELS = [
     (1024, "compress_with_qkv", "false", "", 1, "+second", "gemm_smolgen_compress|"),
     (1024, "compress_with_qkv", "false", "", 16, "+second", "gemm_smolgen_compress|"),
