@@ -15,6 +15,7 @@ import numpy as np
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = None
+_CALLS = None   # the per-position calls without ctypes (csrc/python_calls.cc); None: not built for this interpreter
 
 InputPlane = namedtuple("InputPlane", ["mask", "value"])
 NetworkCapabilities = namedtuple("NetworkCapabilities", ["input_format", "output_format", "moves_left"])
@@ -31,7 +32,7 @@ def library_path():
 
 def load_library():
     """Loads liblc0mi.so (built in-tree by lc0_amd/build.py); never builds it."""
-    global _LIB
+    global _LIB, _CALLS
     if _LIB is not None:
         return _LIB
     path = library_path()
@@ -78,6 +79,11 @@ def load_library():
                       ("lc0mi_pos_encoding", cf)):
         getattr(lib, name).argtypes = [C.POINTER(ci)]
         getattr(lib, name).restype = C.POINTER(typ)
+    try:
+        from . import _calls   # (linked to the library beside it)
+        _CALLS = _calls
+    except ImportError:
+        pass
     _LIB = lib
     return lib
 
@@ -233,17 +239,22 @@ class NetworkComputation:
     The per-sample readers take their values from one bulk read of the library after ComputeBlocking: a call through
     ctypes costs more than the value it fetches."""
 
+    _p = 0   # address of the computation for the extension, 0: none, or no extension
+
     def __init__(self, network):
         self._net = network  # keeps the network alive
         self._lib = load_library()
         self._h = C.c_void_p()
         self._values = self._legal = None   # bulk reads of the last ComputeBlocking
         _check(self._lib.lc0mi_comp_create(network._h, C.byref(self._h)))
+        if _CALLS is not None:
+            self._p = self._h.value
 
     def close(self):
         if getattr(self, "_h", None):
             load_library().lc0mi_comp_destroy(self._h)
             self._h = None
+            self._p = 0
             self._values = self._legal = None
 
     def __del__(self):
@@ -260,11 +271,17 @@ class NetworkComputation:
 
     def AddInputs(self, masks, values):
         """Bulk AddInput: masks u64[n,112], values f32[n,112]."""
+        self._values = self._legal = None
+        if self._p:
+            done = _CALLS.add_inputs(self._p, masks, values)
+            if done == 0:
+                return
+            if done < 0:
+                _check(done)
         masks = np.ascontiguousarray(masks, dtype=np.uint64)
         values = np.ascontiguousarray(values, dtype=np.float32)
         if masks.ndim != 2 or masks.shape[1] != 112 or values.shape != masks.shape:
             raise BackendError("AddInputs expects [n,112] masks and values.")
-        self._values = self._legal = None
         _check(self._lib.lc0mi_comp_add_inputs(self._h, masks.shape[0], _address(masks), _address(values)))
 
     def ComputeBlocking(self):
@@ -290,12 +307,27 @@ class NetworkComputation:
         return v
 
     def GetQVal(self, sample):
+        values = self._values
+        if values is not None and 0 <= sample < len(values[0]):
+            v = values[0][sample]
+            if v == v:
+                return v
         return self._value(0, self._lib.lc0mi_comp_q, sample)
 
     def GetDVal(self, sample):
+        values = self._values
+        if values is not None and 0 <= sample < len(values[1]):
+            v = values[1][sample]
+            if v == v:
+                return v
         return self._value(1, self._lib.lc0mi_comp_d, sample)
 
     def GetMVal(self, sample):
+        values = self._values
+        if values is not None and 0 <= sample < len(values[2]):
+            v = values[2][sample]
+            if v == v:
+                return v
         return self._value(2, self._lib.lc0mi_comp_m, sample)
 
     def GetPVal(self, sample, move_id):
@@ -314,10 +346,16 @@ class NetworkComputation:
         """Policy indices (0..1857) of the legal moves of the input added last. Once used, every input
         needs its list; the policy then comes from GetLegalPolicy (softmax over these moves, computed on
         the device as lc0's search wrapper does on the host) and the raw logits are not downloaded."""
+        self._values = self._legal = None
+        if self._p:
+            done = _CALLS.add_legal_moves(self._p, move_ids)
+            if done == 0:
+                return
+            if done < 0:
+                _check(done)
         ids = np.ascontiguousarray(move_ids, dtype=np.uint16)
         if ids.ndim != 1:
             raise BackendError("AddLegalMoves expects a one-dimensional list of move ids.")
-        self._values = self._legal = None
         _check(self._lib.lc0mi_comp_add_legal_moves(self._h, ids.shape[0], _address(ids)))
 
     def SetPolicySoftmaxTemperature(self, temperature):

@@ -1,11 +1,13 @@
-"""Builds lc0_amd/liblc0mi.so (the C-ABI library: host C++ + gfx950 kernels)."""
+"""Builds lc0_amd/liblc0mi.so (the C-ABI library: host C++ + gfx950 kernels) and the extension of its Python mirror."""
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liblc0mi.so")
+CALLS = os.path.join(HERE, "_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 SOURCES = ["weights.cc", "tables.cc", "network.cc", "capi.cc", "kernel_api.cc", "kernels.hip", "gemm_kernels.hip", "gemm_dma_half.hip",
            "gemm_dma_bf16.hip", "gemm_dma_f8.hip", "gemm_rowpanel.hip", "gemm_resident.hip", "gemm_norm.hip", "gemm_f32.hip", "smolgen_attention.hip", "smolgen_attention_few.hip", "encoder_narrow.hip", "encoder_narrow_f32.hip", "value_heads.hip", "resnet_kernels.hip", "resident_tower.hip", "resident_tower_f32.hip"]
 # -packed-fp32-ops off: packed fp32 forms are not trusted on this hardware pool.
@@ -38,6 +40,8 @@ def build(verbose=False):
         raise RuntimeError("hipcc failed")
     cmd = ["hipcc", "-shared", "-fPIC", "--offload-arch=gfx950", "-o", LIB] + objs + ["-lz"]
     subprocess.check_call(cmd)
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-shared", "-I" + sysconfig.get_path("include"),
+                           os.path.join(CSRC, "python_calls.cc"), "-o", CALLS, "-L" + HERE, "-l:liblc0mi.so", "-Wl,-rpath,$ORIGIN"])
     return LIB
 
 

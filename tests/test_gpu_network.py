@@ -1061,6 +1061,70 @@ def test_narrow_float_layers_on_split_operands_keep_float_precision(emb, heads, 
         assert "encoder_tail" not in names and "qkv_attention" not in names
 
 
+@pytest.mark.parametrize("form", ["plain", "read-only", "strided", "fortran", "int64", "float64", "big-endian", "list", "many"])
+def test_inputs_through_the_extension_and_through_ctypes(form, positions):
+    """Arrays that the extension takes as they are, and those that it leaves to the conversions: the same results, bit for bit."""
+    from lc0_amd import Network, backend
+    net = Network(netgen.cached_config("tiny_attn"))
+    assert backend._CALLS is not None
+    n = 40 if form == "many" else 3
+    masks, values = positions["masks"][:n].copy(), positions["values"][:n].copy()
+    moves = [np.array(sorted(positions["legal"][i]), np.uint16) for i in range(n)]
+    convert = {
+        "read-only": lambda a: (a.setflags(write=False), a)[1],
+        "strided": lambda a: np.repeat(a, 2, axis=-1)[..., ::2],
+        "fortran": np.asfortranarray,
+        "int64": lambda a: a.astype(np.int64) if a.dtype != np.float32 else a,
+        "float64": lambda a: a.astype(np.float64) if a.dtype == np.float32 else a,
+        "big-endian": lambda a: a.astype(a.dtype.newbyteorder(">")),
+        "list": lambda a: a.tolist()}.get(form, lambda a: a)
+    got = []
+    for extension in (True, False):
+        for legal in (False, True):
+            comp = net.NewComputation()
+            assert comp._p
+            if not extension:
+                comp._p = 0
+            if legal:
+                for i in range(n):
+                    comp.AddInputs(convert(masks[i:i + 1]), convert(values[i:i + 1]))
+                    comp.AddLegalMoves(convert(moves[i]))
+            else:
+                comp.AddInputs(convert(masks), convert(values))
+            assert comp.GetBatchSize() == n
+            comp.ComputeBlocking()
+            got.append([comp.GetLegalPolicy(i) for i in range(n)] if legal else [comp.results()["policy"]])
+            comp.close()
+    for one, other in zip(got[0] + got[1], got[2] + got[3]):
+        np.testing.assert_array_equal(one, other)
+
+
+def test_bad_inputs_are_refused_with_and_without_the_extension(positions):
+    from lc0_amd import BackendError, Network
+    net = Network(netgen.cached_config("tiny_attn"), "max_batch=4")
+    masks, values = positions["masks"][:2], positions["values"][:2]
+    for extension in (True, False):
+        comp = net.NewComputation()
+        comp._p = comp._p if extension else 0
+        with pytest.raises(BackendError):
+            comp.AddLegalMoves(np.zeros(1, np.uint16))             # (no input yet)
+        for bad in ((masks[0], values[0]), (masks[:, :111], values[:, :111]), (masks, values[:1])):
+            with pytest.raises(BackendError):
+                comp.AddInputs(*bad)
+        comp.AddInputs(masks[:0], values[:0])
+        assert comp.GetBatchSize() == 0
+        comp.AddInputs(masks[:1], values[:1])
+        for ids in (np.array([1858], np.uint16), np.zeros(257, np.uint16), np.zeros((1, 1), np.uint16)):
+            with pytest.raises(BackendError):
+                comp.AddLegalMoves(ids)
+        comp.AddLegalMoves(np.zeros(0, np.uint16))
+        with pytest.raises(BackendError):
+            comp.AddLegalMoves(np.zeros(1, np.uint16))             # (a second list for one input)
+        comp.close()
+        with pytest.raises(BackendError):
+            comp.AddInputs(masks, values)
+
+
 FUSED_KERNELS = [
     (1024, "compress_with_qkv", "false", "", 1, "+second", "gemm_smolgen_compress|"),
     (1024, "compress_with_qkv", "false", "", 16, "+second", "gemm_smolgen_compress|"),
