@@ -134,8 +134,9 @@ void gemm_dma_kernel(Args p) {
   // that have no second product, e4m3 19200x32x1024 on 128x64 tiles 11.5 us instead of 10.85, 300x8192x256 on 64x64 8.75 instead of 8.45.)
   static_assert(!TWO || (BM < 256 && EPI == 0 && sizeof(OutT) == 2), "small tiles, 16-bit output");
   const int col_tiles = TWO ? (p.N + BN - 1) / BN : 0;
-  const bool second = TWO && (int)blockIdx.y >= col_tiles;
-  const int m0 = blockIdx.x * BM, n0 = (second ? blockIdx.y - col_tiles : blockIdx.y) * BN;
+  const int2 tile = TileOfWorkgroup(p.tile_order);
+  const bool second = TWO && tile.y >= col_tiles;
+  const int m0 = tile.x * BM, n0 = (second ? tile.y - col_tiles : tile.y) * BN;
   const int M = p.M, N = second ? p.N2 : p.N, K = p.K, ldw = second ? p.ldw2 : p.ldw;
   float my_bias = 0.0f;
   [[maybe_unused]] float my_cscale = 0.0f;
@@ -568,7 +569,7 @@ void gemm_dma_kernel(Args p) {
           t.x += part_lds[w * BM + tid].x;
           t.y += part_lds[w * BM + tid].y;
         }
-        reinterpret_cast<float2*>(p.stats_out)[(long long)(m0 + tid) * gridDim.y + blockIdx.y] = t;
+        reinterpret_cast<float2*>(p.stats_out)[(long long)(m0 + tid) * gridDim.y + tile.y] = t;
       }
     }
   }
@@ -594,8 +595,10 @@ inline int OutputStores(int requested, long long m, long long n, long long batch
 }
 
 template <typename ET, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int NSTAGES = 2, bool ALONE = false>
-void LaunchGemmDma(const GemmArgs& a, hipStream_t stream) {
+void LaunchGemmDma(const GemmArgs& args, hipStream_t stream) {
+  GemmArgs a = args;
   dim3 grid((a.M + BM - 1) / BM, (a.N + BN - 1) / BN + (a.N2 + BN - 1) / BN, a.batch);
+  a.tile_order = PickTileOrder(a.M, 1024, grid);
   const dim3 block(WAVES_M * WAVES_N * 64);
   auto launch = [&](auto stores_tag) {
     constexpr int S = decltype(stores_tag)::value;

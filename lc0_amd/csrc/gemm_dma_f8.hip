@@ -5,8 +5,10 @@ namespace lc0mi {
 
 namespace {
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BKB = 128, int NSTAGES = 2, bool ALONE = false>
-void LaunchGemmDmaF8Tile(const GemmF8Args& a, hipStream_t stream) {
+void LaunchGemmDmaF8Tile(const GemmF8Args& args, hipStream_t stream) {
+  GemmF8Args a = args;
   dim3 grid((a.M + BM - 1) / BM, (a.N + BN - 1) / BN + (a.N2 + BN - 1) / BN);
+  a.tile_order = PickTileOrder(a.M, 0, grid);
   const dim3 block(WAVES_M * WAVES_N * 64);
   if constexpr (BM == 256) {
     const int stores = OutputStores(a.out_stores, a.M, a.N, 1, a.out_f8 ? 1 : 2);

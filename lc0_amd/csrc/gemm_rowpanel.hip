@@ -39,8 +39,9 @@ __global__ __launch_bounds__(64 * KS) void gemm_rowpanel_kernel(Args p) {
   const int r = lane & 15, g = lane >> 4;
   // With TWO panels past the columns of the first product belong to a second one.
   const int panels = TWO ? (p.N + COLS - 1) / COLS : 0;
-  const bool second = TWO && (int)blockIdx.y >= panels;
-  const int m0 = blockIdx.x * ROWS, n0 = (second ? blockIdx.y - panels : blockIdx.y) * COLS;
+  const int2 tile = TileOfWorkgroup(p.tile_order);
+  const bool second = TWO && tile.y >= panels;
+  const int m0 = tile.x * ROWS, n0 = (second ? tile.y - panels : tile.y) * COLS;
   const int M = p.M, N = second ? p.N2 : p.N, ldw = second ? p.ldw2 : p.ldw;
   const char* A = reinterpret_cast<const char*>(p.A) + (long long)m0 * p.lda * ES;
   const char* W = (second ? reinterpret_cast<const char*>(p.W2) : reinterpret_cast<const char*>(p.W)) + (long long)n0 * ldw * ES;
@@ -126,11 +127,13 @@ __global__ __launch_bounds__(64 * KS) void gemm_rowpanel_kernel(Args p) {
 template <typename ET> constexpr int kPanelWaves = std::is_same<ET, uint8_t>::value ? 4 : 8;
 
 template <typename ET, typename OutT, typename Args>
-void LaunchPanel(const Args& a, int batch, hipStream_t stream) {
+void LaunchPanel(const Args& args, int batch, hipStream_t stream) {
+  Args a = args;
   const RowPanelShape s = PickRowPanelShape(a.M, a.N, batch);
   auto launch = [&](auto rt_tag, auto ct_tag) {
     constexpr int RT = decltype(rt_tag)::value, CT = decltype(ct_tag)::value, KS = kPanelWaves<ET>;
     dim3 grid((a.M + 16 * RT - 1) / (16 * RT), (a.N + 16 * CT - 1) / (16 * CT) + (a.N2 + 16 * CT - 1) / (16 * CT), batch);
+    a.tile_order = PickTileOrder(a.M, 1024, grid);
     if constexpr (sizeof(OutT) == 2) {
       if (a.N2 > 0) {
         hipLaunchKernelGGL((gemm_rowpanel_kernel<ET, RT, CT, KS, OutT, Args, true>), grid, dim3(64 * KS), 0, stream, a);

@@ -17,6 +17,23 @@ void LaunchGemmDmaF8(GemmVariant v, const GemmF8Args& a, hipStream_t stream);
 // As a value of GemmArgs::out_stores that no longer depends on the size (for the parts of a product).
 int ResolvedOutStores(const GemmArgs& a);
 
+// The order of a launch's tiles. Workgroups go to the eight XCDs in turn, and each XCD's L2 fetches every operand row that one of its
+// tiles reads. In the order of the grid an XCD has tiles of all rows and of all columns, unless the row tiles are a multiple of
+// eight. Neighbouring row tiles per XCD cut the activations fetched to an eighth: from 2048 rows (us of a 15x1024 pass, fp16 36
+// positions 1960 -> 1905, 77 dense 2755 -> 2667, 150 4663 -> 4265, 300 7790 -> 7165, 1000 21550 -> 21050; e4m3 77 2145 -> 2045, 300
+// 5560 -> 5130, 350 7090 -> 6085). With fewer rows the weights, which come
+// from memory, are the larger part: in halves neighbouring column tiles up to 1024 rows (1 position 852 -> 831, 4 1013 -> 988, 16 1236 ->
+// 1221, but 20 1386 -> 1395), in e4m3, with half the bytes, for row panels only (5 positions on tiles 826 -> 841, 16 928 -> 939).
+inline TileOrder PickTileOrder(int M, int columns_max_rows, const dim3& grid) {
+  TileOrder o;
+  const unsigned tiles = grid.x * grid.y;
+  o.columns = M <= columns_max_rows;
+  const unsigned d = o.columns ? grid.x : grid.y;
+  if (grid.z != 1 || tiles < 16 || tiles > 65536 || (!o.columns && (M < 2048 || grid.x % 8 == 0))) return o;
+  if (d > 1) o.inverse = 0xFFFFFFFFu / d + 1;   // (exact division while tiles * d < 2^32)
+  return o;
+}
+
 // Row panels (gemm_rowpanel.hip): panels of 16 rt x 16 ct outputs, and how many of them cover a problem.
 struct RowPanelShape { int rt, ct; };
 constexpr RowPanelShape kRowPanelShapes[] = {{1, 1}, {2, 1}, {1, 2}, {2, 2}, {4, 2}};

@@ -63,6 +63,16 @@ __device__ __forceinline__ void LoadBias4(const float* bias, int n, int N, float
   }
 }
 
+// The (row tile, column tile) of this workgroup in a grid of gridDim.x by gridDim.y of them.
+__device__ __forceinline__ int2 TileOfWorkgroup(const TileOrder& order) {
+  if (order.inverse == 0) return make_int2(blockIdx.x, blockIdx.y);
+  const unsigned nx = gridDim.x, ny = gridDim.y, id = blockIdx.y * nx + blockIdx.x, total = nx * ny;
+  const unsigned xcd = id & 7, at = xcd * (total >> 3) + min(xcd, total & 7) + (id >> 3);
+  const unsigned q = __umulhi(at, order.inverse);   // at / nx or at / ny
+  if (order.columns) return make_int2(at - q * nx, q);
+  return make_int2(q, at - q * ny);
+}
+
 __device__ __forceinline__ float WaveSum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

@@ -29,6 +29,14 @@ enum class Dtype { kHalf, kBf16, kFloat };
 // The last three name a kind of store outright.
 enum OutStores { kStoresAuto = 0, kStoresAutoKeep = 1, kStoresCached = 2, kStoresStream = 3, kStoresWriteThrough = 4 };
 
+// Which output tile a workgroup of a product takes (TileOfWorkgroup): as the grid numbers them, row tiles first (inverse 0), or
+// such that an XCD, which gets every eighth workgroup, has neighbouring row tiles with all their columns, or the other way
+// round. inverse: 2^32 over the number of column tiles (columns: of row tiles), rounded up.
+struct TileOrder {
+  unsigned inverse = 0;
+  bool columns = false;
+};
+
 struct GemmArgs {
   const half_t* A = nullptr; int lda = 0; long long strideA = 0;
   const half_t* W = nullptr; int ldw = 0; long long strideW = 0;
@@ -41,6 +49,7 @@ struct GemmArgs {
   // A, W and (unless out_f32) C hold bfloat16 instead of half values. Not with the folded layer-norm fields.
   bool bf16 = false;
   int out_stores = kStoresAuto;
+  TileOrder tile_order;   // (set by the launchers)
   // split_k > 1: the K range is cut into split_k slices computed by different
   // workgroups; slice s stores its partial sums (float, out_f32 required, no
   // activation, bias only in slice 0) at C + s * split_stride. The consumer adds
@@ -115,6 +124,7 @@ struct GemmF8Args {
   bool out_f8 = false;
   float out_mul = 1.0f;
   int out_stores = kStoresAuto;
+  TileOrder tile_order;   // (set by the launchers)
   // A second product of the same A, as in GemmArgs, with e4m3 output: C2 = e4m3(col_scale2[n] * sum * out_mul2). N2 and ldc2
   // multiples of 4, ldw2 of 16. Only with half output of the first product and where GemmF8TakesSecond().
   const uint8_t* W2 = nullptr; int ldw2 = 0;
