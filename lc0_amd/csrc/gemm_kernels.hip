@@ -220,7 +220,8 @@ int g_variant_override = -1;
 
 GemmVariant PickGemmVariant(const GemmArgs& a);
 
-// Fitted cost model of the five direct-to-LDS tile shapes, in microseconds per launch (see PickGemmVariant).
+// Cost model of the five direct-to-LDS tile shapes in halves, in microseconds per launch (see PickGemmVariant), outside the range of the
+// one below.
 struct FittedCosts {
   double t256, t192, t128, ts, t64;
   double Best() const { return std::min(std::min(std::min(t256, t192), std::min(t128, ts)), t64); }
@@ -242,17 +243,88 @@ inline FittedCosts FitCosts(int M, int N, int K) {
   return c;
 }
 
+// Cost model of the direct-to-LDS tiles in microseconds: fixed + rounds * (round + step * k-tiles), a k-tile being 128 bytes and
+// a round a tile on each of the 256 CUs; a last round that fills a fraction f of the CUs counts partial + (1 - partial) f.
+// (Shapes that share a CU follow it as well: a tile beside others takes proportionally longer.) Fitted to all shapes on 120
+// problems in halves and 140 in e4m3, M 1536 to 57600 in steps of 64, N 512 to 3072, K 512 to 2048, in the order of tiles of
+// PickTileOrder; rms error 2 to 7 %. Back to back the shape it picks is 0.4 % (halves) and 0.5 % (e4m3) behind the fastest one
+// measured, the choice before it 2.5 and 1.9 %.
+// Within a pass that holds only in part: from 80 positions the projection has the smolgen chain beside it, which finds no
+// room on CUs that 256x256 tiles fill (us a pass, choice before -> by this model: fp16 100 positions 3131 -> 3438, e4m3 200 3749
+// -> 4221), and from 16384 rows the other products leave through the cache only from 256-row tiles (e4m3 300 5080 -> 5185). So
+// it decides on wide products up to 2559 rows in halves (32 positions 1621 -> 1573, 36 1888 -> 1782; from there to 64 they are level at
+// best, 46 2010 -> 2026) and up to 5119 in e4m3 (32 1172 -> 1140, 36 1349 -> 1305, 50 1553 -> 1522; the other products of so few
+// rows are level or 1 % slower) and on the others from 5120 to 16383 rows (fp16 90 3047 -> 2988, 150 4240 -> 4008; e4m3 100 2436 -> 2372,
+// 117 2564 -> 2480, 200 3612 -> 3540, but 90 2248 -> 2267).
+struct TileCost {
+  GemmVariant variant;
+  int bm, bn;
+  double fixed, round, step, partial;
+};
+constexpr TileCost kHalfCosts[] = {{kDma256x256, 256, 256, 2.07, 5.95, 1.700, 0.655}, {kDma256x192, 256, 192, 1.92, 4.94, 1.368, 0.634},
+                                   {kDma256x128, 256, 128, 3.59, 1.46, 1.156, 0.536}, {kDma128x128, 128, 128, 3.43, 1.27, 0.531, 0.566},
+                                   {kDma128x64, 128, 64, 2.58, 0.38, 0.365, 0.453}};
+constexpr TileCost kF8Costs[] = {{kDma256x256, 256, 256, 3.64, 5.31, 1.699, 0.647}, {kDma256x192, 256, 192, 2.85, 4.69, 1.369, 0.630},
+                                 {kDma256x128, 256, 128, 2.85, 2.98, 1.021, 0.632}, {kDma128x128, 128, 128, 4.01, 1.37, 0.488, 0.501},
+                                 {kDma128x64, 128, 64, 3.21, 0.61, 0.305, 0.432}, {kDma64x64, 64, 64, 2.56, 0.35, 0.186, 0.476}};
+
+constexpr int kHalfWideEnd = 2560, kF8WideEnd = 5120;
+inline bool InTileCostDomain(int M, int N, int K, int wide_end) {
+  if (K < 512 || N < 512) return false;
+  return N >= 2 * K ? M >= 1536 && M < wide_end : M >= 5120 && M < 16384;
+}
+
+double CostOf(const TileCost& c, int M, int N, int k_tiles) {
+  const double x = (double)((M + c.bm - 1) / c.bm) * (double)((N + c.bn - 1) / c.bn) / 256.0, whole = std::floor(x + 1e-9);
+  const double rounds = whole + (x - whole > 1e-9 ? c.partial + (1.0 - c.partial) * (x - whole) : 0.0);
+  return c.fixed + rounds * (c.round + c.step * k_tiles);
+}
+
+template <size_t COUNT, typename Accept>
+const TileCost* Cheapest(const TileCost (&costs)[COUNT], int M, int N, int k_tiles, Accept&& accept) {
+  const TileCost* best = nullptr;
+  double cost = 0.0;
+  for (const TileCost& c : costs) {
+    if (!accept(c.variant)) continue;
+    const double v = CostOf(c, M, N, k_tiles);
+    if (best == nullptr || v < cost) { best = &c; cost = v; }
+  }
+  return best;
+}
+template <size_t COUNT>
+const TileCost* Cheapest(const TileCost (&costs)[COUNT], int M, int N, int k_tiles) {
+  return Cheapest(costs, M, N, k_tiles, [](GemmVariant) { return true; });
+}
+
 // A large product whose tiles do not fill whole rounds of the 256 CUs, cut along its rows: the rows that make whole
 // rounds of 256x256 (or 256x192) tiles go to one launch and the rest to a second launch on whatever shape suits it
-// (20480x1024x1536: 87 us on 320 tiles of 256x256, one and a quarter rounds, or 78 us on 128x128 tiles, against
+// (20480x1024x1536 in halves: 87 us on 320 tiles of 256x256, one and a quarter rounds, or 78 us on 128x128 tiles, against
 // 49 + 19 us for 16384 rows on one full round of large tiles and 4096 rows on small ones). Returns the rows of the
 // first launch (0: one launch) when the model above prices the pair at least 3 % below the best single shape.
 bool g_row_split = true;   // (profiling and tests switch it off through SetGemmRowSplit)
+int PlanRowSplitByTileCost(int M, int N, int k_tiles, GemmVariant* first) {
+  const auto& costs = kHalfCosts;
+  double best = CostOf(*Cheapest(costs, M, N, k_tiles), M, N, k_tiles) * 0.97;
+  int best_m1 = 0;
+  for (int v = 0; v < 2; v++) {
+    const int col_tiles = (N + costs[v].bn - 1) / costs[v].bn;
+    if (col_tiles > 256) continue;
+    const int rows_per_round = (256 / col_tiles) * 256;
+    for (int m1 = rows_per_round; m1 + 4096 <= M; m1 += rows_per_round) {   // (cut at 2048 rows, 96 positions lost 4 %)
+      const double c = CostOf(costs[v], m1, N, k_tiles) + CostOf(*Cheapest(costs, M - m1, N, k_tiles), M - m1, N, k_tiles) + 1.0;
+      if (c < best) { best = c; best_m1 = m1; *first = costs[v].variant; }
+    }
+  }
+  return best_m1;
+}
+
 int PlanRowSplit(const GemmArgs& a, GemmVariant* first) {
-  if (!g_row_split || g_variant_override >= 0 || !InFittedDomain(a) || a.out_f32 || a.split_k != 1 || a.K % 64 != 0 ||
-      a.skip != nullptr || a.row_stats != nullptr) {
+  if (!g_row_split || g_variant_override >= 0 || a.batch != 1 || a.out_f32 || a.split_k != 1 || a.K % 64 != 0 || a.skip != nullptr ||
+      a.row_stats != nullptr) {
     return 0;
   }
+  if (InTileCostDomain(a.M, a.N, a.K, kHalfWideEnd)) return PlanRowSplitByTileCost(a.M, a.N, a.K / 64, first);
+  if (!InFittedDomain(a)) return 0;
   double best = FitCosts(a.M, a.N, a.K).Best() * 0.97;
   int best_m1 = 0;
   for (int v = 0; v < 2; v++) {
@@ -279,6 +351,33 @@ int PlanRowSplit(const GemmArgs& a, GemmVariant* first) {
 inline GemmVariant OneRoundTile(int M, int N, int batch) {
   auto fits = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch <= 256; };
   return fits(64, 64) ? kDma64x64 : fits(128, 64) ? kDma128x64 : fits(128, 128) ? kDma128x128 : kNoVariant;
+}
+
+// Whether the workgroups of a second product of N2 columns are no more per CU than those of the first one alone: the
+// launch then takes no longer than without them.
+bool SecondFits(GemmVariant v, int M, int N, int N2) {
+  if (v == kRowPanel) {
+    for (const RowPanelShape& c : kRowPanelShapes) {   // (the panel that the first product gets)
+      const long long first = RowPanelWorkgroups(M, N, 1, c);
+      if (first <= kRowPanelWorkgroups) return first + RowPanelWorkgroups(M, N2, 1, c) <= kRowPanelWorkgroups;
+    }
+    return false;
+  }
+  const int bm = v == kDma64x64 ? 64 : 128, bn = v == kDma128x128 ? 128 : 64;
+  if (v != kDma64x64 && v != kDma128x64 && v != kDma128x128) return false;
+  const long long rows = (M + bm - 1) / bm, first = rows * ((N + bn - 1) / bn), both = first + rows * ((N2 + bn - 1) / bn);
+  return (both + 255) / 256 == (first + 255) / 256;
+}
+// The cheapest shape by the cost model. With a second product the cheapest that takes it is allowed 1.5 us more: a launch of its own for
+// the second one costs more, but the smaller tiles lose some of that again (with 4 us 50 positions in halves 2053 -> 2078 a pass).
+template <size_t COUNT, typename Accept>
+GemmVariant PickFitted(const TileCost (&costs)[COUNT], int M, int N, int k_tiles, int N2, Accept&& accept) {
+  const TileCost* best = Cheapest(costs, M, N, k_tiles, accept);
+  if (N2 > 0 && !SecondFits(best->variant, M, N, N2)) {
+    const TileCost* both = Cheapest(costs, M, N, k_tiles, [&](GemmVariant v) { return accept(v) && SecondFits(v, M, N, N2); });
+    if (both != nullptr && CostOf(*both, M, N, k_tiles) <= CostOf(*best, M, N, k_tiles) + 1.5) best = both;
+  }
+  return best->variant;
 }
 
 GemmVariant PickGemmVariant(const GemmArgs& a) {
@@ -316,14 +415,10 @@ GemmVariant PickGemmVariant(const GemmArgs& a) {
     // output element and round (ns per element at K = 1024): 0.60 for 256x256, 0.61 for 256x192;
     // the two small shapes run two workgroups per CU, 0.68 (256x128) and 0.75 (128x128) per element
     // while sharing a CU, 0.84 and 0.95 when a single round leaves every workgroup alone on its CU.
-    // One product of at least 4096 rows with K and N of at least 512 (the encoder layers of the attention bodies
-    // from 64 positions up): a cost model in microseconds fitted to launches of all five shapes on 92 problems
-    // (M 4096 to 65536, N 512 to 3072, K 512 to 2048; the variant it picks is 0.6 % behind the fastest measured one
-    // on average and 9 % at worst, against 3 % and 24 % for the per-element model below, which was set when the
-    // large tiles were slower than they are now). A round of the one-workgroup-per-CU shapes costs a fixed part and
-    // a part per k-tile of 64; a last round that fills only a fraction f of the CUs costs 0.55 + 0.45 f of a full
-    // one (its workgroups find L2 and the memory system less contended); the shapes that share a CU are priced by
-    // tile count.
+    if (a.batch == 1 && InTileCostDomain(a.M, a.N, a.K, kHalfWideEnd)) {
+      auto known = [&](GemmVariant v) { return v != kDma256x192 || a.skip == nullptr; };
+      return PickFitted(kHalfCosts, a.M, a.N, a.K / 64, a.N2, known);
+    }
     if (InFittedDomain(a)) {
       const FittedCosts c = FitCosts(a.M, a.N, a.K);
       GemmVariant best = kDma256x256;
@@ -438,24 +533,6 @@ bool GemmSupportsNormFolding(const GemmArgs& a) {
   return true;
 }
 
-namespace {
-// Whether the workgroups of a second product of N2 columns are no more per CU than those of the first one alone: the
-// launch then takes no longer than without them.
-bool SecondFits(GemmVariant v, int M, int N, int N2) {
-  if (v == kRowPanel) {
-    for (const RowPanelShape& c : kRowPanelShapes) {   // (the panel that the first product gets)
-      const long long first = RowPanelWorkgroups(M, N, 1, c);
-      if (first <= kRowPanelWorkgroups) return first + RowPanelWorkgroups(M, N2, 1, c) <= kRowPanelWorkgroups;
-    }
-    return false;
-  }
-  const int bm = v == kDma64x64 ? 64 : 128, bn = v == kDma128x128 ? 128 : 64;
-  if (v != kDma64x64 && v != kDma128x64 && v != kDma128x128) return false;
-  const long long rows = (M + bm - 1) / bm, first = rows * ((N + bn - 1) / bn), both = first + rows * ((N2 + bn - 1) / bn);
-  return (both + 255) / 256 == (first + 255) / 256;
-}
-}  // namespace
-
 bool GemmTakesSecond(const GemmArgs& a) {
   GemmVariant first = kDma256x256;
   return a.batch == 1 && a.split_k == 1 && !a.out_f32 && a.skip == nullptr && a.row_stats == nullptr && a.N2 % 8 == 0 &&
@@ -536,8 +613,8 @@ bool GemmF8TakesRowPanels(const GemmF8Args& a) {
   return a.K >= 256 && RowPanelWorkgroups(a.M, a.N, 1, kRowPanelShapes[3]) <= kRowPanelWorkgroups;
 }
 
-// kDma256x256, kDma256x192, kDma256x128, kDma128x128 and kDma128x64 (two / three workgroups per CU) by
-// the cost model of the fp16 kernels (the k-tile structure is the same).
+// Outside the fitted range kDma256x256, kDma256x192, kDma256x128, kDma128x128 and kDma128x64 (two / three workgroups per CU) by
+// the cost per element of the fp16 kernels (the k-tile structure is the same).
 GemmVariant PickGemmF8Variant(const GemmF8Args& a) {
   if (g_variant_override >= 0 && (g_variant_override <= 2 || g_variant_override == kDma128x128 ||
                                   g_variant_override == kDma128x64 || g_variant_override == kRowPanel ||
@@ -545,6 +622,7 @@ GemmVariant PickGemmF8Variant(const GemmF8Args& a) {
     return static_cast<GemmVariant>(g_variant_override);
   }
   if (GemmF8TakesRowPanels(a)) return kRowPanel;
+  if (InTileCostDomain(a.M, a.N, a.K, kF8WideEnd)) return PickFitted(kF8Costs, a.M, a.N, (a.K + 127) / 128, a.N2, [](GemmVariant) { return true; });
   // A few hundred to a few thousand rows: 64x64 tiles, up to three workgroups of which share a CU and fill each other's
   // gaps (us against 128x64 tiles: 1024x1024x1536 5.5 / 6.8, 2048x1024x1024 5.5 / 6.3, 2048x1536x1024 on 768 tiles
   // 7.4 / 7.9, 4096x1024x1024 on 1024 tiles 8.9 / 8.5). With several per CU, few rows and weights beyond the 4 MiB of an
