@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256, 2) void qkv_attention_kernel(const half_t* __r
 // 740 -> 471, 1000 1946 -> 1270, with smolgen, where only this kernel is used, 64 654 -> 497, 1000 3721 -> 3166; width 256 with smolgen
 // 64 712 -> 606, 1000 4986 -> 4216. One launch at a width of 512 or more would stream more bytes through every CU than the separate products take.
 // ---------------------------------------------------------------------------
-template <typename ET, int CT, int RT>
+template <typename ET, int CT, int RT, int SPLIT>
 __global__ __launch_bounds__(512) void encoder_tail_kernel(EncoderTailArgs p) {
   using ev8 = typename Vec16<ET>::v8;
   using ev4 = typename Vec16<ET>::v4;
@@ -181,9 +181,11 @@ __global__ __launch_bounds__(512) void encoder_tail_kernel(EncoderTailArgs p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const long long row0 = (long long)blockIdx.x * R;
+  const int block = blockIdx.x / SPLIT, slice = blockIdx.x % SPLIT;
+  const long long row0 = (long long)block * R;
   const int col = wave * 16 * CT + 4 * g;                          // of this lane's four, + 16 c
-  const int att_parts = p.d_model / C, ffn_parts = p.dff / C, parts = att_parts + 2 * ffn_parts;
+  const int att_parts = p.d_model / C, ffn_begin = slice * (p.dff / C) / SPLIT, ffn_end = (slice + 1) * (p.dff / C) / SPLIT;
+  const int parts = att_parts + 2 * (ffn_end - ffn_begin);
 
   // C columns of the attention output into LDS.
   intx4 av[V];
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(512) void encoder_tail_kernel(EncoderTailArgs p) {
       for (int c = 0; c < CT; c++) a[t][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
   };
   auto multiply = [&](const ET* rows, floatx4 (&a)[RT][CT]) {
-    if (++part < parts) next += 8 * S * CT * 64;                   // (after the last part its own weights once more)
+    if (++part < parts) next += 8 * S * CT * 64 * (part == att_parts ? 1 + 2 * ffn_begin : 1);   // (after the last part its own weights once more)
     // Rows DEPTH steps ahead; the order is fixed, or the compiler gathers the loads at the end of a part, where the next part
     // waits for them.
     constexpr int DEPTH = RT == 1 ? S : RT == 2 ? S / 2 : 2;
@@ -326,7 +328,7 @@ __global__ __launch_bounds__(512) void encoder_tail_kernel(EncoderTailArgs p) {
   clear(sum);
   load4(p.ln2_g, col, gamma);
   load4(p.ln2_b, col, beta);
-  for (int f = 0; f < ffn_parts; f++) {
+  for (int f = ffn_begin; f < ffn_end; f++) {
     load4(p.ffn1_b, f * C + col, bias);
     clear(acc);
     multiply(u_lds, acc);
@@ -344,6 +346,44 @@ __global__ __launch_bounds__(512) void encoder_tail_kernel(EncoderTailArgs p) {
     });
     __syncthreads();
     multiply(h, sum);
+  }
+  if constexpr (SPLIT > 1) {
+    // Every slice leaves its sums, written through to memory; the last one of the block to arrive adds all of them, in the order of
+    // the slices whoever that is, and goes on. Nobody waits for another workgroup. (The stores pass by the L2 of their XCD, and
+    // the wait makes them complete before the workgroup counts itself.)
+    __shared__ int last;
+    floatx4* place = reinterpret_cast<floatx4*>(p.partial) + (long long)block * SPLIT * RT * CT * 512 + tid;
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+      for (int c = 0; c < CT; c++) StoreThrough16(place + ((slice * RT + t) * CT + c) * 512, __builtin_bit_cast(intx4, sum[t][c]));
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+    __syncthreads();
+    if (tid == 0) {
+      last = __hip_atomic_fetch_add(p.arrived + block, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == SPLIT - 1;
+      if (last) __hip_atomic_store(p.arrived + block, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (for the next launch)
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();
+    if (!last) return;
+    floatx4 other[SPLIT][RT][CT];
+#pragma unroll
+    for (int j = 0; j < SPLIT; j++)
+#pragma unroll
+      for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int c = 0; c < CT; c++)
+          other[j][t][c] = place[((j * RT + t) * CT + c) * 512];
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+      for (int c = 0; c < CT; c++) {
+        sum[t][c] = other[0][t][c];
+#pragma unroll
+        for (int j = 1; j < SPLIT; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) sum[t][c][e] += other[j][t][c][e];
+      }
   }
   load4(p.ffn2_b, col, bias);
 #pragma unroll
@@ -364,14 +404,22 @@ __global__ __launch_bounds__(512) void encoder_tail_kernel(EncoderTailArgs p) {
 
 template <typename ET, int CT>
 void LaunchTailT(const EncoderTailArgs& a, hipStream_t stream) {
-  const int rt = EncoderTailRows(a.M) / 16;
-  if (rt == 1) {
-    hipLaunchKernelGGL((encoder_tail_kernel<ET, CT, 1>), dim3(a.M / 16), dim3(512), 0, stream, a);
-  } else if (rt == 2) {
-    hipLaunchKernelGGL((encoder_tail_kernel<ET, CT, 2>), dim3(a.M / 32), dim3(512), 0, stream, a);
-  } else {
-    hipLaunchKernelGGL((encoder_tail_kernel<ET, CT, 4>), dim3(a.M / 64), dim3(512), 0, stream, a);
-  }
+  const EncoderTailShape shape = PickEncoderTailShape(a.M, a.emb, a.dff);
+  auto launch = [&](auto rt_tag, auto split_tag) {
+    constexpr int RT = decltype(rt_tag)::value, SPLIT = decltype(split_tag)::value;
+    hipLaunchKernelGGL((encoder_tail_kernel<ET, CT, RT, SPLIT>), dim3(a.M / (16 * RT) * SPLIT), dim3(512), 0, stream, a);
+  };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  using Four = std::integral_constant<int, 4>;
+  auto by_rows = [&](auto split_tag) {
+    if (shape.rows == 16) launch(One{}, split_tag);
+    else if (shape.rows == 32) launch(Two{}, split_tag);
+    else launch(Four{}, split_tag);
+  };
+  if (shape.slices == 4) by_rows(Four{});
+  else if (shape.slices == 2) by_rows(Two{});
+  else by_rows(One{});
 }
 
 template <typename ET>
@@ -407,8 +455,19 @@ bool EncoderTailSupported(int emb, int d_model, int dff) {
 }
 
 // 16 rows per workgroup while they all fit the CUs, else 32, else 64: a workgroup takes the weights through its CU once
-// whatever its rows, so more of them per workgroup cost nothing until their products take longer than the stream.
-int EncoderTailRows(int M) { return M <= 16 * 256 ? 16 : M <= 32 * 256 ? 32 : 64; }
+// whatever its rows, so more of them per workgroup cost nothing until their products take longer than the stream. Where that leaves
+// half of the CUs without work, four or two workgroups (SPLIT) share the FFN of their rows: each takes that much less of the weights, and
+// leaving and adding the sums costs about 3 us, the time of 0.3 MB. us of a ten-layer pass of width 256 with 1024 hidden columns, alone ->
+// shared: by four 5 positions 312 -> 263, 8 312 -> 268, by two 16 318 -> 297. By four up to 16 positions (293) and by two up to 28 (330 -> 321) a
+// pass alone is faster still, but four threads together lose 10 % (16 positions 127k -> 112k evals/s; as it is 123k -> 125k). With 32 rows per
+// workgroup and two slices 64 positions 360 -> 377. Parts of width 128 are a quarter as large: not there.
+EncoderTailShape PickEncoderTailShape(int M, int emb, int dff) {
+  if (emb == 256) {
+    if (M <= 8 * 64 && dff >= 4 * emb) return {16, 4};
+    if (M <= 16 * 64 && dff >= 2 * emb) return {16, 2};
+  }
+  return {M <= 16 * 256 ? 16 : M <= 32 * 256 ? 32 : 64, 1};
+}
 
 // A few workgroups stream all weights through one CU each, whatever the batch, where five launches spread them over the chip;
 // how many positions that costs follows from their bytes. us of a ten-layer pass, layers one by one -> the kernel. Width 256,
@@ -438,6 +497,9 @@ long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_m
 void LaunchEncoderTail(const EncoderTailArgs& a, hipStream_t stream) {
   if (a.M <= 0) return;
   if (!EncoderTailSupported(a.emb, a.d_model, a.dff) || a.M % 64 != 0) throw std::runtime_error("LaunchEncoderTail: unsupported shape");
+  if (PickEncoderTailShape(a.M, a.emb, a.dff).slices > 1 && (a.partial == nullptr || a.arrived == nullptr)) {
+    throw std::runtime_error("LaunchEncoderTail: no place for the slices' sums");
+  }
   if (a.emb == 256) {
     if (a.bf16) LaunchTailT<bf16_t, 2>(a, stream);
     else LaunchTailT<half_t, 2>(a, stream);

@@ -49,10 +49,7 @@ __device__ __forceinline__ void StoreOut16(void* dst, intx4 val) {
   if constexpr (STORES == 1) {
     __builtin_nontemporal_store(val, reinterpret_cast<intx4*>(dst));
   } else if constexpr (STORES == 2) {
-    // (the no-op covers the wait states that the hardware needs between a store of more than eight bytes and a vector
-    // ALU write to its data registers - two on this part; the compiler adds them after its own stores and does not
-    // look into this one: without them the 256x128 tiles, which reuse the registers at once, stored wrong values)
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(dst), "v"(val) : "memory");
+    StoreThrough16(dst, val);
   } else {
     *reinterpret_cast<intx4*>(dst) = val;
   }

@@ -720,6 +720,8 @@ int lc0mi_k_encoder_tail(const uint16_t* att, uint16_t* x, const uint16_t* dense
     const float* n = dev.Put(norms, (size_t)4 * emb);
     a.ln1_g = n; a.ln1_b = n + emb; a.ln2_g = n + 2 * emb; a.ln2_b = n + 3 * emb;
     a.M = M; a.emb = emb; a.d_model = d_model; a.dff = dff; a.alpha = alpha; a.eps = eps; a.act = act; a.bf16 = g_bf16;
+    a.partial = static_cast<float*>(dev.Alloc(sizeof(float) * lc0mi::kEncoderTailPartial));
+    a.arrived = dev.Put(std::vector<int>(lc0mi::kEncoderTailBlocks).data(), lc0mi::kEncoderTailBlocks);
     lc0mi::LaunchEncoderTail(a, nullptr);
     K_CHECK(hipDeviceSynchronize());
     K_CHECK(hipGetLastError());

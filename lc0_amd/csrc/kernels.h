@@ -329,9 +329,15 @@ struct EncoderTailArgs {
   int act = 3;
   bool bf16 = false;
   float *u = nullptr, *partial = nullptr;   // floats with several slices: [M][emb], [slices][M][emb], slices at most dff / emb
+  // 16-bit types: partial holds kEncoderTailPartial floats, arrived kEncoderTailBlocks zeros (and does again after the launch). One
+  // launch at a time may use them.
+  int* arrived = nullptr;
 };
+// Rows of a workgroup, and workgroups that share the FFN of those rows.
+struct EncoderTailShape { int rows, slices; };
+EncoderTailShape PickEncoderTailShape(int M, int emb, int dff);
+constexpr int kEncoderTailBlocks = 64, kEncoderTailPartial = 128 * 16 * 256;   // (several slices: at most 128 workgroups of 16 rows)
 bool EncoderTailSupported(int emb, int d_model, int dff);
-int EncoderTailRows(int M);   // rows of a workgroup
 int EncoderTailMinBatch(int emb, int d_model, int dff);   // smallest batch at which it is faster than its layers one by one
 long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_model);
 void LaunchEncoderTail(const EncoderTailArgs& args, hipStream_t stream);

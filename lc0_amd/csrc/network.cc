@@ -503,6 +503,8 @@ class Mi355xNetwork : public Network, protected ModelState {
   // Partial row sums of the two un-normalised sums of an encoder layer (folded layer norms): [rows][parts][2].
   float *ln_stats_a_ = nullptr, *ln_stats_b_ = nullptr;
   half_t *pol_e_ = nullptr, *pol_qk_ = nullptr, *head1_ = nullptr, *head2_ = nullptr;
+  float* tail_partial_ = nullptr;   // EncoderTailArgs::partial, arrived
+  int* tail_arrived_ = nullptr;
   half_t *pe_qkv_ = nullptr, *pe_att_ = nullptr, *pe_t_ = nullptr, *pe_ffn_ = nullptr;   // policy encoder scratch
   half_t *pe_sg1_ = nullptr, *pe_sg2_ = nullptr, *pe_sg3_ = nullptr, *pe_sbias_ = nullptr;
   float *pol_logits_ = nullptr, *d_policy_ = nullptr, *d_wdl_ = nullptr, *d_mlh_ = nullptr;
@@ -1304,6 +1306,10 @@ void Mi355xNetwork::AllocActivations() {
   qkv_ = AllocH(T * 3 * d_model_);
   att_ = AllocH(T * d_model_);
   ffn_ = AllocH(T * std::max(dff_, emb_dff_));
+  if (dtype_ != Dtype::kFloat && !encoders_.empty() && encoders_[0].tail_packed != nullptr) {
+    tail_partial_ = AllocF(kEncoderTailPartial);
+    tail_arrived_ = arena_.Upload(std::vector<int>(kEncoderTailBlocks));
+  }
   if (pe_dense_) {
     pre_in_ = AllocH(static_cast<size_t>(max_batch_) * 768);
     pre_out_ = AllocH(T * enc_ch_);
@@ -2347,7 +2353,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
         a.ln1_g = e.ln1_g; a.ln1_b = e.ln1_b; a.ln2_g = e.ln2_g; a.ln2_b = e.ln2_b;
         a.M = T; a.emb = emb_; a.d_model = d_model_; a.dff = dff_;
         a.alpha = alpha_; a.eps = eps_; a.act = ffn_act_; a.bf16 = bf16;
-        a.u = reinterpret_cast<float*>(t_); a.partial = reinterpret_cast<float*>(ffn_);
+        a.u = reinterpret_cast<float*>(t_); a.partial = f32 ? reinterpret_cast<float*>(ffn_) : tail_partial_; a.arrived = tail_arrived_;
         const double weights = static_cast<double>(emb_) * (d_model_ + 2 * dff_);
         Timed("encoder_tail", 2.0 * T * weights, (f32 ? 6.0 : 2.0) * weights + es_ * T * (2.0 * emb_ + d_model_), [&] { f32 ? LaunchEncoderTailF32(a, stream_) : LaunchEncoderTail(a, stream_); });
         continue;
