@@ -109,6 +109,9 @@ int lc0mi_k_expand_planes_nchw(const uint64_t* masks, const float* values, int b
  * ppo [4][pd] floats -> policy [B][1858] (network_blas.cc:873-914). */
 int lc0mi_k_attn_policy_gather(const float* logits, const uint16_t* keys, const float* ppo, int pd, int batch,
                                float* out);
+/* The attention policy from its query and key vectors on: qk [B*64][2 depth] halves (bfloat16 bits after lc0mi_k_set_bf16), queries
+ * first, ppo [4][depth] floats -> policy [B][1858] (network_blas.cc:850-914). depth % 8 == 0. */
+int lc0mi_k_policy_tail(const uint16_t* qk, const float* ppo, int depth, int batch, float scale, float* out, int time_iters, double* ms);
 
 /* Softmax over listed moves with lc0's FastExp (NetworkAsBackendComputation::SoftmaxPolicy,
  * src/neural/wrapper.cc:135-156; src/utils/fastmath.h:59-86): policy [batch][1858]; sample b lists

@@ -517,6 +517,26 @@ int lc0mi_k_attn_policy_gather(const float* logits, const uint16_t* keys, const 
   });
 }
 
+int lc0mi_k_policy_tail(const uint16_t* qk, const float* ppo, int depth, int batch, float scale, float* out, int time_iters, double* ms) {
+  return Guard([&] {
+    RequireDevice();
+    if (batch < 1 || depth < 1) throw Error("bad policy shape");
+    Dev dev;
+    lc0mi::PolicyTailArgs a;
+    a.qk = reinterpret_cast<half_t*>(dev.Put(qk, (size_t)batch * 64 * 2 * depth));
+    a.ld = 2 * depth; a.key_offset = a.depth = depth; a.scale = scale;
+    a.ppo = dev.Put(ppo, (size_t)4 * depth);
+    const auto& inv = lc0mi::AttnPolicyInverseMap();
+    a.inv_map = dev.Put(inv.data(), inv.size());
+    a.out = static_cast<float*>(dev.Alloc((size_t)batch * 1858 * 4));
+    lc0mi::LaunchPolicyTail(a, batch, g_bf16, nullptr);
+    K_CHECK(hipDeviceSynchronize());
+    K_CHECK(hipGetLastError());
+    K_CHECK(hipMemcpy(out, a.out, (size_t)batch * 1858 * 4, hipMemcpyDeviceToHost));
+    if (time_iters > 0 && ms) *ms = TimeLaunches(time_iters, [&] { lc0mi::LaunchPolicyTail(a, batch, g_bf16, nullptr); });
+  });
+}
+
 int lc0mi_k_legal_softmax(const float* policy, const int* offsets, const uint16_t* ids, float inv_temperature,
                           int batch, float* probs) {
   return Guard([&] {

@@ -363,10 +363,24 @@ struct HeadLayers {
   int out_act = 3;
   float* out = nullptr;
 };
+// Attention policy of 16-bit networks from its query and key vectors on: qk [B*64][ld], queries from column 0 and keys from
+// key_offset, depth values each; logits scale Q.K, promotion offsets from ppo ([4][depth]), gather by inv_map ([1858], into the 4096 +
+// 192 virtual buffer of LaunchAttnPolicyGather) to out [B][1858].
+struct PolicyTailArgs {
+  const half_t* qk = nullptr;
+  int ld = 0, key_offset = 0, depth = 0;
+  float scale = 1.0f;
+  const float* ppo = nullptr;
+  const int16_t* inv_map = nullptr;
+  float* out = nullptr;
+};
+bool PolicyTailSupported(const PolicyTailArgs& args);
+void LaunchPolicyTail(const PolicyTailArgs& args, int batch, bool bf16, hipStream_t stream);
 struct ValueHeadsArgs {
   const half_t* x = nullptr;
   int ldx = 0, emb = 0, batch = 0, heads = 0, act = 3;
   HeadLayers head[2];
+  PolicyTailArgs policy;   // in the same launch, unless qk is null
   bool bf16 = false;
 };
 long long HeadFragments(bool embed, int emb, int ch);

@@ -758,8 +758,6 @@ void LaunchAttnPolicyGather(const float* logits, const T* kq, int ld_kq, int key
 }
 template void LaunchAttnPolicyGather<half_t>(const float*, const half_t*, int, int, const float*, int, const int16_t*,
                                              float*, int, hipStream_t);
-template void LaunchAttnPolicyGather<bf16_t>(const float*, const bf16_t*, int, int, const float*, int, const int16_t*,
-                                             float*, int, hipStream_t);
 template void LaunchAttnPolicyGather<float>(const float*, const float*, int, int, const float*, int, const int16_t*,
                                             float*, int, hipStream_t);
 

@@ -411,7 +411,7 @@ class Mi355xNetwork : public Network, protected ModelState {
   void ForwardDevice(int batch);
   void ForwardAttentionBody(int B);
   void BuildAttentionPolicy(const NetWeights& w, const PolicyHead& ph, int in_channels);
-  void ForwardAttentionPolicy(const half_t* x, int ld_x, int B);
+  void ForwardAttentionPolicy(const half_t* x, int ld_x, int B, ValueHeadsArgs* beside = nullptr, double beside_flops = 0.0, double beside_bytes = 0.0);
   EncoderDev MakeEncoderLayer(const EncoderLayer& l, int emb, int d_model, int dff);
   // Smolgen weights of one encoder layer; hc / hs / gen receive (or are checked against) the chain's widths.
   void LoadSmolgen(const Smolgen& s, int emb, int heads, EncoderDev* e, int* hc, int* hs, int* gen, bool* any);
@@ -1272,7 +1272,7 @@ void Mi355xNetwork::AllocActivations() {
     const size_t T = static_cast<size_t>(max_batch_) * 64;
     pol_e_ = AllocH(T * pol_emb_);
     pol_qk_ = AllocH(T * 2 * pol_d_);
-    pol_logits_ = AllocF(static_cast<size_t>(max_batch_) * 4096);
+    if (dtype_ == Dtype::kFloat) pol_logits_ = AllocF(static_cast<size_t>(max_batch_) * 4096);
     if (!pol_encoders_.empty()) {
       pe_qkv_ = AllocH(T * 3 * pe_dmodel_);
       pe_att_ = AllocH(T * pe_dmodel_);
@@ -1446,7 +1446,8 @@ void Mi355xNetwork::BuildAttentionPolicy(const NetWeights& w, const PolicyHead& 
   inv_map_ = arena_.Upload(AttnPolicyInverseMap());
 }
 
-void Mi355xNetwork::ForwardAttentionPolicy(const half_t* x, int ld_x, int B) {
+// (beside: value heads that run in the launch of the policy's last kernel)
+void Mi355xNetwork::ForwardAttentionPolicy(const half_t* x, int ld_x, int B, ValueHeadsArgs* beside, double beside_flops, double beside_bytes) {
   const int T = B * 64;
   Gemm("gemm_policy_embed", x, ld_x, pol_emb_lin_, pol_e_, pol_emb_, T, pol_emb_act_);
   for (const EncoderDev& e : pol_encoders_) {   // alpha 1, eps 1e-6 (network_blas.cc:836-842)
@@ -1472,38 +1473,30 @@ void Mi355xNetwork::ForwardAttentionPolicy(const half_t* x, int ld_x, int B) {
   // Per-sample Q.K^T / sqrt(d): 64 x 64 logits, float (network_blas.cc:850-872).
   const float logit_scale = 1.0f / std::sqrt(static_cast<float>(pol_d_));
   const double logit_flops = 2.0 * 64 * 64 * pol_d_ * B, logit_bytes = B * (2.0 * es_ * 64 * pol_d_ + 4.0 * 4096);
-  if (dtype_ == Dtype::kFloat) {
-    GemmArgsF32 g;
-    g.A = reinterpret_cast<const float*>(pol_qk_); g.lda = 2 * pol_d_; g.strideA = 64LL * 2 * pol_d_;
-    g.W = reinterpret_cast<const float*>(ElemAt(pol_qk_, pol_d_)); g.ldw = 2 * pol_d_; g.strideW = 64LL * 2 * pol_d_;
-    g.C = pol_logits_; g.ldc = 64; g.strideC = 4096;
-    g.M = 64; g.N = 64; g.K = pol_d_; g.batch = B;
-    g.scale = logit_scale;
-    g.act = kActNone;
-    Timed("gemm_policy_logits|gemm_f32_mfma_16x16x4", logit_flops, logit_bytes, [&] { LaunchGemmF32(g, stream_); });
-  } else {
-    GemmArgs g;
-    g.A = pol_qk_; g.lda = 2 * pol_d_; g.strideA = 64LL * 2 * pol_d_;
-    g.W = pol_qk_ + pol_d_; g.ldw = 2 * pol_d_; g.strideW = 64LL * 2 * pol_d_;
-    g.C = pol_logits_; g.ldc = 64; g.strideC = 4096;
-    g.M = 64; g.N = 64; g.K = pol_d_; g.batch = B;
-    g.scale = logit_scale;
-    g.act = kActNone;
-    g.out_f32 = true;
-    g.bf16 = dtype_ == Dtype::kBf16;
-    const std::string label = std::string("gemm_policy_logits|") + GemmVariantName(g);
-    Timed(label.c_str(), logit_flops, logit_bytes, [&] { LaunchGemm(g, stream_); });
-  }
-  Timed("policy_gather", 0.0, B * (4.0 * 4288 + 4.0 * 1858), [&] {
-    if (dtype_ == Dtype::kFloat) {
-      LaunchAttnPolicyGather(pol_logits_, reinterpret_cast<const float*>(pol_qk_), 2 * pol_d_, pol_d_, ppo_, pol_d_,
-                             inv_map_, d_policy_, B, stream_);
-    } else if (dtype_ == Dtype::kBf16) {
-      LaunchAttnPolicyGather(pol_logits_, reinterpret_cast<const bf16_t*>(pol_qk_), 2 * pol_d_, pol_d_, ppo_, pol_d_,
-                             inv_map_, d_policy_, B, stream_);
+  if (dtype_ != Dtype::kFloat) {
+    PolicyTailArgs tail;
+    tail.qk = pol_qk_; tail.ld = 2 * pol_d_; tail.key_offset = pol_d_; tail.depth = pol_d_; tail.scale = logit_scale;
+    tail.ppo = ppo_; tail.inv_map = inv_map_; tail.out = d_policy_;
+    const double bytes = B * (2.0 * es_ * 64 * pol_d_ + 4.0 * 1858);
+    if (beside != nullptr) {
+      beside->policy = tail;
+      Timed("value_heads", beside_flops + logit_flops, beside_bytes + bytes, [&] { LaunchValueHeads(*beside, stream_); });
     } else {
-      LaunchAttnPolicyGather(pol_logits_, pol_qk_, 2 * pol_d_, pol_d_, ppo_, pol_d_, inv_map_, d_policy_, B, stream_);
+      Timed("policy_tail", logit_flops, bytes, [&] { LaunchPolicyTail(tail, B, dtype_ == Dtype::kBf16, stream_); });
     }
+    return;
+  }
+  GemmArgsF32 g;
+  g.A = reinterpret_cast<const float*>(pol_qk_); g.lda = 2 * pol_d_; g.strideA = 64LL * 2 * pol_d_;
+  g.W = reinterpret_cast<const float*>(ElemAt(pol_qk_, pol_d_)); g.ldw = 2 * pol_d_; g.strideW = 64LL * 2 * pol_d_;
+  g.C = pol_logits_; g.ldc = 64; g.strideC = 4096;
+  g.M = 64; g.N = 64; g.K = pol_d_; g.batch = B;
+  g.scale = logit_scale;
+  g.act = kActNone;
+  Timed("gemm_policy_logits|gemm_f32_mfma_16x16x4", logit_flops, logit_bytes, [&] { LaunchGemmF32(g, stream_); });
+  Timed("policy_gather", 0.0, B * (4.0 * 4288 + 4.0 * 1858), [&] {
+    LaunchAttnPolicyGather(pol_logits_, reinterpret_cast<const float*>(pol_qk_), 2 * pol_d_, pol_d_, ppo_, pol_d_, inv_map_, d_policy_, B,
+                           stream_);
   });
 }
 
@@ -2430,8 +2423,11 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
   // 1234 -> 1217, 77 2776 -> 2764, 128 level, 256 5603 -> 5633; e4m3 16 934 -> 916. Ten layers with smolgen, width 512 fp16 1 459 -> 447, 64 883 ->
   // 865, 128 1483 -> 1459, 256 2132 -> 2098, 1000 level; width 768 1 530 -> 518, 16 707 -> 695, from 24 on level, 256 3100 -> 3118.
   const int fused_heads_max = fused_heads_max_batch_ >= 0 ? fused_heads_max_batch_ : emb_ <= 256 ? 256 : 128;
+  ValueHeadsArgs heads_args;
+  bool heads_with_policy = false;
+  double head_flops = 0.0, head_bytes = 0.0;
   if (val_packed_[0] != nullptr && B <= fused_heads_max) {
-    ValueHeadsArgs a;
+    ValueHeadsArgs& a = heads_args;
     a.x = x_; a.ldx = emb_; a.emb = emb_; a.batch = B; a.act = default_act_; a.bf16 = dtype_ == Dtype::kBf16;
     double weights = 0.0;
     auto add = [&](half_t* const (&packed)[2], const Linear& embed, const Linear& fc1, const Linear& fc2, int out_act, float* out) {
@@ -2444,8 +2440,10 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
     };
     add(val_packed_, val_emb_lin_, val_fc1_, val_fc2_, kActNone, d_wdl_);
     if (moves_left_) add(mov_packed_, mov_emb_lin_, mov_fc1_, mov_fc2_, kActRelu, d_mlh_);
-    Timed("value_heads", 2.0 * B * (weights + 63.0 * emb_ * (val_ch_ + (moves_left_ ? mov_ch_ : 0))),
-          2.0 * (weights + static_cast<double>(T) * emb_), [&] { LaunchValueHeads(a, hs); }, hs);
+    head_flops = 2.0 * B * (weights + 63.0 * emb_ * (val_ch_ + (moves_left_ ? mov_ch_ : 0)));
+    head_bytes = 2.0 * (weights + static_cast<double>(T) * emb_);
+    heads_with_policy = !heads_beside;
+    if (heads_beside) Timed("value_heads", head_flops, head_bytes, [&] { LaunchValueHeads(a, hs); }, hs);
   } else {
     Gemm("gemm_value_embed", x_, emb_, val_emb_lin_, head1_, val_ch_, T, default_act_, false, hs);
     Gemm("gemm_value_fc1", head1_, 64 * val_ch_, val_fc1_, head2_, val_fc_, B, default_act_, false, hs);
@@ -2458,7 +2456,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
   }
   if (heads_beside) HIP_CHECK(hipEventRecord(heads_join_, hs));
   // Policy head.
-  ForwardAttentionPolicy(x_, emb_, B);
+  ForwardAttentionPolicy(x_, emb_, B, heads_with_policy ? &heads_args : nullptr, head_flops, head_bytes);
   if (heads_beside) HIP_CHECK(hipStreamWaitEvent(stream_, heads_join_, 0));
 }
 

@@ -1,6 +1,11 @@
-// Value and moves-left heads of 16-bit attention bodies in one kernel: embedding layer, first and second dense layer.
-// Replaces three calls of FullyConnectedLayer::Forward1D per head: blas/network_blas.cc:725-772.
+// Heads of 16-bit attention bodies: value and moves-left heads in one kernel (embedding layer, first and second dense layer), the
+// attention policy from its query and key vectors on, and both in one launch.
+// Replaces three calls of FullyConnectedLayer::Forward1D per head: blas/network_blas.cc:725-772, and the logits, promotion
+// offsets and the gather of the policy: blas/network_blas.cc:850-914.
 #include "kernel_common.h"
+#include "row_panel.h"
+
+#include <algorithm>
 
 #include <stdexcept>
 
@@ -21,14 +26,19 @@ constexpr int kHeadWaves = 8, kHeadCh = 32, kHeadFc = 16 * kHeadWaves, kHeadChun
 // first-layer weights. us back to back, both heads: width 256 1 position 8.5, 64 9.2, 256 12.1; width 1024 10.6, 11.5, 22.4.
 // (A form that took row-major weights with the loads of row_panel.h spilled, and took 18 to 29 us at up to 64 positions.)
 // ---------------------------------------------------------------------------
+template <typename ET, int NC> struct ValueHeadLds {
+  __attribute__((aligned(16))) ET rows[NC > 1 ? 2 : 1][64 * (kHeadChunk + 8)];
+  __attribute__((aligned(16))) ET embedded[64 * kHeadCh];
+  float hidden[kHeadFc];
+};
+
 template <typename ET, int NC>   // NC chunks of 256 columns of x
-__global__ __launch_bounds__(64 * kHeadWaves) void value_heads_kernel(ValueHeadsArgs p) {
+__device__ __forceinline__ void ValueHead(const ValueHeadsArgs& p, const HeadLayers& h, ValueHeadLds<ET, NC>& lds) {
   using ev8 = typename Vec16<ET>::v8;
   constexpr int LD = kHeadChunk + 8, VX = 64 * kHeadChunk / 8 / (64 * kHeadWaves), SC = kHeadChunk / 32;
-  __shared__ __attribute__((aligned(16))) ET rows[NC > 1 ? 2 : 1][64 * LD];
-  __shared__ __attribute__((aligned(16))) ET embedded[64 * kHeadCh];
-  __shared__ float hidden[kHeadFc];
-  const HeadLayers& h = p.head[blockIdx.y];
+  auto& rows = lds.rows;
+  auto& embedded = lds.embedded;
+  auto& hidden = lds.hidden;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -111,9 +121,130 @@ __global__ __launch_bounds__(64 * kHeadWaves) void value_heads_kernel(ValueHeads
   }
 }
 
+// ---------------------------------------------------------------------------
+// Policy of one position by a workgroup: logits[q][k] = scale Q_q . K_k (64 x 64, float), the offsets of the three promotion pieces from
+// the last eight keys, and the 1858 moves' values gathered from both. The eight waves share the reduction, 128 columns at a time
+// (with at most 256 columns in all two of them share it, and each of four takes 16 keys); operands straight from memory in the order
+// of row_panel.h, sums of two waves each added in LDS, the four that remain where they are gathered.
+// Bound by latency with few positions, where the products and the gather as launches of their own are 5 to 10 us each in the chain; beside
+// the value heads it is hidden by them. us back to back, depth 1024: 1 position 9.0, 64 9.9, 256 15.8 (the products alone on tiles 14.9, the
+// gather 10 more), 1024 54 (46 and 20); depth 256: 5.9, 6.5, 7.1, 26. us of a pass, three launches -> one: 15x1024 fp16 1 position 828 -> 809, 16
+// 1239 -> 1224, 48 2082 -> 2066, bf16 64 2168 -> 2153, e4m3 16 918 -> 904; 10x256 1 272 -> 255, 64 365 -> 353; level from 100 positions on.
+// ---------------------------------------------------------------------------
+constexpr int kLogitStride = 64 + 4;
+struct PolicyLds {
+  __attribute__((aligned(16))) float part[4][64 * kLogitStride];
+  float offset[4][8];
+};
+
+template <typename ET>
+__device__ __forceinline__ void PolicyTail(const PolicyTailArgs& p, PolicyLds& lds) {
+  using ev8 = typename Vec16<ET>::v8;
+  constexpr int kMoves = 1858, kPerThread = (kMoves + 64 * kHeadWaves - 1) / (64 * kHeadWaves);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const half_t* rows = p.qk + (long long)blockIdx.x * 64 * p.ld;
+  int source[kPerThread];
+#pragma unroll
+  for (int i = 0; i < kPerThread; i++) source[i] = p.inv_map[min(i * 64 * kHeadWaves + tid, kMoves - 1)];
+
+  // Promotion offsets: key 56 + wave against the four rows of ppo.
+  {
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const half_t* key = rows + (long long)(56 + wave) * p.ld + p.key_offset;
+    for (int c = lane; c < p.depth / 8; c += 64) {
+      const ev8 kv = *reinterpret_cast<const ev8*>(key + c * 8);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const floatx4 p0 = *reinterpret_cast<const floatx4*>(p.ppo + (long long)i * p.depth + c * 8);
+        const floatx4 p1 = *reinterpret_cast<const floatx4*>(p.ppo + (long long)i * p.depth + c * 8 + 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[i] += (float)kv[e] * p0[e] + (float)kv[4 + e] * p1[e];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float t = WaveSum(s[i]);
+      if (lane == 0) lds.offset[i][wave] = t;
+    }
+  }
+
+  const int row_bytes = 2 * p.depth, steps = (row_bytes + kStepBytes - 1) / kStepBytes;
+  const char* queries = reinterpret_cast<const char*>(rows);
+  const char* keys = reinterpret_cast<const char*>(rows + p.key_offset);
+  TileOffsets at[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) at[t].Set(16 * t, 64, 2 * p.ld);
+  auto left = [&](int step) { return min(kStepBytes, row_bytes - step * kStepBytes); };
+  int parts = 4;
+  if (steps > 2) {
+    floatx4 acc[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) acc[t][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = wave; s < steps; s += kHeadWaves)
+      OneStep<4, 4>(queries + s * kStepBytes, at, keys + s * kStepBytes, at, left(s), acc, PanelOp<ET>{});
+    // Accumulator lane (r, g) of tile (t, c): query 16 t + r, keys 16 c + 4 g + e.
+    auto place = [&](int t, int c) { return reinterpret_cast<floatx4*>(&lds.part[wave & 3][(16 * t + r) * kLogitStride + 16 * c + 4 * g]); };
+    if (wave >= 4) {
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) *place(t, c) = acc[t][c];
+    }
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) *place(t, c) = acc[t][c] + *place(t, c);
+    }
+  } else {
+    parts = 2;
+    const int s = wave >> 2, c = wave & 3;
+    floatx4 acc[4][1];
+#pragma unroll
+    for (int t = 0; t < 4; t++) acc[t][0] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    TileOffsets mine[1];
+    mine[0].Set(16 * c, 64, 2 * p.ld);
+    if (s < steps) OneStep<4, 1>(queries + s * kStepBytes, at, keys + s * kStepBytes, mine, left(s), acc, PanelOp<ET>{});
+#pragma unroll
+    for (int t = 0; t < 4; t++) *reinterpret_cast<floatx4*>(&lds.part[s][(16 * t + r) * kLogitStride + 16 * c + 4 * g]) = acc[t][0];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPerThread; i++) {
+    const int move = i * 64 * kHeadWaves + tid;
+    const bool plain = source[i] < 4096;
+    const int q = plain ? 0 : source[i] - 4096, k = q / 24, j = q % 24 / 3, piece = q % 3;   // promotion from file k to file j
+    const int cell = plain ? (source[i] >> 6) * kLogitStride + (source[i] & 63) : (48 + k) * kLogitStride + 56 + j;
+    float v = lds.part[0][cell] + lds.part[1][cell];
+    if (parts == 4) v += lds.part[2][cell] + lds.part[3][cell];
+    v *= p.scale;
+    if (!plain) v = v + lds.offset[piece][j] + lds.offset[3][j];
+    if (move < kMoves) p.out[(long long)blockIdx.x * kMoves + move] = v;
+  }
+}
+
+// Value and moves-left head, and with `policy` the policy: a workgroup each per position.
+template <typename ET, int NC>
+__global__ __launch_bounds__(64 * kHeadWaves) void value_heads_kernel(ValueHeadsArgs p) {
+  __shared__ union { ValueHeadLds<ET, NC> head; PolicyLds policy; } lds;
+  if ((int)blockIdx.y < p.heads) ValueHead<ET, NC>(p, p.head[blockIdx.y], lds.head);
+  else PolicyTail<ET>(p.policy, lds.policy);
+}
+
+template <typename ET>
+__global__ __launch_bounds__(64 * kHeadWaves) void policy_tail_kernel(PolicyTailArgs p) {
+  __shared__ PolicyLds lds;
+  PolicyTail<ET>(p, lds);
+}
+
 template <typename ET>
 void LaunchValueHeadsT(const ValueHeadsArgs& a, hipStream_t stream) {
-  const dim3 grid(a.batch, a.heads), block(64 * kHeadWaves);
+  const dim3 grid(a.batch, a.heads + (a.policy.qk != nullptr ? 1 : 0)), block(64 * kHeadWaves);
   switch (a.emb / kHeadChunk) {
     case 1: hipLaunchKernelGGL((value_heads_kernel<ET, 1>), grid, block, 0, stream, a); break;
     case 2: hipLaunchKernelGGL((value_heads_kernel<ET, 2>), grid, block, 0, stream, a); break;
@@ -137,10 +268,23 @@ long long HeadFragmentIndex(bool embed, int row, int col, int emb, int ch) {
   return ((long long)(row / 16 * steps + col / 32) * 64 + row % 16 + 16 * (col % 32 / 8)) * 8 + col % 8;
 }
 
+bool PolicyTailSupported(const PolicyTailArgs& a) {
+  return a.depth >= 8 && a.depth % 8 == 0 && a.ld % 8 == 0 && a.key_offset % 8 == 0 && a.ld <= 1 << 20;
+}
+
+void LaunchPolicyTail(const PolicyTailArgs& a, int batch, bool bf16, hipStream_t stream) {
+  if (batch <= 0) return;
+  if (!PolicyTailSupported(a)) throw std::runtime_error("LaunchPolicyTail: unsupported shape");
+  const dim3 grid(batch), block(64 * kHeadWaves);
+  if (bf16) hipLaunchKernelGGL(policy_tail_kernel<bf16_t>, grid, block, 0, stream, a);
+  else hipLaunchKernelGGL(policy_tail_kernel<half_t>, grid, block, 0, stream, a);
+}
+
 void LaunchValueHeads(const ValueHeadsArgs& a, hipStream_t stream) {
   if (a.batch <= 0) return;
   bool ok = a.heads >= 1 && a.heads <= 2 && a.ldx % 8 == 0;
   for (int i = 0; ok && i < a.heads; i++) ok = ValueHeadSupported(a.emb, a.head[i].ch, a.head[i].fc, a.head[i].out_n);
+  if (a.policy.qk != nullptr) ok = ok && PolicyTailSupported(a.policy);
   if (!ok) throw std::runtime_error("LaunchValueHeads: unsupported shape");
   if (a.bf16) LaunchValueHeadsT<bf16_t>(a, stream);
   else LaunchValueHeadsT<half_t>(a, stream);

@@ -37,6 +37,7 @@ def _lib():
         lib.lc0mi_k_expand_planes_attn.argtypes = [vp, vp, ci, ci, vp, ci, cd]
         lib.lc0mi_k_expand_planes_nchw.argtypes = [vp, vp, ci, vp]
         lib.lc0mi_k_attn_policy_gather.argtypes = [vp, vp, vp, ci, ci, vp]
+        lib.lc0mi_k_policy_tail.argtypes = [vp, vp, ci, ci, C.c_float, vp, ci, cd]
         lib.lc0mi_k_gemm_f8.argtypes = [vp, ci, vp, ci, vp, vp, ci, ci, ci, ci, ci, cf, vp, ci, ci, cd]
         lib.lc0mi_k_norm_gemm.argtypes = [ci] + [vp] * 6 + [ci] * 4 + [cf, cf, ci, vp, ci, cd]
         lib.lc0mi_k_qkv_attention.argtypes = [vp] * 3 + [ci] * 3 + [cf, vp, ci, cd]
@@ -459,6 +460,16 @@ def attn_policy_gather(logits, keys, ppo):
     out = np.zeros((n, 1858), np.float32)
     _check(_lib().lc0mi_k_attn_policy_gather(_ptr(logits), _ptr(keys), _ptr(ppo), keys.shape[1], n, _ptr(out)))
     return out
+
+
+def policy_tail(qk, ppo, scale=1.0, time_iters=0):
+    """qk [B*64, 2 depth] (queries, then keys), ppo f32 [4, depth] -> [B, 1858] (or with ms)."""
+    qk, ppo = _h(qk), np.ascontiguousarray(ppo, np.float32)
+    n, depth = qk.shape[0] // 64, qk.shape[1] // 2
+    out = np.zeros((n, 1858), np.float32)
+    ms = C.c_double(0)
+    _check(_lib().lc0mi_k_policy_tail(_ptr(qk), _ptr(ppo), depth, n, scale, _ptr(out), time_iters, C.byref(ms)))
+    return (out, ms.value) if time_iters else out
 
 
 def legal_softmax(policy, move_lists, temperature=1.359):
