@@ -85,6 +85,10 @@ int lc0mi_k_layer_norm_generic(int dtype, const void* x, const void* skip, const
 /* float variant (fp32 configuration). */
 int lc0mi_k_gemm_f32(const float* A, int lda, const float* W, int ldw, const float* bias, int M, int N, int K,
                      float scale, int act, float* C, int ldc);
+/* Up to three independent products of that kind, in one launch where all of them are small (then *grouped is 1): product i has dims
+ * [5 i] = {M, N, K, batch, act}, A[i] [batch][M][K], W[i] [batch][N][K], bias[i] [N] or null, C[i] [batch][M][N]. */
+int lc0mi_k_gemm_f32_group(int count, const float* const* A, const float* const* W, const float* const* bias, const int* dims, float* const* C,
+                           int* grouped);
 /* y = LN(x * alpha + skip) * gamma + beta, rows of C halves; skip may be NULL.
  * (LayerNorm2DWithSkipConnection, src/neural/backends/blas/encoder.h:29-66) */
 int lc0mi_k_layer_norm(const uint16_t* x, const uint16_t* skip, const float* gamma, const float* beta, int rows,

@@ -3,6 +3,8 @@
 #include "kernel_common.h"
 #include "row_panel.h"
 
+#include <algorithm>
+
 namespace lc0mi {
 
 // ---------------------------------------------------------------------------
@@ -27,19 +29,19 @@ namespace lc0mi {
 // tile keeps one sum per quarter of K (K = 1024 2.9e-7, the form before 4.1e-7): its registers are used up.
 // ---------------------------------------------------------------------------
 namespace {
-template <int RT, int CT, int WM, int WN, int KS, bool ONE_STEP = false>
-__global__ __launch_bounds__(64 * WM * WN * KS, RT * CT == 1 ? 5 : 1) void gemm_f32_mfma_kernel(GemmArgsF32 p) {
+// The workgroup's tile from row m0 and column n0 of product z; part: the waves' sums in LDS, KS times kTileFloats.
+template <int RT, int CT, int WM, int WN> constexpr int kTileFloats = 16 * RT * WM * (16 * CT * WN + 4);   // (rows stay 16-byte aligned)
+template <int RT, int CT, int WM, int WN, int KS, bool ONE_STEP>
+__device__ __forceinline__ void Tile(const GemmArgsF32& p, int m0, int n0, int z, float (*part)[kTileFloats<RT, CT, WM, WN>]) {
   constexpr int ROWS = 16 * RT * WM, COLS = 16 * CT * WN, NT = 64 * WM * WN * KS;
-  constexpr int LD = COLS + 4;   // (rows stay 16-byte aligned)
-  __shared__ __attribute__((aligned(16))) float part[KS][ROWS * LD];
+  constexpr int LD = COLS + 4;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ks = wave % KS, wn = (wave / KS) % WN, wm = wave / (KS * WN);
   const int r = lane & 15, g = lane >> 4;
-  const int m0 = blockIdx.x * ROWS, n0 = blockIdx.y * COLS;
   const int M = p.M, N = p.N, K = p.K;
-  const char* A = reinterpret_cast<const char*>(p.A + (long long)blockIdx.z * p.strideA + (long long)m0 * p.lda);
-  const char* W = reinterpret_cast<const char*>(p.W + (long long)blockIdx.z * p.strideW + (long long)n0 * p.ldw);
+  const char* A = reinterpret_cast<const char*>(p.A + (long long)z * p.strideA + (long long)m0 * p.lda);
+  const char* W = reinterpret_cast<const char*>(p.W + (long long)z * p.strideW + (long long)n0 * p.ldw);
   TileOffsets ta[RT], tw[CT];
 #pragma unroll
   for (int t = 0; t < RT; t++) ta[t].Set(16 * (wm * RT + t), M - m0, 4 * p.lda);
@@ -88,7 +90,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, RT * CT == 1 ? 5 : 1) void gemm_
     for (int c = 0; c < CT; c++)
       *reinterpret_cast<floatx4*>(&part[ks][(16 * (wm * RT + t) + r) * LD + 16 * (wn * CT + c) + 4 * g]) = acc[t][c];
   __syncthreads();
-  float* C = p.C + (long long)blockIdx.z * p.strideC;
+  float* C = p.C + (long long)z * p.strideC;
   DispatchAct(p.act, [&](auto act_fn) {
 #pragma unroll
     for (int i = 0; i < (ROWS * COLS + NT - 1) / NT; i++) {
@@ -98,13 +100,39 @@ __global__ __launch_bounds__(64 * WM * WN * KS, RT * CT == 1 ? 5 : 1) void gemm_
       if (row < ROWS && m < M && n < N) {
         float x = part[0][row * LD + col];
 #pragma unroll
-        for (int z = 1; z < KS; z++) x += part[z][row * LD + col];
+        for (int w = 1; w < KS; w++) x += part[w][row * LD + col];
         x *= p.scale;
         if (p.bias != nullptr) x += p.bias[n];
         C[(long long)m * p.ldc + n] = act_fn(x);
       }
     }
   });
+}
+
+template <int RT, int CT, int WM, int WN, int KS, bool ONE_STEP>
+__global__ __launch_bounds__(64 * WM * WN * KS, RT * CT == 1 ? 5 : 1) void gemm_f32_mfma_kernel(GemmArgsF32 p) {
+  __shared__ __attribute__((aligned(16))) float part[KS][kTileFloats<RT, CT, WM, WN>];
+  Tile<RT, CT, WM, WN, KS, ONE_STEP>(p, blockIdx.x * 16 * RT * WM, blockIdx.y * 16 * CT * WN, blockIdx.z, part);
+}
+
+// Up to three independent products in one launch, in 16x16 tiles: the heads of a float network, whose layers are small and whose
+// chains of dependent launches take 5 to 10 us a launch whatever is in it. Workgroup first[i] is the first of product i.
+struct GroupArgs {
+  GemmArgsF32 p[kGemmF32Group];
+  int first[kGemmF32Group];
+};
+template <int KS>
+__global__ __launch_bounds__(64 * KS, 5) void gemm_f32_group_kernel(GroupArgs a) {
+  __shared__ __attribute__((aligned(16))) float part[KS][kTileFloats<1, 1, 1, 1>];
+  int which = 0;
+#pragma unroll
+  for (int i = 1; i < kGemmF32Group; i++) which = (int)blockIdx.x >= a.first[i] ? i : which;
+  const GemmArgsF32& p = a.p[which];
+  const unsigned t = blockIdx.x - a.first[which], rows = (p.M + 15) / 16, cols = (p.N + 15) / 16;
+  const unsigned q = t / rows, z = q / cols;
+  const int m0 = 16 * (t - q * rows), n0 = 16 * (q - z * cols);
+  if (KS <= 2 || p.K <= 64 * KS) Tile<1, 1, 1, 1, KS, true>(p, m0, n0, z, part);
+  else Tile<1, 1, 1, 1, KS, false>(p, m0, n0, z, part);
 }
 
 template <int RT, int CT, int WM, int WN, int KS, bool ONE_STEP = false>
@@ -114,12 +142,51 @@ void LaunchTile(const GemmArgsF32& a, hipStream_t stream) {
 }
 }  // namespace
 
+namespace {
+long long Tiles(const GemmArgsF32& a, int size) { return (long long)((a.M + size - 1) / size) * ((a.N + size - 1) / size) * a.batch; }
+}  // namespace
+
+// Where a launch of its own would take 16x16 tiles for every product, up to 14 tiles for every CU in all: us of a pass, one by one ->
+// together, 6x64 tower 1 position 129 -> 122, 32 142 -> 136, 100 189 -> 184; 10x256 1 355 -> 336, 20 451 -> 437, 40 619 -> 604, from 64 on level.
+bool GemmF32Grouped(const GemmArgsF32* a, int count) {
+  if (count < 2 || count > kGemmF32Group) return false;
+  long long all = 0;
+  for (int i = 0; i < count; i++) {
+    if (a[i].M <= 0 || a[i].N <= 0 || a[i].K <= 0 || a[i].batch <= 0 || Tiles(a[i], 64) >= 400) return false;
+    if (a[i].K <= 128 && Tiles(a[i], 16) >= 2048) return false;
+    all += Tiles(a[i], 16);
+  }
+  return all <= 14 * 256;
+}
+
+void LaunchGemmF32Group(const GemmArgsF32* a, int count, hipStream_t stream) {
+  if (!GemmF32Grouped(a, count)) {
+    for (int i = 0; i < count; i++) LaunchGemmF32(a[i], stream);
+    return;
+  }
+  GroupArgs g;
+  long long tiles = 0;
+  int k = 0;
+  for (int i = 0; i < kGemmF32Group; i++) {
+    g.first[i] = (int)tiles;   // (beyond the last product: past the grid)
+    if (i >= count) continue;
+    g.p[i] = a[i];
+    tiles += Tiles(a[i], 16);
+    k = std::max(k, a[i].K);
+  }
+  const dim3 grid((unsigned)tiles);
+  // (the waves that share a reduction as for one product of the longest one)
+  if (k <= 64) hipLaunchKernelGGL(gemm_f32_group_kernel<1>, grid, dim3(64), 0, stream, g);
+  else if (k <= 128) hipLaunchKernelGGL(gemm_f32_group_kernel<2>, grid, dim3(128), 0, stream, g);
+  else if (k <= 256 || tiles > 256) hipLaunchKernelGGL(gemm_f32_group_kernel<4>, grid, dim3(256), 0, stream, g);
+  else hipLaunchKernelGGL(gemm_f32_group_kernel<8>, grid, dim3(512), 0, stream, g);
+}
+
 void LaunchGemmF32(const GemmArgsF32& a, hipStream_t stream) {
   if (a.M <= 0 || a.N <= 0 || a.batch <= 0) return;
   // The tile is a matter of filling the CUs: at small sizes many 16x16 tiles balance them best, at large ones operand
   // traffic decides (16384x256x1024: 103 us on 64x64 tiles, 143 on 16x16 ones; 1280x256x1024: 25 against 13).
-  const long long tiles16 = (long long)((a.M + 15) / 16) * ((a.N + 15) / 16) * a.batch;
-  const long long tiles64 = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch;
+  const long long tiles16 = Tiles(a, 16), tiles64 = Tiles(a, 64);
   if (tiles64 >= 400 && a.K >= 512) {
     // Two waves share every operand row in both; a long reduction is worth splitting (16384x1024x256: 125 us unsplit
     // against 137; 16384x256x1024: 117 against 103).

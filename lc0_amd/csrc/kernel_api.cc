@@ -335,6 +335,30 @@ int lc0mi_k_gemm_f32(const float* A, int lda, const float* W, int ldw, const flo
   });
 }
 
+int lc0mi_k_gemm_f32_group(int count, const float* const* A, const float* const* W, const float* const* bias, const int* dims, float* const* C,
+                           int* grouped) {
+  return Guard([&] {
+    RequireDevice();
+    if (count < 1 || count > lc0mi::kGemmF32Group) throw Error("bad count of products");
+    Dev dev;
+    std::vector<lc0mi::GemmArgsF32> g(count);
+    for (int i = 0; i < count; i++) {
+      const int M = dims[5 * i], N = dims[5 * i + 1], K = dims[5 * i + 2], batch = dims[5 * i + 3];
+      if (M < 1 || N < 1 || K < 4 || K % 4 || batch < 1) throw Error("bad gemm shape");
+      g[i].A = dev.Put(A[i], (size_t)batch * M * K); g[i].lda = K; g[i].strideA = (long long)M * K;
+      g[i].W = dev.Put(W[i], (size_t)batch * N * K); g[i].ldw = K; g[i].strideW = (long long)N * K;
+      g[i].C = static_cast<float*>(dev.Alloc(sizeof(float) * batch * M * N)); g[i].ldc = N; g[i].strideC = (long long)M * N;
+      g[i].bias = bias[i] ? dev.Put(bias[i], (size_t)N) : nullptr;
+      g[i].M = M; g[i].N = N; g[i].K = K; g[i].batch = batch; g[i].act = dims[5 * i + 4];
+    }
+    *grouped = lc0mi::GemmF32Grouped(g.data(), count);
+    lc0mi::LaunchGemmF32Group(g.data(), count, nullptr);
+    K_CHECK(hipDeviceSynchronize());
+    K_CHECK(hipGetLastError());
+    for (const auto& a : g) K_CHECK(hipMemcpy(C[&a - g.data()], a.C, sizeof(float) * a.batch * a.M * a.N, hipMemcpyDeviceToHost));
+  });
+}
+
 int lc0mi_k_layer_norm(const uint16_t* x, const uint16_t* skip, const float* gamma, const float* beta, int rows,
                        int C, float alpha, float eps, uint16_t* y, int time_iters, double* ms) {
   return Guard([&] {

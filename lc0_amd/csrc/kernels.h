@@ -154,6 +154,11 @@ struct GemmArgsF32 {
   int act = 3;
 };
 void LaunchGemmF32(const GemmArgsF32& args, hipStream_t stream);
+// Up to kGemmF32Group products that do not depend on each other; in one launch where GemmF32Grouped(): all of them small enough for
+// 16x16 tiles.
+constexpr int kGemmF32Group = 3;
+bool GemmF32Grouped(const GemmArgsF32* args, int count);
+void LaunchGemmF32Group(const GemmArgsF32* args, int count, hipStream_t stream);
 
 // Input planes -> token-major embedding input with the 64 position-encoding
 // channels appended: out[b*64+sq][c], c < 112 plane bits * value, 112..175 the

@@ -466,6 +466,11 @@ class Mi355xNetwork : public Network, protected ModelState {
   void Timed(const char* name, double flops, double bytes, F&& launch, hipStream_t st = nullptr);
   void TimedElsewhere(const std::string& name, double flops, double bytes);
   void AddToProfile(const KernelTime& t);
+  // Independent layers of a float network's heads, in one launch where they are small.
+  void GemmGroup(const std::vector<GemmArgsF32>& list, const char* name);
+  void ForwardHeadsF32(int B);
+  GemmArgsF32 PolicyLogitsF32(int B) const;
+  void PolicyGatherF32(int B);
   bool Gemm(const char* name, const half_t* A, int lda, const Linear& lin, void* C, int ldc, int M, int act,
             bool out_f32 = false, hipStream_t st = nullptr, int split_k = 1, bool latency_first = false,
             const NormFold* fold = nullptr, int out_stores = kStoresAuto, const SecondProduct& second = {});
@@ -502,7 +507,7 @@ class Mi355xNetwork : public Network, protected ModelState {
   float* sg2f_ = nullptr;  // split-K accumulator of smolgen dense1
   // Partial row sums of the two un-normalised sums of an encoder layer (folded layer norms): [rows][parts][2].
   float *ln_stats_a_ = nullptr, *ln_stats_b_ = nullptr;
-  half_t *pol_e_ = nullptr, *pol_qk_ = nullptr, *head1_ = nullptr, *head2_ = nullptr;
+  half_t *pol_e_ = nullptr, *pol_qk_ = nullptr, *head1_ = nullptr, *head2_ = nullptr, *mov_head1_ = nullptr, *mov_head2_ = nullptr;
   float* tail_partial_ = nullptr;   // EncoderTailArgs::partial, arrived
   int* tail_arrived_ = nullptr;
   half_t *pe_qkv_ = nullptr, *pe_att_ = nullptr, *pe_t_ = nullptr, *pe_ffn_ = nullptr;   // policy encoder scratch
@@ -517,7 +522,7 @@ class Mi355xNetwork : public Network, protected ModelState {
   uint8_t *xq_ = nullptr, *attq_ = nullptr, *ffnq_ = nullptr;
   uint8_t *sg1q_ = nullptr, *sg2q_ = nullptr, *sg3q_ = nullptr;   // e4m3 operands of the smolgen chain
   void *r_in_ = nullptr, *r_x_ = nullptr, *r_y_ = nullptr, *r_v_ = nullptr, *r_m_ = nullptr, *r_h1_ = nullptr,
-       *r_h2_ = nullptr;
+       *r_h2_ = nullptr, *r_pol_h1_ = nullptr, *r_mov_h1_ = nullptr, *r_mov_h2_ = nullptr;
 
   // Lanes: further instances that share this network's weights and own their streams and
   // activations, so that computations of several search threads run concurrently on the GPU
@@ -726,6 +731,22 @@ GemmArgs Mi355xNetwork::MakeGemmArgs(const half_t* A, int lda, const Linear& lin
     if (fold->bias != nullptr) g.bias = fold->bias;
   }
   return g;
+}
+
+void Mi355xNetwork::GemmGroup(const std::vector<GemmArgsF32>& list, const char* name) {
+  auto flops = [](const GemmArgsF32& g) { return 2.0 * g.batch * g.M * g.N * g.K; };
+  auto bytes = [](const GemmArgsF32& g) { return 4.0 * g.batch * (static_cast<double>(g.M) * g.K + static_cast<double>(g.N) * g.K + static_cast<double>(g.M) * g.N); };
+  if (GemmF32Grouped(list.data(), static_cast<int>(list.size()))) {
+    double f = 0.0, b = 0.0;
+    for (const GemmArgsF32& g : list) {
+      f += flops(g);
+      b += bytes(g);
+    }
+    Timed((std::string(name) + "|gemm_f32_group").c_str(), f, b, [&] { LaunchGemmF32Group(list.data(), static_cast<int>(list.size()), stream_); });
+    return;
+  }
+  const std::string label = std::string(name) + "|gemm_f32_mfma_16x16x4";
+  for (const GemmArgsF32& g : list) Timed(label.c_str(), flops(g), bytes(g), [&] { LaunchGemmF32(g, stream_); });
 }
 
 bool Mi355xNetwork::Gemm(const char* name, const half_t* A, int lda, const Linear& lin, void* C, int ldc, int M,
@@ -1297,6 +1318,11 @@ void Mi355xNetwork::AllocActivations() {
     r_m_ = arena_.Alloc(ts * 36 * B * 4 * cmax);
     r_h1_ = arena_.Alloc(ts * B * 64 * cmax);
     r_h2_ = arena_.Alloc(ts * B * res_max_fc_);
+    if (fp32_) {   // (the heads run side by side)
+      r_pol_h1_ = arena_.Alloc(ts * B * 64 * cmax);
+      r_mov_h1_ = arena_.Alloc(ts * B * 64 * cmax);
+      r_mov_h2_ = arena_.Alloc(ts * B * res_max_fc_);
+    }
     return;
   }
   const size_t T = static_cast<size_t>(max_batch_) * 64;
@@ -1347,6 +1373,10 @@ void Mi355xNetwork::AllocActivations() {
   }
   head1_ = AllocH(T * std::max(val_ch_, mov_ch_));
   head2_ = AllocH(static_cast<size_t>(max_batch_) * std::max(val_fc_, mov_fc_));
+  if (dtype_ == Dtype::kFloat && moves_left_) {
+    mov_head1_ = AllocH(T * mov_ch_);
+    mov_head2_ = AllocH(static_cast<size_t>(max_batch_) * mov_fc_);
+  }
 }
 
 // Weights of one post-LN encoder layer without smolgen (q, k and v stacked into one matrix).
@@ -1486,14 +1516,23 @@ void Mi355xNetwork::ForwardAttentionPolicy(const half_t* x, int ld_x, int B, Val
     }
     return;
   }
+  const GemmArgsF32 g = PolicyLogitsF32(B);
+  Timed("gemm_policy_logits|gemm_f32_mfma_16x16x4", logit_flops, logit_bytes, [&] { LaunchGemmF32(g, stream_); });
+  PolicyGatherF32(B);
+}
+
+GemmArgsF32 Mi355xNetwork::PolicyLogitsF32(int B) const {
   GemmArgsF32 g;
   g.A = reinterpret_cast<const float*>(pol_qk_); g.lda = 2 * pol_d_; g.strideA = 64LL * 2 * pol_d_;
   g.W = reinterpret_cast<const float*>(ElemAt(pol_qk_, pol_d_)); g.ldw = 2 * pol_d_; g.strideW = 64LL * 2 * pol_d_;
   g.C = pol_logits_; g.ldc = 64; g.strideC = 4096;
   g.M = 64; g.N = 64; g.K = pol_d_; g.batch = B;
-  g.scale = logit_scale;
+  g.scale = 1.0f / std::sqrt(static_cast<float>(pol_d_));
   g.act = kActNone;
-  Timed("gemm_policy_logits|gemm_f32_mfma_16x16x4", logit_flops, logit_bytes, [&] { LaunchGemmF32(g, stream_); });
+  return g;
+}
+
+void Mi355xNetwork::PolicyGatherF32(int B) {
   Timed("policy_gather", 0.0, B * (4.0 * 4288 + 4.0 * 1858), [&] {
     LaunchAttnPolicyGather(pol_logits_, reinterpret_cast<const float*>(pol_qk_), 2 * pol_d_, pol_d_, ppo_, pol_d_, inv_map_, d_policy_, B,
                            stream_);
@@ -2005,14 +2044,42 @@ void Mi355xNetwork::ForwardResnet(int B) {
   auto fc = [&](const char* name, const void* a, const LinearT& l, void* c, int m, int act, bool out_f32) {
     GemmT<T>(name, a, l.ld, 0, l.w, l.ld, 0, c, l.out, 0, l.b, m, l.out, l.ld, 1, act, out_f32);
   };
-  // Value head.
-  fc("gemm_value_conv", r_x_, res_val_conv_, r_h1_, T64, default_act_, false);
-  fc("gemm_value_fc1", r_h1_, res_val_fc1_, r_h2_, B, default_act_, false);
-  fc("gemm_value_fc2", r_h2_, res_val_fc2_, d_wdl_, B, kActNone, true);
-  if (moves_left_) {
-    fc("gemm_mlh_conv", r_x_, res_mov_conv_, r_h1_, T64, default_act_, false);
-    fc("gemm_mlh_fc1", r_h1_, res_mov_fc1_, r_h2_, B, default_act_, false);
-    fc("gemm_mlh_fc2", r_h2_, res_mov_fc2_, d_mlh_, B, kActRelu, true);
+  if constexpr (std::is_same<T, float>::value) {
+    // (layers of the same depth together: GemmF32Grouped)
+    auto layer = [&](const void* a, const LinearT& l, void* c, int m, int act) {
+      GemmArgsF32 g;
+      g.A = static_cast<const float*>(a); g.lda = l.ld;
+      g.W = static_cast<const float*>(l.w); g.ldw = l.ld;
+      g.C = static_cast<float*>(c); g.ldc = l.out;
+      g.bias = l.b; g.M = m; g.N = l.out; g.K = l.ld; g.act = act;
+      return g;
+    };
+    std::vector<GemmArgsF32> conv = {layer(r_x_, res_val_conv_, r_h1_, T64, default_act_)};
+    std::vector<GemmArgsF32> fc1 = {layer(r_h1_, res_val_fc1_, r_h2_, B, default_act_)};
+    std::vector<GemmArgsF32> fc2 = {layer(r_h2_, res_val_fc2_, d_wdl_, B, kActNone)};
+    if (!attn_policy_ && !conv_policy_) {
+      conv.push_back(layer(r_x_, res_pol_conv1x1_, r_pol_h1_, T64, default_act_));
+      fc1.push_back(layer(r_pol_h1_, res_pol_fc_, d_policy_, B, kActNone));
+    }
+    if (moves_left_) {
+      conv.push_back(layer(r_x_, res_mov_conv_, r_mov_h1_, T64, default_act_));
+      fc1.push_back(layer(r_mov_h1_, res_mov_fc1_, r_mov_h2_, B, default_act_));
+      fc2.push_back(layer(r_mov_h2_, res_mov_fc2_, d_mlh_, B, kActRelu));
+    }
+    GemmGroup(conv, "gemm_head_conv");
+    GemmGroup(fc1, "gemm_head_fc1");
+    GemmGroup(fc2, "gemm_head_fc2");
+    if (!attn_policy_ && !conv_policy_) return;
+  } else {
+    // Value head.
+    fc("gemm_value_conv", r_x_, res_val_conv_, r_h1_, T64, default_act_, false);
+    fc("gemm_value_fc1", r_h1_, res_val_fc1_, r_h2_, B, default_act_, false);
+    fc("gemm_value_fc2", r_h2_, res_val_fc2_, d_wdl_, B, kActNone, true);
+    if (moves_left_) {
+      fc("gemm_mlh_conv", r_x_, res_mov_conv_, r_h1_, T64, default_act_, false);
+      fc("gemm_mlh_fc1", r_h1_, res_mov_fc1_, r_h2_, B, default_act_, false);
+      fc("gemm_mlh_fc2", r_h2_, res_mov_fc2_, d_mlh_, B, kActRelu, true);
+    }
   }
   // Policy head.
   if (attn_policy_) {
@@ -2413,6 +2480,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
   const int heads_min = heads_overlap_min_batch_ >= 0 ? heads_overlap_min_batch_
                                                       : (emb_ >= 768 ? std::max(overlap_min_batch_, 16) : 1 << 30);
   const bool heads_beside = !profiling_ && !single_stream_ && B >= heads_min;
+  if (dtype_ == Dtype::kFloat && pol_encoders_.empty() && !heads_beside) return ForwardHeadsF32(B);
   hipStream_t hs = heads_beside ? side_stream_ : stream_;
   if (heads_beside) {
     HIP_CHECK(hipEventRecord(heads_fork_, stream_));
@@ -2458,6 +2526,33 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
   // Policy head.
   ForwardAttentionPolicy(x_, emb_, B, heads_with_policy ? &heads_args : nullptr, head_flops, head_bytes);
   if (heads_beside) HIP_CHECK(hipStreamWaitEvent(stream_, heads_join_, 0));
+}
+
+// Heads of a float attention body, layers of the same depth together (GemmF32Grouped).
+void Mi355xNetwork::ForwardHeadsF32(int B) {
+  const int T = B * 64;
+  auto layer = [&](const void* a, int lda, const Linear& lin, void* c, int M, int act) {
+    GemmArgsF32 g;
+    g.A = static_cast<const float*>(a); g.lda = lda;
+    g.W = reinterpret_cast<const float*>(lin.w); g.ldw = lin.ld;
+    g.C = static_cast<float*>(c); g.ldc = lin.out;
+    g.bias = lin.b;
+    g.M = M; g.N = lin.out; g.K = lin.ld;
+    g.act = act;
+    return g;
+  };
+  std::vector<GemmArgsF32> embed = {layer(x_, emb_, pol_emb_lin_, pol_e_, T, pol_emb_act_), layer(x_, emb_, val_emb_lin_, head1_, T, default_act_)};
+  std::vector<GemmArgsF32> middle = {layer(pol_e_, pol_emb_, pol_qk_lin_, pol_qk_, T, kActNone), layer(head1_, 64 * val_ch_, val_fc1_, head2_, B, default_act_)};
+  std::vector<GemmArgsF32> last = {PolicyLogitsF32(B), layer(head2_, val_fc_, val_fc2_, d_wdl_, B, kActNone)};
+  if (moves_left_) {
+    embed.push_back(layer(x_, emb_, mov_emb_lin_, mov_head1_, T, default_act_));
+    middle.push_back(layer(mov_head1_, 64 * mov_ch_, mov_fc1_, mov_head2_, B, default_act_));
+    last.push_back(layer(mov_head2_, mov_fc_, mov_fc2_, d_mlh_, B, kActRelu));
+  }
+  GemmGroup(embed, "gemm_head_embed");
+  GemmGroup(middle, "gemm_head_fc1");
+  GemmGroup(last, "gemm_head_fc2");
+  PolicyGatherF32(B);
 }
 
 void Mi355xNetwork::LaunchEager(int batch) {

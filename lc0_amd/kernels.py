@@ -31,6 +31,7 @@ def _lib():
         lib.lc0mi_k_layer_norm_rows.argtypes = [vp, vp, ci, vp, vp, vp, ci, ci, cf, cf, vp]
         lib.lc0mi_k_winograd_conv.argtypes = [vp] * 8 + [ci] * 6 + [vp] * 3
         lib.lc0mi_k_expand_planes_nhwc.argtypes = [vp, vp, ci, vp]
+        lib.lc0mi_k_gemm_f32_group.argtypes = [ci, vp, vp, vp, vp, vp, vp]
         lib.lc0mi_k_gemm_f32.argtypes = [vp, ci, vp, ci, vp, ci, ci, ci, cf, ci, vp, ci]
         lib.lc0mi_k_layer_norm.argtypes = [vp, vp, vp, vp, ci, ci, cf, cf, vp, ci, cd]
         lib.lc0mi_k_attention.argtypes = [vp, vp, ci, ci, ci, cf, vp, ci, cd]
@@ -243,6 +244,19 @@ def gemm_f32(a, w, bias=None, scale=1.0, act=ACT_NONE):
     b = np.ascontiguousarray(bias, np.float32) if bias is not None else None
     _check(_lib().lc0mi_k_gemm_f32(_ptr(a), k, _ptr(w), k, _ptr(b), m, n, k, scale, act, _ptr(out), n))
     return out
+
+
+def gemm_f32_group(products):
+    """products: up to three (a [batch, M, K], w [batch, N, K], bias or None, act) -> their results and whether they ran in one launch."""
+    f = lambda v: np.ascontiguousarray(v, np.float32) if v is not None else None
+    products = [(f(a), f(w), f(b), act) for a, w, b, act in products]
+    outs = [np.zeros((a.shape[0], a.shape[1], w.shape[1]), np.float32) for a, w, _, _ in products]
+    dims = np.array([[a.shape[1], w.shape[1], a.shape[2], a.shape[0], act] for a, w, _, act in products], np.int32)
+    table = lambda arrays: (C.c_void_p * len(arrays))(*[v.ctypes.data if v is not None else None for v in arrays])
+    grouped = C.c_int(0)
+    _check(_lib().lc0mi_k_gemm_f32_group(len(products), table([p[0] for p in products]), table([p[1] for p in products]),
+                                         table([p[2] for p in products]), _ptr(dims), table(outs), C.byref(grouped)))
+    return outs, bool(grouped.value)
 
 
 def layer_norm(x, skip, gamma, beta, alpha, eps, time_iters=0):
