@@ -293,6 +293,7 @@ void LaunchSmolgenAttentionF8Out(const half_t* qkv, const half_t* gen, const hal
 // heads * 256 values before the norm, gamma and beta as many floats. out: 16 bits, or with out_f8 e4m3(result * out_mul).
 // SmolgenAttentionFewSupported: head depth 32, a multiple of four heads up to 32, gen_sz 256.
 struct SmolgenFewArgs {
+  int head_groups = 1;   // (set by the launcher)
   const half_t *qkv = nullptr, *gen = nullptr, *wfrag = nullptr;
   const float *gamma = nullptr, *beta = nullptr;
   void* out = nullptr;

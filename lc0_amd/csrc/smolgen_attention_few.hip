@@ -18,7 +18,7 @@ constexpr int kYStride = kGen + 8;                       // 16-bit values per he
 constexpr int kVStride = 256 + 32;                       // bytes per key: the eight rows that 32 lanes read meet different banks
 
 // ---------------------------------------------------------------------------
-// A workgroup of eight waves owns QUERIES (4, 8 or 16) queries of one position and all heads.
+// A workgroup of eight waves owns QUERIES (4, 8 or 16) queries of one position and all heads, or with one to four positions a group of them.
 //   Generator: the 64 QUERIES (query, key) rows are QUERIES / 4 32-row tiles per wave over the 32 heads as columns; weights in
 //     the fragment order of smolgen_attention_kernel, asked for first, and the norm of the vectors while they are on their way.
 //   Attention: four heads per wave. K comes in by 64-byte rows of the four heads and leaves the 4 x 4 transpose of row_panel.h as
@@ -28,7 +28,7 @@ constexpr int kVStride = 256 + 32;                       // bytes per key: the e
 //     head, take probabilities that are zero outside the head's columns. Four queries at a time, K and V^T stay in registers.
 // Logits stay in float with up to 8 queries; with 16 they are rounded to 16 bits, as the generator layer of its own leaves them.
 // Bound by latency and by what a workgroup takes from L2 (32 KiB of weights per query, K and V 256, gamma and beta 64): the
-// fewest queries that give no CU two workgroups are the fastest (us back to back, 32 heads: 4 queries 1 position 10.5, 16 11.6,
+// fewest queries that give no CU two workgroups are the fastest (us back to back, 32 heads in one group: 4 queries 1 position 10.5, 16 11.6,
 // 24 20.5; 8 queries 24 14.0, 32 15.1; 16 queries 33 20.1, 64 22.7).
 // ---------------------------------------------------------------------------
 template <typename ET, typename OutT, int QUERIES>
@@ -47,12 +47,14 @@ __global__ __launch_bounds__(512) void smolgen_attention_few_kernel(SmolgenFewAr
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Workgroups go to the 8 XCDs in turn. From 8 positions on those of a position share an XCD, whose L2 then holds its K and
   // V once; with fewer they are spread, or most of the chip's L2s would have nothing to fetch.
-  const int id = blockIdx.x;
+  // The last grid / groups workgroups do the last group of heads, and so on.
+  const int per_group = gridDim.x / p.head_groups, group = blockIdx.x / per_group, id = blockIdx.x - group * per_group;
   constexpr int MASK = (1 << SHIFT) - 1;
   const int b = p.batch >= 8 ? (id >> (SHIFT + 3)) * 8 + (id & 7) : id >> SHIFT;
   const int q0 = QUERIES * (p.batch >= 8 ? (id >> 3) & MASK : id & MASK);
   if (b >= p.batch) return;
   const int heads = p.heads, d_model = 32 * heads, ld = 3 * d_model;
+  const int first_head = group * (heads / p.head_groups), end_head = first_head + heads / p.head_groups;   // this workgroup's
 
   // What does not depend on anything: weights, generator vectors, gamma and beta, K and Q.
   const intx4* wp = reinterpret_cast<const intx4*>(p.wfrag) + (long long)(2 * q0 + GROUPS * wave) * kNks * 64 + lane;
@@ -61,8 +63,8 @@ __global__ __launch_bounds__(512) void smolgen_attention_few_kernel(SmolgenFewAr
   floatx4 gm[2][2], bt[2][2];
 #pragma unroll
   for (int v = 0; v < 2; v++) {
-    const int at = min(row0 + 16 * v, heads - 1) * kGen + kv;
-    x[v] = *reinterpret_cast<const ev8*>(p.gen + (long long)b * heads * kGen + at);
+    x[v] = *reinterpret_cast<const ev8*>(p.gen + ((long long)b * heads + min(row0 + 16 * v, heads - 1)) * kGen + kv);
+    const int at = min(max(row0 + 16 * v, first_head), end_head - 1) * kGen + kv;   // (other heads' are not used)
 #pragma unroll
     for (int h = 0; h < 2; h++) {
       gm[v][h] = *reinterpret_cast<const floatx4*>(p.gamma + at + 4 * h);
@@ -73,9 +75,9 @@ __global__ __launch_bounds__(512) void smolgen_attention_few_kernel(SmolgenFewAr
 #pragma unroll
   for (int s = 0; s < kNks; s++) w[s] = wp[s * 64];
   const int r = lane & 15, g = lane >> 4;
-  const int head0 = 4 * wave;
-  const bool live = head0 < heads;                       // (a multiple of four heads: whole waves)
-  const half_t* base = p.qkv + (long long)b * 64 * ld + (live ? head0 : 0) * 32;
+  const int head0 = first_head + 4 * wave;
+  const bool live = head0 < end_head;                    // (a multiple of four heads: whole waves)
+  const half_t* base = p.qkv + (long long)b * 64 * ld + (live ? head0 : first_head) * 32;
   intx4 k[4][4];
 #pragma unroll
   for (int t = 0; t < 4; t++)
@@ -252,10 +254,22 @@ __global__ __launch_bounds__(512) void smolgen_attention_few_kernel(SmolgenFewAr
   }
 }
 
+// Workgroups that share the heads of the same queries: K, V, gamma and beta are then spread over as many CUs, weights and the rows of the
+// norm repeated. As many as leave half of the CUs free: us of a 15x1024 pass, one -> shared, 1 position by eight 820 -> 777, 2 by four 890
+// -> 850, 4 by two 994 -> 971, e4m3 1 713 -> 671. By two at 8 positions, on every CU, a pass alone is faster too (1122 -> 1098), but four
+// threads lose 10 % (15.7k -> 14.1k evals/s; 4 positions by two 9.1k -> 9.1k).
+int HeadGroups(int workgroups, int heads) {
+  int groups = 1;
+  while (groups < 8 && 2 * groups * workgroups <= 128 && heads % (8 * groups) == 0) groups *= 2;
+  return groups;
+}
+
 template <int QUERIES>
-void LaunchFew(const SmolgenFewArgs& a, hipStream_t stream) {
+void LaunchFew(const SmolgenFewArgs& args, hipStream_t stream) {
+  SmolgenFewArgs a = args;
   constexpr int PER = 64 / QUERIES;
-  const dim3 grid(a.batch >= 8 ? (a.batch + 7) / 8 * 8 * PER : a.batch * PER), block(512);
+  a.head_groups = HeadGroups(a.batch * PER, a.heads);
+  const dim3 grid((a.batch >= 8 ? (a.batch + 7) / 8 * 8 * PER : a.batch * PER) * a.head_groups), block(512);
   if (a.out_f8) hipLaunchKernelGGL((smolgen_attention_few_kernel<half_t, uint8_t, QUERIES>), grid, block, 0, stream, a);
   else if (a.bf16) hipLaunchKernelGGL((smolgen_attention_few_kernel<bf16_t, half_t, QUERIES>), grid, block, 0, stream, a);
   else hipLaunchKernelGGL((smolgen_attention_few_kernel<half_t, half_t, QUERIES>), grid, block, 0, stream, a);
