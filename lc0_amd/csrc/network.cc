@@ -155,8 +155,7 @@ struct SecondProduct {
   float out_mul = 1.0f;
 };
 
-constexpr int kOverlapMinBatch = 80;                              // option overlap_min_batch
-constexpr int kCompressWithQkvMaxBatch = kOverlapMinBatch - 1;   // largest batch whose compression is such a second product
+constexpr int kCompressWithQkvMaxBatch = 79;   // largest batch whose compression is such a second product
 
 int RoundUp(int v, int m) { return (v + m - 1) / m * m; }
 
@@ -298,7 +297,7 @@ struct ModelState {
   int default_act_ = kActRelu, smolgen_act_ = kActNone, ffn_act_ = kActNone;
   std::string policy_head_, value_head_;
   bool use_graphs_ = true;
-  int overlap_min_batch_ = 0;   // smallest batch whose smolgen chain runs on the side stream
+  int overlap_min_batch_ = -1;   // smallest batch whose smolgen chain runs on the side stream (-1: OverlapMinBatch)
   int heads_overlap_min_batch_ = -1;   // smallest batch whose value and moves-left heads run beside the policy head (-1: automatic)
 
   // Attention body dimensions.
@@ -467,6 +466,7 @@ class Mi355xNetwork : public Network, protected ModelState {
   void TimedElsewhere(const std::string& name, double flops, double bytes);
   void AddToProfile(const KernelTime& t);
   // Independent layers of a float network's heads, in one launch where they are small.
+  int OverlapMinBatch() const;
   void GemmGroup(const std::vector<GemmArgsF32>& list, const char* name);
   void ForwardHeadsF32(int B);
   GemmArgsF32 PolicyLogitsF32(int B) const;
@@ -856,6 +856,16 @@ void Mi355xNetwork::Attention(const half_t* qkv, const half_t* bias, half_t* out
 
 // The smolgen chain of one encoder layer, unfused (network_blas.cc:283-347): compression, two dense layers with
 // their row norms, then the shared generator layer, which leaves the logits in sbias (SmolgenBiasIndex order).
+// Running the smolgen chain beside the QKV projection costs two cross-queue dependencies per layer, and up to here the
+// projection is one round of tiles that leave the chain no room. us of a pass, beside -> on one stream: 15x1024 fp16 80 positions 2925 -> 2755,
+// 84 2950 -> 2800, 85 3136 -> 3135, 150 4200 -> 4544, e4m3 80 2240 -> 2030, 85 2280 -> 2279; ten layers of width 768 fp16 80 1557 -> 1416, 112 1856 ->
+// 1712, 124 1985 -> 1919, 132 2164 -> 2230, e4m3 112 1488 -> 1327, 132 1750 -> 1745; 512 80 1260 -> 1111, 165 1914 -> 1836, 200 2048 -> 2036, 400 3415
+// -> 3468; 384 200 1835 -> 1738, 330 2455 -> 2435.
+int Mi355xNetwork::OverlapMinBatch() const {
+  if (overlap_min_batch_ >= 0) return overlap_min_batch_;
+  return dtype_ == Dtype::kFloat ? 80 : std::max(80, (85 * 1024 + emb_ - 1) / emb_);
+}
+
 void Mi355xNetwork::SmolgenChain(const EncoderDev& e, const half_t* x, int emb, int heads, int hc, int hs, int gen,
                                  half_t* sg1, half_t* sg2, half_t* sg3, half_t* sbias, int B, hipStream_t st,
                                  bool latency_first) {
@@ -1187,12 +1197,7 @@ Mi355xNetwork::Mi355xNetwork(const WeightsFile& file, Options& options) {
   resident_tower_ = options.GetInt("resident_tower", -1);
   if (resident_tower_ < -1 || resident_tower_ > 1) throw Error("resident_tower must be in -1..1.");
   use_graphs_ = options.GetBool("graphs", true);
-  // Running the smolgen chain beside the QKV projection costs two cross-queue dependencies per layer; below
-  // this batch size the chain on the main stream is faster (measured on the 15x1024 net, chain on the main stream
-  // against beside the projection: fp16 batch 8 1.26 against 1.45 ms, batch 64 2.50 against 2.53, batch 96 3.43
-  // against 3.24; fp8 batch 64 2.00 against 2.25, batch 96 2.60 against 2.54).
   overlap_min_batch_ = options.GetInt("overlap_min_batch", -1);
-  if (overlap_min_batch_ < 0) overlap_min_batch_ = kOverlapMinBatch;
   heads_overlap_min_batch_ = options.GetInt("heads_overlap_min_batch", -1);
   lane_count_ = options.GetInt("lanes", 4);
   if (lane_count_ < 1 || lane_count_ > 8) throw Error("lanes must be in 1..8.");
@@ -2199,7 +2204,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
     const bool bf16 = dtype_ == Dtype::kBf16;
     // The smolgen chain depends only on x: it runs on the side stream next to the
     // QKV projection (on the main stream when profiling, for clean per-kernel times).
-    hipStream_t ss = (profiling_ || single_stream_ || B < overlap_min_batch_) ? stream_ : side_stream_;
+    hipStream_t ss = (profiling_ || single_stream_ || B < OverlapMinBatch()) ? stream_ : side_stream_;
     // The generator layer (smolgen_w) runs inside the attention kernel where that kernel serves the shape.
     // (not with e4m3 operands in the chain: the generator is then an fp8 GEMM of its own)
     const bool chain_f8 = f8 && q_smolgen_ && e.has_smolgen;
@@ -2247,6 +2252,15 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
     const bool qkv_before_chain = e.has_smolgen && ss != stream_ && qkv_first_;
     if (e.has_smolgen) {
       const int g = sg_gen_ / heads_;
+      // While the chain beside the projection is the longer of the two, its compression runs before both, on all CUs: beside
+      // 256-row tiles it takes five times as long. us of a pass, beside -> before: 15x1024 fp16 90 positions 3190 -> 3000, 128 3600 -> 3525, 150
+      // 4200 -> 4105, 165 4367 -> 4363 (100, where the projection leaves CUs free in its second round, 3137 -> 3152; 180 4865 -> 4897, 512
+      // 11260 -> 11430), bf16 90 3118 -> 2972, 150 4105 -> 4012; ten layers of width 768 116 1951 -> 1767, 200 2582 -> 2545; 512 256 2247 -> 2182, 512
+      // 3682 -> 3740. (Nothing but the batch decides on its kernel, so that a pass on one stream has the same bits.)
+      const bool compress_first = !chain_f8 && dtype_ != Dtype::kFloat && !with_compress && !norm_in && B * emb_ <= 165 * 1024;
+      if (compress_first) {
+        Gemm("gemm_smolgen_compress", x_, emb_, e.sg_compress, sg1_, sg_hc_, T, kActNone, false, stream_, 1, true);
+      }
       if (ss != stream_) {
         HIP_CHECK(hipEventRecord(fork_events_[li], stream_));
         if (qkv_before_chain && !with_compress) launch_qkv();
@@ -2304,7 +2318,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       } else if (dtype_ == Dtype::kFloat) {
         SmolgenChain(e, x_, emb_, heads_, sg_hc_, sg_hs_, sg_gen_, sg1_, sg2_, sg3_, sbias_, B, ss, chain_first);
       } else {
-      if (!with_compress) {
+      if (!with_compress && !compress_first) {
         Gemm("gemm_smolgen_compress", x_, emb_, norm_in ? e.sg_compress_n : e.sg_compress, sg1_, sg_hc_, T, kActNone,
              false, ss, 1, chain_first, norm_in ? &cons_in : nullptr);
       }
@@ -2478,7 +2492,7 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
   // batch size (its six head GEMMs are shorter than the two dependencies). Hence the automatic rule: wide
   // bodies only, and only where the smolgen chain already runs on the side stream.
   const int heads_min = heads_overlap_min_batch_ >= 0 ? heads_overlap_min_batch_
-                                                      : (emb_ >= 768 ? std::max(overlap_min_batch_, 16) : 1 << 30);
+                                                      : (emb_ >= 768 ? std::max(OverlapMinBatch(), 16) : 1 << 30);
   const bool heads_beside = !profiling_ && !single_stream_ && B >= heads_min;
   if (dtype_ == Dtype::kFloat && pol_encoders_.empty() && !heads_beside) return ForwardHeadsF32(B);
   hipStream_t hs = heads_beside ? side_stream_ : stream_;

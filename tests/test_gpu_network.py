@@ -984,6 +984,20 @@ def test_a_pass_has_the_same_bits_beside_others_on_other_streams_and_profiled(em
                 np.testing.assert_array_equal(res[field], want[n][field], err_msg="%s %s %d" % (what, field, n))
 
 
+@pytest.mark.parametrize("emb", [256, 1024])
+def test_compression_before_the_projection_has_the_same_bits_on_one_stream(emb, smolgen_nets, positions):
+    """Up to 165 positions at width 1024 (660 at 256) the compression runs before the projection and the chain beside it; on one stream, and
+    with the chain always on the other, the results are bitwise the same, on both sides of the line."""
+    from lc0_amd import Network
+    sizes = (84, 85, 129, 165, 166) if emb == 1024 else (339, 340, 660, 661)
+    nets = [Network(smolgen_nets[emb], o) for o in ("", "overlap_min_batch=0", "overlap_min_batch=100000")]
+    for n in sizes:
+        want, *others = [_evaluate(net, positions, n) for net in nets]
+        for res in others:
+            for field in ("policy", "q", "d", "m"):
+                np.testing.assert_array_equal(res[field], want[field], err_msg="%s %d" % (field, n))
+
+
 @pytest.mark.parametrize("heads,inside,outside", [(2, (), (1, 13)), (4, (), (8,)), (8, (1, 13, 32), (33,))])
 def test_generator_layer_normalises_its_rows_itself_where_that_is_faster(heads, inside, outside, positions, tmp_path):
     """Heads of depth 64 have no attention kernel with the generator inside. The layer takes its row norm along from eight heads up
