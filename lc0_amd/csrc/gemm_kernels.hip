@@ -494,6 +494,11 @@ GemmVariant PickGemmVariant(const GemmArgs& a) {
   // (16384x32x1024: 6.8 us against 12.8 on the 64x64 tiles and 9.6 on the 128x32 ones, but with twice the threads on
   // every CU; 4096 rows 4.2 / 9.8 / 6.1).
   if (a.latency_first && a.split_k == 1 && a.N <= 32 && a.K >= 512) return kRowPanel;
+  // Float output has no direct-to-LDS form. 64x32 panels, up to two for every CU, instead of register-staged 64x64 tiles (the
+  // dense policy layer of a tower, 256x1858x2048 10.1 us against 19.6, 512 17.8 / 24.4, 700 25.1 / 26.5, 1024 36.4 / 28.8).
+  if (a.out_f32 && a.split_k == 1 && a.batch == 1 && a.K >= 1024 && RowPanelWorkgroups(a.M, a.N, 1, kRowPanelShapes[4]) <= 2 * kRowPanelWorkgroups) {
+    return kRowPanel;
+  }
   // Many products that each fit a 64x64 tile (the policy head's Q.K^T per position) would leave three quarters of
   // every 128x128 tile empty (256 x 64x64x1024: 14.5 against 21.4 us).
   if (a.M <= 64 && a.N <= 64) return kTile64;
