@@ -213,11 +213,22 @@ __global__ __launch_bounds__(64 * kWaves, 1) void resident_tower_kernel(TowerArg
     const TowerSe se = p.se[conv / 2 - 1];
     if (se.k > 0) {
       // First layer: a wave does 16 hidden values, lane l value l % 16 and every fourth vector of the channels. Second layer: a
-      // thread does four outputs and every KP-th hidden value. The first weights of either are asked for a barrier early.
+      // thread does four outputs and every KP-th hidden value. What comes from memory is asked for ahead: biases and first-layer weights
+      // before the pooling, the second layer's first weights before the first layer with one position (kEarly) and, for want of
+      // registers, after it with two. (Scheduling barriers keep the compiler from reading all of a layer's operands at once with two
+      // positions: 37 spilled registers -> 13. us of a 20x256 pass, biases read where they are added and the weights after the first layer -> this: 17
+      // positions 712 -> 657, 64 712 -> 656, 256 938 -> 890, 400 1384 -> 1306, 512 1533 -> 1498, 1000 2975 -> 2891.)
+      constexpr bool kEarly = POS == 1;
+      constexpr int B2 = 2 * C / THREADS;
+      static_assert(2 * C % THREADS == 0, "whole rounds of threads over the outputs");
       constexpr int S1 = C / 16, O4 = 2 * C / 4, KP = THREADS / O4, U = 16;
       const int k_lane = lane & 15, v_lane = lane >> 4, o4 = tid % O4, kp = tid / O4;
       floatx4 w1[S1], w2[U];
+      float b1, b2[B2];
+#pragma unroll
+      for (int j = 0; j < B2; j++) b2[j] = se.b2[tid + j * THREADS];
       auto load_w1 = [&](int k0) {
+        b1 = se.b1[min(k0 + k_lane, se.k - 1)];
         const float* w = se.w1 + (long long)min(k0 + k_lane, se.k - 1) * C + 4 * v_lane;
 #pragma unroll
         for (int i = 0; i < S1; i++) w1[i] = *reinterpret_cast<const floatx4*>(w + 16 * i);
@@ -245,6 +256,10 @@ __global__ __launch_bounds__(64 * kWaves, 1) void resident_tower_kernel(TowerArg
             }
             if (r == TILE - 16) *reinterpret_cast<floatx4*>(&pool[b][ch0 + TILE * c + 8 * q]) = s;
           }
+      if constexpr (kEarly) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_w2(kp);
+      }
       __syncthreads();
       for (int k0 = 16 * wave; k0 < se.k; k0 += 16 * kWaves) {
         if (k0 > 16 * wave) load_w1(k0);
@@ -254,15 +269,16 @@ __global__ __launch_bounds__(64 * kWaves, 1) void resident_tower_kernel(TowerArg
 #pragma unroll
           for (int i = 0; i < S1; i++) {
             h4 += w1[i] * *reinterpret_cast<const floatx4*>(&pool[b][16 * i + 4 * v_lane]);
+            if (POS > 1 && i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
           }
           float h = (h4[0] + h4[1]) + (h4[2] + h4[3]);
           h += __shfl_xor(h, 16, 64);
           h += __shfl_xor(h, 32, 64);
           const int k = k0 + k_lane;
-          if (v_lane == 0 && k < se.k) TowerAct(p.act, [&](auto act) { hidden[b][k] = act(h + se.b1[k]); });
+          if (v_lane == 0 && k < se.k) TowerAct(p.act, [&](auto act) { hidden[b][k] = act(h + b1); });
         }
       }
-      load_w2(kp);
+      if (!kEarly) load_w2(kp);
       __syncthreads();
       floatx4 out[POS];
 #pragma unroll
@@ -276,6 +292,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void resident_tower_kernel(TowerArg
             const int k = k0 + u * KP;
             const float h = hidden[b][min(k, se.k - 1)];
             out[b] += w2[u] * (k < se.k ? h : 0.0f);
+            if (POS > 1 && b + 1 == POS && u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
           }
       }
       // The partial sums take the place of the block's inner activations: no wave reads those any more.
@@ -283,9 +300,10 @@ __global__ __launch_bounds__(64 * kWaves, 1) void resident_tower_kernel(TowerArg
 #pragma unroll
       for (int b = 0; b < POS; b++) *reinterpret_cast<floatx4*>(part + (kp * POS + b) * 2 * C + 4 * o4) = out[b];
       __syncthreads();
-      for (int i = tid; i < POS * 2 * C; i += THREADS) {
-        const int b = i / (2 * C), o = i % (2 * C);
-        float v = se.b2[o];
+#pragma unroll
+      for (int n = 0; n < POS * B2; n++) {
+        const int i = tid + n * THREADS, b = i / (2 * C), o = i % (2 * C);
+        float v = b2[n % B2];
 #pragma unroll
         for (int j = 0; j < KP; j++) v += part[j * POS * 2 * C + i];
         scale_shift[b][o / C][o % C] = o < C ? 1.0f / (1.0f + __expf(-v)) : v;
