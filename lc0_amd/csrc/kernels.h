@@ -470,7 +470,7 @@ struct TowerArgs {
   int batch = 0, blocks = 0, filters = 0, act = 2;
 };
 bool TowerSupported(int filters, bool f32);
-bool TowerFaster(int batch, int filters, bool f32, int blocks);   // than winograd convolutions
+bool TowerFaster(int batch, int filters, bool f32, int blocks, bool se);   // than winograd convolutions (se: squeeze-and-excitation)
 long long TowerFragments(int blocks, int filters);
 long long TowerFragmentIndex(int blocks, int filters, int conv, int tap, int out, int in);
 void LaunchTower(const TowerArgs& args, hipStream_t stream);

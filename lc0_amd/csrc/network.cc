@@ -2035,7 +2035,7 @@ template <typename T>
 void Mi355xNetwork::ForwardResnet(int B) {
   const int T64 = B * 64;
   bool have_v = false;
-  if (tower_packed_ != nullptr && (resident_tower_ == 1 || TowerFaster(B, filters_, fp32_, static_cast<int>(res_blocks_.size())))) {
+  if (tower_packed_ != nullptr && (resident_tower_ == 1 || TowerFaster(B, filters_, fp32_, static_cast<int>(res_blocks_.size()), res_blocks_[0].has_se))) {
     TowerArgs t;
     t.masks = d_masks_; t.values = d_values_; t.biases = tower_biases_; t.packed = tower_packed_; t.se = tower_se_;
     t.out = r_x_; t.batch = B; t.blocks = static_cast<int>(res_blocks_.size()); t.filters = filters_; t.act = default_act_;

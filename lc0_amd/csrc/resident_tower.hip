@@ -374,7 +374,7 @@ long long TowerFragmentIndex(int blocks, int filters, int conv, int tap, int out
 }
 
 // Where the kernel is faster than winograd convolutions, whose launches spread few positions over more CUs. us a batch through the
-// interface, winograd / this. 20x256 halves 1 position 639 / 683, 13 686 / 726, 32 850 / 702,
+// interface, winograd / this. 20x256 halves 32 positions 850 / 702,
 // 200 1426 / 840, 512 2146 / 1571, 1000 3505 / 3061; 10x256 without squeeze-and-excitation 13 299 / 309, 17 328 / 307, 64 454 / 319, 512
 // 1158 / 876, 1000 1993 / 1606; 10x128 1 284 / 195, 8 302 / 199, 64 392 / 217, 256 655 / 319, 512 915 / 518, 1000 1338 / 963, mish without
 // squeeze-and-excitation 8 261 / 183, 1000 1332 / 929; thousands of evals/s of two and of four threads, 20x256 halves 17 40 / 44 and 58 / 66, 64
@@ -382,9 +382,12 @@ long long TowerFragmentIndex(int blocks, int filters, int conv, int tap, int out
 // 64 floats: 6 blocks 1 position 172 / 124, 32 225 / 139, 256 509 / 269, 512 708 / 486, 1000 1133 / 892, of four threads 1 15.1 / 17.5, 32 349 / 519,
 // 256 1267 / 2018, 1000 1602 / 2352; 2 blocks 1 102 / 86, 24 125 / 94, 1000 848 / 745. One block, more than half of it the input
 // convolution, gains less (24 103 / 84, four threads 508 / 503; 257 263 / 234) and keeps to the batches of one round.
-bool TowerFaster(int batch, int filters, bool f32, int blocks) {
+// 256 half filters with squeeze-and-excitation, since its weights are asked for ahead: 20 blocks 1 position 645 / 630, 4 662 / 667, 8 684 / 670, 16
+// 740 / 660, of four threads 4.3 / 4.5, 8 30.4 / 33.4, 16 55 / 68; 10 blocks 1 337 / 321, 16 369 / 342, 2 blocks 8 126 / 125; without it 20 blocks 1
+// 456 / 500, 16 514 / 528, 4 blocks 8 154 / 160.
+bool TowerFaster(int batch, int filters, bool f32, int blocks, bool se) {
   if (f32) return blocks > 1 || (batch > 24 && batch <= 256);
-  return filters <= 128 || batch > 16;
+  return filters <= 128 || batch > 16 || (se && blocks > 1);
 }
 
 namespace {

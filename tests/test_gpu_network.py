@@ -221,6 +221,19 @@ def test_batches_that_the_tower_kernel_takes_by_itself(filters, options, inside,
         assert any("resident_tower" in k for k in names) == (n in inside) and ("expand_planes" in names) == (n in outside), (n, names)
 
 
+@pytest.mark.parametrize("blocks,se,batch,inside", [(2, 32, 1, True), (2, 70, 16, True), (2, 0, 16, False)])
+def test_wide_half_tower_of_few_positions(blocks, se, batch, inside, positions, tmp_path):
+    """256 half filters: with squeeze-and-excitation of at most and of more hidden values than are asked for at once the kernel takes every
+    batch of more than one block, without it winograd convolutions do up to 16 positions; either against the oracle."""
+    from lc0_amd import Network, netproto
+    path = str(tmp_path / "net.pb.gz")
+    netproto.write_pb_gz(path, netgen.se_resnet(256, blocks, se, seed=7300 + se))
+    names, res = _names_of_a_profiled_pass(Network(path, "precision=fp16"), positions, batch)
+    assert any("resident_tower" in k for k in names) == inside, names
+    idx = (np.arange(batch) * 3) % 320
+    _compare(res, onn.BlasNetwork(nr.load(path)).forward(positions["masks"][idx], positions["values"][idx]), [positions["legal"][i] for i in idx])
+
+
 @pytest.mark.parametrize("se,mish,batch", [(16, False, 1), (0, True, 24), (96, True, 257)])
 def test_float_tower_on_split_operands_keeps_float_precision(se, mish, batch, positions, tmp_path):
     """Two blocks of 64 float filters against the float64 model, at batches that the tower kernel takes by itself, on planes whose
