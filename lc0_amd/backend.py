@@ -8,7 +8,9 @@ compute path: if liblc0mi.so is missing or no GPU is present, construction
 fails; nothing falls back to the CPU.
 """
 import ctypes as C
+import importlib.machinery
 import os
+import warnings
 from collections import namedtuple
 
 import numpy as np
@@ -79,13 +81,21 @@ def load_library():
                       ("lc0mi_pos_encoding", cf)):
         getattr(lib, name).argtypes = [C.POINTER(ci)]
         getattr(lib, name).restype = C.POINTER(typ)
-    try:
-        from . import _calls   # (linked to the library beside it)
-        _CALLS = _calls
-    except ImportError:
-        pass
+    _CALLS = _load_calls()
     _LIB = lib
     return lib
+
+
+def _load_calls():
+    """The extension (linked to the library beside it), or None: without a word where it was not built for this interpreter, with a
+    warning where it is there and does not load."""
+    try:
+        from . import _calls
+        return _calls
+    except ImportError as e:
+        if any(os.path.exists(os.path.join(_HERE, "_calls" + s)) for s in importlib.machinery.EXTENSION_SUFFIXES):
+            warnings.warn("lc0_amd._calls does not load (%s): the calls made per position go through ctypes" % e, RuntimeWarning)
+        return None
 
 
 def _check(rc):

@@ -1,4 +1,5 @@
-"""Builds lc0_amd/liblc0mi.so (the C-ABI library: host C++ + gfx950 kernels) and the extension of its Python mirror."""
+"""Builds lc0_amd/liblc0mi.so (the C-ABI library: host C++ + gfx950 kernels) and, where g++ and Python's headers are there, the
+extension of its Python mirror."""
 import os
 import subprocess
 import sys
@@ -40,9 +41,24 @@ def build(verbose=False):
         raise RuntimeError("hipcc failed")
     cmd = ["hipcc", "-shared", "-fPIC", "--offload-arch=gfx950", "-o", LIB] + objs + ["-lz"]
     subprocess.check_call(cmd)
-    subprocess.check_call(["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-shared", "-I" + sysconfig.get_path("include"),
-                           os.path.join(CSRC, "python_calls.cc"), "-o", CALLS, "-L" + HERE, "-l:liblc0mi.so", "-Wl,-rpath,$ORIGIN"])
+    build_calls()
     return LIB
+
+
+def build_calls():
+    """The extension that spares a Python program ctypes for the calls it makes per position. Nothing depends on it (the library serves
+    C and C++ programs by itself, and backend.py does without), so a machine that cannot compile it gets a warning, and an
+    extension of an earlier build does not stay beside the new library."""
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-shared", "-I" + sysconfig.get_path("include"),
+           os.path.join(CSRC, "python_calls.cc"), "-o", CALLS, "-L" + HERE, "-l:liblc0mi.so", "-Wl,-rpath,$ORIGIN"]
+    try:
+        subprocess.check_call(cmd)
+        return True
+    except (OSError, subprocess.CalledProcessError) as e:
+        if os.path.exists(CALLS):
+            os.remove(CALLS)
+        sys.stderr.write("warning: %s is not built (%s): Python programs go through ctypes\n" % (os.path.basename(CALLS), e))
+        return False
 
 
 if __name__ == "__main__":
