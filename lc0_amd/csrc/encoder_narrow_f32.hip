@@ -102,7 +102,7 @@ __global__ __launch_bounds__(512, 1) void qkv_attention_f32_kernel(const float* 
   auto sums = [&](int c, int n) {
     floatx4 v;
 #pragma unroll
-    for (int e = 0; e < 4; e++) v[e] = hi[c][4 * n + e] + lo[c][4 * n + e];
+    for (int e = 0; e < 4; e++) v[e] = SumOfProducts(hi[c][4 * n + e], lo[c][4 * n + e]);
     return v;
   };
   floatx4 mine[3][N];
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(2 * C, 1) void encoder_tail_f32_kernel(EncoderTailA
   auto sums = [&](const floatx16& hi, const floatx16& lo, int n) {
     floatx4 v;
 #pragma unroll
-    for (int e = 0; e < 4; e++) v[e] = hi[4 * n + e] + lo[4 * n + e];
+    for (int e = 0; e < 4; e++) v[e] = SumOfProducts(hi[4 * n + e], lo[4 * n + e]);
     return v;
   };
   // t <- layer norm of the rows whose values t holds, over the waves.

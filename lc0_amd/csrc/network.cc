@@ -648,15 +648,18 @@ uint16_t Bf16Bits(float v) {
   return static_cast<uint16_t>((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
 
-// v as the exact sum of three bfloat16 (an infinity: its first part).
+// v as the exact sum of three bfloat16, as Split3 (split_bf16.h) has it: the first part of a finite value is finite, an infinity and what is
+// not a number are their first part.
 constexpr int kSplitPartCount = 3;
 void SplitBf16(float v, uint16_t (&part)[kSplitPartCount]) {
+  const bool finite = std::isfinite(v);
   for (uint16_t& b : part) {
     b = Bf16Bits(v);
+    if (finite && (b & 0x7fff) == 0x7f80) b--;   // (the largest bfloat16)
     const uint32_t u = static_cast<uint32_t>(b) << 16;
     float f;
     std::memcpy(&f, &u, 4);
-    v = std::isinf(f) ? 0.0f : v - f;
+    v = finite ? v - f : 0.0f;
   }
 }
 }  // namespace

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kThreads, 1) void resident_tower_f32_kernel(TowerAr
     auto quarter = [&](int q, int i) {
       floatx4 v;
 #pragma unroll
-      for (int e = 0; e < 4; e++) v[e] = hi[q >> 1][8 * (q & 1) + 4 * i + e] + lo[q >> 1][8 * (q & 1) + 4 * i + e];
+      for (int e = 0; e < 4; e++) v[e] = SumOfProducts(hi[q >> 1][8 * (q & 1) + 4 * i + e], lo[q >> 1][8 * (q & 1) + 4 * i + e]);
       return v;
     };
 #pragma unroll

@@ -1088,6 +1088,62 @@ def test_narrow_float_layers_on_split_operands_keep_float_precision(emb, heads, 
         assert "encoder_tail" not in names and "qkv_attention" not in names
 
 
+LARGE = np.float32(3.4e38)   # finite in float, rounded to bfloat16 (largest 3.3895e38) infinite
+
+
+def test_float_tower_on_split_operands_with_extreme_values(positions, tmp_path):
+    """Plane values between the largest bfloat16 and the largest float stay finite, to float precision, and an infinite one arrives as
+    an infinity at every logit that positive weights lead to, as in floats: its products with the lower parts of a weight, which
+    have either sign, do not make it something else."""
+    from blas_model_f64 import BlasModelF64
+    from lc0_amd import Network, netproto
+    net = netgen.se_resnet(64, 2, 0, seed=7400)
+    net["weights"]["input"]["weights"][:, 0] *= np.float32(1e-30)   # (of the plane with the large values)
+    path = str(tmp_path / "large.pb.gz")
+    netproto.write_pb_gz(path, net)
+    masks, values = positions["masks"][:3].copy(), positions["values"][:3].copy()
+    masks[:, 0] = 1 << np.arange(3, dtype=np.uint64) * 17
+    values[:, 0] = LARGE, -LARGE, np.finfo(np.float32).max
+    gpu, res = _run_gpu(path, masks, values, "precision=fp32")
+    want = np.asarray(BlasModelF64(net).forward(masks, values)["policy"])
+    for got, w in zip(res["policy"], want):
+        assert np.linalg.norm(got - w) <= 1e-6 * np.linalg.norm(w)
+    names, _ = _names_of_a_profiled_pass(gpu, positions, 3)
+    assert any("resident_tower" in k for k in names)
+
+    w = net["weights"]
+    for layer in [w["input"], w["policy"]] + [block[c] for block in w["residual"] for c in ("conv1", "conv2")]:
+        layer["weights"] = np.maximum(np.abs(layer["weights"]), np.float32(1e-35))   # (some are zero)
+    w["ip_pol_w"] = np.maximum(np.abs(w["ip_pol_w"]), np.float32(1e-35))
+    path = str(tmp_path / "infinite.pb.gz")
+    netproto.write_pb_gz(path, net)
+    values[:, 0] = np.inf
+    comp = Network(path, "precision=fp32").NewComputation()
+    comp.AddInputs(masks, values)
+    comp.ComputeBlocking()
+    assert all((comp.GetPolicyRow(i) == np.inf).all() for i in range(3))
+
+
+def test_narrow_float_layers_on_split_operands_with_large_hidden_values(positions, tmp_path):
+    """Hidden values of the FFN between the largest bfloat16 and the largest float, against the float64 model."""
+    from blas_model_f64 import BlasModelF64
+    from lc0_amd import netproto
+    net = netgen.attention_body(128, 2, 4, 256, seed=2400, perturb_ln=True, std=0.05, d_model=128)
+    net["format"]["network_format"]["default_activation"] = netgen.DEFAULT_ACTIVATION_RELU
+    rng = np.random.default_rng(24)
+    for layer in net["weights"]["encoder"]:
+        ffn, large = layer["ffn"], slice(3, 256, 40)
+        ffn["dense1_w"][large], ffn["dense1_b"][large] = 0.0, LARGE
+        ffn["dense2_w"][:, large] = rng.standard_normal(ffn["dense2_w"][:, large].shape) * 1e-30
+    path = str(tmp_path / "net.pb.gz")
+    netproto.write_pb_gz(path, net)
+    gpu, res = _run_gpu(path, positions["masks"][:5], positions["values"][:5], "precision=fp32")
+    want = np.asarray(BlasModelF64(net).forward(positions["masks"][:5], positions["values"][:5])["policy"])
+    assert np.linalg.norm(res["policy"] - want) <= 1e-6 * np.linalg.norm(want)
+    names, _ = _names_of_a_profiled_pass(gpu, positions, 5)
+    assert "encoder_tail" in names and "qkv_attention" in names
+
+
 @pytest.mark.parametrize("form", ["plain", "read-only", "strided", "fortran", "int64", "float64", "big-endian", "list", "many"])
 def test_inputs_through_the_extension_and_through_ctypes(form, positions):
     """Arrays that the extension takes as they are, and those that it leaves to the conversions: the same results, bit for bit."""
