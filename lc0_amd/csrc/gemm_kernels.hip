@@ -299,34 +299,51 @@ const TileCost* Cheapest(const TileCost (&costs)[COUNT], int M, int N, int k_til
 // A large product whose tiles do not fill whole rounds of the 256 CUs, cut along its rows: the rows that make whole
 // rounds of 256x256 (or 256x192) tiles go to one launch and the rest to a second launch on whatever shape suits it
 // (20480x1024x1536 in halves: 87 us on 320 tiles of 256x256, one and a quarter rounds, or 78 us on 128x128 tiles, against
-// 49 + 19 us for 16384 rows on one full round of large tiles and 4096 rows on small ones). Returns the rows of the
-// first launch (0: one launch) when the model above prices the pair at least 3 % below the best single shape.
+// 49 + 19 us for 16384 rows on one full round of large tiles and 4096 rows on small ones). Cut when the model above prices the
+// pair at least 3 % below the best single shape.
 bool g_row_split = true;   // (profiling and tests switch it off through SetGemmRowSplit)
-int PlanRowSplitByTileCost(int M, int N, int k_tiles, GemmVariant* first) {
+struct RowSplit {
+  int rows = 0;                                    // of the first launch (0: one launch)
+  GemmVariant first = kDma256x256, rest = kNoVariant;   // (rest kNoVariant: as a product of its own)
+};
+// (Below 5120 rows a product of its own can get another shape than the cheapest of this table, by which the rest is priced. The rest runs
+// on the cheapest where the other is priced more than the model's error above it: us of a product, rest as of its own -> this, 12608x2048x2048
+// 130 -> 124, one launch 124, 12416x1984x1856 119 -> 112 and 113; where they are close its own shape is the faster one, 4096x1088x1728 26.9 on
+// 128x128 tiles against 28.7 on 128x64.)
+RowSplit PlanRowSplitByTileCost(const GemmArgs& a) {
   const auto& costs = kHalfCosts;
+  const int M = a.M, N = a.N, k_tiles = a.K / 64;
   double best = CostOf(*Cheapest(costs, M, N, k_tiles), M, N, k_tiles) * 0.97;
-  int best_m1 = 0;
+  RowSplit plan;
   for (int v = 0; v < 2; v++) {
     const int col_tiles = (N + costs[v].bn - 1) / costs[v].bn;
     if (col_tiles > 256) continue;
     const int rows_per_round = (256 / col_tiles) * 256;
     for (int m1 = rows_per_round; m1 + 4096 <= M; m1 += rows_per_round) {   // (cut at 2048 rows, 96 positions lost 4 %)
-      const double c = CostOf(costs[v], m1, N, k_tiles) + CostOf(*Cheapest(costs, M - m1, N, k_tiles), M - m1, N, k_tiles) + 1.0;
-      if (c < best) { best = c; best_m1 = m1; *first = costs[v].variant; }
+      const TileCost& rest = *Cheapest(costs, M - m1, N, k_tiles);
+      const double c = CostOf(costs[v], m1, N, k_tiles) + CostOf(rest, M - m1, N, k_tiles) + 1.0;
+      if (c < best) { best = c; plan = {m1, costs[v].variant, rest.variant}; }
     }
   }
-  return best_m1;
+  if (plan.rows > 0) {
+    GemmArgs rest = a;
+    rest.M = M - plan.rows;
+    const GemmVariant own = PickGemmVariant(rest);
+    const TileCost* c = Cheapest(costs, rest.M, N, k_tiles, [&](GemmVariant v) { return v == own; });
+    if (c != nullptr && CostOf(*c, rest.M, N, k_tiles) <= 1.05 * CostOf(*Cheapest(costs, rest.M, N, k_tiles), rest.M, N, k_tiles)) plan.rest = own;
+  }
+  return plan;
 }
 
-int PlanRowSplit(const GemmArgs& a, GemmVariant* first) {
+RowSplit PlanRowSplit(const GemmArgs& a) {
   if (!g_row_split || g_variant_override >= 0 || a.batch != 1 || a.out_f32 || a.split_k != 1 || a.K % 64 != 0 || a.skip != nullptr ||
       a.row_stats != nullptr) {
-    return 0;
+    return {};
   }
-  if (InTileCostDomain(a.M, a.N, a.K, kHalfWideEnd)) return PlanRowSplitByTileCost(a.M, a.N, a.K / 64, first);
-  if (!InFittedDomain(a)) return 0;
+  if (InTileCostDomain(a.M, a.N, a.K, kHalfWideEnd)) return PlanRowSplitByTileCost(a);
+  if (!InFittedDomain(a)) return {};
   double best = FitCosts(a.M, a.N, a.K).Best() * 0.97;
-  int best_m1 = 0;
+  RowSplit plan;
   for (int v = 0; v < 2; v++) {
     const int bn = v == 0 ? 256 : 192;
     const int col_tiles = (a.N + bn - 1) / bn;
@@ -337,10 +354,10 @@ int PlanRowSplit(const GemmArgs& a, GemmVariant* first) {
     for (int m1 = rows_per_round; m1 + 4096 <= a.M; m1 += rows_per_round) {
       const FittedCosts top = FitCosts(m1, a.N, a.K);
       const double c = (v == 0 ? top.t256 : top.t192) + FitCosts(a.M - m1, a.N, a.K).Best() + 1.0;
-      if (c < best) { best = c; best_m1 = m1; *first = v == 0 ? kDma256x256 : kDma256x192; }
+      if (c < best) { best = c; plan = {m1, v == 0 ? kDma256x256 : kDma256x192, kNoVariant}; }
     }
   }
-  return best_m1;
+  return plan;
 }
 
 // The smallest direct-to-LDS tile with which an output fits the CUs with one workgroup each (kNoVariant: none does). A
@@ -539,9 +556,8 @@ bool GemmSupportsNormFolding(const GemmArgs& a) {
 }
 
 bool GemmTakesSecond(const GemmArgs& a) {
-  GemmVariant first = kDma256x256;
   return a.batch == 1 && a.split_k == 1 && !a.out_f32 && a.skip == nullptr && a.row_stats == nullptr && a.N2 % 8 == 0 &&
-         a.ldw2 % 8 == 0 && a.ldc2 % 8 == 0 && PlanRowSplit(a, &first) == 0 && SecondFits(PickGemmVariant(a), a.M, a.N, a.N2);
+         a.ldw2 % 8 == 0 && a.ldc2 % 8 == 0 && PlanRowSplit(a).rows == 0 && SecondFits(PickGemmVariant(a), a.M, a.N, a.N2);
 }
 
 int GemmStatsParts(const GemmArgs& a) {
@@ -550,14 +566,12 @@ int GemmStatsParts(const GemmArgs& a) {
 }
 
 int GemmRowSplit(const GemmArgs& a) {
-  GemmVariant first = kDma256x256;
-  return PlanRowSplit(a, &first);
+  return PlanRowSplit(a).rows;
 }
 
-const char* GemmVariantName(const GemmArgs& a) {
-  GemmVariant first = kDma256x256;
-  if (PlanRowSplit(a, &first) > 0) return first == kDma256x256 ? "gemm_dma_256x256x64+rest" : "gemm_dma_256x192x64+rest";
-  switch (PickGemmVariant(a)) {
+namespace {
+const char* NameOf(GemmVariant v, const GemmArgs& a) {
+  switch (v) {
     case kDma256x256: return "gemm_dma_256x256x64";
     case kDma256x192: return "gemm_dma_256x192x64";
     case kDma256x128: return "gemm_dma_256x128x32";
@@ -572,14 +586,36 @@ const char* GemmVariantName(const GemmArgs& a) {
   }
 }
 
+GemmArgs RestOf(const GemmArgs& a, int rows) {
+  GemmArgs rest = a;
+  rest.M = a.M - rows;
+  rest.A = a.A + static_cast<long long>(rows) * a.lda;
+  rest.C = static_cast<half_t*>(a.C) + static_cast<long long>(rows) * a.ldc;
+  return rest;
+}
+GemmVariant RestVariant(const RowSplit& plan, const GemmArgs& rest) { return plan.rest != kNoVariant ? plan.rest : PickGemmVariant(rest); }
+}  // namespace
+
+const char* GemmVariantName(const GemmArgs& a) {
+  const RowSplit plan = PlanRowSplit(a);
+  if (plan.rows > 0) return plan.first == kDma256x256 ? "gemm_dma_256x256x64+rest" : "gemm_dma_256x192x64+rest";
+  return NameOf(PickGemmVariant(a), a);
+}
+
+const char* GemmRestVariantName(const GemmArgs& a) {
+  const RowSplit plan = PlanRowSplit(a);
+  GemmArgs rest = a;
+  rest.M = a.M - plan.rows;
+  return plan.rows > 0 ? NameOf(RestVariant(plan, rest), rest) : "";
+}
+
 namespace {
 void LaunchDma(GemmVariant v, const GemmArgs& a, hipStream_t stream) {
   if (a.bf16) LaunchGemmDmaBf16(v, a, stream);
   else LaunchGemmDmaHalf(v, a, stream);
 }
 
-void LaunchGemmOne(const GemmArgs& a, hipStream_t stream) {
-  const GemmVariant v = PickGemmVariant(a);
+void LaunchGemmOne(GemmVariant v, const GemmArgs& a, hipStream_t stream) {
   switch (v) {
     case kRowPanel: LaunchGemmRowPanel(a, stream); break;
     case kResident: LaunchGemmResident(a, stream); break;
@@ -596,20 +632,16 @@ void LaunchGemm(const GemmArgs& a, hipStream_t stream) {
   if ((a.skip != nullptr || a.row_stats != nullptr) && !GemmSupportsNormFolding(a)) {
     throw std::runtime_error("LaunchGemm: no kernel variant with the folded layer-norm epilogue for this shape");
   }
-  GemmVariant first = kDma256x256;
-  const int m1 = PlanRowSplit(a, &first);
-  if (m1 > 0) {
-    GemmArgs top = a, rest = a;
+  const RowSplit plan = PlanRowSplit(a);
+  if (plan.rows > 0) {
+    GemmArgs top = a, rest = RestOf(a, plan.rows);
     top.out_stores = rest.out_stores = ResolvedOutStores(a);   // as for the whole product
-    top.M = m1;
-    rest.M = a.M - m1;
-    rest.A = a.A + static_cast<long long>(m1) * a.lda;
-    rest.C = static_cast<half_t*>(a.C) + static_cast<long long>(m1) * a.ldc;
-    LaunchDma(first, top, stream);
-    LaunchGemmOne(rest, stream);   // (the rest is below one round of the large tiles: one launch)
+    top.M = plan.rows;
+    LaunchDma(plan.first, top, stream);
+    LaunchGemmOne(RestVariant(plan, rest), rest, stream);   // (the rest is below one round of the large tiles: one launch)
     return;
   }
-  LaunchGemmOne(a, stream);
+  LaunchGemmOne(PickGemmVariant(a), a, stream);
 }
 
 namespace {

@@ -107,6 +107,7 @@ bool GemmTakesSecond(const GemmArgs& args);
 // along its rows into whole rounds of large tiles and a rest, GemmRowSplit() rows in the first launch).
 const char* GemmVariantName(const GemmArgs& args);
 int GemmRowSplit(const GemmArgs& args);
+const char* GemmRestVariantName(const GemmArgs& args);   // of the rest (empty: not cut)
 
 // e4m3 (OCP fp8, "fn": max 448, no infinities) GEMM with fp32 accumulation:
 //   C[m][n] = act(col_scale[n] * sum_k A[m][k] * W[n][k] + bias[n])

@@ -23,6 +23,8 @@ def _lib():
         lib.lc0mi_k_gemm_f8_variant_name.argtypes = [ci, ci, ci]
         lib.lc0mi_k_gemm_f8_variant_name.restype = C.c_char_p
         lib.lc0mi_k_gemm_row_split.argtypes = [ci, ci, ci]
+        lib.lc0mi_k_gemm_rest_variant_name.argtypes = [ci, ci, ci]
+        lib.lc0mi_k_gemm_rest_variant_name.restype = C.c_char_p
         lib.lc0mi_k_set_gemm_row_split.argtypes = [ci]
         lib.lc0mi_k_set_gemm_row_split.restype = None
         lib.lc0mi_k_gemm_norm_producer.argtypes = [vp, ci, vp, ci, vp, ci, ci, ci, cf, vp, vp, ci, vp, vp, cf, vp, vp, ci,
@@ -144,6 +146,11 @@ def set_gemm_row_split(on):
 def gemm_row_split(m, n, k):
     """Rows of the first launch when the launcher cuts a product of this shape along its rows (0: one launch)."""
     return _lib().lc0mi_k_gemm_row_split(m, n, k)
+
+
+def gemm_rest_variant_name(m, n, k):
+    """Tile shape of the second launch of such a product (empty: not cut)."""
+    return _lib().lc0mi_k_gemm_rest_variant_name(m, n, k).decode()
 
 
 STORES_AUTO, STORES_AUTO_KEEP, STORES_CACHED, STORES_STREAM, STORES_WRITE_THROUGH = range(5)

@@ -65,6 +65,18 @@ def test_products_that_leave_a_partial_round_are_cut_along_their_rows():
     assert K.gemm_row_split(20480, 64, 1024) == 0 and K.gemm_row_split(1 << 20, 1024, 256) == 0   # outside the model
 
 
+def test_the_rest_of_a_cut_product_runs_on_the_shape_it_is_priced_with():
+    """4416 rows of 2048 columns would get 128x128 tiles as a product of their own (55 us; 256x192 tiles, by which the cut is priced, 46.5):
+    with them the pair is slower than one launch. A shape priced as high as the cheapest stays."""
+    assert K.gemm_variant_name(4416, 2048, 2048) == "gemm_dma_128x128x64"
+    for m, n, k, m1, rest in ((12608, 2048, 2048, 8192, "256x192"), (12416, 1984, 1856, 8192, "256x192"), (11648, 2176, 1792, 7168, "256x192"),
+                              (14848, 1088, 1728, 10752, "128x128"), (13312, 1792, 1024, 9216, "128x128")):
+        assert K.gemm_row_split(m, n, k) == m1
+        assert K.gemm_rest_variant_name(m, n, k) == "gemm_dma_%sx64" % rest, (m, n, k)
+    assert K.gemm_rest_variant_name(20480, 1024, 1536) == K.gemm_variant_name(4096, 1024, 1536)   # (the model of 16384 rows and more)
+    assert K.gemm_rest_variant_name(16384, 1024, 1024) == ""
+
+
 def test_small_and_batched_products_keep_their_kernels():
     assert K.gemm_variant_name(1, 3072, 1024) == "gemm_rowpanel"
     assert K.gemm_variant_name(64, 64, 1024, batch=256) == "gemm_64x64x64"    # policy logits, one product per position
