@@ -1326,10 +1326,11 @@ void Mi355xNetwork::AllocActivations() {
     r_m_ = arena_.Alloc(ts * 36 * B * 4 * cmax);
     r_h1_ = arena_.Alloc(ts * B * 64 * cmax);
     r_h2_ = arena_.Alloc(ts * B * res_max_fc_);
-    if (fp32_) {   // (the heads run side by side)
-      r_pol_h1_ = arena_.Alloc(ts * B * 64 * cmax);
-      r_mov_h1_ = arena_.Alloc(ts * B * 64 * cmax);
-      r_mov_h2_ = arena_.Alloc(ts * B * res_max_fc_);
+    // (in floats the heads run side by side, each with buffers of its own)
+    if (fp32_ && !attn_policy_ && !conv_policy_) r_pol_h1_ = arena_.Alloc(ts * B * 64 * res_pol_conv1x1_.out);
+    if (fp32_ && moves_left_) {
+      r_mov_h1_ = arena_.Alloc(ts * B * 64 * res_mov_conv_.out);
+      r_mov_h2_ = arena_.Alloc(ts * B * res_mov_fc1_.out);
     }
     return;
   }

@@ -1144,6 +1144,31 @@ def test_narrow_float_layers_on_split_operands_with_large_hidden_values(position
     assert "encoder_tail" in names and "qkv_attention" in names
 
 
+def test_float_tower_has_buffers_of_the_heads_it_has_only(tmp_path):
+    """Without a moves-left head and without a dense policy layer a float tower keeps the buffers that a half tower keeps, with twice the
+    bytes each. (Weights are small here; a buffer of the other heads would be 21 MB.)"""
+    import ctypes
+    from lc0_amd import Network, netproto
+    from lc0_amd.backend import load_library
+    path = str(tmp_path / "net.pb.gz")
+    netproto.write_pb_gz(path, netgen.se_resnet(64, 2, 8, seed=77, conv_policy=True))
+    hip = load_library()   # (and, through it, the HIP runtime that it is linked to)
+
+    def used(options):
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        before = free.value
+        network = Network(path, options + ",max_batch=1024,lanes=1")
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        network.close()
+        return before - free.value
+
+    used("precision=fp32"), used("precision=fp16")   # (what a process allocates once)
+    half, single = used("precision=fp16"), used("precision=fp32")
+    assert half > 64 << 20
+    assert single <= 2 * half + (8 << 20)
+
+
 @pytest.mark.parametrize("form", ["plain", "read-only", "strided", "fortran", "int64", "float64", "big-endian", "list", "many"])
 def test_inputs_through_the_extension_and_through_ctypes(form, positions):
     """Arrays that the extension takes as they are, and those that it leaves to the conversions: the same results, bit for bit."""
