@@ -186,6 +186,10 @@ int lc0mi_k_gemm_row_split(int M, int N, int K) {
   return lc0mi::GemmRowSplit(g);
 }
 
+int lc0mi_k_smolgen_overlap_min_batch(int f32, int f8, int emb, int d_model) {
+  return lc0mi::SmolgenOverlapMinBatch(f32 != 0, f8 != 0, emb, d_model);
+}
+
 const char* lc0mi_k_gemm_rest_variant_name(int M, int N, int K) {
   lc0mi::GemmArgs g;
   g.M = M; g.N = N; g.K = K; g.batch = 1;

@@ -486,4 +486,7 @@ void LaunchTowerF32(const TowerArgs& args, hipStream_t stream);
 template <typename T>
 void LaunchConvPolicyGather(const T* t, int ld, const int16_t* inv_map, float* out, int batch, hipStream_t stream);
 
+// Smallest batch whose smolgen chain runs beside the Q/K/V projection (network.cc).
+int SmolgenOverlapMinBatch(bool f32, bool f8, int emb, int d_model);
+
 }  // namespace lc0mi

@@ -857,18 +857,29 @@ void Mi355xNetwork::Attention(const half_t* qkv, const half_t* bias, half_t* out
   }
 }
 
-// The smolgen chain of one encoder layer, unfused (network_blas.cc:283-347): compression, two dense layers with
-// their row norms, then the shared generator layer, which leaves the logits in sbias (SmolgenBiasIndex order).
+}  // namespace
+
 // Running the smolgen chain beside the QKV projection costs two cross-queue dependencies per layer, and up to here the
 // projection is one round of tiles that leave the chain no room. us of a pass, beside -> on one stream: 15x1024 fp16 80 positions 2925 -> 2755,
 // 84 2950 -> 2800, 85 3136 -> 3135, 150 4200 -> 4544, e4m3 80 2240 -> 2030, 85 2280 -> 2279; ten layers of width 768 fp16 80 1557 -> 1416, 112 1856 ->
 // 1712, 124 1985 -> 1919, 132 2164 -> 2230, e4m3 112 1488 -> 1327, 132 1750 -> 1745; 512 80 1260 -> 1111, 165 1914 -> 1836, 200 2048 -> 2036, 400 3415
-// -> 3468; 384 200 1835 -> 1738, 330 2455 -> 2435.
-int Mi355xNetwork::OverlapMinBatch() const {
-  if (overlap_min_batch_ >= 0) return overlap_min_batch_;
-  return dtype_ == Dtype::kFloat ? 80 : std::max(80, (85 * 1024 + emb_ - 1) / emb_);
+// -> 3468; 384 200 1835 -> 1738, 330 2455 -> 2435. Its tiles cover the 3 d_model columns of the projection, so the line goes by that width where it
+// is not the body's. Six layers, fp16, body 1024 and d_model 512 84 positions 1002 -> 897, 120 1146 -> 1088, 150 1432 -> 1450, 170 1592 -> 1652; body 512 and
+// d_model 1024 84 837 -> 750, 90 814 -> 830, 100 855 -> 828, 165 1225 -> 1243, 170 1218 -> 1295. In e4m3 the projection of a narrower body, whose
+// reduction is a few steps, is too short to hide the chain: body 1024 and d_model 512 90 884 -> 795, 165 1287 -> 1223; 512 and 1024 90 740 ->
+// 683, 165 1045 -> 1021.
+int SmolgenOverlapMinBatch(bool f32, bool f8, int emb, int d_model) {
+  const int width = f8 ? std::min(emb, d_model) : d_model;
+  return f32 ? 80 : std::max(80, (85 * 1024 + width - 1) / width);
 }
 
+namespace {
+int Mi355xNetwork::OverlapMinBatch() const {
+  return overlap_min_batch_ >= 0 ? overlap_min_batch_ : SmolgenOverlapMinBatch(dtype_ == Dtype::kFloat, fp8_, emb_, d_model_);
+}
+
+// The smolgen chain of one encoder layer, unfused (network_blas.cc:283-347): compression, two dense layers with
+// their row norms, then the shared generator layer, which leaves the logits in sbias (SmolgenBiasIndex order).
 void Mi355xNetwork::SmolgenChain(const EncoderDev& e, const half_t* x, int emb, int heads, int hc, int hs, int gen,
                                  half_t* sg1, half_t* sg2, half_t* sg3, half_t* sbias, int B, hipStream_t st,
                                  bool latency_first) {
@@ -2260,7 +2271,9 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
       // 256-row tiles it takes five times as long. us of a pass, beside -> before: 15x1024 fp16 90 positions 3190 -> 3000, 128 3600 -> 3525, 150
       // 4200 -> 4105, 165 4367 -> 4363 (100, where the projection leaves CUs free in its second round, 3137 -> 3152; 180 4865 -> 4897, 512
       // 11260 -> 11430), bf16 90 3118 -> 2972, 150 4105 -> 4012; ten layers of width 768 116 1951 -> 1767, 200 2582 -> 2545; 512 256 2247 -> 2182, 512
-      // 3682 -> 3740. (Nothing but the batch decides on its kernel, so that a pass on one stream has the same bits.)
+      // 3682 -> 3740. Where the two widths differ that of the body decides: six layers of body 512 and d_model 1024 170 1240 -> 1218, 256 1508 ->
+      // 1471, 330 1925 -> 1911; of body 1024 and d_model 512 it would pay further (200 1660 -> 1602, 300 2350 -> 2296).
+      // (Nothing but the batch decides on its kernel, so that a pass on one stream has the same bits.)
       const bool compress_first = !chain_f8 && dtype_ != Dtype::kFloat && !with_compress && !norm_in && B * emb_ <= 165 * 1024;
       if (compress_first) {
         Gemm("gemm_smolgen_compress", x_, emb_, e.sg_compress, sg1_, sg_hc_, T, kActNone, false, stream_, 1, true);

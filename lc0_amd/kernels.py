@@ -25,6 +25,7 @@ def _lib():
         lib.lc0mi_k_gemm_row_split.argtypes = [ci, ci, ci]
         lib.lc0mi_k_gemm_rest_variant_name.argtypes = [ci, ci, ci]
         lib.lc0mi_k_gemm_rest_variant_name.restype = C.c_char_p
+        lib.lc0mi_k_smolgen_overlap_min_batch.argtypes = [ci, ci, ci, ci]
         lib.lc0mi_k_set_gemm_row_split.argtypes = [ci]
         lib.lc0mi_k_set_gemm_row_split.restype = None
         lib.lc0mi_k_gemm_norm_producer.argtypes = [vp, ci, vp, ci, vp, ci, ci, ci, cf, vp, vp, ci, vp, vp, cf, vp, vp, ci,
@@ -151,6 +152,11 @@ def gemm_row_split(m, n, k):
 def gemm_rest_variant_name(m, n, k):
     """Tile shape of the second launch of such a product (empty: not cut)."""
     return _lib().lc0mi_k_gemm_rest_variant_name(m, n, k).decode()
+
+
+def smolgen_overlap_min_batch(emb, d_model, f32=False, f8=False):
+    """Smallest batch whose smolgen chain runs beside the Q/K/V projection, by default."""
+    return _lib().lc0mi_k_smolgen_overlap_min_batch(int(f32), int(f8), emb, d_model)
 
 
 STORES_AUTO, STORES_AUTO_KEEP, STORES_CACHED, STORES_STREAM, STORES_WRITE_THROUGH = range(5)

@@ -102,6 +102,19 @@ def test_few_rows_with_many_columns_or_products():
     assert K.gemm_variant_name(64, 64, 256, batch=77) == "gemm_dma_64x64x64"
 
 
+def test_the_smolgen_chain_leaves_the_projection_where_that_has_more_than_one_round_of_tiles():
+    """256x256 tiles over the 64 rows of every position and the 3 d_model columns of the projection, whatever the width of the body; in
+    e4m3 that of the narrower of the two."""
+    for emb in (384, 512, 1024):
+        for d_model in (384, 512, 768, 1024, 1088):
+            batch = K.smolgen_overlap_min_batch(emb, d_model)
+            tiles = 64 * batch / 256 * 3 * d_model / 256
+            assert batch == 80 or 255 <= tiles <= 258, (emb, d_model, batch)
+    assert [K.smolgen_overlap_min_batch(d, d) for d in (384, 512, 768, 1024, 1536)] == [227, 170, 114, 85, 80]
+    assert [K.smolgen_overlap_min_batch(e, d, f8=True) for e, d in ((512, 1024), (1024, 512), (1024, 1024))] == [170, 170, 85]
+    assert K.smolgen_overlap_min_batch(512, 512, f32=True) == 80
+
+
 def test_e4m3_products_of_few_rows_with_large_weights():
     """More than one 64x64 tile per CU and weights beyond an XCD's 4 MiB of L2: 128x64 tiles; otherwise 64x64."""
     for m, n, k in ((512, 3072, 1536), (256, 8192, 2048), (300, 8192, 1024), (640, 3072, 2048)):
