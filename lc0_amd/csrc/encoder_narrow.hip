@@ -412,14 +412,13 @@ void LaunchTailT(const EncoderTailArgs& a, hipStream_t stream) {
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;
   using Four = std::integral_constant<int, 4>;
-  auto by_rows = [&](auto split_tag) {
-    if (shape.rows == 16) launch(One{}, split_tag);
-    else if (shape.rows == 32) launch(Two{}, split_tag);
-    else launch(Four{}, split_tag);
-  };
-  if (shape.slices == 4) by_rows(Four{});
-  else if (shape.slices == 2) by_rows(Two{});
-  else by_rows(One{});
+  if constexpr (CT == 2) {   // (slices at width 256 only, with 16 rows each)
+    if (shape.slices == 4) return launch(One{}, Four{});
+    if (shape.slices == 2) return launch(One{}, Two{});
+  }
+  if (shape.rows == 16) launch(One{}, One{});
+  else if (shape.rows == 32) launch(Two{}, One{});
+  else launch(Four{}, One{});
 }
 
 template <typename ET>
