@@ -113,7 +113,7 @@ int lc0mi_k_expand_planes_attn(const uint64_t* masks, const float* values, int b
                                int time_iters, double* ms);
 /* Input planes -> [B][112][64] floats (EncodePlanes, network_blas.cc:973-981). */
 int lc0mi_k_expand_planes_nchw(const uint64_t* masks, const float* values, int batch, float* out);
-/* Attention-policy tail: logits [B][4096] floats, keys [B*64][pd] halves,
+/* Attention-policy tail of a float network: logits [B][4096] floats, keys [B*64][pd] given as halves,
  * ppo [4][pd] floats -> policy [B][1858] (network_blas.cc:873-914). */
 int lc0mi_k_attn_policy_gather(const float* logits, const uint16_t* keys, const float* ppo, int pd, int batch,
                                float* out);

@@ -540,7 +540,8 @@ int lc0mi_k_attn_policy_gather(const float* logits, const uint16_t* keys, const 
     if (batch < 1 || pd < 1) throw Error("bad policy shape");
     Dev dev;
     float* dl = dev.Put(logits, (size_t)batch * 4096);
-    auto* dk = reinterpret_cast<half_t*>(dev.Put(keys, (size_t)batch * 64 * pd));
+    const half_t* k = reinterpret_cast<const half_t*>(keys);
+    float* dk = dev.Put(std::vector<float>(k, k + (size_t)batch * 64 * pd).data(), (size_t)batch * 64 * pd);
     float* dp = dev.Put(ppo, (size_t)4 * pd);
     const auto& inv = lc0mi::AttnPolicyInverseMap();
     int16_t* di = dev.Put(inv.data(), inv.size());

@@ -396,11 +396,11 @@ bool ValueHeadSupported(int emb, int ch, int fc, int out_n);
 void LaunchValueHeads(const ValueHeadsArgs& args, hipStream_t stream);
 
 // Attention policy tail: promotion offsets + gather to 1858 moves.
-// logits: [B][64*64] float (already scaled), kq: [B*64][ld_kq] with keys at column
+// logits: [B][64*64] float (already scaled), kq: [B*64][ld_kq] floats with keys at column
 // offset key_off, ppo: [4][pd] float, inv_map: [1858] source index into the
 // 4096+192 virtual buffer. out: [B][1858] float.
-template <typename T>   // T: element type of kq (half_t, bf16_t, float)
-void LaunchAttnPolicyGather(const float* logits, const T* kq, int ld_kq, int key_off, const float* ppo,
+// (16-bit networks: LaunchPolicyTail)
+void LaunchAttnPolicyGather(const float* logits, const float* kq, int ld_kq, int key_off, const float* ppo,
                             int pd, const int16_t* inv_map, float* out, int batch, hipStream_t stream);
 
 // Most legal moves one sample may list for LaunchLegalSoftmax (chess positions have at most 218).

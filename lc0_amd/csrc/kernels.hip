@@ -689,9 +689,8 @@ void LaunchAttentionF8Out(const half_t* qkv, const half_t* bias, uint8_t* out, f
 // Attention policy tail.
 // ---------------------------------------------------------------------------
 namespace {
-template <typename T>   // element type of kq: half_t, bf16_t or float
 __global__ __launch_bounds__(256) void attn_policy_gather_kernel(const float* __restrict__ logits,
-                                                                 const T* __restrict__ kq, int ld_kq,
+                                                                 const float* __restrict__ kq, int ld_kq,
                                                                  int key_off, const float* __restrict__ ppo, int pd,
                                                                  const int16_t* __restrict__ inv_map,
                                                                  float* __restrict__ out) {
@@ -701,30 +700,12 @@ __global__ __launch_bounds__(256) void attn_policy_gather_kernel(const float* __
   // with the loads of the eight products in flight together.
   {
     const int i = wave;
-    const T* krow = kq + (long long)(b * 64 + 56) * ld_kq + key_off;
+    const float* krow = kq + (long long)(b * 64 + 56) * ld_kq + key_off;
     float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    bool done = false;
-    if constexpr (sizeof(T) == 2) {
-      if (((pd | ld_kq | key_off) & 7) == 0) {
-        done = true;
-      for (int c = lane; c < pd / 8; c += 64) {
-        const floatx4 p0 = *reinterpret_cast<const floatx4*>(ppo + (long long)i * pd + c * 8);
-        const floatx4 p1 = *reinterpret_cast<const floatx4*>(ppo + (long long)i * pd + c * 8 + 4);
+    for (int k = lane; k < pd; k += 64) {
+      const float pw = ppo[(long long)i * pd + k];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-          const auto kv = *reinterpret_cast<const typename Vec16<T>::v8*>(krow + (long long)j * ld_kq + c * 8);
-#pragma unroll
-          for (int e = 0; e < 4; e++) s[j] += (float)kv[e] * p0[e] + (float)kv[4 + e] * p1[e];
-        }
-      }
-      }
-    }
-    if (!done) {
-      for (int k = lane; k < pd; k += 64) {
-        const float pw = ppo[(long long)i * pd + k];
-#pragma unroll
-        for (int j = 0; j < 8; j++) s[j] += (float)krow[(long long)j * ld_kq + k] * pw;
-      }
+      for (int j = 0; j < 8; j++) s[j] += krow[(long long)j * ld_kq + k] * pw;
     }
 #pragma unroll
     for (int j = 0; j < 8; j++) {
@@ -749,17 +730,12 @@ __global__ __launch_bounds__(256) void attn_policy_gather_kernel(const float* __
 }
 }  // namespace
 
-template <typename T>
-void LaunchAttnPolicyGather(const float* logits, const T* kq, int ld_kq, int key_off, const float* ppo, int pd,
+void LaunchAttnPolicyGather(const float* logits, const float* kq, int ld_kq, int key_off, const float* ppo, int pd,
                             const int16_t* inv_map, float* out, int batch, hipStream_t stream) {
   if (batch <= 0) return;
-  hipLaunchKernelGGL(attn_policy_gather_kernel<T>, dim3(batch), dim3(256), 0, stream, logits, kq, ld_kq, key_off, ppo,
+  hipLaunchKernelGGL(attn_policy_gather_kernel, dim3(batch), dim3(256), 0, stream, logits, kq, ld_kq, key_off, ppo,
                      pd, inv_map, out);
 }
-template void LaunchAttnPolicyGather<half_t>(const float*, const half_t*, int, int, const float*, int, const int16_t*,
-                                             float*, int, hipStream_t);
-template void LaunchAttnPolicyGather<float>(const float*, const float*, int, int, const float*, int, const int16_t*,
-                                            float*, int, hipStream_t);
 
 // ---------------------------------------------------------------------------
 // Layer norm and attention for any element type and any row length / head depth: the forms the float
