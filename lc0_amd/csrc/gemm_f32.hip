@@ -4,6 +4,7 @@
 #include "row_panel.h"
 
 #include <algorithm>
+#include <stdexcept>
 
 namespace lc0mi {
 
@@ -160,10 +161,7 @@ bool GemmF32Grouped(const GemmArgsF32* a, int count) {
 }
 
 void LaunchGemmF32Group(const GemmArgsF32* a, int count, hipStream_t stream) {
-  if (!GemmF32Grouped(a, count)) {
-    for (int i = 0; i < count; i++) LaunchGemmF32(a[i], stream);
-    return;
-  }
+  if (!GemmF32Grouped(a, count)) throw std::runtime_error("LaunchGemmF32Group: not products for one launch");
   GroupArgs g;
   long long tiles = 0;
   int k = 0;

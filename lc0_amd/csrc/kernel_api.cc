@@ -363,7 +363,8 @@ int lc0mi_k_gemm_f32_group(int count, const float* const* A, const float* const*
       g[i].M = M; g[i].N = N; g[i].K = K; g[i].batch = batch; g[i].act = dims[5 * i + 4];
     }
     *grouped = lc0mi::GemmF32Grouped(g.data(), count);
-    lc0mi::LaunchGemmF32Group(g.data(), count, nullptr);
+    if (*grouped) lc0mi::LaunchGemmF32Group(g.data(), count, nullptr);
+    else for (const auto& a : g) lc0mi::LaunchGemmF32(a, nullptr);
     K_CHECK(hipDeviceSynchronize());
     K_CHECK(hipGetLastError());
     for (const auto& a : g) K_CHECK(hipMemcpy(C[&a - g.data()], a.C, sizeof(float) * a.batch * a.M * a.N, hipMemcpyDeviceToHost));

@@ -155,7 +155,7 @@ struct GemmArgsF32 {
   int act = 3;
 };
 void LaunchGemmF32(const GemmArgsF32& args, hipStream_t stream);
-// Up to kGemmF32Group products that do not depend on each other; in one launch where GemmF32Grouped(): all of them small enough for
+// Up to kGemmF32Group products that do not depend on each other in one launch. Only where GemmF32Grouped(): all of them small enough for
 // 16x16 tiles.
 constexpr int kGemmF32Group = 3;
 bool GemmF32Grouped(const GemmArgsF32* args, int count);

@@ -465,8 +465,8 @@ class Mi355xNetwork : public Network, protected ModelState {
   void Timed(const char* name, double flops, double bytes, F&& launch, hipStream_t st = nullptr);
   void TimedElsewhere(const std::string& name, double flops, double bytes);
   void AddToProfile(const KernelTime& t);
+  int OverlapMinBatch() const;   // smallest batch whose smolgen chain runs on the side stream
   // Independent layers of a float network's heads, in one launch where they are small.
-  int OverlapMinBatch() const;
   void GemmGroup(const std::vector<GemmArgsF32>& list, const char* name);
   void ForwardHeadsF32(int B);
   GemmArgsF32 PolicyLogitsF32(int B) const;
