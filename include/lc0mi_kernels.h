@@ -69,7 +69,7 @@ int lc0mi_k_set_bf16(int on);
 /* Test hook, process-wide: the kind of output stores of lc0mi_k_gemm and lc0mi_k_gemm_f8 (256-row tiles of the
  * direct-to-LDS kernel; others always store ordinarily) and of lc0mi_k_layer_norm: 0 by output size (ordinary or
  * streaming), 1 by output size (ordinary or written through), 2 ordinary, 3 streaming (non-temporal), 4 written
- * through at system scope (the layer norm then also reads x with non-temporal loads). The network picks 1 and the
+ * through at device scope (the layer norm then also reads x with non-temporal loads). The network picks 1 and the
  * written-through layer norm for the big tensors of an encoder layer while a layer's activations fit the memory-side
  * cache. No counterpart in the reference. */
 int lc0mi_k_set_out_stores(int kind);

@@ -349,8 +349,9 @@ __global__ __launch_bounds__(512) void encoder_tail_kernel(EncoderTailArgs p) {
   }
   if constexpr (SPLIT > 1) {
     // Every slice leaves its sums, written through to memory; the last one of the block to arrive adds all of them, in the order of
-    // the slices whoever that is, and goes on. Nobody waits for another workgroup. (The stores pass by the L2 of their XCD, and
-    // the wait makes them complete before the workgroup counts itself.)
+    // the slices whoever that is, and goes on. Nobody waits for another workgroup. (The counter is relaxed and no release fence precedes it:
+    // stores at device scope, which pass by the L2 of their XCD, and the wait for them before the barrier and the count take its place.
+    // Ordinary or streaming stores would not do here.)
     __shared__ int last;
     floatx4* place = reinterpret_cast<floatx4*>(p.partial) + (long long)block * SPLIT * RT * CT * 512 + tid;
 #pragma unroll
@@ -469,10 +470,15 @@ EncoderTailShape PickEncoderTailShape(int M, int emb, int dff) {
 }
 
 // A few workgroups stream all weights through one CU each, whatever the batch, where five launches spread them over the chip;
-// how many positions that costs follows from their bytes. us of a ten-layer pass, layers one by one -> the kernel. Width 256,
-// 0.66 MB (512 hidden columns) 1 position 275 -> 255; 1.2 MB (1024) 1 287 -> 304, 4 302 -> 311, 8 341 -> 310, with smolgen 1 440 ->
-// 453, 4 463 -> 469, 8 559 -> 522; 2.2 MB (2048) 1 305 -> 406, 12 392 -> 411, 16 386 -> 410, 24 460 -> 418. Width 128, whose own
-// products have short reductions, 0.3 MB 1 292 -> 200, 1.1 MB (2048) 1 330 -> 319, 16 378 -> 329.
+// how many positions that costs follows from their bytes. us of a ten-layer pass, layers one by one -> the kernel with one workgroup per
+// row. Width 256, 0.66 MB (512 hidden columns) 1 position 275 -> 255; 1.2 MB (1024) 1 287 -> 304, 4 302 -> 311, 8 341 -> 310, with
+// smolgen 1 440 -> 453, 4 463 -> 469, 8 559 -> 522; 2.2 MB (2048) 1 305 -> 406, 12 392 -> 411, 16 386 -> 410, 24 460 -> 418. Width 128, whose
+// own products have short reductions, 0.3 MB 1 292 -> 200, 1.1 MB (2048) 1 330 -> 319, 16 378 -> 329.
+// Where workgroups share the FFN the kernel is ahead below this line too for one thread and for two, and from 3 positions for four threads,
+// unless there is smolgen: 1024 1 252 -> 232, 3 278 -> 239, 4 281 -> 240, with smolgen 1 447 -> 415, 4 484 -> 436; 2048 1 281 -> 262, 4 332 -> 268, 8
+// 362 -> 272, 16 393 -> 323; thousands of evals/s of four threads 1024 1 9.4 -> 8.7, 3 25.1 -> 25.3, 4 31.5 -> 32.2, with smolgen 1 5.4 -> 4.7, 4
+// 17.9 -> 18.0; 2048 1 8.5 -> 7.9, 4 28.5 -> 28.7, 16 80 -> 90, with smolgen 4 17.8 -> 17.0, 12 38.7 -> 34.0. The line is that of one workgroup
+// per row all the same.
 int EncoderTailMinBatch(int emb, int d_model, int dff) {
   const int kib = 2 * emb * (d_model + 2 * dff) / 1024;
   return emb <= 128 ? 1 : std::max(1, (kib - 768 + 79) / 80);

@@ -60,7 +60,7 @@ __device__ __forceinline__ void StoreOut16(void* dst, intx4 val) {
 // GemmF8Args: 128 bytes = 128 values per row, v_mfma_f32_32x32x64_f8f6f4);
 // BKB is the k-tile in bytes. OutT is half_t or uint8_t (e4m3, fp8 operands only).
 // STORES: how the 16-byte output vectors are stored: 0 ordinary stores (the output stays in L2 and the memory-side
-// cache), 1 streaming (non-temporal) stores, 2 stores written through at system scope (they leave L2 alone like the
+// cache), 1 streaming (non-temporal) stores, 2 stores written through at device scope (they leave L2 alone like the
 // streaming ones, but what they wrote is found faster by the next kernel; plain epilogue only).
 // EPI (fp16 operands only): 0 the plain epilogue, 1 the consumer and 2 the producer side of a folded layer norm
 // (GemmArgs::row_stats / GemmArgs::skip).

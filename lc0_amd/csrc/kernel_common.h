@@ -38,7 +38,7 @@ __device__ __forceinline__ floatx4 Mfma16(bf16x8 a, bf16x8 b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// 16 bytes written through at system scope: past the L2 of the XCD, to where every XCD finds them.
+// 16 bytes written through at device scope: past the L2 of the XCD, to where every XCD finds them.
 __device__ __forceinline__ void StoreThrough16(void* dst, intx4 val) {
   // (the no-op covers the wait states that the hardware needs between a store of more than eight bytes and a vector
   // ALU write to its data registers - two on this part; the compiler adds them after its own stores and does not

@@ -23,7 +23,7 @@ enum class Dtype { kHalf, kBf16, kFloat };
 // How a large GEMM writes its output (GemmArgs::out_stores, GemmF8Args::out_stores; only the 256-row tiles of the
 // direct-to-LDS kernel know more than ordinary stores). kStoresAuto: ordinary stores, or streaming (non-temporal)
 // ones for an output so large that it would push the operands out of L2. kStoresAutoKeep: the same size rule, but
-// with stores written through at system scope in place of the streaming ones: they leave L2 alone as well, and the
+// with stores written through at device scope in place of the streaming ones: they leave L2 alone as well, and the
 // kernel that reads the output next finds it in the memory-side cache, which streamed data is not. For outputs
 // whose reader is bound by memory (attention, layer norm) as long as a layer's activations fit that cache.
 // The last three name a kind of store outright.
@@ -247,7 +247,7 @@ void LaunchNormGemm(const NormGemmArgs& args, hipStream_t stream);
 // t = x * alpha + skip (skip may be null). x, skip, y may alias. C % 8 == 0, C <= 8192.
 // y_f8 (optional): also receives e4m3(y * f8_mul), saturating, the operand of a following fp8 GEMM.
 // through: for tensors far larger than L2 inside a pass whose activations fit the memory-side cache: x (not read
-// again) comes in with non-temporal loads, y goes out with stores written through at system scope, where the
+// again) comes in with non-temporal loads, y goes out with stores written through at device scope, where the
 // kernels that read it next find it (GemmArgs::out_stores has the measurements).
 void LaunchLayerNorm(const half_t* x, const half_t* skip, half_t* y, const float* gamma, const float* beta,
                      int rows, int C, float alpha, float eps, hipStream_t stream, uint8_t* y_f8 = nullptr,
@@ -345,7 +345,7 @@ struct EncoderTailShape { int rows, slices; };
 EncoderTailShape PickEncoderTailShape(int M, int emb, int dff);
 constexpr int kEncoderTailBlocks = 64, kEncoderTailPartial = 128 * 16 * 256;   // (several slices: at most 128 workgroups of 16 rows)
 bool EncoderTailSupported(int emb, int d_model, int dff);
-int EncoderTailMinBatch(int emb, int d_model, int dff);   // smallest batch at which it is faster than its layers one by one
+int EncoderTailMinBatch(int emb, int d_model, int dff);   // smallest batch that it is used for
 long long EncoderTailFragmentIndex(int layer, int row, int col, int emb, int d_model);
 void LaunchEncoderTail(const EncoderTailArgs& args, hipStream_t stream);
 // The same two for floats (encoder_narrow_f32.hip): x, att and out hold floats, u stays one. packed: bfloat16, the first of a weight's

@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const half_t* __restric
         f[e] = beta[v * 8 + e] + gamma[v * 8 + e] * (t[i][e] - mean) * den;
         o[e] = (ET)f[e];
       }
-      if (through) {   // written through at system scope: past L2, into the memory-side cache (the no-op: the wait
+      if (through) {   // written through at device scope: past L2, into the memory-side cache (the no-op: the wait
                        // states between a 16-byte store and a vector ALU write to its data registers)
         asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(yr + v * 8), "v"(o) : "memory");
       } else {

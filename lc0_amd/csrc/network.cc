@@ -2250,7 +2250,10 @@ void Mi355xNetwork::ForwardAttentionBody(int B) {
     // 15x1024 pass, own launch -> with the projection: fp16 1 position 923 -> 833, 13 1296 -> 1230, 21 1574 -> 1502, 48 2219 ->
     // 2136; e4m3 1 791 -> 729, 16 979 -> 929, 48 1545 -> 1486. Its sums are added in another order than in a launch of its own, so
     // nothing but the batch decides: a pass has the same bits on one stream and on two, beside other passes and when profiled. The
-    // limit is where the chain leaves the projection's stream by default: beside the projection it has no launch to save.
+    // limit was set where the chain left the projection's stream. Between it and SmolgenOverlapMinBatch, where the compression is a launch of
+    // its own before the projection, the two are level but for the last batches of one round of tiles: us of a pass, own launch -> with the
+    // projection, six layers of width 1024 fp16 84 1128 -> 1137, e4m3 871 -> 872; eight of 768 fp16 100 1263 -> 1265, 113 1513 -> 1480, e4m3 113 1105
+    // -> 1069; ten of 512 fp16 140 1597 -> 1597, e4m3 165 1390 -> 1387.
     bool with_compress = false;
     if (e.has_smolgen && B <= kCompressWithQkvMaxBatch && compress_with_qkv_ && !norm_in && !calibrating_ && chain_f8 == (f8 && q_qkv_)) {
       SecondProduct compress;

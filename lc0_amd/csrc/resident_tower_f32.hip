@@ -261,7 +261,7 @@ __global__ __launch_bounds__(kThreads, 1) void resident_tower_f32_kernel(TowerAr
 }  // namespace
 
 // Elements of the packed weights (a few steps' worth is asked for past the end), and the index of the first part of one of them;
-// the others are kTowerF32Part further each.
+// the others are kSplitPart further each.
 long long TowerF32Fragments(int blocks) { return (8 * (2LL * kTaps + 2LL * kTaps * blocks) + kRing) * kParts * 512; }
 
 long long TowerF32FragmentIndex(int blocks, int conv, int tap, int out, int in) {
