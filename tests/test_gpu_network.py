@@ -1040,7 +1040,7 @@ def test_attention_kernel_of_few_positions_where_it_is_faster(heads, inside, out
         _compare(res, bn.forward(positions["masks"][idx], positions["values"][idx]), [positions["legal"][i] for i in idx])
 
 
-@pytest.mark.parametrize("dff,smolgen,first", [(512, None, 1), (1024, None, 5), (1024, (32, 256, 256), 5), (2048, None, 18)])
+@pytest.mark.parametrize("dff,smolgen,first", [(512, None, 1), (1024, None, 5), (1024, (32, 256, 256), 5), (1536, None, 12), (2048, None, 18)])
 def test_rest_of_a_layer_is_one_kernel_from_as_many_positions_as_its_weights_need(dff, smolgen, first, positions, tmp_path):
     """The kernel streams a layer's weights through every CU that it uses: with few positions and many weights the layers one by
     one are faster. Both sides of the line against the oracle, by the names in the profile."""
