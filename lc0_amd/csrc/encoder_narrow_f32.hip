@@ -21,8 +21,8 @@ namespace {
 // Attention with its projection: a workgroup computes Q, K and V of one position and one or two heads of depth 32 (64 x 96 outputs
 // each) and their attention, which stay in LDS. Projection: wave (share of the inputs, head, row tile) multiplies 32 rows by the 96
 // columns of its head; the shares are exchanged through LDS. Attention as attention_f32_kernel, 16 queries of a head per wave.
-// Bound by latency (16 KiB of rows and 74 KiB of weights per position and head) up to one round, then by the products: 20 positions of
-// 8 heads 11 us, where projection and attention on their own took 15.6.
+// Bound by latency (16 KiB of rows and 74 KiB of weights per position and head: 6.7 k of a wave's 21.6 k cycles are products) up to one
+// round, then by the products: 20 positions of 8 heads 11 us, where projection and attention on their own took 15.6.
 // ---------------------------------------------------------------------------
 template <int C, int HEADS>
 __global__ __launch_bounds__(512, 1) void qkv_attention_f32_kernel(const float* __restrict__ x, const intx4* __restrict__ packed,
@@ -189,8 +189,9 @@ __global__ __launch_bounds__(512, 1) void qkv_attention_f32_kernel(const float* 
 // 32 rows; its waves share the columns of every product (32 each of the C that are in work at a time) and stream the layer's
 // weights once, from L2, kRing steps of 16 inputs ahead. Activations stay in LDS as their three parts, that is, exactly.
 // With few rows several workgroups share the FFN's hidden columns; each leaves its sums to encoder_tail_sum_kernel.
-// Bound by the products (55 k cycles at width 256 and 1024 hidden columns, as many as the 3.5 MB of weights take at 64 bytes a cycle) and by
-// what lies between them, norms, activations and splits, 40 k. us for 20 positions of a 10x256 body: five
+// Bound by the products (55 k cycles at width 256 and 1024 hidden columns, as many as the 3.5 MB of weights take at 64 bytes a cycle, for one
+// workgroup per row; with four that share the FFN 18.4 k of a wave's 40.7 k, counted) and by what lies between them, norms, activations
+// and splits. us for 20 positions of a 10x256 body: five
 // launches on the float instructions 40, this with one workgroup per row 42, with four that share its FFN and the launch after it 23.
 // ---------------------------------------------------------------------------
 template <int C>

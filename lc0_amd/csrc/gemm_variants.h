@@ -19,11 +19,11 @@ int ResolvedOutStores(const GemmArgs& a);
 
 // The order of a launch's tiles. Workgroups go to the eight XCDs in turn, and each XCD's L2 fetches every operand row that one of its
 // tiles reads. In the order of the grid an XCD has tiles of all rows and of all columns, unless the row tiles are a multiple of
-// eight. Neighbouring row tiles per XCD cut the activations fetched to an eighth: from 2048 rows (us of a 15x1024 pass, fp16 36
-// positions 1960 -> 1905, 77 dense 2755 -> 2667, 150 4663 -> 4265, 300 7790 -> 7165, 1000 21550 -> 21050; e4m3 77 2145 -> 2045, 300
-// 5560 -> 5130, 350 7090 -> 6085). With fewer rows the weights, which come
-// from memory, are the larger part: in halves neighbouring column tiles up to 1024 rows (1 position 852 -> 831, 4 1013 -> 988, 16 1236 ->
-// 1221, but 20 1386 -> 1395), in e4m3, with half the bytes, for row panels only (5 positions on tiles 826 -> 841, 16 928 -> 939).
+// eight. Neighbouring row tiles per XCD cut the activations fetched to an eighth: from 2048 rows (us of a 15x1024 pass
+// with the tiles chosen now, fp16 36 positions 1733 -> 1756, 77 dense 2740 -> 2645, 150 3913 -> 3815, 300 7661 -> 7032, 1000 21300 -> 20768; e4m3 77
+// 2091 -> 1987, 300 5495 -> 5044, 350 7019 -> 6140). With fewer rows the weights, which come
+// from memory, are the larger part: in halves neighbouring column tiles up to 1024 rows (1 position 779 -> 761, 4 968 -> 947, 16 1204 ->
+// 1196, but 20 1386 -> 1395), in e4m3, with half the bytes, for row panels only (5 positions on tiles 826 -> 841, 16 928 -> 939).
 inline TileOrder PickTileOrder(int M, int columns_max_rows, const dim3& grid) {
   TileOrder o;
   const unsigned tiles = grid.x * grid.y;

@@ -45,10 +45,10 @@ template <int C> struct TowerShape {
 // twice or more (two positions, a 64-byte step: 512 cycles of products, 256 of LDS reads, 256 of weights at 64 bytes a cycle); half
 // the channels per wave would read the rows twice as often. One position per workgroup has half the products for the same
 // weights and serves up to one round of the CUs.
-// What bounds it: with two positions the matrix cores are busy 60 % of a wave's 2.5 M cycles (20x256 tower, 512 positions). By phases the
-// convolutions take 69 % (their waits included), squeeze-and-excitation 22 % (192 KiB of float weights per block and workgroup, four
-// barriers: 28 k cycles a block where the weights alone take 3 k), biases, skip and activations 9 %; with all CUs busy the clock falls to
-// 1.9 GHz on top. One position: 65, 28 and 7 %. A round of 512 positions takes 1.25 ms (1.2 PFLOP/s of direct products), where 41
+// What bounds it: with two positions the matrix cores are busy 64 % of a wave's 2.34 M cycles (20x256 tower, 512 positions). By phases the
+// convolutions take 75 % (their waits included), squeeze-and-excitation 16 % (192 KiB of float weights per block and workgroup, four
+// barriers: 19 k cycles a block where the weights alone take 3 k), biases, skip and activations 9 %; with all CUs busy the clock falls to
+// 1.9 GHz on top. One position: 71, 20 and 8 %. A round of 512 positions takes 1.21 ms (1.3 PFLOP/s of direct products), where 41
 // transforms of 24 us and 40 launches of 36 x 2048x256x256 of 22 us took 1.86.
 // Tried and not kept: the next squeeze-and-excitation weights touched during a convolution, so that they wait in the L2 (the stream
 // waits for them in order: 512 positions 1558 -> 1727 us a pass); zeros in the banks of the rows they stand for (level).
