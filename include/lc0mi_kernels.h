@@ -32,7 +32,8 @@ const char* lc0mi_k_gemm_f8_variant_name(int M, int N, int K);
 int lc0mi_k_gemm_row_split(int M, int N, int K);
 /* Kernel variant of the second launch of such a product (empty: not cut). Host-side choice. */
 const char* lc0mi_k_gemm_rest_variant_name(int M, int N, int K);
-/* Smallest batch whose smolgen chain runs on a second stream beside the Q/K/V projection, by default. Host-side choice. */
+/* Smallest batch whose smolgen chain runs on a second stream beside the Q/K/V projection, by default (0: no such widths). Host-side
+ * choice. */
 int lc0mi_k_smolgen_overlap_min_batch(int f32, int f8, int emb, int d_model);
 /* Switches that cut off (0) or on (1, the default), for measurements and tests; process-wide, like lc0mi_k_set_gemm_variant. */
 void lc0mi_k_set_gemm_row_split(int on);

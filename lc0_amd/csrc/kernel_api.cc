@@ -187,6 +187,7 @@ int lc0mi_k_gemm_row_split(int M, int N, int K) {
 }
 
 int lc0mi_k_smolgen_overlap_min_batch(int f32, int f8, int emb, int d_model) {
+  if (emb < 1 || d_model < 1) return 0;
   return lc0mi::SmolgenOverlapMinBatch(f32 != 0, f8 != 0, emb, d_model);
 }
 

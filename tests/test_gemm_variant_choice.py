@@ -113,6 +113,8 @@ def test_the_smolgen_chain_leaves_the_projection_where_that_has_more_than_one_ro
     assert [K.smolgen_overlap_min_batch(d, d) for d in (384, 512, 768, 1024, 1536)] == [227, 170, 114, 85, 80]
     assert [K.smolgen_overlap_min_batch(e, d, f8=True) for e, d in ((512, 1024), (1024, 512), (1024, 1024))] == [170, 170, 85]
     assert K.smolgen_overlap_min_batch(512, 512, f32=True) == 80
+    for emb, d_model in ((0, 0), (1024, 0), (0, 1024), (-1, 512)):
+        assert K.smolgen_overlap_min_batch(emb, d_model, f8=True) == 0
 
 
 def test_e4m3_products_of_few_rows_with_large_weights():
